@@ -594,6 +594,13 @@ struct GemmTile
     static constexpr bool USE_LUT = DT == DT_I8 && LDS_CU / (NST * STAGE) == LDS_CU / (NST * STAGE + 256);
     static constexpr int LUT     = USE_LUT ? 256 : 0;
     static constexpr int LDS     = NST * STAGE + LUT;
+    // Workgroups of this instance that a CU's LDS and thread slots hold -- what launch_tile() sizes the persistent grid for --
+    // and the waves per SIMD they come to. The register allocator is held to that many: a few registers more and the second
+    // workgroup of every CU runs after the first instead of beside it. Left alone it gave fp16 128 x 128 with D operands 265
+    // registers, one workgroup per CU where two fit: 1x1 conv C 256 -> K 128 at 56 x 56, N = 256, bias + ReLU 148 -> 127 us,
+    // with a residual 200 -> 163 (plain: 124). It also keeps the accumulators out of AccVGPRs, which saves their copies.
+    static constexpr int PER_CU   = LDS_CU / LDS < 2048 / NT ? LDS_CU / LDS : 2048 / NT;
+    static constexpr int WAVES_EU = PER_CU * NW / 4 > 0 ? PER_CU * NW / 4 : 1;
     static constexpr int NLA     = BM * CPR / NT; // 16-byte loads per thread and K tile, A
     static constexpr int NLB     = BN * CPR / NT;
     static constexpr int LPT     = NLA + NLB;
@@ -1482,7 +1489,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs p)
 
 template <int DT, int BM, int BN, int WM, int WN, int BKB, int NST, int IM2COL, bool TA = false, bool TB = false,
           bool FUSED = false>
-__global__ __launch_bounds__(WM* WN * 64) void gemm_tile_kernel(const GemmArgs p)
+__global__ __launch_bounds__((WM * WN * 64), (GemmTile<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED>::WAVES_EU))
+void gemm_tile_kernel(const GemmArgs p)
 {
     extern __shared__ __attribute__((aligned(1024))) uint8_t ckx_smem[];
     GemmTile<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED>::run(p, ckx_smem);

@@ -54,10 +54,7 @@ hipError_t launch_tile(const GemmArgs& a, int tiles, hipStream_t s)
     });
     if(attr_err != hipSuccess)
         return attr_err;
-    int per_cu = 160 * 1024 / T::LDS;
-    per_cu     = per_cu > 2048 / T::NT ? 2048 / T::NT : per_cu;
-    per_cu     = per_cu < 1 ? 1 : per_cu;
-    int grid   = num_cus() * per_cu;
+    int grid = num_cus() * T::PER_CU;
     grid -= grid % 8;
     grid = tiles < grid ? tiles : grid;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(T::NT), T::LDS, s, a);
