@@ -91,7 +91,6 @@ __global__ __launch_bounds__(256) void conv_rows_kernel(const ConvRowsArgs p)
                                rsrc_in, m < (uint32_t)p.M ? m * (uint32_t)(64 * KS) + 64u * ks + 16u * q : kOutOfRange, 0, 0));
         }
     };
-    const bool vec_ok = ((reinterpret_cast<uintptr_t>(p.out) | ((uintptr_t)p.Kout * ES)) & 15u) == 0;
     const bool nt     = p.nt_store != 0;
     auto finish_rows  = [&](int grp, const i32x4(&a)[U][KS]) {
 #pragma unroll
@@ -124,11 +123,11 @@ __global__ __launch_bounds__(256) void conv_rows_kernel(const ConvRowsArgs p)
                         int8_t* crow      = reinterpret_cast<int8_t*>(p.out) + (size_t)m * p.Kout;
                         const i32x4 v[4] = {acc[0], acc[1], acc[2], acc[3]};
                         if(p.epi == EPI_REQUANT_RND)
-                            store_row16_i8<EPI_REQUANT_RND>(crow, n0, p.Kout, vec_ok, v, p.scale_gemm, p.scale_relu, nt);
+                            store_row16_i8<EPI_REQUANT_RND>(crow, n0, p.Kout, v, p.scale_gemm, p.scale_relu, nt);
                         else if(p.epi == EPI_REQUANT_CK)
-                            store_row16_i8<EPI_REQUANT_CK>(crow, n0, p.Kout, vec_ok, v, p.scale_gemm, p.scale_relu, nt);
+                            store_row16_i8<EPI_REQUANT_CK>(crow, n0, p.Kout, v, p.scale_gemm, p.scale_relu, nt);
                         else
-                            store_row16_i8<EPI_PASSTHROUGH>(crow, n0, p.Kout, vec_ok, v, p.scale_gemm, p.scale_relu, nt);
+                            store_row16_i8<EPI_PASSTHROUGH>(crow, n0, p.Kout, v, p.scale_gemm, p.scale_relu, nt);
                     }
                     else
                     {
@@ -145,7 +144,7 @@ __global__ __launch_bounds__(256) void conv_rows_kernel(const ConvRowsArgs p)
                                     v[t][j] = epi_f16_value<false>(EPI_ADD_RELU, v[t][j], (float)(e < 8 ? b_lo[g][e & 7] : b_hi[g][e & 7]), 0.0f);
                                 }
                         }
-                        store_row16_f16(crow, n0, p.Kout, vec_ok, v, nt);
+                        store_row16_f16(crow, n0, p.Kout, v, nt);
                     }
                 }
             }

@@ -108,7 +108,6 @@ struct ConvStem
 
         const uint32_t smem_lds = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
         const bool nt           = p.nt_store != 0;
-        const bool vec_ok       = (reinterpret_cast<uintptr_t>(p.out) & 15u) == 0;
 
         for(int unit = (int)blockIdx.x; unit < nunits; unit += (int)gridDim.x)
         {
@@ -198,16 +197,16 @@ struct ConvStem
                             for(int j = 0; j < 4; ++j)
                                 acc[t][j] = __builtin_fmaxf(acc[t][j] + bias[t][j], 0.0f);
                     }
-                    store_row16_f16(crow, 16 * (int)q, KOUT, vec_ok, acc, nt);
+                    store_row16_f16(crow, 16 * (int)q, KOUT, acc, nt);
                 }
                 else
                 {
                     if(p.epi == EPI_REQUANT_RND)
-                        store_row16_i8<EPI_REQUANT_RND>(crow, 16 * (int)q, KOUT, vec_ok, acc, p.scale_gemm, p.scale_relu, nt);
+                        store_row16_i8<EPI_REQUANT_RND>(crow, 16 * (int)q, KOUT, acc, p.scale_gemm, p.scale_relu, nt);
                     else if(p.epi == EPI_REQUANT_CK)
-                        store_row16_i8<EPI_REQUANT_CK>(crow, 16 * (int)q, KOUT, vec_ok, acc, p.scale_gemm, p.scale_relu, nt);
+                        store_row16_i8<EPI_REQUANT_CK>(crow, 16 * (int)q, KOUT, acc, p.scale_gemm, p.scale_relu, nt);
                     else
-                        store_row16_i8<EPI_PASSTHROUGH>(crow, 16 * (int)q, KOUT, vec_ok, acc, p.scale_gemm, p.scale_relu, nt);
+                        store_row16_i8<EPI_PASSTHROUGH>(crow, 16 * (int)q, KOUT, acc, p.scale_gemm, p.scale_relu, nt);
                 }
             }
         }

@@ -367,7 +367,6 @@ __global__ __launch_bounds__(NW * 64)
         }
     }
 
-    const bool vec_ok = ((reinterpret_cast<uintptr_t>(C) | ((uintptr_t)p.sc * 2)) & 15u) == 0;
     if constexpr(SOFTMAX)
     {
 #pragma unroll
@@ -394,7 +393,7 @@ __global__ __launch_bounds__(NW * 64)
                 continue;
             const f32x4 v[4] = {acc1[mt][og * 4], acc1[mt][og * 4 + 1], acc1[mt][og * 4 + 2],
                                 acc1[mt][og * 4 + 3]};
-            store_row16_f16(C + (int64_t)m * p.sc, o0, p.O, vec_ok, v);
+            store_row16_f16(C + (int64_t)m * p.sc, o0, p.O, v);
         }
     }
 }

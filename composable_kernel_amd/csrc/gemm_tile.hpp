@@ -74,14 +74,90 @@ __host__ __device__ constexpr bool epi_has_d1(int epi) { return epi == EPI_ADD_R
 // and the store acknowledgements stall the K pipeline of the next tile.
 // (Written as inline assembly: two stores that differ only in the non-temporal hint get merged
 // into one plain store by the optimiser.)
+//
+// The address needs no alignment beyond an element's: an odd leading dimension (N = 6719) or base puts every row on another
+// offset, and the part takes 16-byte accesses at any byte (unaligned access mode, the mode every HSA kernel runs in). Such
+// rows once fell back to one store per element: fp16 6349 x 6718 x 784 150 us, int8 6422 x 5607 x 544 111 us.
 template <typename V>
-__device__ __forceinline__ void store_vec(V* ptr, V val, bool nt)
+struct __attribute__((packed)) AnyAlign
+{
+    V v;
+};
+template <typename V>
+__device__ __forceinline__ void store_vec(void* ptr, V val, bool nt)
 {
     static_assert(sizeof(V) == 16, "16-byte vector store");
     if(nt)
         asm volatile("global_store_dwordx4 %0, %1, off nt" ::"v"(ptr), "v"(val) : "memory");
     else
-        *ptr = val;
+        reinterpret_cast<AnyAlign<V>*>(ptr)->v = val;
+}
+template <typename V>
+__device__ __forceinline__ V load_vec(const void* ptr)
+{
+    return reinterpret_cast<const AnyAlign<V>*>(ptr)->v;
+}
+
+// The ragged end of a row: the first nb bytes (0 < nb < 16, a multiple of the element size UNIT) of a 16-byte vector as at
+// most four accesses of 8, 4, 2 and 1 bytes. (One guarded access per ELEMENT instead, unrolled into every epilogue copy, made
+// up two thirds of the D-operand kernels' code: 38 000 instructions in the four-wave body, fetched once per tile.)
+template <int UNIT, typename V>
+__device__ __forceinline__ void store_head(void* ptr, const V& val, int nb)
+{
+    const i32x4 x = __builtin_bit_cast(i32x4, val);
+    uint8_t* dst  = reinterpret_cast<uint8_t*>(ptr);
+    int lo = x[0], hi = x[1];
+    if(nb & 8)
+    {
+        reinterpret_cast<AnyAlign<i32x2>*>(dst)->v = i32x2{lo, hi};
+        lo = x[2], hi = x[3], dst += 8;
+    }
+    if(nb & 4)
+    {
+        reinterpret_cast<AnyAlign<int>*>(dst)->v = lo;
+        lo = hi, dst += 4;
+    }
+    if constexpr(UNIT <= 2)
+        if(nb & 2)
+        {
+            reinterpret_cast<AnyAlign<int16_t>*>(dst)->v = (int16_t)lo;
+            lo >>= 16, dst += 2;
+        }
+    if constexpr(UNIT == 1)
+        if(nb & 1)
+            *dst = (uint8_t)lo;
+}
+// ... and its load, zeros behind the nb bytes (nb <= 0: nothing but zeros, nothing read)
+template <typename V>
+__device__ __forceinline__ V load_head16(const void* ptr, int nb) // 16-bit elements
+{
+    const uint8_t* src = reinterpret_cast<const uint8_t*>(ptr);
+    if(nb >= 16)
+        return load_vec<V>(src);
+    nb             = nb < 0 ? 0 : nb;
+    i32x2 first    = {0, 0}, rest = {0, 0};
+    const int big  = nb & 8;
+    if(big)
+        first = reinterpret_cast<const AnyAlign<i32x2>*>(src)->v;
+    const int at4 = big, at2 = big + (nb & 4);
+    if(nb & 4)
+        rest[0] = reinterpret_cast<const AnyAlign<int>*>(src + at4)->v;
+    if(nb & 2)
+    {
+        const int last = reinterpret_cast<const AnyAlign<uint16_t>*>(src + at2)->v;
+        rest           = (nb & 4) ? i32x2{rest[0], last} : i32x2{last, 0};
+    }
+    const i32x4 x = big ? i32x4{first[0], first[1], rest[0], rest[1]} : i32x4{rest[0], rest[1], 0, 0};
+    return __builtin_bit_cast(V, x);
+}
+// as much of a 16-byte vector as the row has room for
+template <int UNIT, typename V>
+__device__ __forceinline__ void store_room(void* ptr, const V& val, int room_bytes, bool nt)
+{
+    if(room_bytes >= 16)
+        store_vec(ptr, val, nt);
+    else if(room_bytes > 0)
+        store_head<UNIT>(ptr, val, room_bytes);
 }
 
 // q = n / d for 0 <= n < 2^31 (include/ck/utility/magic_division.hpp:28-54,132-137)
@@ -325,31 +401,21 @@ __device__ __forceinline__ void requant_lut(const i32x4 (&v)[NQ], float sg, uint
     __builtin_amdgcn_sched_barrier(0);
 }
 // 16 consecutive int8 outputs of one row, rounded requant through the table
-__device__ __forceinline__ void store_row16_i8_lut(int8_t* crow, int n0, int N, bool vec_ok, const i32x4 (&v)[4], float sg,
+__device__ __forceinline__ void store_row16_i8_lut(int8_t* crow, int n0, int N, const i32x4 (&v)[4], float sg,
                                                    uint32_t lut_lds, bool nt)
 {
     int b[16];
     requant_lut<4>(v, sg, lut_lds, b);
-    if(vec_ok && n0 + 16 <= N)
-    {
-        i32x4 pk;
+    i32x4 pk;
 #pragma unroll
-        for(int w = 0; w < 4; ++w)
-            pk[w] = pack4_low_bytes(b[4 * w], b[4 * w + 1], b[4 * w + 2], b[4 * w + 3]);
-        store_vec(reinterpret_cast<i32x4*>(crow + n0), pk, nt);
-    }
-    else
-    {
-#pragma unroll
-        for(int e = 0; e < 16; ++e)
-            if(n0 + e < N)
-                crow[n0 + e] = (int8_t)b[e];
-    }
+    for(int w = 0; w < 4; ++w)
+        pk[w] = pack4_low_bytes(b[4 * w], b[4 * w + 1], b[4 * w + 2], b[4 * w + 3]);
+    store_room<1>(crow + n0, pk, N - n0, nt);
 }
 
 // 16 consecutive int8 outputs of one row
 template <int EPI>
-__device__ __forceinline__ void store_row16_i8(int8_t* crow, int n0, int N, bool vec_ok, const i32x4 (&v)[4],
+__device__ __forceinline__ void store_row16_i8(int8_t* crow, int n0, int N, const i32x4 (&v)[4],
                                                float sg, float sr, bool nt = false)
 {
     int b[16];
@@ -358,25 +424,15 @@ __device__ __forceinline__ void store_row16_i8(int8_t* crow, int n0, int N, bool
 #pragma unroll
         for(int j = 0; j < 4; ++j)
             b[t * 4 + j] = epilogue_i8<EPI>(v[t][j], sg, sr);
-    if(vec_ok && n0 + 16 <= N)
-    {
-        i32x4 pk;
+    i32x4 pk;
 #pragma unroll
-        for(int w = 0; w < 4; ++w)
-            pk[w] = pack4_low_bytes(b[4 * w], b[4 * w + 1], b[4 * w + 2], b[4 * w + 3]);
-        store_vec(reinterpret_cast<i32x4*>(crow + n0), pk, nt);
-    }
-    else
-    {
-#pragma unroll
-        for(int e = 0; e < 16; ++e)
-            if(n0 + e < N)
-                crow[n0 + e] = (int8_t)b[e];
-    }
+    for(int w = 0; w < 4; ++w)
+        pk[w] = pack4_low_bytes(b[4 * w], b[4 * w + 1], b[4 * w + 2], b[4 * w + 3]);
+    store_room<1>(crow + n0, pk, N - n0, nt);
 }
 
 // 16 consecutive int8 outputs of one row under per-column scales sc[0..15] (columns n0 .. n0 + 15)
-__device__ __forceinline__ void store_row16_i8_cols(int8_t* crow, int n0, int N, bool vec_ok, const i32x4 (&v)[4],
+__device__ __forceinline__ void store_row16_i8_cols(int8_t* crow, int n0, int N, const i32x4 (&v)[4],
                                                     const float (&sc)[16], bool relu, bool nt = false)
 {
     int b[16];
@@ -385,21 +441,11 @@ __device__ __forceinline__ void store_row16_i8_cols(int8_t* crow, int n0, int N,
 #pragma unroll
         for(int j = 0; j < 4; ++j)
             b[t * 4 + j] = mul2_clamp(v[t][j], sc[t * 4 + j], relu);
-    if(vec_ok && n0 + 16 <= N)
-    {
-        i32x4 pk;
+    i32x4 pk;
 #pragma unroll
-        for(int w = 0; w < 4; ++w)
-            pk[w] = pack4_low_bytes(b[4 * w], b[4 * w + 1], b[4 * w + 2], b[4 * w + 3]);
-        store_vec(reinterpret_cast<i32x4*>(crow + n0), pk, nt);
-    }
-    else
-    {
-#pragma unroll
-        for(int e = 0; e < 16; ++e)
-            if(n0 + e < N)
-                crow[n0 + e] = (int8_t)b[e];
-    }
+    for(int w = 0; w < 4; ++w)
+        pk[w] = pack4_low_bytes(b[4 * w], b[4 * w + 1], b[4 * w + 2], b[4 * w + 3]);
+    store_room<1>(crow + n0, pk, N - n0, nt);
 }
 
 // the 16 scales of columns n0 .. n0 + 15 (zeros past N: a bounds-checked buffer read, no alignment beyond a float's)
@@ -471,76 +517,58 @@ struct FunctorOf
 
 // 16 consecutive fp16 outputs of one row with D operands; d0row / d1row point at column 0 of the
 // row's D values (d1row may be null)
-__device__ __forceinline__ void store_row16_f16_fused(_Float16* crow, int n0, int N, bool vec_ok, f32x4 (&v)[4],
+__device__ __forceinline__ void store_row16_f16_fused(_Float16* crow, int n0, int N, f32x4 (&v)[4],
                                                       int mode, const _Float16* d0row, const _Float16* d1row,
-                                                      bool dvec_ok, bool nt, float alpha, float beta);
+                                                      bool nt, float alpha, float beta);
 
 // T = _Float16 or __bf16
 template <typename T>
-__device__ __forceinline__ void store_row16_f16(T* crow, int n0, int N, bool vec_ok, const f32x4 (&v)[4],
+__device__ __forceinline__ void store_row16_f16(T* crow, int n0, int N, const f32x4 (&v)[4],
                                                 bool nt = false)
 {
     typedef T tx8 __attribute__((ext_vector_type(8)));
-    if(vec_ok && n0 + 16 <= N)
-    {
-        tx8 lo, hi;
+    tx8 lo, hi;
 #pragma unroll
-        for(int j = 0; j < 4; ++j)
-        {
-            lo[j]     = (T)v[0][j];
-            lo[4 + j] = (T)v[1][j];
-            hi[j]     = (T)v[2][j];
-            hi[4 + j] = (T)v[3][j];
-        }
-        store_vec(reinterpret_cast<tx8*>(crow + n0), lo, nt);
-        store_vec(reinterpret_cast<tx8*>(crow + n0 + 8), hi, nt);
+    for(int j = 0; j < 4; ++j)
+    {
+        lo[j]     = (T)v[0][j];
+        lo[4 + j] = (T)v[1][j];
+        hi[j]     = (T)v[2][j];
+        hi[4 + j] = (T)v[3][j];
+    }
+    if(n0 + 16 <= N)
+    {
+        store_vec(crow + n0, lo, nt);
+        store_vec(crow + n0 + 8, hi, nt);
     }
     else
     {
-#pragma unroll
-        for(int t = 0; t < 4; ++t)
-#pragma unroll
-            for(int j = 0; j < 4; ++j)
-                if(n0 + t * 4 + j < N)
-                    crow[n0 + t * 4 + j] = (T)v[t][j];
+        store_room<2>(crow + n0, lo, (N - n0) * 2, nt);
+        store_room<2>(crow + n0 + 8, hi, (N - n0 - 8) * 2, nt);
     }
 }
 
-__device__ __forceinline__ void store_row16_f16_fused(_Float16* crow, int n0, int N, bool vec_ok, f32x4 (&v)[4],
+__device__ __forceinline__ void store_row16_f16_fused(_Float16* crow, int n0, int N, f32x4 (&v)[4],
                                                       int mode, const _Float16* d0row, const _Float16* d1row,
-                                                      bool dvec_ok, bool nt, float alpha, float beta)
+                                                      bool nt, float alpha, float beta)
 {
     const bool has_d1 = epi_has_d1(mode);
-    if(dvec_ok && n0 + 16 <= N)
-    {
-        const f16x8 z   = {0, 0, 0, 0, 0, 0, 0, 0};
-        const f16x8 b_lo = *reinterpret_cast<const f16x8*>(d0row + n0);
-        const f16x8 b_hi = *reinterpret_cast<const f16x8*>(d0row + n0 + 8);
-        const f16x8 r_lo = has_d1 ? *reinterpret_cast<const f16x8*>(d1row + n0) : z;
-        const f16x8 r_hi = has_d1 ? *reinterpret_cast<const f16x8*>(d1row + n0 + 8) : z;
+    const f16x8 z     = {0, 0, 0, 0, 0, 0, 0, 0};
+    const int room    = (N - n0) * 2;
+    const f16x8 b_lo = load_head16<f16x8>(d0row + n0, room);
+    const f16x8 b_hi = load_head16<f16x8>(d0row + n0 + 8, room - 16);
+    const f16x8 r_lo = has_d1 ? load_head16<f16x8>(d1row + n0, room) : z;
+    const f16x8 r_hi = has_d1 ? load_head16<f16x8>(d1row + n0 + 8, room - 16) : z;
 #pragma unroll
-        for(int t = 0; t < 4; ++t)
+    for(int t = 0; t < 4; ++t)
 #pragma unroll
-            for(int j = 0; j < 4; ++j)
-            {
-                const int e = t * 4 + j;
-                v[t][j]     = epi_f16_value(mode, v[t][j], (float)(e < 8 ? b_lo[e] : b_hi[e - 8]),
-                                            (float)(e < 8 ? r_lo[e] : r_hi[e - 8]), alpha, beta);
-            }
-    }
-    else
-    {
-#pragma unroll
-        for(int t = 0; t < 4; ++t)
-#pragma unroll
-            for(int j = 0; j < 4; ++j)
-            {
-                const int n = n0 + t * 4 + j;
-                if(n < N)
-                    v[t][j] = epi_f16_value(mode, v[t][j], (float)d0row[n], has_d1 ? (float)d1row[n] : 0.0f, alpha, beta);
-            }
-    }
-    store_row16_f16(crow, n0, N, vec_ok, v, nt);
+        for(int j = 0; j < 4; ++j)
+        {
+            const int e = t * 4 + j;
+            v[t][j]     = epi_f16_value(mode, v[t][j], (float)(e < 8 ? b_lo[e] : b_hi[e - 8]),
+                                        (float)(e < 8 ? r_lo[e] : r_hi[e - 8]), alpha, beta);
+        }
+    store_row16_f16(crow, n0, N, v, nt);
 }
 
 // ------------------------------------------------------------------- kernel
@@ -1027,11 +1055,7 @@ struct GemmTile
         };
 
         // ---- epilogue: registers -> global, 16 consecutive columns per lane -------------
-        const bool vec_ok = ((reinterpret_cast<uintptr_t>(p.c) | ((uintptr_t)p.ldc * ES) |
-                              (nbatch > 1 ? (uintptr_t)p.bsc * ES : 0)) & 15u) == 0;
         const bool nt     = p.nt_store != 0;
-        const bool dvec_ok = ((reinterpret_cast<uintptr_t>(p.d0) | ((uintptr_t)p.ldd0 * ES) |
-                               reinterpret_cast<uintptr_t>(p.d1) | ((uintptr_t)p.ldd1 * ES)) & 15u) == 0;
         auto epilogue = [&](int unit) {
             int tm, tn, bi;
             tile_of_block(unit % ntiles_all, p.tiles_m, p.tiles_n, nbatch, bi, tm, tn);
@@ -1065,7 +1089,7 @@ struct GemmTile
                             if(m < p.M && n0 < p.N)
                             {
                                 const i32x4 v[4] = {acc[i][g * 4], acc[i][g * 4 + 1], acc[i][g * 4 + 2], acc[i][g * 4 + 3]};
-                                store_row16_i8_cols(reinterpret_cast<int8_t*>(c_batch) + (size_t)m * p.ldc, n0, p.N, vec_ok,
+                                store_row16_i8_cols(reinterpret_cast<int8_t*>(c_batch) + (size_t)m * p.ldc, n0, p.N,
                                                     v, sc, relu, nt);
                             }
 #pragma unroll
@@ -1090,19 +1114,9 @@ struct GemmTile
                         {
                             // raw accumulators, 16 consecutive columns = 64 bytes per lane
                             uint8_t* wrow = reinterpret_cast<uint8_t*>(slice) + ((size_t)m * p.N + n0) * 4;
-                            if(n0 + 16 <= p.N && (p.N & 3) == 0)
-                            {
 #pragma unroll
-                                for(int t = 0; t < 4; ++t)
-                                    reinterpret_cast<acc_t*>(wrow)[t] = acc[i][g * 4 + t];
-                            }
-                            else
-                            {
-#pragma unroll
-                                for(int e = 0; e < 16; ++e)
-                                    if(n0 + e < p.N)
-                                        reinterpret_cast<decltype(acc[0][0][0] + 0)*>(wrow)[e] = acc[i][g * 4 + e / 4][e % 4];
-                            }
+                            for(int t = 0; t < 4; ++t)
+                                store_room<4>(wrow + 16 * t, acc[i][g * 4 + t], (p.N - n0 - 4 * t) * 4, false);
                         }
                         else if constexpr(DT == DT_I8)
                         {
@@ -1110,25 +1124,25 @@ struct GemmTile
                             const i32x4 v[4] = {acc[i][g * 4], acc[i][g * 4 + 1], acc[i][g * 4 + 2],
                                                 acc[i][g * 4 + 3]};
                             if(p.epi == EPI_REQUANT_RND && USE_LUT)
-                                store_row16_i8_lut(crow, n0, p.N, vec_ok, v, p.scale_gemm,
+                                store_row16_i8_lut(crow, n0, p.N, v, p.scale_gemm,
                                                    (uint32_t)(uintptr_t)(lds_ptr_t)smem + (uint32_t)(NST * STAGE), nt);
                             else if(p.epi == EPI_REQUANT_RND)
-                                store_row16_i8<EPI_REQUANT_RND>(crow, n0, p.N, vec_ok, v, p.scale_gemm, p.scale_relu, nt);
+                                store_row16_i8<EPI_REQUANT_RND>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu, nt);
                             else if(p.epi == EPI_REQUANT_CK)
-                                store_row16_i8<EPI_REQUANT_CK>(crow, n0, p.N, vec_ok, v, p.scale_gemm, p.scale_relu, nt);
+                                store_row16_i8<EPI_REQUANT_CK>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu, nt);
                             else
-                                store_row16_i8<EPI_PASSTHROUGH>(crow, n0, p.N, vec_ok, v, p.scale_gemm, p.scale_relu, nt);
+                                store_row16_i8<EPI_PASSTHROUGH>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu, nt);
                         }
                         else
                         {
                             const f32x4 v[4] = {acc[i][g * 4], acc[i][g * 4 + 1], acc[i][g * 4 + 2],
                                                 acc[i][g * 4 + 3]};
                             if constexpr(DT == DT_BF16)
-                                store_row16_f16(reinterpret_cast<__bf16*>(c_batch) + (size_t)m * p.ldc, n0, p.N, vec_ok,
+                                store_row16_f16(reinterpret_cast<__bf16*>(c_batch) + (size_t)m * p.ldc, n0, p.N,
                                                 v, nt);
                             else
                                 store_row16_f16(reinterpret_cast<_Float16*>(c_batch) + (size_t)m * p.ldc, n0, p.N,
-                                                vec_ok, v, nt);
+                                                v, nt);
                         }
                     }
 #pragma unroll
@@ -1159,20 +1173,19 @@ struct GemmTile
             const _Float16* d0 = reinterpret_cast<const _Float16*>(p.d0);
             const _Float16* d1 = reinterpret_cast<const _Float16*>(p.d1);
             const f16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-            auto load16 = [&](const _Float16* row, int n0, f16x8& lo, f16x8& hi) {
-                if(dvec_ok && n0 + 16 <= p.N)
+            auto load16 = [&](const _Float16* d, size_t at, int n0, f16x8& lo, f16x8& hi) {
+                if constexpr(BM * BN >= 256 * 256)
+                    asm volatile("" : "+v"(at)); // (as for the stores' row offsets below)
+                const _Float16* row = d + at;
+                if(n0 + 16 <= p.N)
                 {
-                    lo = *reinterpret_cast<const f16x8*>(row + n0);
-                    hi = *reinterpret_cast<const f16x8*>(row + n0 + 8);
+                    lo = load_vec<f16x8>(row + n0);
+                    hi = load_vec<f16x8>(row + n0 + 8);
                 }
                 else
                 {
-#pragma unroll
-                    for(int e = 0; e < 8; ++e)
-                    {
-                        lo[e] = n0 + e < p.N ? row[n0 + e] : (_Float16)0;
-                        hi[e] = n0 + 8 + e < p.N ? row[n0 + 8 + e] : (_Float16)0;
-                    }
+                    lo = load_head16<f16x8>(row + n0, (p.N - n0) * 2);
+                    hi = load_head16<f16x8>(row + n0 + 8, (p.N - n0 - 8) * 2);
                 }
             };
             auto col0 = [&](int g) { return tn * BN + wn * WTN + 64 * g + 16 * (lane >> 4); };
@@ -1182,7 +1195,7 @@ struct GemmTile
             {
                 b_lo[g] = b_hi[g] = zero8;
                 if(!d0_per_row && col0(g) < p.N)
-                    load16(d0, col0(g), b_lo[g], b_hi[g]);
+                    load16(d0, 0, col0(g), b_lo[g], b_hi[g]);
             }
             // The D values are awaited where every lane passes, right behind their loads (they are the youngest
             // requests, so the first use would wait for as much). Left to the uses, which sit under the same conditions
@@ -1207,13 +1220,13 @@ struct GemmTile
                         {
                             x_lo[c][g] = x_hi[c][g] = zero8;
                             if(live)
-                                load16(d0 + (size_t)m * p.ldd0, col0(g), x_lo[c][g], x_hi[c][g]);
+                                load16(d0, (size_t)m * p.ldd0, col0(g), x_lo[c][g], x_hi[c][g]);
                         }
                         if constexpr(has_d1)
                         {
                             y_lo[c][g] = y_hi[c][g] = zero8;
                             if(live)
-                                load16(d1 + (size_t)m * p.ldd1, col0(g), y_lo[c][g], y_hi[c][g]);
+                                load16(d1, (size_t)m * p.ldd1, col0(g), y_lo[c][g], y_hi[c][g]);
                         }
                     }
                 if constexpr(d0_per_row || has_d1)
@@ -1240,8 +1253,13 @@ struct GemmTile
                                     const float y = has_d1 ? (float)(e < 8 ? y_lo[cy][g][e & 7] : y_hi[cy][g][e & 7]) : 0.0f;
                                     v[t][j] = epi_f16_value<EXT>(mode, acc[i][g * 4 + t][j], x, y, p.scale_gemm, p.scale_relu);
                                 }
-                            _Float16* crow = reinterpret_cast<_Float16*>(p.c) + (size_t)m * p.ldc;
-                            store_row16_f16(crow, col0(g), p.N, vec_ok, v, nt);
+                            // (the row's offset as a value of this place: the 256 x 256 instance has no registers for the
+                            // addresses of several rows worked out ahead, and spilled)
+                            size_t at = (size_t)m * p.ldc;
+                            if constexpr(BM * BN >= 256 * 256)
+                                asm volatile("" : "+v"(at));
+                            _Float16* crow = reinterpret_cast<_Float16*>(p.c) + at;
+                            store_row16_f16(crow, col0(g), p.N, v, nt);
                         }
 #pragma unroll
                         for(int t = 0; t < 4; ++t)
@@ -1349,12 +1367,15 @@ struct GemmTile
                         using std::integral_constant;
                         using std::false_type;
                         using std::true_type;
-                        const bool d0_rows = p.ldd0 != 0;
                         // chunks of fragment rows whose D values are fetched together: all of them for a bias row alone,
                         // two with one per-row tensor, one with two
                         auto with_functor = [&](auto mode_c) {
                             constexpr bool resi = decltype(mode_c)::has_d1;
-                            if(!d0_rows)
+                            // (a conv's first D operand is the bias row; one residual row at a time in the im2col kernels whose
+                            // registers are full)
+                            if constexpr(IM2COL != 0)
+                                epilogue_fused(unit, integral_constant<int, (resi ? (BM >= 256 ? 1 : 2) : MT)>{}, false_type{}, mode_c);
+                            else if(p.ldd0 == 0)
                                 epilogue_fused(unit, integral_constant<int, (resi ? 2 : MT)>{}, false_type{}, mode_c);
                             else
                                 epilogue_fused(unit, integral_constant<int, (resi ? 1 : 2)>{}, true_type{}, mode_c);
@@ -1430,7 +1451,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs p)
 #pragma unroll
     for(int t = 0; t < 4; ++t)
         v[t] = acc_t{0, 0, 0, 0};
-    const bool full = n0 + 16 <= p.N && (p.N & 3) == 0;
+    const bool full = n0 + 16 <= p.N;
     for(int sp = 0; sp < p.ksplit; ++sp)
     {
         const uint8_t* wrow = reinterpret_cast<const uint8_t*>(p.ws) + (((size_t)sp * p.M + m) * p.N + n0) * 4;
@@ -1439,7 +1460,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs p)
 #pragma unroll
             for(int t = 0; t < 4; ++t)
             {
-                const acc_t w = reinterpret_cast<const acc_t*>(wrow)[t];
+                const acc_t w = load_vec<acc_t>(wrow + 16 * t);
                 v[t][0] += w[0], v[t][1] += w[1], v[t][2] += w[2], v[t][3] += w[3];
             }
         }
@@ -1451,7 +1472,6 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs p)
                     v[e / 4][e % 4] += reinterpret_cast<const decltype(v[0][0] + 0)*>(wrow)[e];
         }
     }
-    const bool vec_ok = ((reinterpret_cast<uintptr_t>(p.c) | ((uintptr_t)p.ldc * ES)) & 15u) == 0;
     if constexpr(DT == DT_I8)
     {
         int8_t* crow = reinterpret_cast<int8_t*>(p.c) + (size_t)m * p.ldc;
@@ -1459,30 +1479,28 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs p)
         {
             float sc[16];
             load_col_scales(make_rsrc(p.d0, (uint32_t)p.N * 4u), n0, sc);
-            store_row16_i8_cols(crow, n0, p.N, vec_ok, v, sc, p.epi == EPI_RELU_MUL2_CLAMP);
+            store_row16_i8_cols(crow, n0, p.N, v, sc, p.epi == EPI_RELU_MUL2_CLAMP);
         }
         else if(p.epi == EPI_REQUANT_RND)
-            store_row16_i8<EPI_REQUANT_RND>(crow, n0, p.N, vec_ok, v, p.scale_gemm, p.scale_relu);
+            store_row16_i8<EPI_REQUANT_RND>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu);
         else if(p.epi == EPI_REQUANT_CK)
-            store_row16_i8<EPI_REQUANT_CK>(crow, n0, p.N, vec_ok, v, p.scale_gemm, p.scale_relu);
+            store_row16_i8<EPI_REQUANT_CK>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu);
         else
-            store_row16_i8<EPI_PASSTHROUGH>(crow, n0, p.N, vec_ok, v, p.scale_gemm, p.scale_relu);
+            store_row16_i8<EPI_PASSTHROUGH>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu);
     }
     else if constexpr(DT == DT_BF16)
-        store_row16_f16(reinterpret_cast<__bf16*>(p.c) + (size_t)m * p.ldc, n0, p.N, vec_ok, v);
+        store_row16_f16(reinterpret_cast<__bf16*>(p.c) + (size_t)m * p.ldc, n0, p.N, v);
     else
     {
         _Float16* crow = reinterpret_cast<_Float16*>(p.c) + (size_t)m * p.ldc;
         if(p.epi == EPI_PASSTHROUGH)
-            store_row16_f16(crow, n0, p.N, vec_ok, v);
+            store_row16_f16(crow, n0, p.N, v);
         else
         {
-            const bool dvec_ok = ((reinterpret_cast<uintptr_t>(p.d0) | ((uintptr_t)p.ldd0 * ES) |
-                                   reinterpret_cast<uintptr_t>(p.d1) | ((uintptr_t)p.ldd1 * ES)) & 15u) == 0;
-            store_row16_f16_fused(crow, n0, p.N, vec_ok, v, p.epi,
+            store_row16_f16_fused(crow, n0, p.N, v, p.epi,
                                   reinterpret_cast<const _Float16*>(p.d0) + (size_t)m * p.ldd0,
                                   p.d1 ? reinterpret_cast<const _Float16*>(p.d1) + (size_t)m * p.ldd1 : nullptr,
-                                  dvec_ok, false, p.scale_gemm, p.scale_relu);
+                                  false, p.scale_gemm, p.scale_relu);
         }
     }
 }

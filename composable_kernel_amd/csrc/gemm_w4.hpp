@@ -176,49 +176,29 @@ struct GemmW4
     }
     // the lane's 16 outputs of one row and 64-column group (first column n64) as two runs of 8 consecutive 16-bit values
     template <typename T>
-    __device__ static __forceinline__ void store_2x8(T* crow, int n64, int q, int N, bool vec_ok, const f32x4 (&v)[4], bool nt)
+    __device__ static __forceinline__ void store_2x8(T* crow, int n64, int q, int N, const f32x4 (&v)[4], bool nt)
     {
         typedef T tx8 __attribute__((ext_vector_type(8)));
 #pragma unroll
         for(int h = 0; h < 2; ++h)
         {
             const int n0 = n64 + 32 * h + 8 * q;
-            if(vec_ok && n0 + 8 <= N)
-            {
-                tx8 x;
+            tx8 x;
 #pragma unroll
-                for(int j = 0; j < 4; ++j)
-                    x[j] = (T)v[2 * h][j], x[4 + j] = (T)v[2 * h + 1][j];
-                store_vec(reinterpret_cast<tx8*>(crow + n0), x, nt);
-            }
-            else
-            {
-#pragma unroll
-                for(int e = 0; e < 8; ++e)
-                    if(n0 + e < N)
-                        crow[n0 + e] = (T)v[2 * h + e / 4][e % 4];
-            }
+            for(int j = 0; j < 4; ++j)
+                x[j] = (T)v[2 * h][j], x[4 + j] = (T)v[2 * h + 1][j];
+            store_room<2>(crow + n0, x, (N - n0) * 2, nt);
         }
     }
 
     // 16 consecutive int8 outputs of one row from their (already requantised) values b[0..15]
-    __device__ static __forceinline__ void store_bytes16(int8_t* crow, int n0, int N, bool vec_ok, const int* b, bool nt)
+    __device__ static __forceinline__ void store_bytes16(int8_t* crow, int n0, int N, const int* b, bool nt)
     {
-        if(vec_ok && n0 + 16 <= N)
-        {
-            i32x4 pk;
+        i32x4 pk;
 #pragma unroll
-            for(int w = 0; w < 4; ++w)
-                pk[w] = pack4_low_bytes(b[4 * w], b[4 * w + 1], b[4 * w + 2], b[4 * w + 3]);
-            store_vec(reinterpret_cast<i32x4*>(crow + n0), pk, nt);
-        }
-        else
-        {
-#pragma unroll
-            for(int e = 0; e < 16; ++e)
-                if(n0 + e < N)
-                    crow[n0 + e] = (int8_t)b[e];
-        }
+        for(int w = 0; w < 4; ++w)
+            pk[w] = pack4_low_bytes(b[4 * w], b[4 * w + 1], b[4 * w + 2], b[4 * w + 3]);
+        store_room<1>(crow + n0, pk, N - n0, nt);
     }
 
     __device__ static __forceinline__ void run(const GemmArgs& p, uint8_t* smem)
@@ -256,8 +236,6 @@ struct GemmW4
         const uint32_t fa[2] = {smem_lds + frag_part(wm * 128, 0), smem_lds + frag_part(wm * 128, 1)};
         const uint32_t fb[2] = {smem_lds + B_AT(0) + frag_part(wn * 128, 0), smem_lds + B_AT(0) + frag_part(wn * 128, 1)};
 
-        const bool vec_ok = ((reinterpret_cast<uintptr_t>(p.c) | ((uintptr_t)p.ldc * ES) |
-                              (nbatch > 1 ? (uintptr_t)p.bsc * ES : 0)) & 15u) == 0;
         const bool nt     = p.nt_store != 0;
 
         for(int unit = (int)blockIdx.x; unit < ntiles; unit += (int)gridDim.x)
@@ -454,9 +432,9 @@ struct GemmW4
                         {
                             int8_t* crow = reinterpret_cast<int8_t*>(c_batch) + (size_t)m * p.ldc;
                             if(nb < p.N)
-                                store_bytes16(crow, nb, p.N, vec_ok, b, nt);
+                                store_bytes16(crow, nb, p.N, b, nt);
                             if(nb + 64 < p.N)
-                                store_bytes16(crow, nb + 64, p.N, vec_ok, b + 16, nt);
+                                store_bytes16(crow, nb + 64, p.N, b + 16, nt);
                         }
                     }
                     else
@@ -466,7 +444,7 @@ struct GemmW4
                         int b[16];
                         requant_lut<4>(v, p.scale_gemm, lut_lds, b);
                         if(m < p.M && nb + 64 * G < p.N)
-                            store_bytes16(reinterpret_cast<int8_t*>(c_batch) + (size_t)m * p.ldc, nb + 64 * G, p.N, vec_ok, b, nt);
+                            store_bytes16(reinterpret_cast<int8_t*>(c_batch) + (size_t)m * p.ldc, nb + 64 * G, p.N, b, nt);
                     }
                     return;
                 }
@@ -481,7 +459,7 @@ struct GemmW4
                             acc_t v[4];
                             fetch_acc(in_vgpr{}, acc[i], g, v);
                             int8_t* crow = reinterpret_cast<int8_t*>(c_batch) + (size_t)m * p.ldc;
-                            store_row16_i8<EPI>(crow, n0, p.N, vec_ok, v, p.scale_gemm, p.scale_relu, nt);
+                            store_row16_i8<EPI>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu, nt);
                         }
                     }
                     else
@@ -492,9 +470,9 @@ struct GemmW4
                             acc_t v[4];
                             fetch_acc(in_vgpr{}, acc[i], g, v);
                             if constexpr(DT == DT_BF16)
-                                store_2x8(reinterpret_cast<__bf16*>(c_batch) + (size_t)m * p.ldc, n64, lane >> 4, p.N, vec_ok, v, nt);
+                                store_2x8(reinterpret_cast<__bf16*>(c_batch) + (size_t)m * p.ldc, n64, lane >> 4, p.N, v, nt);
                             else
-                                store_2x8(reinterpret_cast<_Float16*>(c_batch) + (size_t)m * p.ldc, n64, lane >> 4, p.N, vec_ok, v, nt);
+                                store_2x8(reinterpret_cast<_Float16*>(c_batch) + (size_t)m * p.ldc, n64, lane >> 4, p.N, v, nt);
                         }
                     }
                 }
@@ -518,23 +496,9 @@ struct GemmW4
                     const _Float16* d0  = reinterpret_cast<const _Float16*>(p.d0);
                     const _Float16* d1  = reinterpret_cast<const _Float16*>(p.d1);
                     const bool d0_rows  = p.ldd0 != 0;
-                    const bool dvec_ok  = ((reinterpret_cast<uintptr_t>(p.d0) | ((uintptr_t)p.ldd0 * ES) |
-                                           reinterpret_cast<uintptr_t>(p.d1) | ((uintptr_t)p.ldd1 * ES)) & 15u) == 0;
                     const int q         = lane >> 4;
                     const f16x8 zero8   = {0, 0, 0, 0, 0, 0, 0, 0};
-                    auto load8          = [&](const _Float16* row, int n0) {
-                        f16x8 x = zero8;
-                        if(dvec_ok && n0 + 8 <= p.N)
-                            x = *reinterpret_cast<const f16x8*>(row + n0);
-                        else
-                        {
-#pragma unroll
-                            for(int e = 0; e < 8; ++e)
-                                if(n0 + e < p.N)
-                                    x[e] = row[n0 + e];
-                        }
-                        return x;
-                    };
+                    auto load8          = [&](const _Float16* row, int n0) { return load_head16<f16x8>(row + n0, (p.N - n0) * 2); };
                     auto col0 = [&](int g, int h) { return tn * BN + wn * 128 + 64 * g + 32 * h + 8 * q; };
                     auto with_functor = [&](auto mode_c) {
                         constexpr int MODE    = decltype(mode_c)::value;
@@ -584,7 +548,7 @@ struct GemmW4
                                                                                           p.scale_gemm, p.scale_relu);
                                         }
                                     if(m < p.M && n64 < p.N)
-                                        store_2x8(reinterpret_cast<_Float16*>(c_batch) + (size_t)m * p.ldc, n64, q, p.N, vec_ok, v, nt);
+                                        store_2x8(reinterpret_cast<_Float16*>(c_batch) + (size_t)m * p.ldc, n64, q, p.N, v, nt);
                                 }
                             });
                         });
