@@ -21,6 +21,7 @@
 #include "conv_stem.hpp"
 #include "gemm_skinny.hpp"
 #include "gemm_generic.hpp"
+#include "gemm_ragged.hpp"
 
 // Workspace of ckx_gemm_i8_splitk_noalloc: device memory that belongs to the library, one copy per GPU,
 // held from the time the code object is loaded on that GPU until the process ends. In host code the name
@@ -624,14 +625,10 @@ int run_gemm(int dt, const void* a, const void* b, void* c, int M, int N, int K,
         g.d0 = dops.d0, g.d1 = uses_d1(epi) ? dops.d1 : nullptr;
         g.ldd0 = dops.ldd0, g.ldd1 = dops.ldd1;
         g.ksplit  = 1;
-        g.tiles_m = (M + 63) / 64, g.tiles_n = (N + 63) / 64;
         if(batch > 65535)
             return fail(CKX_UNSUPPORTED, "the element-granular instance (operands that are not 16-byte aligned vectors) "
                                          "takes at most 65535 batches per launch");
-        ckx::GenericLayout lay{};
-        lay.a_sm = ta ? 1 : sa, lay.a_sk = ta ? sa : 1;
-        lay.b_sn = tb ? 1 : sb, lay.b_sk = tb ? sb : 1;
-        hipError_t e = ckx::launch_generic(dt, 0, g, lay, (hipStream_t)stream);
+        hipError_t e = ckx::launch_ragged(dt, ta, tb, g, (hipStream_t)stream);
         return e == hipSuccess ? CKX_OK : hip_fail(e, kGenericName);
     }
     if(misaligned)
@@ -963,7 +960,6 @@ int run_conv(int op, const void* in, const void* wei, void* out, const ckx_conv2
         g.cv.div_xc   = make_magic((uint32_t)(d->X * d->C));
         g.cv.div_c    = make_magic((uint32_t)d->C);
         ckx::GenericLayout lay{};
-        lay.b_sn = K, lay.b_sk = 1;
         lay.X = d->X, lay.Y = d->Y;
         hipError_t e = ckx::launch_generic(es == 1 ? ckx::DT_I8 : ckx::DT_F16, 1, g, lay, (hipStream_t)stream);
         return e == hipSuccess ? CKX_OK : hip_fail(e, kGenericName);
@@ -1233,7 +1229,6 @@ int run_convnd(int op, const void* in, const void* wei, void* out, const ckx_con
         g.tiles_m = (M + 63) / 64, g.tiles_n = (N + 63) / 64;
         g.ksplit  = 1;
         ckx::GenericLayout lay{};
-        lay.b_sn = K, lay.b_sk = 1;
         lay.X = d->filter[2], lay.Y = d->filter[1];
         hipError_t e = ckx::launch_generic(es == 1 ? ckx::DT_I8 : ckx::DT_F16, 2, g, lay, (hipStream_t)stream);
         return e == hipSuccess ? CKX_OK : hip_fail(e, kGenericName);

@@ -1,22 +1,17 @@
-// Element-granular GEMM / implicit-GEMM conv forward for gfx950: the instance that takes what the vectorised
-// instances refuse -- a K (or, for a K-major operand, an M / N) extent, a leading dimension, a channel count
-// or a base address that is not a whole 16-byte vector.
+// Element-granular implicit-GEMM conv forward for gfx950: the instance that takes what the vectorised conv instances
+// refuse -- a channel count or a base address that is not a whole 16-byte vector.
 //
-// Takes the place of the reference's padded GEMM instances (GemmSpecialization::KPadding / MNKPadding,
-// include/ck/tensor_operation/gpu/device/gemm_specialization.hpp:10-20, device_gemm_xdl_cshuffle.hpp:99-184)
-// and of its odd-channel conv instances (ConvolutionForwardSpecialization::OddC,
+// Takes the place of the reference's odd-channel conv instances (ConvolutionForwardSpecialization::OddC,
 // convolution_forward_specialization.hpp:13-19; device test case C = 3, test/convnd_fwd/conv2d_fwd.cpp:111),
-// which load with SrcScalarPerVector = 1. As there, the price is bandwidth: every operand element is its own
-// load instruction unless a whole 16-byte chunk happens to be in range, contiguous and aligned.
+// which load with SrcScalarPerVector = 1. As there, the price is bandwidth: every pixel element is its own load instruction.
 //
 // One workgroup of 4 waves (2 x 2) computes a 64 x 64 tile of C; a K tile is ONE MFMA k-step (64 int8 /
-// 32 fp16 or bf16 values = 64 bytes of every row). Thread t gathers 16 bytes of row t / 4 of the A tile and of
-// the B tile into registers -- zeros where the row, the K index or the conv window is out of range, which is the
-// whole of "padding" -- and writes them to LDS (rows padded to 80 bytes); after a barrier every wave reads two A and
-// two B fragments and issues four MFMAs (D^T = B_frag x A_frag, so a lane owns 4 consecutive columns of one row).
-// Operand layouts are run-time element strides, so all four GEMM layouts, a strided batch and the 1-D / 2-D / 3-D
-// im2col view go through the same code. Epilogues: PassThrough, both requant forms (int8), the add / ReLU functors
-// with D operands (fp16), applied per element.
+// 32 fp16 values = 64 bytes of every row). Thread t gathers 16 bytes of row t / 4 of the pixel tile and of
+// the weight tile into registers -- zeros where the row, the K index or the conv window is out of range, which is the
+// whole of "padding" -- and writes them to LDS (rows padded to 80 bytes); after a barrier every wave reads two pixel and
+// two weight fragments and issues four MFMAs (D^T = weights x pixels, so a lane owns 4 consecutive columns of one row).
+// The 1-D / 2-D and the 3-D im2col view go through the same code. Epilogues: PassThrough, both requant forms (int8), the
+// add / ReLU functors with D operands (fp16), applied per element.
 #pragma once
 
 #include "gemm_tile.hpp"
@@ -25,9 +20,7 @@ namespace ckx {
 
 struct GenericLayout
 {
-    long a_sm, a_sk; // element strides of A(m, k)
-    long b_sn, b_sk; // element strides of B(k, n)
-    int X, Y;        // filter extents of the two innermost spatial dimensions (im2col only)
+    int X, Y; // filter extents of the two innermost spatial dimensions
 };
 
 template <int DT, int IM2COL>
@@ -45,10 +38,9 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const GemmArgs p, con
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int tm = (int)(blockIdx.x % (unsigned)p.tiles_m), tn = (int)(blockIdx.x / (unsigned)p.tiles_m);
-    const long g = blockIdx.y;
 
-    const elem_t* A = reinterpret_cast<const elem_t*>(p.a) + g * p.bsa;
-    const elem_t* B = reinterpret_cast<const elem_t*>(p.b) + g * p.bsb;
+    const elem_t* A = reinterpret_cast<const elem_t*>(p.a);
+    const elem_t* B = reinterpret_cast<const elem_t*>(p.b);
 
     // this thread's slot of both staged tiles: row lrow, 16-byte chunk lchunk
     const int lrow = tid >> 2, lchunk = tid & 3;
@@ -58,30 +50,27 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const GemmArgs p, con
     // im2col: window origin of output pixel gm (device_conv2d_fwd_xdl_nhwc_kyxc_nhwk.hpp:224-301 in closed form)
     long img = 0;
     int hi0 = 0, wi0 = 0, d0 = 0;
-    if constexpr(IM2COL != 0)
+    if(m_ok)
     {
-        if(m_ok)
+        uint32_t rem = (uint32_t)gm, n;
+        if constexpr(IM2COL == 2)
         {
-            uint32_t rem = (uint32_t)gm, n;
-            if constexpr(IM2COL == 2)
-            {
-                n                 = magic_div(rem, p.cv.div_dhowo);
-                const uint32_t r3 = rem - n * p.cv.div_dhowo.d;
-                const uint32_t od = magic_div(r3, p.cv.div_howo);
-                rem               = r3 - od * p.cv.div_howo.d;
-                d0                = (int)od * p.cv.sD - p.cv.pF;
-            }
-            else
-            {
-                n   = magic_div(rem, p.cv.div_howo);
-                rem = rem - n * p.cv.div_howo.d;
-            }
-            const uint32_t ho = magic_div(rem, p.cv.div_wo);
-            const uint32_t wo = rem - ho * p.cv.div_wo.d;
-            hi0               = (int)ho * p.cv.sH - p.cv.pT;
-            wi0               = (int)wo * p.cv.sW - p.cv.pL;
-            img               = n;
+            n                 = magic_div(rem, p.cv.div_dhowo);
+            const uint32_t r3 = rem - n * p.cv.div_dhowo.d;
+            const uint32_t od = magic_div(r3, p.cv.div_howo);
+            rem               = r3 - od * p.cv.div_howo.d;
+            d0                = (int)od * p.cv.sD - p.cv.pF;
         }
+        else
+        {
+            n   = magic_div(rem, p.cv.div_howo);
+            rem = rem - n * p.cv.div_howo.d;
+        }
+        const uint32_t ho = magic_div(rem, p.cv.div_wo);
+        const uint32_t wo = rem - ho * p.cv.div_wo.d;
+        hi0               = (int)ho * p.cv.sH - p.cv.pT;
+        wi0               = (int)wo * p.cv.sW - p.cv.pL;
+        img               = n;
     }
 
     acc_t acc[2][2];
@@ -98,19 +87,6 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const GemmArgs p, con
         __attribute__((aligned(16))) elem_t va[EPC];
         __attribute__((aligned(16))) elem_t vb[EPC];
         // ---- A chunk ----
-        if constexpr(IM2COL == 0)
-        {
-            const elem_t* src = A + gm * lay.a_sm + (long)k0 * lay.a_sk;
-            if(m_ok && lay.a_sk == 1 && k0 + EPC <= p.K && (reinterpret_cast<uintptr_t>(src) & 15) == 0)
-                *reinterpret_cast<i32x4*>(va) = *reinterpret_cast<const i32x4*>(src);
-            else
-            {
-#pragma unroll
-                for(int e = 0; e < EPC; ++e)
-                    va[e] = (m_ok && k0 + e < p.K) ? src[(long)e * lay.a_sk] : (elem_t)0;
-            }
-        }
-        else
         {
             // k -> ([z,] y, x, c), c fastest; then step element by element
             uint32_t kyx = (uint32_t)k0;
@@ -151,14 +127,14 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const GemmArgs p, con
         }
         // ---- B chunk ----
         {
-            const elem_t* src = B + gn * lay.b_sn + (long)k0 * lay.b_sk;
-            if(n_ok && lay.b_sk == 1 && k0 + EPC <= p.K && (reinterpret_cast<uintptr_t>(src) & 15) == 0)
+            const elem_t* src = B + gn * p.K + k0;
+            if(n_ok && k0 + EPC <= p.K && (reinterpret_cast<uintptr_t>(src) & 15) == 0)
                 *reinterpret_cast<i32x4*>(vb) = *reinterpret_cast<const i32x4*>(src);
             else
             {
 #pragma unroll
                 for(int e = 0; e < EPC; ++e)
-                    vb[e] = (n_ok && k0 + e < p.K) ? src[(long)e * lay.b_sk] : (elem_t)0;
+                    vb[e] = (n_ok && k0 + e < p.K) ? src[e] : (elem_t)0;
             }
         }
         __syncthreads(); // the previous K tile has been read by every wave
@@ -179,9 +155,6 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const GemmArgs p, con
             {
                 if constexpr(DT == DT_I8)
                     acc[i][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bf[t], af[i], acc[i][t], 0, 0, 0);
-                else if constexpr(DT == DT_BF16)
-                    acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, bf[t]),
-                                                                     __builtin_bit_cast(bf16x8, af[i]), acc[i][t], 0, 0, 0);
                 else
                     acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, bf[t]),
                                                                     __builtin_bit_cast(f16x8, af[i]), acc[i][t], 0, 0, 0);
@@ -203,7 +176,7 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const GemmArgs p, con
                 const long n = (long)tn * 64 + wn * 32 + 16 * t + 4 * (lane >> 4) + j;
                 if(m >= p.M || n >= p.N)
                     continue;
-                const long ci = g * p.bsc + m * p.ldc + n;
+                const long ci = m * p.ldc + n;
                 if constexpr(DT == DT_I8)
                 {
                     const int v = acc[i][t][j];
@@ -214,8 +187,6 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const GemmArgs p, con
                                                              : v;
                     reinterpret_cast<int8_t*>(p.c)[ci] = (int8_t)o;
                 }
-                else if constexpr(DT == DT_BF16)
-                    reinterpret_cast<__bf16*>(p.c)[ci] = (__bf16)acc[i][t][j];
                 else
                 {
                     float v = acc[i][t][j];
@@ -229,8 +200,8 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const GemmArgs p, con
     }
 }
 
-// dt: DT_*, im2col: 0 (dense A), 1 (one or two spatial dimensions), 2 (three). The grid is
-// (C tiles of 64 x 64, batches); GemmArgs::tiles_m / tiles_n must be set for 64 x 64 tiles.
+// dt: DT_I8 / DT_F16, im2col: 1 (one or two spatial dimensions), 2 (three). The grid is the C tiles of 64 x 64, which
+// GemmArgs::tiles_m / tiles_n must be set for.
 hipError_t launch_generic(int dt, int im2col, const GemmArgs& a, const GenericLayout& lay, hipStream_t s);
 
 } // namespace ckx
