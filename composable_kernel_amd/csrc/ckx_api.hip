@@ -15,6 +15,7 @@
 #include "tile_launch.hpp"
 #include "conv_rows.hpp"
 #include "gemm_gemm.hpp"
+#include "conv_few.hpp"
 #include "conv_patch.hpp"
 #include "conv_patch_wide.hpp"
 #include "conv_pointwise.hpp"
@@ -942,6 +943,22 @@ int run_conv(int op, const void* in, const void* wei, void* out, const ckx_conv2
         if((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(wei) | reinterpret_cast<uintptr_t>(out) |
             (f16_fused(epi) ? reinterpret_cast<uintptr_t>(dops.d0) | reinterpret_cast<uintptr_t>(dops.d1) : 0)) & (es - 1))
             return fail(CKX_UNSUPPORTED, "operands must be aligned to their element size");
+        // pixels of a few channels: padded to four or eight in LDS (conv_few.hpp); a bias is a row there (D0 stride 0)
+        ckx::ConvFewArgs f;
+        std::memset(&f, 0, sizeof(f));
+        f.N = d->N, f.Hi = d->Hi, f.Wi = d->Wi, f.C = d->C, f.Ho = d->Ho, f.Wo = d->Wo, f.K = d->K, f.X = d->X;
+        f.sH = d->stride_h, f.sW = d->stride_w, f.dH = d->dilation_h, f.dW = d->dilation_w, f.pT = d->pad_top, f.pL = d->pad_left;
+        const int dt = es == 1 ? ckx::DT_I8 : ckx::DT_F16;
+        if(dops.ldd0 == 0 && ckx::plan_conv_few(dt, f, d->Y))
+        {
+            f.in = in, f.wei = wei, f.out = out;
+            f.d0 = dops.d0, f.d1 = uses_d1(epi) ? dops.d1 : nullptr, f.ldd1 = dops.ldd1;
+            f.div_pc = make_magic((uint32_t)f.PC), f.div_tw = make_magic((uint32_t)f.TW);
+            f.epi = epi, f.scale_gemm = sg, f.scale_relu = sr;
+            f.nt_store   = es == 1 && (long)M * N * es >= stream_output_bytes();
+            hipError_t e = ckx::launch_conv_few(dt, f, (hipStream_t)stream);
+            return e == hipSuccess ? CKX_OK : hip_fail(e, kGenericName);
+        }
         ckx::GemmArgs g;
         std::memset(&g, 0, sizeof(g));
         g.a = in, g.b = wei, g.c = out;
@@ -961,7 +978,7 @@ int run_conv(int op, const void* in, const void* wei, void* out, const ckx_conv2
         g.cv.div_c    = make_magic((uint32_t)d->C);
         ckx::GenericLayout lay{};
         lay.X = d->X, lay.Y = d->Y;
-        hipError_t e = ckx::launch_generic(es == 1 ? ckx::DT_I8 : ckx::DT_F16, 1, g, lay, (hipStream_t)stream);
+        hipError_t e = ckx::launch_generic(dt, 1, g, lay, (hipStream_t)stream);
         return e == hipSuccess ? CKX_OK : hip_fail(e, kGenericName);
     }
     if(misaligned)

@@ -21,7 +21,7 @@ template <int DT, bool TA, bool TB>
 static hipError_t launch_tile_size(const GemmArgs& a, hipStream_t s)
 {
     // One 128 x 128 tile per CU and more: half the operand bytes per product. 4001 x 4003 x 4095 fp16 197 us against 323 on
-    // 64 x 64, int8 122 against 192; 1000 x 4001 x 513 (exactly 256 tiles) 15.5 against 16.4; 2049 x 2047 x 2047 K-major
+    // 64 x 64, int8 118 against 192; 1000 x 4001 x 513 (exactly 256 tiles) 15.5 against 16.4; 2049 x 2047 x 2047 K-major
     // (272) level at 55. Below, the smaller tile fills CUs that would idle: 2001 x 1003 x 1025 fp16 (128 tiles) 16.1 us
     // against 21.3, int8 1500 x 1501 x 1025 K-major B (144) 14.2 against 17.8, 122 x 1283 x 3001 17.4 against 43.7.
     const long tiles128 = (long)((a.M + 127) / 128) * ((a.N + 127) / 128) * (a.batch > 1 ? a.batch : 1);

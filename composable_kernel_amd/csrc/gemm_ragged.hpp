@@ -20,7 +20,7 @@
 // What bounds it: with the 128 x 128 tile the operand bytes through a CU's L1 (32 KB per K tile; 0.27 of the MFMA rate at
 // 4001 x 4003 x 4095 fp16), with few tiles the latency of one K tile after the other. Against the element-by-element gather
 // that served these shapes (one load instruction per element), fp16: 2001 x 1003 x 1025 90.4 -> 16.1 us, 4001 x 4003 x 4095
-// 2623 -> 197, 122 x 1283 x 3001 148 -> 17.4, 2049 x 2047 x 2047 with a K-major A 290 -> 55; int8 4001 x 4003 x 4095 3019 -> 122,
+// 2623 -> 197, 122 x 1283 x 3001 148 -> 17.4, 2049 x 2047 x 2047 with a K-major A 290 -> 55; int8 4001 x 4003 x 4095 3019 -> 118,
 // 40 x 333 x 3999 156 -> 16; bf16 3000 x 2999 x 1001 275 -> 47; one tile (32 x 33 x 65) 5.7, as before.
 //
 // Two tiles: 128 x 128 reads half the operand bytes per product, 64 x 64 gives four times the workgroups; launch_ragged() says
@@ -191,27 +191,6 @@ struct RaggedOperand
     }
 };
 
-// NW dwords to any element address, as many bytes of them as the row has room for
-template <int UNIT, int NW>
-__device__ __forceinline__ void store_run(uint8_t* dst, const int (&w)[NW], int room)
-{
-    if constexpr(NW >= 4)
-    {
-#pragma unroll
-        for(int i = 0; i < NW / 4; ++i)
-            store_room<UNIT>(dst + 16 * i, i32x4{w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]}, room - 16 * i, false);
-    }
-    else if(room >= NW * 4)
-    {
-        if constexpr(NW == 2)
-            reinterpret_cast<AnyAlign<i32x2>*>(dst)->v = i32x2{w[0], w[1]};
-        else
-            reinterpret_cast<AnyAlign<int>*>(dst)->v = w[0];
-    }
-    else if(room > 0)
-        store_head<UNIT>(dst, i32x4{w[0], NW == 2 ? w[NW - 1] : 0, 0, 0}, room);
-}
-
 template <int DT, int BM, int BN, bool TA, bool TB>
 __global__ __launch_bounds__(256, 2) void gemm_ragged_kernel(const GemmArgs p)
 {
@@ -356,17 +335,9 @@ __global__ __launch_bounds__(256, 2) void gemm_ragged_kernel(const GemmArgs p)
             if constexpr(DT == DT_I8)
             {
                 int o[RUN];
-#pragma unroll
-                for(int e = 0; e < RUN; ++e)
-                {
-                    const int v = acc[i][r * TPR + e / 4][e % 4];
-                    if(epi_per_column_scale(p.epi))
-                        o[e] = mul2_clamp(v, n + e < p.N ? reinterpret_cast<const float*>(p.d0)[n + e] : 0.0f, p.epi == EPI_RELU_MUL2_CLAMP);
-                    else
-                        o[e] = p.epi == EPI_REQUANT_RND  ? requant_rnd(v, p.scale_gemm, p.scale_relu)
-                               : p.epi == EPI_REQUANT_CK ? requant_ck(v, p.scale_gemm, p.scale_relu)
-                                                         : v;
-                }
+                int8_results(GemmEpilogue{p.epi, p.scale_gemm, p.scale_relu}, o,
+                             [&](int e) { return acc[i][r * TPR + e / 4][e % 4]; },
+                             [&](int e) { return n + e < p.N ? reinterpret_cast<const float*>(p.d0)[n + e] : 0.0f; });
 #pragma unroll
                 for(int e = 0; e < RUN / 4; ++e)
                     w[e] = pack4_low_bytes(o[4 * e], o[4 * e + 1], o[4 * e + 2], o[4 * e + 3]);

@@ -160,6 +160,27 @@ __device__ __forceinline__ void store_room(void* ptr, const V& val, int room_byt
         store_head<UNIT>(ptr, val, room_bytes);
 }
 
+// NW dwords to any element address, as many bytes of them as the row has room for
+template <int UNIT, int NW>
+__device__ __forceinline__ void store_run(uint8_t* dst, const int (&w)[NW], int room, bool nt = false)
+{
+    if constexpr(NW >= 4)
+    {
+#pragma unroll
+        for(int i = 0; i < NW / 4; ++i)
+            store_room<UNIT>(dst + 16 * i, i32x4{w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]}, room - 16 * i, nt);
+    }
+    else if(room >= NW * 4)
+    {
+        if constexpr(NW == 2)
+            reinterpret_cast<AnyAlign<i32x2>*>(dst)->v = i32x2{w[0], w[1]};
+        else
+            reinterpret_cast<AnyAlign<int>*>(dst)->v = w[0];
+    }
+    else if(room > 0)
+        store_head<UNIT>(dst, i32x4{w[0], NW == 2 ? w[NW - 1] : 0, 0, 0}, room);
+}
+
 // q = n / d for 0 <= n < 2^31 (include/ck/utility/magic_division.hpp:28-54,132-137)
 struct MagicDiv
 {
@@ -446,6 +467,41 @@ __device__ __forceinline__ void store_row16_i8_cols(int8_t* crow, int n0, int N,
     for(int w = 0; w < 4; ++w)
         pk[w] = pack4_low_bytes(b[4 * w], b[4 * w + 1], b[4 * w + 2], b[4 * w + 3]);
     store_room<1>(crow + n0, pk, N - n0, nt);
+}
+
+struct GemmEpilogue
+{
+    int epi;
+    float scale_gemm, scale_relu;
+};
+// RUN accumulators to their int8 results, the functor of the launch asked for once per run and not once per element
+template <int RUN, typename Acc, typename Scale>
+__device__ __forceinline__ void int8_results(const GemmEpilogue& ep, int (&o)[RUN], Acc&& acc, Scale&& scale)
+{
+    if(ep.epi == EPI_REQUANT_RND)
+    {
+#pragma unroll
+        for(int e = 0; e < RUN; ++e)
+            o[e] = requant_rnd(acc(e), ep.scale_gemm, ep.scale_relu);
+    }
+    else if(ep.epi == EPI_REQUANT_CK)
+    {
+#pragma unroll
+        for(int e = 0; e < RUN; ++e)
+            o[e] = requant_ck(acc(e), ep.scale_gemm, ep.scale_relu);
+    }
+    else if(epi_per_column_scale(ep.epi))
+    {
+#pragma unroll
+        for(int e = 0; e < RUN; ++e)
+            o[e] = mul2_clamp(acc(e), scale(e), ep.epi == EPI_RELU_MUL2_CLAMP);
+    }
+    else
+    {
+#pragma unroll
+        for(int e = 0; e < RUN; ++e)
+            o[e] = acc(e);
+    }
 }
 
 // the 16 scales of columns n0 .. n0 + 15 (zeros past N: a bounds-checked buffer read, no alignment beyond a float's)
