@@ -76,6 +76,16 @@ def test_gemm_softmax_gemm_shapes(shape, mask, instance):
     _close(out, lit.batched_gemm_softmax_gemm_f16(a, b0_gnk.transpose(0, 2, 1), b1, scale, mask))
 
 
+@pytest.mark.parametrize("G, M, N", [(1, 300, 300), (8, 260, 260), (65, 140, 140), (127, 129, 60), (128, 257, 257),
+                                     (130, 130, 130), (200, 129, 200)])
+def test_gemm_softmax_gemm_masked_slab_order(G, M, N):
+    """The masked launch deals its slabs out over groups of 64 to 127 batches: batch counts at the groups' edges."""
+    a, b0_gnk, b1 = (uniform_f16((G, x, 16), -1, 1, 1950 + i) for i, x in enumerate((M, N, N)))
+    for instance in (capi.INSTANCE_AUTO, 1):
+        _close(_run(a, b0_gnk, b1, 0.25, True, instance),
+               lit.batched_gemm_softmax_gemm_f16(a, b0_gnk.transpose(0, 2, 1), b1, 0.25, True))
+
+
 def test_gemm_softmax_gemm_closed_forms():
     """Zero scores: the uniform distribution, C = mean of B1's rows (exact: small integers over a power of
     two). Upper-triangle mask: row m averages rows 0..m, row 0 is B1[0] exactly. A dominant score selects
