@@ -64,14 +64,15 @@ __device__ __forceinline__ float quad_rows_sum(float x)
 // MFMA result, a lane swap) canonicalised by a v_max_f32 x, x, x of its own; the 2019 maximumNumber has not, and two of
 // them are one v_max3_f32. (A NaN score makes its row of the output NaN through the exponentials whatever the maximum is.)
 __device__ __forceinline__ float score_max(float a, float b) { return __builtin_elementwise_maximumnum(a, b); }
+// (of two operands only maximumNumber is canonicalised after all; maximum, which a NaN wins, is one v_maximum3_f32)
 __device__ __forceinline__ float quad_rows_max(float x)
 {
     auto a = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
     const uint32_t a0 = a[0], a1 = a[1];
-    x      = score_max(__builtin_bit_cast(float, a0), __builtin_bit_cast(float, a1));
+    x      = __builtin_elementwise_maximum(__builtin_bit_cast(float, a0), __builtin_bit_cast(float, a1));
     auto b = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
     const uint32_t b0 = b[0], b1 = b[1];
-    return score_max(__builtin_bit_cast(float, b0), __builtin_bit_cast(float, b1));
+    return __builtin_elementwise_maximum(__builtin_bit_cast(float, b0), __builtin_bit_cast(float, b1));
 }
 
 // (batch, slab of rows) of workgroup `bid`. Workgroups of one batch share B0[g] and B1[g]: they are kept on one XCD (ids are
@@ -174,7 +175,7 @@ __global__ __launch_bounds__(NW * 64)
 
     const int tid  = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int fr   = lane & 15; // MFMA row/col index supplied by this lane
     const int q    = lane >> 4; // K-slot group
 
@@ -319,6 +320,20 @@ __global__ __launch_bounds__(NW * 64)
     // with the upper-triangle mask, columns past the slab's last row are masked for every row of it
     const int n_end = (SOFTMAX && p.mask_upper && m0 + Cfg::BM < p.N) ? m0 + Cfg::BM : p.N;
 
+    // A step with masked columns for any row of this wave runs the EDGE form of the step (wave-uniform). Only the form without
+    // compares and guards is straight-line code, and a wave has one EDGE step; there the 32-column pairs past the wave's last
+    // unmasked column are left out. 32 x 2048 x 2048 x 128 with softmax 147.0 -> 138.4 us, causal 56.0 -> 53.6; 100 x 1000 x 1500
+    // x 80 97.0 -> 93.7; causal 200 x 300 x 300 x 128 27.0 -> 26.0; without softmax 64 x 512 x 512 x 64 7.9 -> 7.5.
+    // RAISE: MFMA sections at raised wave priority, so that the other wave of the SIMD does its softmax meanwhile: with K of 33
+    // to 64 355.8 -> 348.3 us at 64 x 4096 x 4096 x 64 (without the two forms 351.9 -> 344.6); slower with K of 128
+    // (147 -> 153) and 32 (72.1 -> 73.0) and without softmax (128 x 1024 x 1024 x 64 38.2 -> 39.2).
+    constexpr bool RAISE = SOFTMAX && KS == 2;
+    const int wave_m0    = m0 + wave * 16 * MT;
+    const int wave_n_end = (p.mask_upper && wave_m0 + 16 * MT < p.N) ? wave_m0 + 16 * MT : p.N;
+    const int full_end   = (p.mask_upper && wave_m0 + 1 < p.N) ? wave_m0 + 1 : p.N;
+    auto edge_step       = [&](int n0) { return n0 + Cfg::BNC > full_end; };
+    auto pairs_of        = [&](int n0) { return (wave_n_end - n0 + 31) >> 5; };
+
     // ---- main loop over the steps ---------------------------------------------------------------------------
     // A step's MFMAs take well under a microsecond, a load out of HBM longer: with one step of register prefetch
     // every step of a short problem (N = 512: four steps) ends waiting for its successor's slices. Where the
@@ -334,7 +349,18 @@ __global__ __launch_bounds__(NW * 64)
             __syncthreads();
             if(n0 + Cfg::BNC < n_end)
                 load_step(n0 + Cfg::BNC); // in flight while this step is multiplied
+                if(SOFTMAX && edge_step(n0))
+                {
+                    constexpr bool EDGE  = SOFTMAX;
+                    const int edge_pairs = pairs_of(n0);
 #include "gemm_gemm_step.inc"
+                }
+                else
+                {
+                    constexpr bool EDGE  = false;
+                    constexpr int edge_pairs = 4;
+#include "gemm_gemm_step.inc"
+                }
         }
     }
     else
@@ -351,7 +377,18 @@ __global__ __launch_bounds__(NW * 64)
                 __syncthreads();
                 if(n0 + 2 * Cfg::BNC < n_end)
                     load_into(n0 + 2 * Cfg::BNC, rb0, rb1);
+                if(SOFTMAX && edge_step(n0))
+                {
+                    constexpr bool EDGE  = SOFTMAX;
+                    const int edge_pairs = pairs_of(n0);
 #include "gemm_gemm_step.inc"
+                }
+                else
+                {
+                    constexpr bool EDGE  = false;
+                    constexpr int edge_pairs = 4;
+#include "gemm_gemm_step.inc"
+                }
             }
             if(nb + Cfg::BNC < n_end)
             {
@@ -361,7 +398,18 @@ __global__ __launch_bounds__(NW * 64)
                 __syncthreads();
                 if(n0 + 2 * Cfg::BNC < n_end)
                     load_into(n0 + 2 * Cfg::BNC, rb0b, rb1b);
+                if(SOFTMAX && edge_step(n0))
+                {
+                    constexpr bool EDGE  = SOFTMAX;
+                    const int edge_pairs = pairs_of(n0);
 #include "gemm_gemm_step.inc"
+                }
+                else
+                {
+                    constexpr bool EDGE  = false;
+                    constexpr int edge_pairs = 4;
+#include "gemm_gemm_step.inc"
+                }
             }
         }
     }

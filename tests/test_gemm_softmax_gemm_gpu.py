@@ -86,6 +86,18 @@ def test_gemm_softmax_gemm_masked_slab_order(G, M, N):
                lit.batched_gemm_softmax_gemm_f16(a, b0_gnk.transpose(0, 2, 1), b1, 0.25, True))
 
 
+@pytest.mark.parametrize("N", [1, 31, 32, 33, 64, 65, 96, 97, 127, 129, 160, 225, 256])
+@pytest.mark.parametrize("K", [32, 64, 128])
+def test_gemm_softmax_gemm_edge_pairs(N, K):
+    """Steps with masked columns multiply only the 32-column pairs that hold an unmasked one: N around the pairs' edges, rows
+    above, on and below the diagonal of every wave."""
+    a, b0_gnk, b1 = (uniform_f16((2, x, K), -1, 1, 1960 + i) for i, x in enumerate((161, N, N)))
+    for mask in (False, True):
+        ref = lit.batched_gemm_softmax_gemm_f16(a, b0_gnk.transpose(0, 2, 1), b1, 0.3, mask)
+        for instance in (0, 1, 2):
+            _close(_run(a, b0_gnk, b1, 0.3, mask, instance), ref)
+
+
 def test_gemm_softmax_gemm_closed_forms():
     """Zero scores: the uniform distribution, C = mean of B1's rows (exact: small integers over a power of
     two). Upper-triangle mask: row m averages rows 0..m, row 0 is B1[0] exactly. A dominant score selects
