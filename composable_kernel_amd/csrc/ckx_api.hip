@@ -270,7 +270,11 @@ Plan make_plan(long M, int N, int kbytes, int only_tile, long workspace_bytes, i
             // 128 x 64 tiles at three per CU were rated 43 us on fp16 512 x 11008 x 4096 and took 60 (256 x 128: 48).
             // (GEMM launches only: an im2col A operand re-reads its pixels out of L1 / L2 tap after tap, and with the term
             // the 3-D layer 4 x 28^3 x 64 -> 256, stride 2, went from the 64 x 64 tile, 24.7 us, to 256 x 64 at 35.9)
-            if(per_cu >= 3 && !conv)
+            // (two four-stage 64 x 64 workgroups per CU on a long K without a split are bound by it as well: fp16 1222 x 960 x 8288
+            // was rated 44 us and took 63, bf16 1100 x 1088 x 10000 52 and 87; 45 and 54 on the 128 x 64 tile with three K runs.
+            // Up to 94 K tiles that tile stays the best or within 4 % of it, with or without the term: 1024 x 1280 x 4096
+            // 25.4 against 33.1, 512 x 4000 x 5120 37.6 against 42.0, 700 x 2896 x 6000 55.7 against 54.0)
+            if((per_cu >= 3 || (per_cu == 2 && nst > 2 && nk_per >= 128 && !kmajor)) && !conv)
             {
                 const double load_us = per_cu * (double)(t.bm + t.bn) * 128.0 / 85.0e3;
                 iter_us              = iter_us < load_us ? load_us : iter_us;

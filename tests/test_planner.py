@@ -86,3 +86,12 @@ def test_plan_queries_validate_like_the_launchers():
         assert capi.gemm_plan(capi.OP_GEMM_I8, 256, 256, 4096, workspace_bytes=WORKSPACE)[1] == 3
     finally:
         assert L.ckx_set_forced_k_runs(0) == 3
+
+
+def test_long_k_leaves_the_four_stage_64x64_tile():
+    """Two of its workgroups on a CU are bound by their operand bytes from 128 K tiles on (both sides measured: ckx_api.hip)."""
+    def plan(op, M, N, K):
+        return capi.gemm_plan(op, M, N, K, workspace_bytes=WORKSPACE)
+    assert plan(capi.OP_GEMM_F16, 1222, 960, 8288) == (3, 3)
+    assert plan(capi.OP_GEMM_F16, 1222, 960, 8128)[0] == 8    # 127 K tiles
+    assert plan(capi.OP_GEMM_F16, 1024, 1280, 4096) == (8, 1)
