@@ -161,9 +161,13 @@ struct GemmGemmCfg
 
 template <int KS, int OG, int MT, int NW, bool SOFTMAX = false>
 // (the 32-row-per-wave softmax variant for small K and O is held to 256 registers, two waves per SIMD: one
-// wave's exponentials then overlap the other's MFMAs; left alone the compiler takes 340 and runs one)
+// wave's exponentials then overlap the other's MFMAs; left alone the compiler takes 340 and runs one. The 8-wave variant for
+// K up to 32 is held to 128, two workgroups per CU)
 __global__ __launch_bounds__(NW * 64)
-    __attribute__((amdgpu_waves_per_eu(SOFTMAX && MT == 2 && KS <= 2 && OG == 1 ? 2 : 1))) void gemm_gemm_kernel(
+    __attribute__((amdgpu_waves_per_eu(!SOFTMAX || OG != 1   ? 1
+                                       : MT == 2 && KS <= 2 ? 2
+                                       : NW == 8 && KS == 1 ? 4
+                                                            : 1))) void gemm_gemm_kernel(
         const GemmGemmArgs p)
 {
     using Cfg = GemmGemmCfg<KS, OG, MT, NW>;
@@ -328,6 +332,10 @@ __global__ __launch_bounds__(NW * 64)
     // to 64 355.8 -> 348.3 us at 64 x 4096 x 4096 x 64 (without the two forms 351.9 -> 344.6); slower with K of 128
     // (147 -> 153) and 32 (72.1 -> 73.0) and without softmax (128 x 1024 x 1024 x 64 38.2 -> 39.2).
     constexpr bool RAISE = SOFTMAX && KS == 2;
+    // One form, with the compares behind a branch, where the second one's registers cost a co-resident workgroup: 8 waves with
+    // K up to 32 and O up to 64 (122 registers, 150 with two forms: 200 x 500 x 500 x 32 24.4 -> 32.7 us, 256 x 2000 x 300 x 32 69 ->
+    // 93) and the 64-row instances.
+    constexpr bool TWO_FORMS = SOFTMAX && (NW == 8 ? !(KS == 1 && OG == 1) : MT == 2);
     const int wave_m0    = m0 + wave * 16 * MT;
     const int wave_n_end = (p.mask_upper && wave_m0 + 16 * MT < p.N) ? wave_m0 + 16 * MT : p.N;
     const int full_end   = (p.mask_upper && wave_m0 + 1 < p.N) ? wave_m0 + 1 : p.N;
@@ -349,9 +357,9 @@ __global__ __launch_bounds__(NW * 64)
             __syncthreads();
             if(n0 + Cfg::BNC < n_end)
                 load_step(n0 + Cfg::BNC); // in flight while this step is multiplied
-                if(SOFTMAX && edge_step(n0))
+                if(TWO_FORMS && edge_step(n0))
                 {
-                    constexpr bool EDGE  = SOFTMAX;
+                    constexpr bool EDGE  = TWO_FORMS;
                     const int edge_pairs = pairs_of(n0);
 #include "gemm_gemm_step.inc"
                 }
@@ -377,9 +385,9 @@ __global__ __launch_bounds__(NW * 64)
                 __syncthreads();
                 if(n0 + 2 * Cfg::BNC < n_end)
                     load_into(n0 + 2 * Cfg::BNC, rb0, rb1);
-                if(SOFTMAX && edge_step(n0))
+                if(TWO_FORMS && edge_step(n0))
                 {
-                    constexpr bool EDGE  = SOFTMAX;
+                    constexpr bool EDGE  = TWO_FORMS;
                     const int edge_pairs = pairs_of(n0);
 #include "gemm_gemm_step.inc"
                 }
@@ -398,9 +406,9 @@ __global__ __launch_bounds__(NW * 64)
                 __syncthreads();
                 if(n0 + 2 * Cfg::BNC < n_end)
                     load_into(n0 + 2 * Cfg::BNC, rb0b, rb1b);
-                if(SOFTMAX && edge_step(n0))
+                if(TWO_FORMS && edge_step(n0))
                 {
-                    constexpr bool EDGE  = SOFTMAX;
+                    constexpr bool EDGE  = TWO_FORMS;
                     const int edge_pairs = pairs_of(n0);
 #include "gemm_gemm_step.inc"
                 }
