@@ -2,8 +2,6 @@
 // compile beside the others).
 #include "gemm_ragged.hpp"
 
-#include "tile_launch.hpp"
-
 namespace ckx {
 
 template <int DT, int B, bool TA, bool TB>
@@ -13,7 +11,7 @@ static hipError_t launch_one(GemmArgs a, hipStream_t s)
     const long blocks = (long)a.tiles_m * a.tiles_n * (a.batch > 1 ? a.batch : 1);
     if(blocks >= (1l << 31))
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemm_ragged_kernel<DT, B, B, TA, TB>), dim3((unsigned)blocks), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((gemm_ragged_kernel<DT, B, B, TA, TB>), linear_grid(blocks), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

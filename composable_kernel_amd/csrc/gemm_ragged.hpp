@@ -28,6 +28,7 @@
 #pragma once
 
 #include "gemm_tile.hpp"
+#include "tile_launch.hpp"
 
 namespace ckx {
 
@@ -209,7 +210,9 @@ __global__ __launch_bounds__(256, 2) void gemm_ragged_kernel(const GemmArgs p)
     const int wm = wave >> 1, wn = wave & 1;
     const uint32_t frow = lane & 15, fq = lane >> 4;
     int g, tm, tn;
-    tile_of_block((int)blockIdx.x, p.tiles_m, p.tiles_n, p.batch > 1 ? p.batch : 1, g, tm, tn);
+    if(linear_block() >= (uint32_t)p.tiles_m * p.tiles_n * (p.batch > 1 ? p.batch : 1))
+        return;
+    tile_of_block((int)linear_block(), p.tiles_m, p.tiles_n, p.batch > 1 ? p.batch : 1, g, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
     const uint8_t* A = reinterpret_cast<const uint8_t*>(p.a) + (int64_t)g * p.bsa * ES;
     const uint8_t* B = reinterpret_cast<const uint8_t*>(p.b) + (int64_t)g * p.bsb * ES;

@@ -62,3 +62,20 @@ def test_k_around_the_k_tiles(kind, layout):
 def test_tile_edges(kind, layout, shape):
     _run(kind, layout, *shape, off=0)
     _run(kind, layout, *shape, off=3)
+
+
+def test_batches_past_one_launch_dimension():
+    """More than 2^24 workgroups of 256 threads in one launch: the threads along a grid dimension are counted in 32 bits."""
+    import torch
+    import gpu_util
+    G, N = 65281, 32769
+    g = torch.Generator(device="cuda").manual_seed(5)
+    a, b = (torch.randint(-9, 10, (n,), generator=g, device="cuda").to(torch.int8) for n in (G, N))
+    c = torch.full((G, N), 77, dtype=torch.int8, device="cuda")
+    op = ck.DeviceBatchedGemmInt8()
+    arg = op.MakeArgumentPointer(a, b, c, 1, N, 1, 1, 1, N, 1, 0, N, G)
+    assert op.IsSupportedArgument(arg), capi.last_error()
+    op.MakeInvokerPointer().Run(arg, ck.StreamConfig(gpu_util.stream()))
+    torch.cuda.synchronize()
+    for i in range(0, G, 8192):
+        assert torch.equal(c[i:i + 8192], a[i:i + 8192, None] * b[None, :]), f"batches from {i} on differ"
