@@ -23,7 +23,7 @@
 // 2623 -> 197, 122 x 1283 x 3001 148 -> 17.4, 2049 x 2047 x 2047 with a K-major A 290 -> 55; int8 4001 x 4003 x 4095 3019 -> 118,
 // 40 x 333 x 3999 156 -> 16; bf16 3000 x 2999 x 1001 275 -> 47; one tile (32 x 33 x 65) 5.7, as before.
 //
-// Two tiles: 128 x 128 reads half the operand bytes per product, 64 x 64 gives four times the workgroups; launch_ragged() says
+// Two tiles: 128 x 128 reads half the operand bytes per product, 64 x 64 gives four times the workgroups; ragged_tile() says
 // where the line lies.
 #pragma once
 
@@ -376,6 +376,8 @@ __global__ __launch_bounds__(256, 2) void gemm_ragged_kernel(const GemmArgs p)
     }
 }
 
+// rows and columns of the C tile a problem runs on: 128 or 64
+int ragged_tile(int M, int N, int batch);
 // ta / tb: the operand is K-major. tiles_m / tiles_n are set here.
 hipError_t launch_ragged(int dt, bool ta, bool tb, GemmArgs a, hipStream_t s);
 

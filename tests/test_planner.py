@@ -95,3 +95,11 @@ def test_long_k_leaves_the_four_stage_64x64_tile():
     assert plan(capi.OP_GEMM_F16, 1222, 960, 8288) == (3, 3)
     assert plan(capi.OP_GEMM_F16, 1222, 960, 8128)[0] == 8    # 127 K tiles
     assert plan(capi.OP_GEMM_F16, 1024, 1280, 4096) == (8, 1)
+
+
+def test_ragged_tile_covers_little_padding():
+    """128 x 128 tiles of the ragged GEMM: from 256 of them on, and only where they cover at most a fifth more than 64 x 64 ones."""
+    tile = capi.lib()._ZN3ckx11ragged_tileEiii
+    assert tile(4001, 4003, 1) == 128 and tile(1000, 4001, 1) == 128 and tile(2001, 1003, 1) == 64
+    assert [tile(m, n, 20000) for m, n in ((3, 5), (33, 35), (64, 64), (65, 64), (129, 131), (150, 500), (300, 300))] == [64] * 7
+    assert [tile(m, n, 300) for m, n in ((128, 128), (200, 200), (449, 449), (700, 321))] == [128] * 4
