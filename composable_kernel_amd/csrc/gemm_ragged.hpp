@@ -110,6 +110,15 @@ struct RaggedOperand
         for(int i = 0; i < NCH; ++i)
             v[i] = load_vec<i32x4>(src + off[i]);
     }
+    // Row and chunk of slot idx of a checked K tile. across: an operand that is read element by element; int8 (16 loads a
+    // chunk) then has the rows across the lanes, so that the chunks past K are whole waves', which skip them: 147 x 869 x 15 5.7
+    // -> 5.0 us, 3621 x 2 x 7 4.8 -> 4.2. In 16 bits (8 loads) it costs as much as it saves: 20000 x (3 x 5 x 7) 45.0 -> 47.7.
+    __device__ static __forceinline__ void slot(int idx, bool across, int& r, int& c)
+    {
+        across = across && !KM && ES == 1;
+        r      = across ? idx % BX : idx / CPR;
+        c      = across ? idx / BX : idx % CPR;
+    }
     // K tile `kt` with every bound checked; vec: at least one vector in the contiguous direction
     __device__ __forceinline__ void load_checked(const uint8_t* base, int kt, int tid, int x0, int X, int K, int ld, bool vec,
                                                  i32x4 (&v)[NCH]) const
@@ -118,7 +127,8 @@ struct RaggedOperand
 #pragma unroll
         for(int i = 0; i < NCH; ++i)
         {
-            const int idx = tid + 256 * i, r = idx / CPR, c = idx % CPR;
+            int r, c;
+            slot(tid + 256 * i, !vec, r, c);
             // the chunk is elements [e0, e0 + EPC) of a contiguous line of `extent` elements
             const int line   = KM ? kt * KE + r : x0 + row_of(r);
             const int e0     = KM ? x0 + c * EPC : kt * KE + c * EPC;
@@ -142,12 +152,14 @@ struct RaggedOperand
             }
         }
     }
-    __device__ __forceinline__ void store_lds(uint8_t* s, int tid, const i32x4 (&v)[NCH]) const
+    __device__ __forceinline__ void store_lds(uint8_t* s, int tid, const i32x4 (&v)[NCH], bool across = false) const
     {
 #pragma unroll
         for(int i = 0; i < NCH; ++i)
         {
-            const uint32_t idx = (uint32_t)(tid + 256 * i), r = idx / CPR, c = idx % CPR;
+            int ri, ci;
+            slot(tid + 256 * i, across, ri, ci);
+            const uint32_t r = (uint32_t)ri, c = (uint32_t)ci;
             uint32_t at;
             if constexpr(KM)
                 at = r * (BX * ES) + ((((c * EPC) >> 4) ^ tswz(r)) << SEGSH) + (ES == 2 ? (c & 1u) << 4 : 0u);
@@ -234,10 +246,12 @@ __global__ __launch_bounds__(256, 2) void gemm_ragged_kernel(const GemmArgs p)
         for(int t = 0; t < NTL; ++t)
             acc[i][t] = acc_t{0, 0, 0, 0};
 
-    auto multiply = [&](const uint8_t* s) {
+    auto multiply = [&](const uint8_t* s, int ksteps) {
 #pragma unroll
         for(int ks = 0; ks < 2; ++ks)
         {
+            if(ks >= ksteps)
+                break;
             i32x4 af[MT], bf[NTL];
 #pragma unroll
             for(int t = 0; t < NTL; ++t)
@@ -264,17 +278,17 @@ __global__ __launch_bounds__(256, 2) void gemm_ragged_kernel(const GemmArgs p)
     i32x4 ra0[OpA::NCH], rb0[OpB::NCH], ra1[OpA::NCH], rb1[OpB::NCH];
     // registers -> stage, the next load into the freed registers, multiply. One barrier per K tile: a stage is written
     // again only after the barrier of the tile in between, which every wave passes when it is done reading.
-    auto step = [&](int stage, i32x4(&ra)[OpA::NCH], i32x4(&rb)[OpB::NCH], int next) {
+    auto step = [&](int stage, i32x4(&ra)[OpA::NCH], i32x4(&rb)[OpB::NCH], int next, int ksteps = 2, bool across_a = false, bool across_b = false) {
         uint8_t* s = smem + stage * STAGE;
-        opa.store_lds(s, tid, ra);
-        opb.store_lds(s + OpA::BYTES, tid, rb);
+        opa.store_lds(s, tid, ra, across_a);
+        opb.store_lds(s + OpA::BYTES, tid, rb, across_b);
         if(next >= 0)
         {
             opa.load(A, next, ra);
             opb.load(B, next, rb);
         }
         __syncthreads();
-        multiply(s);
+        multiply(s, ksteps);
     };
 
     // the checked K tiles: the last one, or all of them; the first unchecked ones are in flight meanwhile
@@ -291,7 +305,8 @@ __global__ __launch_bounds__(256, 2) void gemm_ragged_kernel(const GemmArgs p)
         i32x4 ra[OpA::NCH], rb[OpB::NCH];
         opa.load_checked(A, kt, tid, m0, p.M, p.K, p.lda, vec_a, ra);
         opb.load_checked(B, kt, tid, n0, p.N, p.K, p.ldb, vec_b, rb);
-        step((nk - 1 - kt) & 1 ? 0 : 1, ra, rb, -1); // (stages alternate, the last checked tile in stage 1)
+        // (stages alternate, the last checked tile in stage 1; a second k-step past K is left out)
+        step((nk - 1 - kt) & 1 ? 0 : 1, ra, rb, -1, p.K - kt * KE <= KE / 2 ? 1 : 2, !vec_a, !vec_b);
     }
     if(nfull > 0)
     {

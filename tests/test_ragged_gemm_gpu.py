@@ -79,3 +79,14 @@ def test_batches_past_one_launch_dimension():
     torch.cuda.synchronize()
     for i in range(0, G, 8192):
         assert torch.equal(c[i:i + 8192], a[i:i + 8192, None] * b[None, :]), f"batches from {i} on differ"
+
+
+@pytest.mark.parametrize("kind", ["i8", "f16", "bf16"])
+@pytest.mark.parametrize("K", [1, 7, 15, 31, 33, 63, 65])
+def test_k_below_one_vector_and_half_a_k_tile(kind, K):
+    """Rows of less than one vector are read element by element (int8 with another order of the slots), and a second k-step past
+    K is left out, in C tiles of full, partial and single rows."""
+    for M, N in ((147, 869), (64, 65), (1, 63), (130, 3)):
+        _run(kind, "mk_nk", M, N, K, off=1)
+        _run(kind, "km_nk", M, N, K, off=0)
+        _run(kind, "mk_kn", M, N, K, off=1)
