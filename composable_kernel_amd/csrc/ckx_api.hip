@@ -952,13 +952,13 @@ int run_conv(int op, const void* in, const void* wei, void* out, const ckx_conv2
         std::memset(&f, 0, sizeof(f));
         f.N = d->N, f.Hi = d->Hi, f.Wi = d->Wi, f.C = d->C, f.Ho = d->Ho, f.Wo = d->Wo, f.K = d->K, f.X = d->X;
         f.sH = d->stride_h, f.sW = d->stride_w, f.dH = d->dilation_h, f.dW = d->dilation_w, f.pT = d->pad_top, f.pL = d->pad_left;
+        f.epi = epi, f.scale_gemm = sg, f.scale_relu = sr;
         const int dt = es == 1 ? ckx::DT_I8 : ckx::DT_F16;
         if(dops.ldd0 == 0 && ckx::plan_conv_few(dt, f, d->Y))
         {
             f.in = in, f.wei = wei, f.out = out;
             f.d0 = dops.d0, f.d1 = uses_d1(epi) ? dops.d1 : nullptr, f.ldd1 = dops.ldd1;
             f.div_pc = make_magic((uint32_t)f.PC), f.div_tw = make_magic((uint32_t)f.TW);
-            f.epi = epi, f.scale_gemm = sg, f.scale_relu = sr;
             f.nt_store   = es == 1 && (long)M * N * es >= stream_output_bytes();
             hipError_t e = ckx::launch_conv_few(dt, f, (hipStream_t)stream);
             return e == hipSuccess ? CKX_OK : hip_fail(e, kGenericName);

@@ -4,6 +4,7 @@
 #include "tile_launch.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 
 namespace ckx {
@@ -96,7 +97,28 @@ bool plan_conv_few(int dt, ConvFewArgs& a, int filter_h)
     if(units >= (1l << 31) - 65536)
         return false;
     a.units  = (int)units;
-    return true;
+    // Refused where the element-by-element gather (gemm_generic.hpp) is rated faster: few output pixels for many weights to lay out
+    // in every workgroup, or a patch of many more pixels than it multiplies (a stride or a dilation past the filter). Both times in
+    // us, fitted to 1458 layers (C 1 ... 8, K 1 ... 1000, filters 1 ... 11, strides to 16, dilations to 45, with and without D
+    // operands) timed on both kernels, with an rms error of 14 and 22 %. int8 2 x 10^2, C 3 -> K 1000, 3 x 3 stride 8: 27.8 us
+    // here, 5.8 gathered; fp16 1 x 78^2, C 2 -> K 64, 3 x 3 dilation 20: 16.5 and 5.4; fp16 52 x 10^2, C 7 -> K 1000, 2 x 2:
+    // 38.8 and 13.9. 289 of them were more than 3 % slower here than gathered, at worst 5.3 times; with this line 66 are, at worst
+    // 1.6 times, and 5 that are faster here, at worst 1.27 times, are refused.
+    const int mt       = nt == 4 ? 2 : 4;
+    const long lds     = fixed + ((long)a.patch_pixels * px + 15) / 16 * 16, per_cu = std::min(4l, kLdsCu / lds);
+    const long slots   = std::max(1l, num_cus() * per_cu / groups), per_wg = (units + slots - 1) / slots;
+    const long rounds  = std::max(1l, (groups + num_cus() * per_cu - 1) / (num_cus() * per_cu));
+    const double here  = std::max(1.0, std::min((double)per_cu, (double)(std::min(units, slots) * groups) / num_cus()));
+    const int d_ops    = a.epi == EPI_ADD_RELU_ADD ? 2 : a.epi >= EPI_ADD_RELU ? 1 : 0;
+    const double lay   = 0.045 * a.nks * a.kblocks * nt * 64 / 256 * (16 / es);
+    const long turns   = ((long)a.R * a.TW + 64 * mt - 1) / (64 * mt);
+    const double patch = turns * a.kblocks * (0.024 * mt * nt * a.nks + 0.83 + 0.13 * d_ops) + 0.12 * a.patch_pixels / 256;
+    const double few_us = 2.5 + rounds * std::pow(here, 2.0 / 3) * (lay + per_wg * patch);
+    const double waves  = (double)(((long)a.N * a.Ho * a.Wo + 63) / 64) * ((a.K + 63) / 64) / (2.0 * num_cus());
+    const int ksteps    = (int)(((long)a.taps * a.C * es + 63) / 64);
+    const double gather_us = 2.3 + (ksteps * (es == 1 ? 2.9 : 1.5) + 0.9 + (d_ops ? 1.2 + 0.4 * d_ops : 0.0)) *
+                                       std::max(1.0, waves > 3.0 ? waves : std::ceil(waves));
+    return groups <= 65535 && few_us <= 1.3 * gather_us;
 }
 
 hipError_t launch_conv_few(int dt, const ConvFewArgs& a, hipStream_t s)

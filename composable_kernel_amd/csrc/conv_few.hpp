@@ -310,8 +310,9 @@ __global__ __launch_bounds__(256, 4) void conv_few_kernel(const ConvFewArgs p)
     ConvFew<DT, CP, NT>::run(p, ckx_smem);
 }
 
-// (conv_few.hip) Fills the tiling of `a`, div_pc and div_tw apart, whose problem is set: false if it is not one of few channels
-// (a pixel of less than 16 bytes, at most 8 channels) or the filter or its reach does not fit the LDS.
+// (conv_few.hip) Fills the tiling of `a`, div_pc and div_tw apart, whose problem and epilogue are set: false if it is not one of few channels
+// (a pixel of less than 16 bytes, at most 8 channels), the filter or its reach does not fit the LDS, or the gather is
+// rated faster on it.
 bool plan_conv_few(int dt, ConvFewArgs& a, int filter_h);
 hipError_t launch_conv_few(int dt, const ConvFewArgs& a, hipStream_t s);
 

@@ -92,3 +92,18 @@ def test_an_infinite_pixel_stays_in_its_windows(f):
     hit[0, 10 - f // 2:11 + f // 2, 12 - f // 2:13 + f // 2] = True
     assert np.all(np.isposinf(out[hit]))
     np.testing.assert_array_equal(out[~hit], clean[~hit])
+
+
+@pytest.mark.parametrize("dtype", ["i8", "f16"])
+@pytest.mark.parametrize("layer", [(8, 90, 50, 49, 5, 3, (1, 1), (1, 1), (1, 1)), (8, 257, 60, 60, 3, 5, (1, 1), (2, 2), (1, 1)),
+                                   (6, 600, 30, 31, 7, 7, (1, 1), (1, 1), (3, 3)), (2, 1000, 10, 10, 3, 3, (8, 8), (1, 1), (0, 0))])
+def test_several_channel_blocks(dtype, layer):
+    """Output channels of more than one block with enough pixels for the few-channel kernel; the last layer is one of too few
+    pixels, which the gather takes."""
+    import gpu_util
+    from conv_few_plan import takes
+    N, K, H, W, C, f, s, d, p = layer
+    assert takes(dtype, N, H, W, C, K, f, f, s, d, p)[0] == (K != 1000)
+    inp, wei = _ints((N, H, W, C), K, dtype), _ints((K, f, f, C), K + 1, dtype)
+    out = gpu_util.conv2d_fwd(inp, wei, s, d, p)
+    np.testing.assert_array_equal(out, (fast.conv2d_fwd_i8 if dtype == "i8" else fast.conv2d_fwd_f16)(inp, wei, s, d, p))

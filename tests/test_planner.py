@@ -103,3 +103,18 @@ def test_ragged_tile_covers_little_padding():
     assert tile(4001, 4003, 1) == 128 and tile(1000, 4001, 1) == 128 and tile(2001, 1003, 1) == 64
     assert [tile(m, n, 20000) for m, n in ((3, 5), (33, 35), (64, 64), (65, 64), (129, 131), (150, 500), (300, 300))] == [64] * 7
     assert [tile(m, n, 300) for m, n in ((128, 128), (200, 200), (449, 449), (700, 321))] == [128] * 4
+
+
+def test_few_channel_layers_that_the_gather_is_faster_on():
+    """First layers run on the few-channel conv kernel; few output pixels for many channels, or a patch of many more pixels than
+    are multiplied, on the element-by-element gather (both sides measured: csrc/conv_few.hip)."""
+    from conv_few_plan import takes
+    for dtype in ("i8", "f16"):
+        assert takes(dtype, 64, 224, 224, 3, 32, 3, 3, (2, 2), (1, 1), (1, 1))[0]
+        assert takes(dtype, 16, 200, 200, 6, 96, 7, 7, (1, 1), (1, 1), (3, 3))[0]
+        assert takes(dtype, 1, 28, 28, 1, 16, 3, 3, (1, 1), (1, 1), (1, 1))[0]
+    assert not takes("i8", 2, 10, 10, 3, 1000, 3, 3, (8, 8))[0]
+    assert not takes("f16", 52, 10, 10, 7, 1000, 2, 2)[0]
+    assert not takes("f16", 1, 78, 78, 2, 64, 3, 3, (2, 2), (20, 20), (20, 20))[0]
+    assert not takes("i8", 11, 140, 140, 1, 8, 2, 2, (4, 4), (45, 45), (22, 22))[0]
+    assert not takes("i8", 3, 188, 188, 8, 256, 5, 5, (8, 8), (2, 2))[0]
