@@ -222,12 +222,8 @@ int splitk_runs(int kbytes, int k_batch)
 // 128 x 64 one by 10 - 17 % (ResNet-like layers at N = 32 and 256), which the GEMM-calibrated figures did not say; the
 // 1 x 1 layers of the same networks follow the GEMM figures (256 x 64 rated up sent C 256 -> K 128 at 56 x 56 to it, 20 %
 // behind the 256 x 128 tile)
-// d_epilogue: a conv launch with D operands (bias / residual). On K loops of a few tiles the 128 x 128 instance -- two
-// co-resident workgroups of one wave per SIMD, each held at the epilogue's wait for its D values with nobody to cover
-// for it -- measured 30 - 100 % behind its plain self (C 256 -> K 128, 1x1, 56 x 56, N = 256: 169 us against 128; the
-// 256 x 128 instance 132 against 127), so it is left out there.
 Plan make_plan(long M, int N, int kbytes, int only_tile, long workspace_bytes, int k_batch = 0, bool kmajor = false,
-               bool conv = false, int taps = 2, bool d_epilogue = false)
+               bool conv = false, int taps = 2)
 {
     Plan best;
     double best_us  = 1e30;
@@ -240,8 +236,6 @@ Plan make_plan(long M, int N, int kbytes, int only_tile, long workspace_bytes, i
             continue;
         const TileInstance& t = kTiles[i];
         if(kmajor && t.bm < 64)
-            continue;
-        if(conv && d_epilogue && only_tile < 0 && t.bm == 128 && t.bn == 128 && nk <= 8)
             continue;
         const long tiles      = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
         for(int sp = 1; sp <= 8; ++sp)
@@ -1056,7 +1050,7 @@ int run_conv(int op, const void* in, const void* wei, void* out, const ckx_conv2
     if(conv_is_dense_gemm(op, d))
         return run_gemm(es == 1 ? ckx::DT_I8 : ckx::DT_F16, in, wei, out, M, N, K, K, K, N, CKX_ROW_MAJOR, CKX_COL_MAJOR,
                         CKX_ROW_MAJOR, epi, sg, sr, instance, ws, ws_bytes, stream, dops);
-    const Plan pl = make_plan(M, N, K * es, instance, ws ? ws_bytes : 0, 0, false, true, d->Y * d->X, f16_fused(epi));
+    const Plan pl = make_plan(M, N, K * es, instance, ws ? ws_bytes : 0, 0, false, true, d->Y * d->X);
     const TileInstance& t = kTiles[pl.tile];
     ckx::GemmArgs g;
     std::memset(&g, 0, sizeof(g));
@@ -1393,8 +1387,7 @@ int ckx_conv2d_fwd_plan(int op, const ckx_conv2d_desc* d, int epilogue, int64_t 
     else if(*instance == CKX_INSTANCE_AUTO || *instance < kNumTiles)
     {
         const Plan pl = make_plan((long)d->N * d->Ho * d->Wo, d->K, d->Y * d->X * d->C * es, *instance,
-                                  workspace_bytes > 0 ? workspace_bytes : 0, 0, false, true, d->Y * d->X,
-                                  f16_fused(epilogue));
+                                  workspace_bytes > 0 ? workspace_bytes : 0, 0, false, true, d->Y * d->X);
         *instance = pl.tile, *k_runs = pl.ksplit;
     }
     return CKX_OK;

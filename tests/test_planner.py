@@ -118,3 +118,13 @@ def test_few_channel_layers_that_the_gather_is_faster_on():
     assert not takes("f16", 1, 78, 78, 2, 64, 3, 3, (2, 2), (20, 20), (20, 20))[0]
     assert not takes("i8", 11, 140, 140, 1, 8, 2, 2, (4, 4), (45, 45), (22, 22))[0]
     assert not takes("i8", 3, 188, 188, 8, 256, 5, 5, (8, 8), (2, 2))[0]
+
+
+def test_short_conv_loops_with_d_operands_take_the_128x128_tile():
+    """1x1 stride-2 layers with a bias (and residual): the 128 x 128 instance, 2, measured 86.1 us against 106.5 on the 256 x 64
+    instance, 102.5 against 127.3 and 58.8 against 70.8, since its registers let two of its workgroups share a CU."""
+    for N, C, K, hw, epi in ((174, 56, 336, 67, capi.EPI_ADD_RELU_ADD), (180, 120, 368, 77, capi.EPI_ADD_RELU),
+                             (155, 64, 112, 107, capi.EPI_ADD_RELU_ADD)):
+        ho = (hw - 1) // 2 + 1
+        d = capi.Conv2dDesc(N, K, C, hw, hw, 1, 1, ho, ho, 2, 2, 1, 1, 0, 0, 0, 0)
+        assert capi.conv2d_fwd_plan(capi.OP_CONV2D_FWD_F16, d, epi, WORKSPACE) == (2, 1)
