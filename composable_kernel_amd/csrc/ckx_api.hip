@@ -264,16 +264,22 @@ Plan make_plan(long M, int N, int kbytes, int only_tile, long workspace_bytes, i
             // 128 x 64 tiles at three per CU were rated 43 us on fp16 512 x 11008 x 4096 and took 60 (256 x 128: 48).
             // (GEMM launches only: an im2col A operand re-reads its pixels out of L1 / L2 tap after tap, and with the term
             // the 3-D layer 4 x 28^3 x 64 -> 256, stride 2, went from the 64 x 64 tile, 24.7 us, to 256 x 64 at 35.9)
-            // (two four-stage 64 x 64 workgroups per CU on a long K without a split are bound by it as well: fp16 1222 x 960 x 8288
-            // was rated 44 us and took 63, bf16 1100 x 1088 x 10000 52 and 87; 45 and 54 on the 128 x 64 tile with three K runs.
-            // Up to 94 K tiles that tile stays the best or within 4 % of it, with or without the term: 1024 x 1280 x 4096
-            // 25.4 against 33.1, 512 x 4000 x 5120 37.6 against 42.0, 700 x 2896 x 6000 55.7 against 54.0)
-            if((per_cu >= 3 || (per_cu == 2 && nst > 2 && nk_per >= 128 && !kmajor)) && !conv)
+            if(per_cu >= 3 && !conv)
             {
                 const double load_us = per_cu * (double)(t.bm + t.bn) * 128.0 / 85.0e3;
                 iter_us              = iter_us < load_us ? load_us : iter_us;
             }
             double us      = rounds * (iter_us * nk_per + 6.0 / per_cu + 2.0);
+            // Two four-stage 64 x 64 workgroups per CU without a split: 3 us and their K tiles' bytes at 82 GB/s, which is above the
+            // estimate so far from 20 K tiles on. Measured over 257 ... 512 such tiles: 13 us at 24 K tiles, 16 ... 17 at 32, 25 ... 27
+            // at 64, 32 ... 37 at 80, 49 ... 57 at 127, 80 at 200; half as much again with K-major operands, which keep this rate as
+            // their other instances are slower too. fp16 1222 x 960 x 8288 63 -> 45 us (three K runs of 128 x 64 tiles), bf16 2266 x
+            // 488 x 6656 K-major B 48.2 -> 39.0, int8 2800 x 376 x 16256 52.0 -> 45.3; 1024 x 1280 x 4096 stays (25.4, next 33.1).
+            if(per_cu == 2 && nst > 2 && sp == 1 && !conv)
+            {
+                const double load_us = rounds * (per_cu * (double)(t.bm + t.bn) * 128.0 / 82.0e3 * nk_per + 3.0);
+                us                   = us < load_us ? load_us : us;
+            }
             // a single, partly filled round of one four-stage workgroup per CU: measured fixed cost ~4 us, not 8 (M = 64,
             // N = 11008, K = 4096 int8 on the four-stage 64 x 64 tile: 14.4 us = 3.8 + 0.33 per K tile; the 8 sent
             // such problems to one-wave tiles at 20 us)

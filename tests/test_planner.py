@@ -89,12 +89,18 @@ def test_plan_queries_validate_like_the_launchers():
 
 
 def test_long_k_leaves_the_four_stage_64x64_tile():
-    """Two of its workgroups on a CU are bound by their operand bytes from 128 K tiles on (both sides measured: ckx_api.hip)."""
-    def plan(op, M, N, K):
-        return capi.gemm_plan(op, M, N, K, workspace_bytes=WORKSPACE)
-    assert plan(capi.OP_GEMM_F16, 1222, 960, 8288) == (3, 3)
-    assert plan(capi.OP_GEMM_F16, 1222, 960, 8128)[0] == 8    # 127 K tiles
-    assert plan(capi.OP_GEMM_F16, 1024, 1280, 4096) == (8, 1)
+    """Two of its workgroups on a CU are bound by their operand bytes, more so the longer K is and K-major or not. us on that
+    instance, 8, and on the one chosen instead (3: 128 x 64 with three K runs), 1222 x 960 fp16: 64 K tiles 25.8 / 37.7, 110
+    42.1 / 35.6, 120 48.1 / 37.6, 127 51.8 / 42.2, 130 48.6 / 39.1 (80 to 100, where 8 is still chosen: 34.4 / 30.0, 38.9 / 34.3)."""
+    def plan(op, M, N, K, **kw):
+        return capi.gemm_plan(op, M, N, K, workspace_bytes=WORKSPACE, **kw)
+    assert [plan(capi.OP_GEMM_F16, 1222, 960, 64 * n) for n in (110, 120, 127, 130)] == [(3, 3)] * 4
+    assert [plan(capi.OP_GEMM_BF16, 1100, 1088, 64 * n) for n in (120, 127, 130)] == [(3, 3)] * 3    # 49.2 / 37.5, 53.1 / 43.2
+    assert plan(capi.OP_GEMM_F16, 1222, 960, 64 * 64) == (8, 1) and plan(capi.OP_GEMM_F16, 1024, 1280, 4096) == (8, 1)
+    assert plan(capi.OP_GEMM_I8, 700, 2896, 128 * 100) == (8, 1)                                     # 44.9 / 59.1
+    # K-major B: 368 x 2704 with 112 K tiles 59.3 / 46.3; 288 x 12208, both K-major, 147 K tiles 161 / 108 on 256 x 128
+    assert plan(capi.OP_GEMM_I8, 368, 2704, 128 * 112, b_layout=capi.ROW_MAJOR, sb=2704) == (3, 3)
+    assert plan(capi.OP_GEMM_F16, 288, 12208, 64 * 147, a_layout=capi.COL_MAJOR, sa=288, b_layout=capi.ROW_MAJOR, sb=12208) == (1, 1)
 
 
 def test_ragged_tile_covers_little_padding():
