@@ -294,6 +294,22 @@ __global__ __launch_bounds__(NW * 64)
     const uint32_t b1_lane =
         (uint32_t)(8 * q + (fr >> 2)) * Cfg::B1RS + ((uint32_t)(32 * (fr & 3)) ^ Cfg::b1_key((uint32_t)(8 * q + (fr >> 2))));
 
+    // byte offsets of this lane's B0 fragments of score tiles 0 and 1: rows 8 * (fr / 4) + fr % 4 and 4 more. Tile t is 32 * (t / 2)
+    // rows on, and neither step changes ab_key (bits 0, 1 and 3 of the row): immediates of the read. Worked out tile by tile
+    // they became eight address registers and, in some of the kernels, a slower order of the step: without softmax 45 x 32 x
+    // 1046 x 16 9.6 -> 11.3 us, 12 x 54 x 3073 x 32 22.6 -> 28.1. (Two registers in the plain 8-wave kernel for K up to 32, where
+    // one reads fewer fragments ahead: 231 x 45 x 2741 x 16 20.8 -> 20.0, 57 x 1934 x 61 x 32 7.3 -> 7.4, 7.7 with eight.)
+    uint32_t b0_lane[KS][2];
+#pragma unroll
+    for(int ks = 0; ks < KS; ++ks)
+    {
+        const uint32_t row = (uint32_t)(8 * (fr >> 2) + (fr & 3));
+        b0_lane[ks][0]     = row * Cfg::AST + ((uint32_t)(ks * 4 + q) ^ Cfg::ab_key(row)) * 16;
+        b0_lane[ks][1]     = b0_lane[ks][0] + 4 * Cfg::AST;
+        if constexpr(!SOFTMAX && NW == 8 && KS == 1)
+            asm volatile("" : "+v"(b0_lane[ks][1]));
+    }
+
     f32x4 acc1[MT][OG * 4];
 #pragma unroll
     for(int mt = 0; mt < MT; ++mt)

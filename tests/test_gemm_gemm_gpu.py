@@ -84,3 +84,26 @@ def test_gemm_gemm_unsupported():
     assert not op.IsSupportedArgument(arg)          # K > 128
     with pytest.raises(RuntimeError):
         op.MakeInvokerPointer().Run(arg)
+
+
+@pytest.mark.parametrize("K", [8, 32, 64, 128])
+@pytest.mark.parametrize("instance", [0, 1, 2])
+def test_columns_of_the_intermediate_in_order(K, instance):
+    """Every column of the intermediate meets its own row of B1: B0 is a scaled selection, so that the intermediate holds one value
+    of A per column, and B1's rows are all different. Small integers, exact in fp16: one misplaced fragment row shows."""
+    import torch
+    import gpu_util
+    M, N, O = 130, 300, 64
+    a = torch.randint(-2, 3, (1, M, K), device="cuda").half()
+    b0 = torch.zeros((1, N, K), device="cuda", dtype=torch.float16)
+    n = torch.arange(N, device="cuda")
+    b0[0, n, (n * 7 + n // K) % K] = (n % 3 - 1).half()
+    b1 = ((n[:, None] * 5 + torch.arange(O, device="cuda")[None, :] * 3) % 7 - 3).half()[None].contiguous()
+    c = torch.full((1, M, O), float("nan"), device="cuda", dtype=torch.float16)
+    op = ck.DeviceBatchedGemmGemmF16(instance)
+    arg = op.MakeArgumentPointer(a, b0, b1, c, M, N, K, O, 1, K, K, O, O, M * K, N * K, N * O, M * O)
+    assert op.IsSupportedArgument(arg)
+    op.MakeInvokerPointer().Run(arg, ck.StreamConfig(gpu_util.stream()))
+    torch.cuda.synchronize()
+    want = (a[0].double() @ b0[0].double().T) @ b1[0].double()  # |sums| <= 300 * 2 * 3: exact
+    assert torch.equal(c[0].double(), want)
