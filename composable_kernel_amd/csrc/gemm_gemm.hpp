@@ -159,15 +159,23 @@ struct GemmGemmCfg
     static_assert(NB0 >= 1 && NB1 >= 1, "too many threads for one step");
 };
 
+// Waves per SIMD that the registers are allocated for. The 32-row-per-wave softmax variant for small K and O is held to 256
+// registers, two waves per SIMD: one wave's exponentials then overlap the other's MFMAs; left alone the compiler takes 340 and
+// runs one. The 8-wave softmax variant for K up to 32 is held to 128, two workgroups per CU. The 8-wave variants past K or O of 64 take
+// more than 128 registers and a whole CU, two waves per SIMD, whatever they do: told so, the compiler spends up to 256 on reads
+// ahead instead of saving some for a third wave that no workgroup has. Without softmax K 64, O 128: 16 x 20 x 1000 17.2 -> 14.9
+// us, 60 x 300 x 256 8.0 -> 7.3; K 128, O 32 and K 32, O 128 0.88 and 0.94 of the time; with softmax level.
+constexpr int gemm_gemm_min_waves(int KS, int OG, int MT, int NW, bool SOFTMAX)
+{
+    if(NW == 8 && (KS == 4 || OG == 2))
+        return 2;
+    return !SOFTMAX || OG != 1 ? 1 : MT == 2 && KS <= 2 ? 2 : NW == 8 && KS == 1 ? 4 : 1;
+}
+constexpr int gemm_gemm_max_waves(int KS, int OG, int NW) { return NW == 8 && (KS == 4 || OG == 2) ? 2 : 8; }
+
 template <int KS, int OG, int MT, int NW, bool SOFTMAX = false>
-// (the 32-row-per-wave softmax variant for small K and O is held to 256 registers, two waves per SIMD: one
-// wave's exponentials then overlap the other's MFMAs; left alone the compiler takes 340 and runs one. The 8-wave variant for
-// K up to 32 is held to 128, two workgroups per CU)
 __global__ __launch_bounds__(NW * 64)
-    __attribute__((amdgpu_waves_per_eu(!SOFTMAX || OG != 1   ? 1
-                                       : MT == 2 && KS <= 2 ? 2
-                                       : NW == 8 && KS == 1 ? 4
-                                                            : 1))) void gemm_gemm_kernel(
+    __attribute__((amdgpu_waves_per_eu(gemm_gemm_min_waves(KS, OG, MT, NW, SOFTMAX), gemm_gemm_max_waves(KS, OG, NW)))) void gemm_gemm_kernel(
         const GemmGemmArgs p)
 {
     using Cfg = GemmGemmCfg<KS, OG, MT, NW>;
