@@ -85,22 +85,9 @@ long stream_output_bytes()
     return v;
 }
 
-ckx::MagicDiv make_magic(uint32_t d)
-{
-    // include/ck/utility/magic_division.hpp:28-54
-    uint32_t shift = 0;
-    while(shift < 32 && (1ull << shift) < d)
-        ++shift;
-    const uint64_t one = 1;
-    ckx::MagicDiv m;
-    m.mul   = (uint32_t)(((one << 32) * ((one << shift) - d)) / d + 1);
-    m.shift = shift;
-    m.d     = d;
-    return m;
-}
-
 // ------------------------------------------------------------ tile instances
 using ckx::launch_tile;
+using ckx::make_magic;
 using ckx::num_cus;
 using ckx::tile_launch_fn;
 

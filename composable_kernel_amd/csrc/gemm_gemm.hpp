@@ -33,6 +33,13 @@
 
 namespace ckx {
 
+// Order of a masked launch (slab_order()): batches go out in groups, the slabs of a group heaviest first.
+struct SlabOrder
+{
+    MagicDiv group, in_group, in_last; // by: workgroups of a group, batches of a group, batches of the last one
+    int groups;
+};
+
 struct GemmGemmArgs
 {
     const _Float16* a;
@@ -45,6 +52,7 @@ struct GemmGemmArgs
     int slabs; // ceil(M / rows per workgroup)
     float scale;   // softmax variant: scores are scale * (A * B0)
     int mask_upper; // softmax variant: scores with n > m are masked out
+    SlabOrder order; // masked launches only
 };
 
 // maximum / sum over the four lanes l, l^16, l^32, l^48 (every one of them gets the result)
@@ -78,27 +86,23 @@ __device__ __forceinline__ float quad_rows_max(float x)
 // (batch, slab of rows) of workgroup `bid`. Workgroups of one batch share B0[g] and B1[g]: they are kept on one XCD (ids are
 // dealt round-robin over 8 XCDs) where the batch count allows, so that those panels are fetched into one L2 only.
 // With the upper-triangle mask slab i has i + 1 times the work of slab 0, and the launch lasts until its last slab is
-// through: the slabs go out heaviest first, over groups of batches at once (batch by batch the heavy slabs of the last
-// batch started when the rest was done: half of the CUs idle for the last third). A group is 64 to 127 batches: 8
-// per XCD and up keep both of a CU's places filled to the end, and more would only widen what the L2s hold at a time.
-// Causal 64 x 4096 x 4096 x 64: 246.8 -> 202.8 us (550 -> 678 TFLOP/s counting the unmasked products).
-__host__ __device__ __forceinline__ void slab_of_block_masked(int bid, int slabs, int batch, int& g, int& slab)
+// through: the slabs go out heaviest first, over groups of batches at once, in the order that slab_order() lays out on the host
+// (three divisions of the kernel's own took 0.15 us of every launch: 2 x 55 x 55 x 32 3.6 -> 3.8).
+__device__ __forceinline__ void slab_of_block_masked(int bid, int slabs, const SlabOrder& o, int& g, int& slab)
 {
-    const int groups = batch >= 128 ? batch / 64 : 1;
-    int size         = (batch + groups - 1) / groups;
-    if((batch & 7) == 0)
-        size = (size + 7) & ~7; // (every group starts at XCD 0)
-    const int group = bid / (size * slabs), in = bid - group * size * slabs;
-    const int left  = batch - group * size, here = left < size ? left : size;
-    slab            = slabs - 1 - in / here;
-    g               = group * size + in % here;
+    const uint32_t group = magic_div((uint32_t)bid, o.group), in = (uint32_t)bid - group * o.group.d;
+    const bool last      = group == (uint32_t)o.groups - 1;
+    const MagicDiv here  = {last ? o.in_last.mul : o.in_group.mul, last ? o.in_last.shift : o.in_group.shift, last ? o.in_last.d : o.in_group.d};
+    const uint32_t up    = magic_div(in, here);
+    slab                 = slabs - 1 - (int)up;
+    g                    = (int)(group * o.in_group.d + in - up * here.d);
 }
 
 template <bool SOFTMAX>
 __device__ __forceinline__ void slab_of_block(int bid, const GemmGemmArgs& p, int& g, int& slab)
 {
     if(SOFTMAX && p.mask_upper)
-        slab_of_block_masked(bid, p.slabs, p.batch, g, slab);
+        slab_of_block_masked(bid, p.slabs, p.order, g, slab);
     else if((p.batch & 7) == 0)
     {
         const int xcd = bid & 7, local = bid >> 3;
@@ -510,6 +514,19 @@ inline bool gemm_gemm_supported(int M, int N, int K, int O, int batch, int sa, i
     return true;
 }
 
+// A group is 64 to 127 batches: 8 per XCD and up keep both of a CU's places filled to the end, and more would only widen what the
+// L2s hold at a time. (Batch by batch the heavy slabs of the last batch started when the rest was done: half of the CUs idle for
+// the last third. Causal 64 x 4096 x 4096 x 64: 246.8 -> 202.8 us.)
+inline SlabOrder slab_order(int slabs, int batch)
+{
+    const int wanted = batch >= 128 ? batch / 64 : 1;
+    int size         = (batch + wanted - 1) / wanted;
+    if((batch & 7) == 0)
+        size = (size + 7) & ~7; // (every group starts at XCD 0)
+    const int groups = (batch + size - 1) / size;
+    return SlabOrder{make_magic((uint32_t)size * (uint32_t)slabs), make_magic((uint32_t)size), make_magic((uint32_t)(batch - (groups - 1) * size)), groups};
+}
+
 template <int KS, int OG, int MT, int NW, bool SOFTMAX>
 inline hipError_t gemm_gemm_launch_t(GemmGemmArgs a, hipStream_t s)
 {
@@ -524,6 +541,8 @@ inline hipError_t gemm_gemm_launch_t(GemmGemmArgs a, hipStream_t s)
     if(attr_err != hipSuccess)
         return attr_err;
     a.slabs = (a.M + Cfg::BM - 1) / Cfg::BM;
+    if(a.mask_upper)
+        a.order = slab_order(a.slabs, a.batch);
     hipLaunchKernelGGL(kern, dim3(a.slabs * a.batch), dim3(Cfg::NT), Cfg::LDS, s, a);
     return hipGetLastError();
 }
@@ -551,7 +570,7 @@ inline hipError_t gemm_gemm_launch(const void* a, const void* b0, const void* b1
     g.M = M, g.N = N, g.K = K, g.O = O, g.batch = batch;
     g.sa = sa, g.sb0 = sb0, g.sb1 = sb1, g.sc = sc;
     g.bsa = bsa, g.bsb0 = bsb0, g.bsb1 = bsb1, g.bsc = bsc;
-    g.slabs = 0;
+    g.slabs = 0, g.order = SlabOrder{};
     g.scale = scale, g.mask_upper = mask_upper;
     if(instance < 0)
     {

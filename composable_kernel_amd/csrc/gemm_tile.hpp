@@ -189,6 +189,19 @@ struct MagicDiv
     uint32_t d;
 };
 
+inline MagicDiv make_magic(uint32_t d)
+{
+    // include/ck/utility/magic_division.hpp:28-54
+    uint32_t shift = 0;
+    while(shift < 32 && (1ull << shift) < d)
+        ++shift;
+    const uint64_t one = 1;
+    MagicDiv m;
+    m.mul   = (uint32_t)(((one << 32) * ((one << shift) - d)) / d + 1);
+    m.shift = shift;
+    m.d     = d;
+    return m;
+}
 __device__ __forceinline__ uint32_t magic_div(uint32_t n, const MagicDiv& m)
 {
     return (__umulhi(n, m.mul) + n) >> m.shift;
