@@ -352,18 +352,20 @@ __global__ __launch_bounds__(NW * 64)
     // with the upper-triangle mask, columns past the slab's last row are masked for every row of it
     const int n_end = (SOFTMAX && p.mask_upper && m0 + Cfg::BM < p.N) ? m0 + Cfg::BM : p.N;
 
-    // A step with masked columns for any row of this wave runs the EDGE form of the step (wave-uniform). Only the form without
-    // compares and guards is straight-line code, and a wave has one EDGE step; there the 32-column pairs past the wave's last
-    // unmasked column are left out. 32 x 2048 x 2048 x 128 with softmax 147.0 -> 138.4 us, causal 56.0 -> 53.6; 100 x 1000 x 1500
-    // x 80 97.0 -> 93.7; causal 200 x 300 x 300 x 128 27.0 -> 26.0; without softmax 64 x 512 x 512 x 64 7.9 -> 7.5.
+    // The softmax step is compiled in three forms, chosen per step and wave (wave-uniform): without a masked column it is straight-line
+    // code without compares; with masked columns in all of its four 32-column pairs it compares, in straight-line code still; past
+    // the wave's last unmasked column (EDGE) the pairs that lie there are left out, behind branches. With the first and the last:
+    // 32 x 2048 x 2048 x 128 147.0 -> 138.4 us, causal 56.0 -> 53.6; 100 x 1000 x 1500 x 80 97.0 -> 93.7; causal 200 x 300 x 300 x 128
+    // 27.0 -> 26.0. With the middle one, which most steps of a single-step problem and the last of N % 128 > 96 take: 26 x 66 x
+    // 121 x 64 4.83 -> 4.62, 53 x 226 x 363 x 64 -> 128 11.3 -> 10.7.
     // RAISE: MFMA sections at raised wave priority, so that the other wave of the SIMD does its softmax meanwhile: with K of 33
-    // to 64 355.8 -> 348.3 us at 64 x 4096 x 4096 x 64 (without the two forms 351.9 -> 344.6); slower with K of 128
+    // to 64 355.8 -> 348.3 us at 64 x 4096 x 4096 x 64 (without the forms 351.9 -> 344.6); slower with K of 128
     // (147 -> 153) and 32 (72.1 -> 73.0) and without softmax (128 x 1024 x 1024 x 64 38.2 -> 39.2).
     constexpr bool RAISE = SOFTMAX && KS == 2;
-    // One form, with the compares behind a branch, where the second one's registers cost a co-resident workgroup: 8 waves with
+    // One form, with the compares behind a branch, where more forms' registers cost a co-resident workgroup: 8 waves with
     // K up to 32 and O up to 64 (122 registers, 150 with two forms: 200 x 500 x 500 x 32 24.4 -> 32.7 us, 256 x 2000 x 300 x 32 69 ->
     // 93) and the 64-row instances.
-    constexpr bool TWO_FORMS = SOFTMAX && (NW == 8 ? !(KS == 1 && OG == 1) : MT == 2);
+    constexpr bool FORMS = SOFTMAX && (NW == 8 ? !(KS == 1 && OG == 1) : MT == 2);
     const int wave_m0    = m0 + wave * 16 * MT;
     const int wave_n_end = (p.mask_upper && wave_m0 + 16 * MT < p.N) ? wave_m0 + 16 * MT : p.N;
     const int full_end   = (p.mask_upper && wave_m0 + 1 < p.N) ? wave_m0 + 1 : p.N;
@@ -385,18 +387,7 @@ __global__ __launch_bounds__(NW * 64)
             __syncthreads();
             if(n0 + Cfg::BNC < n_end)
                 load_step(n0 + Cfg::BNC); // in flight while this step is multiplied
-                if(TWO_FORMS && edge_step(n0))
-                {
-                    constexpr bool EDGE  = TWO_FORMS;
-                    const int edge_pairs = pairs_of(n0);
-#include "gemm_gemm_step.inc"
-                }
-                else
-                {
-                    constexpr bool EDGE  = false;
-                    constexpr int edge_pairs = 4;
-#include "gemm_gemm_step.inc"
-                }
+#include "gemm_gemm_forms.inc"
         }
     }
     else
@@ -413,18 +404,7 @@ __global__ __launch_bounds__(NW * 64)
                 __syncthreads();
                 if(n0 + 2 * Cfg::BNC < n_end)
                     load_into(n0 + 2 * Cfg::BNC, rb0, rb1);
-                if(TWO_FORMS && edge_step(n0))
-                {
-                    constexpr bool EDGE  = TWO_FORMS;
-                    const int edge_pairs = pairs_of(n0);
-#include "gemm_gemm_step.inc"
-                }
-                else
-                {
-                    constexpr bool EDGE  = false;
-                    constexpr int edge_pairs = 4;
-#include "gemm_gemm_step.inc"
-                }
+#include "gemm_gemm_forms.inc"
             }
             if(nb + Cfg::BNC < n_end)
             {
@@ -434,18 +414,7 @@ __global__ __launch_bounds__(NW * 64)
                 __syncthreads();
                 if(n0 + 2 * Cfg::BNC < n_end)
                     load_into(n0 + 2 * Cfg::BNC, rb0b, rb1b);
-                if(TWO_FORMS && edge_step(n0))
-                {
-                    constexpr bool EDGE  = TWO_FORMS;
-                    const int edge_pairs = pairs_of(n0);
-#include "gemm_gemm_step.inc"
-                }
-                else
-                {
-                    constexpr bool EDGE  = false;
-                    constexpr int edge_pairs = 4;
-#include "gemm_gemm_step.inc"
-                }
+#include "gemm_gemm_forms.inc"
             }
         }
     }
