@@ -150,11 +150,13 @@ __device__ __forceinline__ V load_head16(const void* ptr, int nb) // 16-bit elem
     const i32x4 x = big ? i32x4{first[0], first[1], rest[0], rest[1]} : i32x4{rest[0], rest[1], 0, 0};
     return __builtin_bit_cast(V, x);
 }
-// as much of a 16-byte vector as the row has room for
+// as much of a 16-byte vector as the row has room for (whole: known to be all of it, for every lane)
 template <int UNIT, typename V>
-__device__ __forceinline__ void store_room(void* ptr, const V& val, int room_bytes, bool nt)
+__device__ __forceinline__ void store_room(void* ptr, const V& val, int room_bytes, bool nt, bool whole = false)
 {
-    if(room_bytes >= 16)
+    if(whole)
+        store_vec(ptr, val, nt);
+    else if(room_bytes >= 16)
         store_vec(ptr, val, nt);
     else if(room_bytes > 0)
         store_head<UNIT>(ptr, val, room_bytes);
@@ -436,7 +438,7 @@ __device__ __forceinline__ void requant_lut(const i32x4 (&v)[NQ], float sg, uint
 }
 // 16 consecutive int8 outputs of one row, rounded requant through the table
 __device__ __forceinline__ void store_row16_i8_lut(int8_t* crow, int n0, int N, const i32x4 (&v)[4], float sg,
-                                                   uint32_t lut_lds, bool nt)
+                                                   uint32_t lut_lds, bool nt, bool whole = false)
 {
     int b[16];
     requant_lut<4>(v, sg, lut_lds, b);
@@ -444,13 +446,13 @@ __device__ __forceinline__ void store_row16_i8_lut(int8_t* crow, int n0, int N, 
 #pragma unroll
     for(int w = 0; w < 4; ++w)
         pk[w] = pack4_low_bytes(b[4 * w], b[4 * w + 1], b[4 * w + 2], b[4 * w + 3]);
-    store_room<1>(crow + n0, pk, N - n0, nt);
+    store_room<1>(crow + n0, pk, N - n0, nt, whole);
 }
 
 // 16 consecutive int8 outputs of one row
 template <int EPI>
 __device__ __forceinline__ void store_row16_i8(int8_t* crow, int n0, int N, const i32x4 (&v)[4],
-                                               float sg, float sr, bool nt = false)
+                                               float sg, float sr, bool nt = false, bool whole = false)
 {
     int b[16];
 #pragma unroll
@@ -462,7 +464,7 @@ __device__ __forceinline__ void store_row16_i8(int8_t* crow, int n0, int N, cons
 #pragma unroll
     for(int w = 0; w < 4; ++w)
         pk[w] = pack4_low_bytes(b[4 * w], b[4 * w + 1], b[4 * w + 2], b[4 * w + 3]);
-    store_room<1>(crow + n0, pk, N - n0, nt);
+    store_room<1>(crow + n0, pk, N - n0, nt, whole);
 }
 
 // 16 consecutive int8 outputs of one row under per-column scales sc[0..15] (columns n0 .. n0 + 15)
@@ -1132,6 +1134,11 @@ struct GemmTile
             acc_t* slice = reinterpret_cast<acc_t*>(reinterpret_cast<uint8_t*>(p.ws) +
                                                     (size_t)(unit / ntiles_all) * p.M * p.N * 4);
             uint8_t* c_batch = reinterpret_cast<uint8_t*>(p.c) + (size_t)bi * p.bsc * ES;
+            // Output channels in whole groups of 16: no lane's row ends inside its vector, and the branches of store_head are passed by
+            // with one scalar one. The 256 x 256 instance of the 3-D im2col kernel has no scalar registers left for their lane masks:
+            // int8 16 x 28^3, C 112 -> K 240 235.5 -> 229.6 us, 31 x 37^3, C 16 -> K 224 248.9 -> 234.3, 11 x 18^3, C 48 -> K 144 23.9
+            // -> 23.1. (The smaller ones have, and get 1 % slower by it: 9 x 33^3, C 32 -> K 80 58.6 -> 59.3.)
+            const bool whole = IM2COL == 2 && BM * BN >= 256 * 256 && (p.N & 15) == 0;
             // Per-column requant scales (the FUSED variant of the int8 kernel: compiled into the plain one it cost the
             // im2col instances ten more spilled SGPRs and 7 - 10 % on the conv and LLM shapes): a loop nest of its own,
             // column group outermost, so that the 16 scales of the lane's columns are fetched once per group and before
@@ -1194,13 +1201,13 @@ struct GemmTile
                                                 acc[i][g * 4 + 3]};
                             if(p.epi == EPI_REQUANT_RND && USE_LUT)
                                 store_row16_i8_lut(crow, n0, p.N, v, p.scale_gemm,
-                                                   (uint32_t)(uintptr_t)(lds_ptr_t)smem + (uint32_t)(NST * STAGE), nt);
+                                                   (uint32_t)(uintptr_t)(lds_ptr_t)smem + (uint32_t)(NST * STAGE), nt, whole);
                             else if(p.epi == EPI_REQUANT_RND)
-                                store_row16_i8<EPI_REQUANT_RND>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu, nt);
+                                store_row16_i8<EPI_REQUANT_RND>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu, nt, whole);
                             else if(p.epi == EPI_REQUANT_CK)
-                                store_row16_i8<EPI_REQUANT_CK>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu, nt);
+                                store_row16_i8<EPI_REQUANT_CK>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu, nt, whole);
                             else
-                                store_row16_i8<EPI_PASSTHROUGH>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu, nt);
+                                store_row16_i8<EPI_PASSTHROUGH>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu, nt, whole);
                         }
                         else
                         {

@@ -147,3 +147,15 @@ def test_convnd_unsupported_arguments_are_refused():
     with pytest.raises(ValueError):
         ck.DeviceConvNdFwdF16(3).MakeArgumentPointer(0, 0, 0, 1, 16, 16, [6, 6], [3, 3], [4, 4], [1, 1], [1, 1], [0, 0], [0, 0])
     assert len(ck.DeviceConvNdFwdF16.GetInstances(3)) == n
+
+
+@pytest.mark.parametrize("K", [1, 15, 16, 17, 32, 48, 144, 250, 257, 272])
+@pytest.mark.parametrize("instance", [capi.INSTANCE_AUTO, 0, 1, 4, 7])
+def test_conv3d_int8_output_channels_around_groups_of_16(K, instance):
+    """Whole groups of 16 output channels are stored without a look at the row's end, others in pieces; every epilogue."""
+    import gpu_util
+    inp, wei = uniform_int8((1, 4, 5, 6, 16), -5, 5, 1300), uniform_int8((K, 3, 3, 3, 16), -5, 5, 1301 + K)
+    geom = ((1, 1, 1), (1, 1, 1), (1, 1, 1))
+    for op, epi in ((None, {}), (ck.RequantReluRequant(0.05, 0.7, rounded=True), dict(epi=lit.EPI_REQUANT_RND, scale_gemm=0.05, scale_relu=0.7)),
+                    (ck.RequantReluRequant(0.05, 0.7), dict(epi=lit.EPI_REQUANT_CK, scale_gemm=0.05, scale_relu=0.7))):
+        np.testing.assert_array_equal(gpu_util.convnd_fwd(inp, wei, *geom, out_op=op, instance=instance), lit.convnd_fwd(inp, wei, *geom, **epi))
