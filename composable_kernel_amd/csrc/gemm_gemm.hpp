@@ -309,8 +309,9 @@ __global__ __launch_bounds__(NW * 64)
     // byte offsets of this lane's B0 fragments of score tiles 0 and 1: rows 8 * (fr / 4) + fr % 4 and 4 more. Tile t is 32 * (t / 2)
     // rows on, and neither step changes ab_key (bits 0, 1 and 3 of the row): immediates of the read. Worked out tile by tile
     // they became eight address registers and, in some of the kernels, a slower order of the step: without softmax 45 x 32 x
-    // 1046 x 16 9.6 -> 11.3 us, 12 x 54 x 3073 x 32 22.6 -> 28.1. (Two registers in the plain 8-wave kernel for K up to 32, where
-    // one reads fewer fragments ahead: 231 x 45 x 2741 x 16 20.8 -> 20.0, 57 x 1934 x 61 x 32 7.3 -> 7.4, 7.7 with eight.)
+    // 1046 x 16 9.6 -> 11.3 us, 12 x 54 x 3073 x 32 22.6 -> 28.1. (Two registers for K up to 32 in the plain 8-wave and in the
+    // softmax 32-row kernel, where one reads fewer fragments ahead: plain 231 x 45 x 2741 x 16 20.8 -> 20.0, 57 x 1934 x 61 x 32 7.3
+    // -> 7.4, 7.7 with eight; softmax 128 x 2539 x 2539 x 32 238.9 -> 235.5, 19 x 3046 x 3046 causal 42.9 -> 42.4.)
     uint32_t b0_lane[KS][2];
 #pragma unroll
     for(int ks = 0; ks < KS; ++ks)
@@ -318,7 +319,7 @@ __global__ __launch_bounds__(NW * 64)
         const uint32_t row = (uint32_t)(8 * (fr >> 2) + (fr & 3));
         b0_lane[ks][0]     = row * Cfg::AST + ((uint32_t)(ks * 4 + q) ^ Cfg::ab_key(row)) * 16;
         b0_lane[ks][1]     = b0_lane[ks][0] + 4 * Cfg::AST;
-        if constexpr(!SOFTMAX && NW == 8 && KS == 1)
+        if constexpr(KS == 1 && (SOFTMAX ? MT == 2 : NW == 8))
             asm volatile("" : "+v"(b0_lane[ks][1]));
     }
 
@@ -357,7 +358,8 @@ __global__ __launch_bounds__(NW * 64)
     // the wave's last unmasked column (EDGE) the pairs that lie there are left out, behind branches. With the first and the last:
     // 32 x 2048 x 2048 x 128 147.0 -> 138.4 us, causal 56.0 -> 53.6; 100 x 1000 x 1500 x 80 97.0 -> 93.7; causal 200 x 300 x 300 x 128
     // 27.0 -> 26.0. With the middle one, which most steps of a single-step problem and the last of N % 128 > 96 take: 26 x 66 x
-    // 121 x 64 4.83 -> 4.62, 53 x 226 x 363 x 64 -> 128 11.3 -> 10.7.
+    // 121 x 64 4.83 -> 4.62, 53 x 226 x 363 x 64 -> 128 11.3 -> 10.7; not for K and O past 64, whose other forms it slows down: 206 x 1803
+    // x 1803 x 128 560 -> 582.
     // RAISE: MFMA sections at raised wave priority, so that the other wave of the SIMD does its softmax meanwhile: with K of 33
     // to 64 355.8 -> 348.3 us at 64 x 4096 x 4096 x 64 (without the forms 351.9 -> 344.6); slower with K of 128
     // (147 -> 153) and 32 (72.1 -> 73.0) and without softmax (128 x 1024 x 1024 x 64 38.2 -> 39.2).
@@ -366,6 +368,7 @@ __global__ __launch_bounds__(NW * 64)
     // K up to 32 and O up to 64 (122 registers, 150 with two forms: 200 x 500 x 500 x 32 24.4 -> 32.7 us, 256 x 2000 x 300 x 32 69 ->
     // 93) and the 64-row instances.
     constexpr bool FORMS = SOFTMAX && (NW == 8 ? !(KS == 1 && OG == 1) : MT == 2);
+    constexpr bool MIDDLE_FORM = FORMS && !(KS == 4 && OG == 2);
     const int wave_m0    = m0 + wave * 16 * MT;
     const int wave_n_end = (p.mask_upper && wave_m0 + 16 * MT < p.N) ? wave_m0 + 16 * MT : p.N;
     const int full_end   = (p.mask_upper && wave_m0 + 1 < p.N) ? wave_m0 + 1 : p.N;
