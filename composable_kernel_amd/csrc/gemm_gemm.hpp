@@ -513,10 +513,24 @@ inline hipError_t gemm_gemm_launch_t(GemmGemmArgs a, hipStream_t s)
     if(attr_err != hipSuccess)
         return attr_err;
     a.slabs = (a.M + Cfg::BM - 1) / Cfg::BM;
-    if(a.mask_upper)
-        a.order = slab_order(a.slabs, a.batch);
-    hipLaunchKernelGGL(kern, dim3(a.slabs * a.batch), dim3(Cfg::NT), Cfg::LDS, s, a);
-    return hipGetLastError();
+    // (the threads of a grid dimension are counted in 32 bits, and a launch past them wraps around without an error: more batches
+    // than fit go out in launches of their own, whole groups of eight of them for the XCD mapping)
+    const long fit = ((1l << 32) - 1) / Cfg::NT / a.slabs;
+    if(fit < 1)
+        return hipErrorInvalidValue;
+    const int most = (int)(fit >= a.batch ? a.batch : fit >= 8 ? fit & ~7l : fit);
+    for(int left = a.batch; left > 0; left -= most)
+    {
+        a.batch = left < most ? left : most;
+        if(a.mask_upper)
+            a.order = slab_order(a.slabs, a.batch);
+        hipLaunchKernelGGL(kern, dim3(a.slabs * a.batch), dim3(Cfg::NT), Cfg::LDS, s, a);
+        const hipError_t e = hipGetLastError();
+        if(e != hipSuccess)
+            return e;
+        a.a += most * a.bsa, a.b0 += most * a.bsb0, a.b1 += most * a.bsb1, a.c += most * a.bsc;
+    }
+    return hipSuccess;
 }
 
 template <int MT, int NW, bool SOFTMAX>

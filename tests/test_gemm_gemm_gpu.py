@@ -107,3 +107,27 @@ def test_columns_of_the_intermediate_in_order(K, instance):
     torch.cuda.synchronize()
     want = (a[0].double() @ b0[0].double().T) @ b1[0].double()  # |sums| <= 300 * 2 * 3: exact
     assert torch.equal(c[0].double(), want)
+
+
+@pytest.mark.parametrize("softmax", [False, True])
+def test_batches_past_one_launch(softmax):
+    """More workgroups than one launch has threads for in 32 bits (2^23 of 512 threads)."""
+    import torch
+    import gpu_util
+    G, K = (1 << 23) + 24, 8
+    n = torch.arange(G, device="cuda")
+    a, b0, b1 = (((n % m)[:, None] + torch.arange(K, device="cuda")[None, :] % 3 - 3).half() for m in (5, 7, 11))
+    c = torch.full((G, K), float("nan"), device="cuda", dtype=torch.float16)
+    dims = (1, 1, K, K, G, K, K, K, K, K, K, K, K)
+    if softmax:  # one column: its probability is 1
+        op = ck.DeviceBatchedGemmSoftmaxGemmF16(MaskOutUpperTriangle=True)
+        arg = op.MakeArgumentPointer(a, b0, b1, c, *dims, ck.PassThrough(), ck.PassThrough(), ck.Scale(1.0))
+        want = b1
+    else:
+        op = ck.DeviceBatchedGemmGemmF16()
+        arg = op.MakeArgumentPointer(a, b0, b1, c, *dims)
+        want = ((a.float() * b0.float()).sum(1, keepdim=True) * b1.float()).half()  # (small integers: exact)
+    assert op.IsSupportedArgument(arg)
+    op.MakeInvokerPointer().Run(arg, ck.StreamConfig(gpu_util.stream()))
+    torch.cuda.synchronize()
+    assert torch.equal(c, want)
