@@ -90,3 +90,96 @@ def test_k_below_one_vector_and_half_a_k_tile(kind, K):
         _run(kind, "mk_nk", M, N, K, off=1)
         _run(kind, "km_nk", M, N, K, off=0)
         _run(kind, "mk_kn", M, N, K, off=1)
+
+
+# ---- the 128 x 128 tile (256 of them and more): its epilogue has 16 columns per lane where B is K-contiguous
+def _big(kind, M, N, K, lda, ldb, seed):
+    """Small integers with leading dimensions of their own: fp16 results and int8 accumulators are exact."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    dt = torch.int8 if kind == "i8" else torch.float16
+    a = torch.randint(-3, 4, (M, lda), generator=g, device="cuda").to(dt)
+    b = torch.randint(-3, 4, (N, ldb), generator=g, device="cuda").to(dt)
+    return a, b, a[:, :K].float() @ b[:, :K].float().T.contiguous()
+
+
+def _requant(acc, sg, sr, rounded):
+    """The two requantisations in fp32, operation by operation."""
+    import torch
+    sg, sr = torch.tensor(sg, device="cuda"), torch.tensor(sr, device="cuda")  # fp32, as the kernel's arguments
+    if rounded:
+        x = (acc * sg).round().clamp(-128, 127).clamp_min(0)
+        return (x * sr).round().clamp(-128, 127).to(torch.int8)
+    x = (acc * sg).clamp(-128, 127).clamp_min(0)
+    return (x * sr).clamp(-128, 127).to(torch.int8)  # (truncating)
+
+
+@pytest.mark.parametrize("epilogue", ["rounded", "literal", "per_column", "per_column_relu"])
+@pytest.mark.parametrize("shape", [(2047, 2049, 195, 201, 197, 2051), (2100, 2000, 65, 65, 67, 2003)])
+def test_large_tile_int8_epilogues(epilogue, shape):
+    import torch
+    import gpu_util
+    M, N, K, lda, ldb, ldc = shape
+    assert capi.lib()._ZN3ckx11ragged_tileEiii(M, N, 1) == 128
+    a, b, acc = _big("i8", M, N, K, lda, ldb, 21)
+    c = torch.full((M, ldc), 77, dtype=torch.int8, device="cuda")
+    if epilogue.startswith("per_column"):
+        scales = torch.rand((N,), device="cuda") * 0.4
+        relu = epilogue == "per_column_relu"
+        op = ck.DeviceGemmMultipleDInt8()
+        arg = op.MakeArgumentPointer(a, b, [scales], c, M, N, K, lda, ldb, [0], ldc, None, None,
+                                     ck.ActivationMul2Clamp(ck.Relu() if relu else ck.PassThrough()))
+        want = (scales * (acc.clamp_min(0) if relu else acc)).clamp(-128, 127).to(torch.int8)
+    else:
+        op = ck.DeviceGemmInt8()
+        arg = op.MakeArgumentPointer(a, b, c, M, N, K, lda, ldb, ldc, None, None, ck.RequantReluRequant(0.3, 0.7, rounded=epilogue == "rounded"))
+        want = _requant(acc, 0.3, 0.7, epilogue == "rounded")
+    assert op.IsSupportedArgument(arg), capi.last_error()
+    op.MakeInvokerPointer().Run(arg, ck.StreamConfig(gpu_util.stream()))
+    torch.cuda.synchronize()
+    assert torch.equal(c[:, :N], want), f"{int((c[:, :N] != want).sum())} elements differ"
+    assert bool((c[:, N:] == 77).all()), "wrote outside the C rows"
+
+
+@pytest.mark.parametrize("functor", ["relu_add", "bilinear"])
+def test_large_tile_d_operands_on_any_element(functor):
+    import torch
+    import gpu_util
+    M, N, K, ldd, ldc = 2049, 2047, 131, 2053, 2049
+    assert capi.lib()._ZN3ckx11ragged_tileEiii(M, N, 1) == 128
+    a, b, acc = _big("f16", M, N, K, K + 2, K + 4, 22)
+    d = [torch.randint(-50, 51, (M * ldd + 1,), device="cuda").half() for _ in range(2)]
+    rows = [x[1:].reshape(M, ldd)[:, :N].float() for x in d]
+    cde, nd, want = (ck.AddReluAdd(), 2, (acc + rows[0]).clamp_min(0) + rows[1]) if functor == "relu_add" else \
+        (ck.Bilinear(0.5, 2.0), 1, 0.5 * acc + 2.0 * rows[0])
+    e = torch.full((M, ldc), 7, dtype=torch.float16, device="cuda")
+    op = ck.DeviceGemmMultipleDF16()
+    arg = op.MakeArgumentPointer(a, b, [x.data_ptr() + 2 for x in d[:nd]], e, M, N, K, K + 2, K + 4, [ldd] * nd, ldc, None, None, cde)
+    assert op.IsSupportedArgument(arg), capi.last_error()
+    op.MakeInvokerPointer().Run(arg, ck.StreamConfig(gpu_util.stream()))
+    torch.cuda.synchronize()
+    assert torch.equal(e[:, :N], want.half()) and bool((e[:, N:] == 7).all())
+
+
+@pytest.mark.parametrize("kind", ["i8", "f16"])
+@pytest.mark.parametrize("G, M, N, K, large", [(70, 250, 255, 67, True), (70, 129, 131, 67, False), (300, 127, 121, 33, True)])
+def test_batches_on_both_tiles(kind, G, M, N, K, large):
+    """Batches whose tiles add up past 256 although one has a few; odd batch strides, the gaps between the C batches untouched."""
+    import torch
+    import gpu_util
+    assert capi.lib()._ZN3ckx11ragged_tileEiii(M, N, G) == (128 if large else 64)
+    g = torch.Generator(device="cuda").manual_seed(23)
+    dt = torch.int8 if kind == "i8" else torch.float16
+    bsa, bsb, bsc = M * K + 3, N * K + 5, M * N + 7
+    a, b = (torch.randint(-3, 4, (G, bs), generator=g, device="cuda").to(dt) for bs in (bsa, bsb))
+    c = torch.full((G, bsc), 77, dtype=dt, device="cuda")
+    op = (ck.DeviceBatchedGemmInt8 if kind == "i8" else ck.DeviceBatchedGemmF16)()
+    arg = op.MakeArgumentPointer(a, b, c, M, N, K, K, K, N, bsa, bsb, bsc, G)
+    assert op.IsSupportedArgument(arg), capi.last_error()
+    op.MakeInvokerPointer().Run(arg, ck.StreamConfig(gpu_util.stream()))
+    torch.cuda.synchronize()
+    for i in range(G):
+        want = a[i, :M * K].reshape(M, K).float() @ b[i, :N * K].reshape(N, K).float().T.contiguous()
+        want = want.to(torch.int32).to(torch.int8) if kind == "i8" else want.half()
+        assert torch.equal(c[i, :M * N].reshape(M, N), want), f"batch {i}"
+    assert bool((c[:, M * N:] == 77).all()), "wrote between the C batches"

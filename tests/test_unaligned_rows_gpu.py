@@ -105,3 +105,50 @@ def test_split_k_slices_of_odd_rows(kind, N):
     want = fast.gemm_i8(a, b.T, lit.EPI_REQUANT_RND, 0.02, 0.4) if kind == "i8" else \
         (a.astype(np.float32) @ b.astype(np.float32).T).astype(np.float16)
     np.testing.assert_array_equal(dc.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("K", [64, 65])
+@pytest.mark.parametrize("instance", [-1, 1, 7])
+def test_streamed_int8_rows_on_any_element(K, instance):
+    """int8 outputs of 64 MiB and more are stored with the non-temporal hint, also at odd addresses and next to row ends in pieces
+    (K = 65: the last instance of the family, which is the automatic choice)."""
+    import torch
+    import gpu_util
+    if K % 16 and instance >= 0:
+        pytest.skip("the tile instances take whole 16-byte vectors of K")
+    M, N, ldc, off = 8300, 8191, 8193, 1
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a, b = (torch.randint(-3, 4, (n, K), generator=g, device="cuda").to(torch.int8) for n in (M, N))
+    buf, pc = _rows(M, N, ldc, off, 77, torch.int8)
+    op = ck.DeviceGemmInt8(instance)
+    arg = op.MakeArgumentPointer(a, b, pc, M, N, K, K, K, ldc)
+    assert op.IsSupportedArgument(arg), capi.last_error()
+    op.MakeInvokerPointer().Run(arg, ck.StreamConfig(gpu_util.stream()))
+    torch.cuda.synchronize()
+    rows = buf[off:off + M * ldc].reshape(M, ldc)
+    want = (a.float() @ b.float().T.contiguous()).to(torch.int32).to(torch.int8)
+    assert torch.equal(rows[:, :N], want) and bool((rows[:, N:] == 77).all())
+    assert bool((buf[:off] == 77).all()) and bool((buf[off + M * ldc:] == 77).all())
+
+
+@pytest.mark.parametrize("C, K", [(3, 45), (16, 43)])
+def test_streamed_int8_conv_outputs_on_any_element(C, K):
+    """The same for convolutions: the few-channel kernel and the im2col tile kernels, an odd number of output channels."""
+    import torch
+    import gpu_util
+    N, H = 32, 224
+    g = torch.Generator(device="cuda").manual_seed(C)
+    x = torch.randint(-3, 4, (N, H, H, C), generator=g, device="cuda").to(torch.int8)
+    w = torch.randint(-3, 4, (K, 3, 3, C), generator=g, device="cuda").to(torch.int8)
+    y = torch.full((N * H * H * K + 1,), 77, dtype=torch.int8, device="cuda")
+    op = ck.DeviceConv2dFwdInt8()
+    arg = op.MakeArgumentPointer(x, w, y.data_ptr() + 1, N, K, C, [H, H], [3, 3], [H, H], [1, 1], [1, 1], [1, 1], [1, 1], None, None, None)
+    assert op.IsSupportedArgument(arg), capi.last_error()
+    op.MakeInvokerPointer().Run(arg, ck.StreamConfig(gpu_util.stream()))
+    torch.cuda.synchronize()
+    assert int(y[0]) == 77
+    out = y[1:].reshape(N, H, H, K)
+    for i in range(N):
+        pixels = torch.nn.functional.pad(x[i].float(), (0, 0, 1, 1, 1, 1))
+        want = sum(pixels[r:r + H, s:s + H] @ w[:, r, s].float().T.contiguous() for r in range(3) for s in range(3))
+        assert torch.equal(out[i], want.to(torch.int32).to(torch.int8)), f"image {i}"
