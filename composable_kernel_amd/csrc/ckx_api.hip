@@ -348,11 +348,11 @@ const SkinnyInstance kSkinny[] = {
 };
 constexpr int kAStream = 8; // (position in kSkinny)
 constexpr int kNumSkinny    = sizeof(kSkinny) / sizeof(kSkinny[0]);
-// the element-granular instance (gemm_generic.hpp) closes every GEMM and conv instance list: any extent, leading
-// dimension, channel count and base address, all four GEMM layouts, every epilogue of the data type
+// the padding instance closes every GEMM and conv instance list: any extent, leading dimension, channel count and base
+// address, all four GEMM layouts, every epilogue of the data type (gemm_ragged.hpp; conv_few.hpp and gemm_generic.hpp)
 constexpr int kGenericGemmInstance = kNumTiles + kNumSkinny;
 constexpr int kNumGemmInsts        = kNumTiles + kNumSkinny + 1;
-const char* const kGenericName     = "MI355X_Mfma16_Generic<64, 64, one k-step, waves 2x2, element-wise loads>";
+const char* const kGenericName     = "MI355X_Mfma16_Generic<padding: any extent, stride, channel count and base address>";
 
 const char* family_prefix(int op)
 {
@@ -447,7 +447,7 @@ int check_gemm_shape(int dt, int M, int N, int K, int sa, int sb, int sc, int al
         return fail(CKX_UNSUPPORTED, "C is row-major in every instance (as in the reference's instance lists)");
     // K-major operands: A column-major (element (m,k) at k*sa + m), B row-major ((k,n) at k*sb + n)
     const bool ta = al == CKX_COL_MAJOR, tb = bl == CKX_ROW_MAJOR;
-    // what only the element-granular instance takes (AUTO sends it there)
+    // what only the padding instance takes (AUTO sends it there)
     const bool fast = instance != CKX_INSTANCE_AUTO && instance != kGenericGemmInstance;
     if(fast && (ta || tb) && (f16_fused(epi) || per_column_scale(epi)))
         return fail(CKX_UNSUPPORTED, "the D-operand epilogues of this instance are built for A row-major, B column-major");
@@ -457,7 +457,7 @@ int check_gemm_shape(int dt, int M, int N, int K, int sa, int sb, int sc, int al
         return fail(CKX_UNSUPPORTED, "stride smaller than the contiguous extent");
     if(fast && gemm_needs_generic(dt, M, N, K, sa, sb, ta, tb, epi))
         return fail(CKX_UNSUPPORTED, "the contiguous extents of A and B and their strides must be multiples of 16 bytes "
-                                     "for this instance (the element-wise instance and AUTO take any)");
+                                     "for this instance (the padding instance and AUTO take any)");
     if((long)(ta ? K : M) * sa * es >= (1l << 31) || (long)(tb ? K : N) * sb * es >= (1l << 31) ||
        (long)M * sc * es >= (1l << 31))
         return fail(CKX_UNSUPPORTED, "operands of 2 GiB or more are not addressed");
@@ -493,7 +493,7 @@ int check_batch(int dt, int M, int N, int K, int sa, int sb, int sc, bool ta, bo
     {
         const int es = dt == ckx::DT_I8 ? 1 : 2;
         if(instance >= kNumTiles && instance != kGenericGemmInstance)
-            return fail(CKX_UNSUPPORTED, "batched GEMM runs on the tile instances and the element-wise instance");
+            return fail(CKX_UNSUPPORTED, "batched GEMM runs on the tile instances and the padding instance");
         if(epi >= CKX_EPI_ADD_RELU || k_batch > 1)
             return fail(CKX_UNSUPPORTED, "batched GEMM has neither D operands nor a K split");
         if(bsa < 0 || bsb < 0 || bsc < 0)
@@ -502,7 +502,7 @@ int check_batch(int dt, int M, int N, int K, int sa, int sb, int sc, bool ta, bo
             return fail(CKX_UNSUPPORTED, "batch strides of A and B must be multiples of 16 bytes for this instance");
         if(batch > 65535 && (instance == kGenericGemmInstance || (bsa * es) % 16 || (bsb * es) % 16 ||
                              gemm_needs_generic(dt, M, N, K, sa, sb, ta, tb, epi)))
-            return fail(CKX_UNSUPPORTED, "the element-wise instance takes at most 65535 batches");
+            return fail(CKX_UNSUPPORTED, "the padding instance takes at most 65535 batches");
         if(bsc < (long)(M - 1) * sc + N && M > 0 && N > 0)
             return fail(CKX_UNSUPPORTED, "C batches overlap");
         const long ea = operand_extent(batch, bsa, ta ? K : M, ta ? M : K, sa, es);
@@ -603,7 +603,7 @@ int run_gemm(int dt, const void* a, const void* b, void* c, int M, int N, int K,
     if(instance == kGenericGemmInstance ||
        (instance == CKX_INSTANCE_AUTO && (misaligned || gemm_needs_generic(dt, M, N, K, sa, sb, ta, tb, epi))))
     {
-        // element-granular instance: one pass over K whatever KBatch says (the result does not depend on the split)
+        // padding instance: one pass over K whatever KBatch says (the result does not depend on the split)
         if((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c) |
             (f16_fused(epi) ? reinterpret_cast<uintptr_t>(dops.d0) | reinterpret_cast<uintptr_t>(dops.d1) : 0)) & (es - 1))
             return fail(CKX_UNSUPPORTED, "operands must be aligned to their element size");
@@ -617,8 +617,8 @@ int run_gemm(int dt, const void* a, const void* b, void* c, int M, int N, int K,
         g.d0 = dops.d0, g.d1 = uses_d1(epi) ? dops.d1 : nullptr;
         g.ldd0 = dops.ldd0, g.ldd1 = dops.ldd1;
         g.ksplit  = 1;
-        if(batch > 65535)
-            return fail(CKX_UNSUPPORTED, "the element-granular instance (operands that are not 16-byte aligned vectors) "
+        if(batch > 65535) // (the documented limit; the kernel itself counts batches in its linear grid)
+            return fail(CKX_UNSUPPORTED, "the padding instance (operands that are not 16-byte aligned vectors) "
                                          "takes at most 65535 batches per launch");
         hipError_t e = ckx::launch_ragged(dt, ta, tb, g, (hipStream_t)stream);
         return e == hipSuccess ? CKX_OK : hip_fail(e, kGenericName);
@@ -852,9 +852,9 @@ int check_conv(int op, const ckx_conv2d_desc* d, int epi, int instance)
         return fail(CKX_UNSUPPORTED, "output spatial lengths do not match the conv geometry");
     // a 16-byte vector along c must not cross a filter tap
     // (device_conv2d_fwd_xdl_nhwc_kyxc_nhwk.hpp:595-601)
-    // (ConvolutionForwardSpecialization::OddC is the element-wise instance; AUTO sends such layers there)
+    // (ConvolutionForwardSpecialization::OddC is the padding instance; AUTO sends such layers there)
     if(((long)d->C * es) % 16 && instance != CKX_INSTANCE_AUTO && instance != kConvGenericInstance && instance != kConvStemInstance)
-        return fail(CKX_UNSUPPORTED, "C must be a multiple of 16 bytes for this instance (the element-wise instance and AUTO take any)");
+        return fail(CKX_UNSUPPORTED, "C must be a multiple of 16 bytes for this instance (the padding instance and AUTO take any)");
     const long in_b  = (long)d->N * d->Hi * d->Wi * d->C * es;
     const long wei_b = (long)d->K * d->Y * d->X * d->C * es;
     const long out_b = (long)d->N * d->Ho * d->Wo * d->K * es;
@@ -1154,7 +1154,7 @@ int check_convnd(int op, const ckx_convnd_desc* d, int epi, int instance, ckx_co
             return fail(CKX_UNSUPPORTED, "tensors of 2 GiB or more are not addressed");
     }
     if(((long)d->C * es) % 16 && instance != CKX_INSTANCE_AUTO && instance != kConvGenericInstance)
-        return fail(CKX_UNSUPPORTED, "C must be a multiple of 16 bytes for this instance (the element-wise instance and AUTO take any)");
+        return fail(CKX_UNSUPPORTED, "C must be a multiple of 16 bytes for this instance (the padding instance and AUTO take any)");
     // (device_convnd_fwd_xdl_nhwc_kyxc_nhwk.hpp:883-890 refuses tensors above 2 GB as well)
     if(in_px * d->C * es >= (1l << 31) || (long)d->K * taps * d->C * es >= (1l << 31) ||
        out_px * d->K * es >= (1l << 31) || taps * d->C >= (1l << 31))
@@ -1266,7 +1266,7 @@ int ckx_num_instances(int op)
     if(op == CKX_OP_GEMM_SPLITK)
         return kNumTiles;
     if(op == CKX_OP_CONV2D_FWD_F16 || op == CKX_OP_CONV2D_FWD_I8)
-        return kNumConvInsts; // + the input-patch, the pointwise, the stem, the streaming 1x1 and the element-wise kernel
+        return kNumConvInsts; // + the input-patch, the pointwise, the stem, the streaming 1x1 and the padding kernels
     if(op == CKX_OP_BATCHED_GEMM_GEMM || op == CKX_OP_BATCHED_GEMM_SOFTMAX_GEMM)
         return ckx::kNumGemmGemmInstances;
     return 0;

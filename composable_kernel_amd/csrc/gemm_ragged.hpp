@@ -19,7 +19,7 @@
 //
 // What bounds it: with the 128 x 128 tile the operand bytes through a CU's L1 (32 KB per K tile; 0.27 of the MFMA rate at
 // 4001 x 4003 x 4095 fp16), with few tiles the latency of one K tile after the other. Against the element-by-element gather
-// that served these shapes (one load instruction per element), fp16: 2001 x 1003 x 1025 90.4 -> 16.1 us, 4001 x 4003 x 4095
+// that served these shapes (one load instruction per element), fp16: 2001 x 1003 x 1025 98.7 -> 15.4 us, 4001 x 4003 x 4095
 // 2623 -> 197, 122 x 1283 x 3001 148 -> 17.4, 2049 x 2047 x 2047 with a K-major A 290 -> 55; int8 4001 x 4003 x 4095 3019 -> 118,
 // 40 x 333 x 3999 156 -> 16; bf16 3000 x 2999 x 1001 275 -> 47; one tile (32 x 33 x 65) 5.7, as before.
 //

@@ -126,7 +126,7 @@ const char* ckx_instance_name(int op, int instance);
  * base addresses to be whole 16-byte vectors, and report CKX_UNSUPPORTED otherwise -- the reference's
  * GemmSpecialization::Default instances (gemm_specialization.hpp:10-20). mk_nk runs on every instance; a
  * K-major operand (km / kn) on the tile instances of 64 rows and more, with the PassThrough / requant
- * epilogues. The LAST instance of every GEMM family is element-granular (any K, M, N, strides and base
+ * epilogues. The LAST instance of every GEMM family is the padding instance (any K, M, N, strides and base
  * addresses, all four layouts, every epilogue of the data type: the reference's KPadding / MNKPadding
  * instances, device_gemm_xdl_cshuffle.hpp:99-184) and CKX_INSTANCE_AUTO sends there exactly the problems
  * the vectorised instances refuse, so AUTO supports every shape. This holds for every ckx_gemm_* and
@@ -171,9 +171,9 @@ int64_t ckx_gemm_bf16_workspace_bytes(int32_t M, int32_t N, int32_t K, int insta
  * Batch, ...) + Run (device_batched_gemm.hpp:24-45; batch offsets as ComputePtrOffsetOfStridedBatch,
  * device_batched_gemm_xdl.hpp:256-285). Batch strides are in elements. The batches share one launch:
  * the persistent workgroups walk the C tiles of all batches. Shapes as for ckx_gemm_*_is_supported on a
- * tile instance, the element-granular instance or AUTO; the C batches must not overlap and the whole A, B, C
+ * tile instance, the padding instance or AUTO; the C batches must not overlap and the whole A, B, C
  * extents stay below 2 GiB. On the tile instances the A / B batch strides must be multiples of 16 bytes; AUTO
- * sends other strides (up to 65535 batches) to the element-granular instance. */
+ * sends other strides (up to 65535 batches) to the padding instance. */
 int ckx_batched_gemm_is_supported(int op, int32_t M, int32_t N, int32_t K, int32_t stride_a, int32_t stride_b,
                                   int32_t stride_c, int64_t batch_stride_a, int64_t batch_stride_b,
                                   int64_t batch_stride_c, int32_t batch, int a_layout, int b_layout, int c_layout,
@@ -228,7 +228,7 @@ int ckx_gemm_i8_splitk_noalloc(const void* p_a, const void* p_b, void* p_c, int3
  * CKX_EPI_ADD_RELU / _ADD_RELU_ADD / _CSHUFFLE_ADD_RELU / _ADD_ADD_FASTGELU (and, for the query, _BILINEAR). D0, D1 are
  * [M,N] row-major fp16 with row strides stride_d0 / stride_d1 in elements; stride 0 broadcasts one row (a bias
  * vector), as examples 03 and 04 do. p_d1 is ignored unless cde_op uses it. With a K-major operand (A column-major
- * or B row-major) these run on CKX_INSTANCE_AUTO or the element-granular instance only; an explicit tile or skinny
+ * or B row-major) these run on CKX_INSTANCE_AUTO or the padding instance only; an explicit tile or skinny
  * instance answers CKX_UNSUPPORTED. CKX_EPI_ADD_ADD_FASTGELU agrees with the reference's functor
  * (element_wise_operation.hpp:113-140) within rtol = atol = 1e-2, not bit for bit: the device evaluates
  * x / (1 + exp(-u)); the reference's 0.5 + 0.5 * (2 / (1 + exp(-u)) - 1) cancels to a coarse or zero factor for
@@ -255,8 +255,8 @@ int ckx_gemm_f16_bilinear(const void* p_a, const void* p_b, const void* p_d, voi
  * Activation_Mul2_Clamp<Act>>::MakeArgumentPointer + Run (device_gemm_multiple_d.hpp:14-55) for cde_op in
  * CKX_EPI_MUL2_CLAMP / CKX_EPI_RELU_MUL2_CLAMP. D0 is one contiguous row of N floats, broadcast over the rows
  * (stride_d0 must be 0, as a per-channel scale is passed upstream). Every instance of the int8 GEMM family takes it
- * (tile, skinny, element-wise; K runs through the workspace) with A row-major and B column-major; with a K-major
- * operand (A column-major or B row-major) it runs on CKX_INSTANCE_AUTO or the element-granular instance only -- an
+ * (tile, skinny, padding; K runs through the workspace) with A row-major and B column-major; with a K-major
+ * operand (A column-major or B row-major) it runs on CKX_INSTANCE_AUTO or the padding instance only -- an
  * explicit tile or skinny instance answers CKX_UNSUPPORTED. Batches do not take it. */
 int ckx_gemm_i8_multiple_d_is_supported(int32_t M, int32_t N, int32_t K, int32_t stride_a, int32_t stride_b,
                                         int32_t stride_d0, int32_t stride_e, int a_layout, int b_layout, int e_layout,
@@ -276,7 +276,7 @@ int ckx_gemm_i8_multiple_d(const void* p_a, const void* p_b, const void* p_d0, v
  * dilations = {dH, dW}, left pads = {pad_top, pad_left}, right pads = {pad_bottom, pad_right}.
  * The vectorised instances need C to fill whole 16-byte vectors (C % 16 for int8, C % 8 for fp16; the
  * reference: C % SrcScalarPerVector, device_conv2d_fwd_xdl_nhwc_kyxc_nhwk.hpp:595-601) and 16-byte aligned
- * input and weight addresses. The LAST instance of both conv families is element-granular -- any C, the
+ * input and weight addresses. The LAST instance of both conv families is the padding instance -- any C, the
  * reference's ConvolutionForwardSpecialization::OddC instances (convolution_forward_specialization.hpp:13-19)
  * -- for one, two and three spatial dimensions and every epilogue; CKX_INSTANCE_AUTO sends it the layers the
  * vectorised instances refuse. */
@@ -392,7 +392,7 @@ int ckx_batched_gemm_softmax_gemm_f16(const void* p_a, const void* p_b0, const v
  * the instance and the number of K runs that ckx_gemm_* / ckx_batched_gemm_* (op = CKX_OP_GEMM_I8 / _F16 / _BF16) or
  * ckx_conv2d_fwd_* would use for this problem with `workspace_bytes` of 16-byte aligned workspace (0: none).
  * *instance is in / out: CKX_INSTANCE_AUTO asks for the automatic choice, an instance index for that instance's K
- * split. Operand addresses are taken to be 16-byte aligned (a launch sends misaligned ones to the element-granular
+ * split. Operand addresses are taken to be 16-byte aligned (a launch sends misaligned ones to the padding
  * instance). The automatic choice is a cost model; tests/golden/planner_audit.json holds what it was measured against. */
 int ckx_gemm_plan(int op, int32_t M, int32_t N, int32_t K, int32_t stride_a, int32_t stride_b, int32_t stride_c,
                   int a_layout, int b_layout, int c_layout, int epilogue, int32_t batch, int64_t workspace_bytes,

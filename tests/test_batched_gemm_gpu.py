@@ -81,7 +81,7 @@ def test_batched_gemm_argument_checks():
     ok = lambda *x: L.ckx_batched_gemm_is_supported(*x)
     assert ok(capi.OP_GEMM_F16, 64, 64, 64, 64, 64, 64, 4096, 4096, 4096, 4, 0, 1, 0, 0, -1) == capi.OK
     assert ok(capi.OP_GEMM_F16, 64, 64, 64, 64, 64, 64, 4096, 4096, 100, 4, 0, 1, 0, 0, -1) == capi.UNSUPPORTED   # C overlap
-    # a batch stride of A that is not a whole 16-byte vector: the element-wise instance (and AUTO through it) only
+    # a batch stride of A that is not a whole 16-byte vector: the padding instance (and AUTO through it) only
     assert ok(capi.OP_GEMM_F16, 64, 64, 64, 64, 64, 64, 4100, 4096, 4096, 4, 0, 1, 0, 0, 0) == capi.UNSUPPORTED
     assert ok(capi.OP_GEMM_F16, 64, 64, 64, 64, 64, 64, 4100, 4096, 4096, 4, 0, 1, 0, 0, -1) == capi.OK
     assert ok(capi.OP_GEMM_F16, 64, 64, 64, 64, 64, 64, -8, 4096, 4096, 4, 0, 1, 0, 0, -1) == capi.UNSUPPORTED

@@ -55,7 +55,7 @@ def test_gemm_argument_validation_is_pure_host_logic():
     f16 = ck.DeviceGemmF16()
     assert f16.IsSupportedArgument(f16.MakeArgumentPointer(0, 0, 0, 4096, 4096, 4096, 4096, 4096, 4096))
     # K not a multiple of 16 bytes (the reference's KPadding / MNKPadding instances): the vectorised instances
-    # refuse, the element-wise instance -- the last of the list -- and the automatic choice accept
+    # refuse, the padding instance -- the last of the list -- and the automatic choice accept
     last = capi.lib().ckx_num_instances(capi.OP_GEMM_I8) - 1
     assert b"Generic" in capi.lib().ckx_instance_name(capi.OP_GEMM_I8, last)
     for cls, (M, N, K) in ((ck.DeviceGemmInt8, (64, 64, 100)), (ck.DeviceGemmF16, (64, 64, 60))):
@@ -174,7 +174,7 @@ conv_patch_wide.hpp:390:1: remark:     ScratchSize [bytes/lane]: 0 [-Rpass-analy
 def test_d_operand_epilogues_with_k_major_operands_run_on_auto_or_the_element_granular_instance_only():
     """The is_supported answers per instance and layout, as include/ckx.h states them: with A column-major or B
     row-major the D-operand epilogues (per-column requant scales, the fp16 add / scale / GELU functors) are
-    supported by CKX_INSTANCE_AUTO and by the element-granular instance (the last of the family) and by no explicit
+    supported by CKX_INSTANCE_AUTO and by the padding instance (the last of the family) and by no explicit
     tile or skinny instance; with A row-major and B column-major every instance that takes the shape supports them."""
     L = capi.lib()
     M, N, K = 16, 256, 512   # (16 rows: within the reach of every skinny instance)

@@ -23,7 +23,7 @@ LAYOUTS = {"mk_nk": (ck.RowMajor, ck.ColumnMajor), "mk_kn": (ck.RowMajor, ck.Row
 
 
 def _instance(tag):
-    """'generic': the element-wise instance, the last of the family"""
+    """'generic': the padding instance, the last of the family"""
     if tag != "generic":
         return tag
     L = capi.lib()
@@ -202,7 +202,7 @@ def test_k_runs_apply_the_functor_in_the_second_pass(force_k_runs, runs):
 
 @pytest.mark.parametrize("layout", list(LAYOUTS))
 def test_every_operand_layout_and_ragged_extents(layout):
-    """K = 100, N = 50 (no whole 16-byte vectors) and K-major operands go to the element-wise instance."""
+    """K = 100, N = 50 (no whole 16-byte vectors) and K-major operands go to the padding instance."""
     M, N, K = 90, 50, 100
     a = uniform_f16((M, K), -1, 1, 1400)
     b_kn = uniform_f16((K, N), -1, 1, 1401)

@@ -73,7 +73,7 @@ def test_conv2d_reference_golden_vectors_fp16():
         N, K, C = case["N"], case["K"], case["C"]
         Hi, Wi = case["input"]
         Y, X = case["filter"]
-        # C = 2 as in the reference case (4-byte pixels: the element-wise instance), and the same two channels
+        # C = 2 as in the reference case (4-byte pixels: the padding instance), and the same two channels
         # embedded in 8 (zeros elsewhere leave every sum unchanged: the vectorised instances)
         want = np.array(case["expected"], np.float32).astype(np.float16)
         for cpad in (C, 8):

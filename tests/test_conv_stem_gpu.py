@@ -3,7 +3,7 @@ reference's ResNet-50 script (script/profile_resnet50.sh:46), which its own inst
 specialisation. Through the C ABI against the CPU oracle (ReferenceConvFwd restated, oracle/ck_oracle.cpp): int8
 bit-exact with every requant form, fp16 within rtol = atol = 1e-2 and bit-exact on integer operands, the fused
 bias + ReLU form against the reference's conv + AddRelu; image sizes whose output rows and columns are not whole bands
-and tiles; the automatic choice and the element-granular instance on the same inputs."""
+and tiles; the automatic choice and the padding instance on the same inputs."""
 import numpy as np
 import pytest
 
@@ -60,7 +60,7 @@ def test_stem_fp16(size):
     inp = uniform_int8((N, Hi, Wi, 3), -5, 5, 7102).astype(np.float16)
     wei = uniform_int8((64, 7, 7, 3), -5, 5, 7103).astype(np.float16)
     np.testing.assert_array_equal(gpu_util.conv2d_fwd(inp, wei, S, D, P, instance=inst), lit.conv2d_fwd(inp, wei, S, D, P))
-    # ... and the element-granular instance (the reference's OddC route) agrees on the same inputs
+    # ... and the padding instance (the reference's OddC route) agrees on the same inputs
     generic = gpu_util.conv_instance(capi.OP_CONV2D_FWD_F16, "Generic")
     np.testing.assert_array_equal(gpu_util.conv2d_fwd(inp, wei, S, D, P, instance=inst),
                                   gpu_util.conv2d_fwd(inp, wei, S, D, P, instance=generic))

@@ -74,7 +74,7 @@ GOLD_ND = json.load(open(os.path.join(HERE, "golden", "reference_convnd_fwd_vect
                          ids=lambda c: c["name"])
 def test_convnd_reference_golden_vectors_fp16(case):
     """The reference's golden cases with integer inputs: exactly representable in fp16. Run with the case's own
-    channel count (C = 2: the element-wise instance) and with C padded to a whole 16-byte vector by zero channels,
+    channel count (C = 2: the padding instance) and with C padded to a whole 16-byte vector by zero channels,
     which add nothing (the vectorised instances)."""
     import gpu_util
     N, K, Cc = case["N"], case["K"], case["C"]

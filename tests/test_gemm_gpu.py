@@ -125,7 +125,7 @@ def test_int8_gemm_unsupported_arguments_are_refused():
     op = ck.DeviceGemmInt8()
     d = torch.zeros(1 << 16, dtype=torch.int8, device="cuda")
     # K not a multiple of 16 bytes: the vectorised instances refuse (as the reference's Default-specialisation
-    # instances do), the element-wise instance and the automatic choice take it (its KPadding instances)
+    # instances do), the padding instance and the automatic choice take it (its KPadding instances)
     for instance in range(N_INSTANCES - 1):
         fast = ck.DeviceGemmInt8(instance)
         arg = fast.MakeArgumentPointer(d, d, d, 16, 64, 100, 100, 100, 64)

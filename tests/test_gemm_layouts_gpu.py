@@ -178,7 +178,7 @@ def test_layouts_refused_arguments(layout):
         _run("i8", layout, a_st, b_st, M, N, K, instance, expect_unsupported=True)
     al, bl = LAYOUTS[layout]
     # contiguous extent of the K-major operand not a whole 16-byte vector: refused by the vectorised tile instances,
-    # taken by the element-wise instance and by the automatic choice; a stride below the extent by nobody
+    # taken by the padding instance and by the automatic choice; a stride below the extent by nobody
     lib = capi.lib()
     if al is ck.ColumnMajor:
         assert lib.ckx_gemm_f16_is_supported(60, 64, 64, 64, 64, 64, al.code, bl.code, ck.RowMajor.code, 0) == capi.UNSUPPORTED

@@ -96,7 +96,7 @@ def test_profiler_batched_gemm_gemm(tmp_path):
 
 def test_profiler_reports_unsupported_problems(tmp_path):
     """K = 100 is not a whole 16-byte vector: every vectorised instance says it does not support the problem (as the
-    reference's profiler prints, profile_gemm_impl.hpp:205-208), the element-wise instance runs it; a leading
+    reference's profiler prints, profile_gemm_impl.hpp:205-208), the padding instance runs it; a leading
     dimension below K is supported by no instance and the profiler fails."""
     M, N, K = 64, 64, 100
     out, dump = _run("ckx_profiler", ["gemm", 3, 1, 1, 1, 0, 0, M, N, K, -1, -1, -1], "CKX_PROFILER_DUMP", tmp_path)

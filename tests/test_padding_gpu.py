@@ -1,4 +1,4 @@
-"""GPU parity of the element-granular instance, through the C ABI: what the reference covers with its padded GEMM
+"""GPU parity of the padding instance, through the C ABI: what the reference covers with its padded GEMM
 instances (GemmSpecialization::KPadding / MNKPadding, gemm_specialization.hpp:10-20) and its odd-channel conv
 instances (ConvolutionForwardSpecialization::OddC; device test case C = 3, test/convnd_fwd/conv2d_fwd.cpp:111):
 K, leading dimensions, channel counts and base addresses that are not whole 16-byte vectors. The automatic choice

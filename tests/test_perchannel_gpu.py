@@ -125,7 +125,7 @@ def test_k_major_operands(layouts):
 
 
 def test_padding_shapes_take_the_element_wise_instance():
-    """K = 100 and an odd N: the element-granular instance, chosen by AUTO"""
+    """K = 100 and an odd N: the padding instance, chosen by AUTO"""
     a = uniform_int8((70, 100), -8, 8, 51)
     b_nk = uniform_int8((45, 100), -8, 8, 52)
     s = scales_for(45, 53)
@@ -180,7 +180,7 @@ def _conv(x, w, s, act, strides, pads, instance=capi.INSTANCE_AUTO, allow_unsupp
                                    (2, 3, 24, 3, 20, 1, 1)])
 def test_conv2d_per_output_channel(layer):
     """N, C, K, filter, HW, stride, pad: the patch-window and pointwise shapes (which fall back to the tile instances
-    for this functor), a ragged layer, and the reference's C = 3 case on the element-wise instance"""
+    for this functor), a ragged layer, and the reference's C = 3 case on the padding instance"""
     n, c, k, f, hw, st, pd = layer
     x = uniform_int8((n, hw, hw, c), -5, 5, 81)
     w = uniform_int8((k, f, f, c), -5, 5, 82)

@@ -75,7 +75,7 @@ def test_plan_queries_validate_like_the_launchers():
     inst, runs = C.c_int(-1), C.c_int(0)
     assert L.ckx_gemm_plan(capi.OP_GEMM_I8, 64, 64, 128, 64, 128, 64, 0, 1, 0, 0, 1, 0, C.byref(inst), C.byref(runs)) == capi.UNSUPPORTED
     assert L.ckx_gemm_plan(99, 64, 64, 128, 128, 128, 64, 0, 1, 0, 0, 1, 0, C.byref(inst), C.byref(runs)) == capi.INVALID_VALUE
-    # a K that is not a whole vector: the element-wise instance, one pass
+    # a K that is not a whole vector: the padding instance, one pass
     n = L.ckx_num_instances(capi.OP_GEMM_I8)
     assert capi.gemm_plan(capi.OP_GEMM_I8, 64, 64, 100) == (n - 1, 1)
     # no workspace: never more than one K run
