@@ -361,8 +361,9 @@ __global__ __launch_bounds__(NW * 64)
     // 121 x 64 4.83 -> 4.62, 53 x 226 x 363 x 64 -> 128 11.3 -> 10.7; not for K and O past 64, whose other forms it slows down: 206 x 1803
     // x 1803 x 128 560 -> 582.
     // RAISE: MFMA sections at raised wave priority, so that the other wave of the SIMD does its softmax meanwhile: with K of 33
-    // to 64 355.8 -> 348.3 us at 64 x 4096 x 4096 x 64 (without the forms 351.9 -> 344.6); slower with K of 128
-    // (147 -> 153) and 32 (72.1 -> 73.0) and without softmax (128 x 1024 x 1024 x 64 38.2 -> 39.2).
+    // to 64 355.8 -> 348.3 us at 64 x 4096 x 4096 x 64 (without the forms 351.9 -> 344.6); slower with K of 72 ... 128
+    // (32 x 2048 x 2048 x 72 90.2 -> 91.8, x 96 90.4 -> 92.8, x 128 93.3 -> 94.6; causal 64 x 1024 x 1024 x 80 32.2 -> 32.4) and 32 (72.1
+    // -> 73.0) and without softmax (128 x 1024 x 1024 x 64 38.2 -> 39.2).
     constexpr bool RAISE = SOFTMAX && KS == 2;
     // One form, with the compares behind a branch, where more forms' registers cost a co-resident workgroup: 8 waves with
     // K up to 32 and O up to 64 (122 registers, 150 with two forms: 200 x 500 x 500 x 32 24.4 -> 32.7 us, 256 x 2000 x 300 x 32 69 ->
@@ -488,7 +489,9 @@ inline bool gemm_gemm_supported(int M, int N, int K, int O, int batch, int sa, i
 
 // A group is 64 to 127 batches: 8 per XCD and up keep both of a CU's places filled to the end, and more would only widen what the
 // L2s hold at a time. (Batch by batch the heavy slabs of the last batch started when the rest was done: half of the CUs idle for
-// the last third. Causal 64 x 4096 x 4096 x 64: 246.8 -> 202.8 us.)
+// the last third. Causal 64 x 4096 x 4096 x 64: 246.8 -> 202.8 us.) Groups of 32 to 63 and of 128 to 255, over 20 causal problems of
+// 128 to 512 batches, N 1024 to 4096: heads of 64 1.02 and 0.97 of the time (128 x 1024: 1.10 and 1.05, 200 x 1024: 1.00 and
+// 0.91), heads of 128, whose B0 and B1 take twice the L2, 0.98 and 1.01.
 inline SlabOrder slab_order(int slabs, int batch)
 {
     const int wanted = batch >= 128 ? batch / 64 : 1;
