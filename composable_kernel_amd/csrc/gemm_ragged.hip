@@ -4,15 +4,34 @@
 
 namespace ckx {
 
+// The threads of a grid dimension are counted in 32 bits, and a launch past them wraps around without an error.
+constexpr long kMostBlocks = ((1l << 32) - 1) / 256;
+
 template <int DT, int B, bool TA, bool TB>
 static hipError_t launch_one(GemmArgs a, hipStream_t s)
 {
+    constexpr long es = DT == DT_I8 ? 1 : 2;
     a.tiles_m = (a.M + B - 1) / B, a.tiles_n = (a.N + B - 1) / B;
-    const long blocks = (long)a.tiles_m * a.tiles_n * (a.batch > 1 ? a.batch : 1);
-    if(blocks >= (1l << 31))
+    const long per_batch = (long)a.tiles_m * a.tiles_n, fit = kMostBlocks / per_batch;
+    if(fit < 1)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemm_ragged_kernel<DT, B, B, TA, TB>), linear_grid(blocks), dim3(256), 0, s, a);
-    return hipGetLastError();
+    // (more batches than fit a launch go out in launches of their own; an earlier 1 x 32769 x 1 in 65281 batches, 2^24 + 1 workgroups,
+    // computed one of them. A second grid dimension instead, with a check of its last row in the kernel, cost up to 2 % everywhere)
+    int left = a.batch > 1 ? a.batch : 1;
+    while(left > 0)
+    {
+        const int n = left < fit ? left : (int)fit;
+        a.batch     = n;
+        hipLaunchKernelGGL((gemm_ragged_kernel<DT, B, B, TA, TB>), dim3((unsigned)(per_batch * n)), dim3(256), 0, s, a);
+        const hipError_t e = hipGetLastError();
+        if(e != hipSuccess)
+            return e;
+        a.a = reinterpret_cast<const uint8_t*>(a.a) + n * a.bsa * es;
+        a.b = reinterpret_cast<const uint8_t*>(a.b) + n * a.bsb * es;
+        a.c = reinterpret_cast<uint8_t*>(a.c) + n * a.bsc * es;
+        left -= n;
+    }
+    return hipSuccess;
 }
 
 int ragged_tile(int M, int N, int batch)
@@ -27,7 +46,8 @@ int ragged_tile(int M, int N, int batch)
     // x 7) 116 us against 45, 2000 x (33 x 35 x 37) 17.7 against 8.4.
     const long n        = batch > 1 ? batch : 1;
     const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128) * n, tiles64 = (long)((M + 63) / 64) * ((N + 63) / 64) * n;
-    return tiles128 >= 256 && 10 * tiles128 <= 3 * tiles64 ? 128 : 64;
+    // (... or where one batch of the small ones is more than a launch holds)
+    return (tiles128 >= 256 && 10 * tiles128 <= 3 * tiles64) || tiles64 / n > kMostBlocks ? 128 : 64;
 }
 
 template <int DT, bool TA, bool TB>

@@ -28,7 +28,6 @@
 #pragma once
 
 #include "gemm_tile.hpp"
-#include "tile_launch.hpp"
 
 namespace ckx {
 
@@ -222,9 +221,7 @@ __global__ __launch_bounds__(256, 2) void gemm_ragged_kernel(const GemmArgs p)
     const int wm = wave >> 1, wn = wave & 1;
     const uint32_t frow = lane & 15, fq = lane >> 4;
     int g, tm, tn;
-    if(linear_block() >= (uint32_t)p.tiles_m * p.tiles_n * (p.batch > 1 ? p.batch : 1))
-        return;
-    tile_of_block((int)linear_block(), p.tiles_m, p.tiles_n, p.batch > 1 ? p.batch : 1, g, tm, tn);
+    tile_of_block((int)blockIdx.x, p.tiles_m, p.tiles_n, p.batch > 1 ? p.batch : 1, g, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
     const uint8_t* A = reinterpret_cast<const uint8_t*>(p.a) + (int64_t)g * p.bsa * ES;
     const uint8_t* B = reinterpret_cast<const uint8_t*>(p.b) + (int64_t)g * p.bsb * ES;
@@ -246,12 +243,10 @@ __global__ __launch_bounds__(256, 2) void gemm_ragged_kernel(const GemmArgs p)
         for(int t = 0; t < NTL; ++t)
             acc[i][t] = acc_t{0, 0, 0, 0};
 
-    auto multiply = [&](const uint8_t* s, int ksteps) {
+    auto multiply = [&](const uint8_t* s) {
 #pragma unroll
         for(int ks = 0; ks < 2; ++ks)
         {
-            if(ks >= ksteps)
-                break;
             i32x4 af[MT], bf[NTL];
 #pragma unroll
             for(int t = 0; t < NTL; ++t)
@@ -278,7 +273,7 @@ __global__ __launch_bounds__(256, 2) void gemm_ragged_kernel(const GemmArgs p)
     i32x4 ra0[OpA::NCH], rb0[OpB::NCH], ra1[OpA::NCH], rb1[OpB::NCH];
     // registers -> stage, the next load into the freed registers, multiply. One barrier per K tile: a stage is written
     // again only after the barrier of the tile in between, which every wave passes when it is done reading.
-    auto step = [&](int stage, i32x4(&ra)[OpA::NCH], i32x4(&rb)[OpB::NCH], int next, int ksteps = 2, bool across_a = false, bool across_b = false) {
+    auto step = [&](int stage, i32x4(&ra)[OpA::NCH], i32x4(&rb)[OpB::NCH], int next, bool across_a = false, bool across_b = false) {
         uint8_t* s = smem + stage * STAGE;
         opa.store_lds(s, tid, ra, across_a);
         opb.store_lds(s + OpA::BYTES, tid, rb, across_b);
@@ -288,7 +283,7 @@ __global__ __launch_bounds__(256, 2) void gemm_ragged_kernel(const GemmArgs p)
             opb.load(B, next, rb);
         }
         __syncthreads();
-        multiply(s, ksteps);
+        multiply(s);
     };
 
     // the checked K tiles: the last one, or all of them; the first unchecked ones are in flight meanwhile
@@ -305,8 +300,7 @@ __global__ __launch_bounds__(256, 2) void gemm_ragged_kernel(const GemmArgs p)
         i32x4 ra[OpA::NCH], rb[OpB::NCH];
         opa.load_checked(A, kt, tid, m0, p.M, p.K, p.lda, vec_a, ra);
         opb.load_checked(B, kt, tid, n0, p.N, p.K, p.ldb, vec_b, rb);
-        // (stages alternate, the last checked tile in stage 1; a second k-step past K is left out)
-        step((nk - 1 - kt) & 1 ? 0 : 1, ra, rb, -1, p.K - kt * KE <= KE / 2 ? 1 : 2, !vec_a, !vec_b);
+        step((nk - 1 - kt) & 1 ? 0 : 1, ra, rb, -1, !vec_a, !vec_b); // (stages alternate, the last checked tile in stage 1)
     }
     if(nfull > 0)
     {

@@ -38,16 +38,6 @@ inline int num_cus()
     return n;
 }
 
-// Grid of `blocks` workgroups (of up to 512 threads), one tile each: the threads along a grid dimension are counted in 32 bits,
-// and a launch past them wraps around without an error, so larger grids go on in y. linear_block() is the workgroup's number;
-// the last row of such a grid has numbers past `blocks`, whose workgroups leave at once.
-inline dim3 linear_grid(long blocks)
-{
-    constexpr long kRow = 1l << 22; // (a multiple of 8: workgroup b stays on XCD b % 8)
-    return blocks <= kRow ? dim3((unsigned)blocks) : dim3((unsigned)kRow, (unsigned)((blocks + kRow - 1) / kRow));
-}
-__device__ __forceinline__ uint32_t linear_block() { return blockIdx.y * gridDim.x + blockIdx.x; }
-
 // Persistent launch: at most (workgroups that fit a CU) x (CUs) workgroups, a multiple of 8 so
 // that workgroup b always lands on XCD b % 8 together with the tiles b, b + grid, ...
 template <int DT, int BM, int BN, int WM, int WN, int BKB, int NST, int IM2COL, bool TA = false, bool TB = false,
