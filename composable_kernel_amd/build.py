@@ -9,8 +9,7 @@ Three guards protect the kernels' hand-managed waits (the MFMA fragment reads of
 conv_pointwise.hpp are inline-assembly LDS reads that the compiler does not count in lgkmcnt; the kernels wait for
 them themselves, so no compiler-made copy or spill of such a register may run before that wait):
   * every kernel's register report (-Rpass-analysis=kernel-resource-usage) is read, and the build FAILS if one of
-    those kernels spills vector registers (the fused two-GEMM kernel, which reads LDS through compiler-known
-    builtins, is allowed its four spilled registers in the long-sequence softmax variant);
+    those kernels spills vector registers;
   * the four-wave GEMM body (gemm_w4.hpp) also issues its MFMAs and direct loads as inline assembly: its kernels must
     use no scratch memory and exactly the AccVGPRs the source ties accumulators to (a compiler that moved an
     accumulator or fragment through another register between the assembly and its wait would show up there);

@@ -13,7 +13,8 @@
 //   round-to-nearest-even conversion to fp16. B1 is transposed while it is staged into LDS
 //   so that its fragment is one 16-byte read as well.
 //
-// SOFTMAX variant (upstream's DeviceBatchedGemmSoftmaxGemm, "attention"):
+// SOFTMAX variant (upstream's DeviceBatchedGemmSoftmaxGemm, "attention") on 16 rows per wave, for problems too small to give every
+// SIMD two waves of 32 (gemm_softmax_gemm.hpp has the kernel for all others):
 //   C[g] = half( half(softmax_n(scale * A[g] * B0[g], masked)) * B1[g] )
 // with the softmax along N in one pass over N (running row maximum and running sum): a step's
 // scores become p = exp(s - running max), the output accumulators and the running sum are rescaled
@@ -163,23 +164,22 @@ struct GemmGemmCfg
     static_assert(NB0 >= 1 && NB1 >= 1, "too many threads for one step");
 };
 
-// Waves per SIMD that the registers are allocated for. The 32-row-per-wave softmax variant for small K and O is held to 256
-// registers, two waves per SIMD: one wave's exponentials then overlap the other's MFMAs; left alone the compiler takes 340 and
-// runs one. The 8-wave softmax variant for K up to 32 is held to 128, two workgroups per CU. The 8-wave variants past K or O of 64 take
-// more than 128 registers and a whole CU, two waves per SIMD, whatever they do: told so, the compiler spends up to 256 on reads
-// ahead instead of saving some for a third wave that no workgroup has. Without softmax K 64, O 128: 16 x 20 x 1000 17.2 -> 14.9
-// us, 60 x 300 x 256 8.0 -> 7.3; K 128, O 32 and K 32, O 128 0.88 and 0.94 of the time; with softmax level.
-constexpr int gemm_gemm_min_waves(int KS, int OG, int MT, int NW, bool SOFTMAX)
+// Waves per SIMD that the registers are allocated for. The 8-wave softmax variant for K up to 32 is held to 128, two workgroups per
+// CU. The 8-wave variants past K or O of 64 take more than 128 registers and a whole CU, two waves per SIMD, whatever they do: told
+// so, the compiler spends up to 256 on reads ahead instead of saving some for a third wave that no workgroup has. Without softmax
+// K 64, O 128: 16 x 20 x 1000 17.2 -> 14.9 us, 60 x 300 x 256 8.0 -> 7.3; K 128, O 32 and K 32, O 128 0.88 and 0.94 of the time; with
+// softmax level.
+constexpr int gemm_gemm_min_waves(int KS, int OG, int NW, bool SOFTMAX)
 {
     if(NW == 8 && (KS == 4 || OG == 2))
         return 2;
-    return !SOFTMAX || OG != 1 ? 1 : MT == 2 && KS <= 2 ? 2 : NW == 8 && KS == 1 ? 4 : 1;
+    return SOFTMAX && OG == 1 && NW == 8 && KS == 1 ? 4 : 1;
 }
 constexpr int gemm_gemm_max_waves(int KS, int OG, int NW) { return NW == 8 && (KS == 4 || OG == 2) ? 2 : 8; }
 
 template <int KS, int OG, int MT, int NW, bool SOFTMAX = false>
 __global__ __launch_bounds__(NW * 64)
-    __attribute__((amdgpu_waves_per_eu(gemm_gemm_min_waves(KS, OG, MT, NW, SOFTMAX), gemm_gemm_max_waves(KS, OG, NW)))) void gemm_gemm_kernel(
+    __attribute__((amdgpu_waves_per_eu(gemm_gemm_min_waves(KS, OG, NW, SOFTMAX), gemm_gemm_max_waves(KS, OG, NW)))) void gemm_gemm_kernel(
         const GemmGemmArgs p)
 {
     using Cfg = GemmGemmCfg<KS, OG, MT, NW>;
@@ -309,9 +309,8 @@ __global__ __launch_bounds__(NW * 64)
     // byte offsets of this lane's B0 fragments of score tiles 0 and 1: rows 8 * (fr / 4) + fr % 4 and 4 more. Tile t is 32 * (t / 2)
     // rows on, and neither step changes ab_key (bits 0, 1 and 3 of the row): immediates of the read. Worked out tile by tile
     // they became eight address registers and, in some of the kernels, a slower order of the step: without softmax 45 x 32 x
-    // 1046 x 16 9.6 -> 11.3 us, 12 x 54 x 3073 x 32 22.6 -> 28.1. (Two registers for K up to 32 in the plain 8-wave and in the
-    // softmax 32-row kernel, where one reads fewer fragments ahead: plain 231 x 45 x 2741 x 16 20.8 -> 20.0, 57 x 1934 x 61 x 32 7.3
-    // -> 7.4, 7.7 with eight; softmax 128 x 2539 x 2539 x 32 238.9 -> 235.5, 19 x 3046 x 3046 causal 42.9 -> 42.4.)
+    // 1046 x 16 9.6 -> 11.3 us, 12 x 54 x 3073 x 32 22.6 -> 28.1. (Two registers for K up to 32 in the plain 8-wave
+    // kernel, where one reads fewer fragments ahead: 231 x 45 x 2741 x 16 20.8 -> 20.0, 57 x 1934 x 61 x 32 7.3 -> 7.4, 7.7 with eight.)
     uint32_t b0_lane[KS][2];
 #pragma unroll
     for(int ks = 0; ks < KS; ++ks)
@@ -319,7 +318,7 @@ __global__ __launch_bounds__(NW * 64)
         const uint32_t row = (uint32_t)(8 * (fr >> 2) + (fr & 3));
         b0_lane[ks][0]     = row * Cfg::AST + ((uint32_t)(ks * 4 + q) ^ Cfg::ab_key(row)) * 16;
         b0_lane[ks][1]     = b0_lane[ks][0] + 4 * Cfg::AST;
-        if constexpr(KS == 1 && (SOFTMAX ? MT == 2 : NW == 8))
+        if constexpr(KS == 1 && !SOFTMAX && NW == 8)
             asm volatile("" : "+v"(b0_lane[ks][1]));
     }
 
@@ -356,19 +355,16 @@ __global__ __launch_bounds__(NW * 64)
     // The softmax step is compiled in three forms, chosen per step and wave (wave-uniform): without a masked column it is straight-line
     // code without compares; with masked columns in all of its four 32-column pairs it compares, in straight-line code still; past
     // the wave's last unmasked column (EDGE) the pairs that lie there are left out, behind branches. With the first and the last:
-    // 32 x 2048 x 2048 x 128 147.0 -> 138.4 us, causal 56.0 -> 53.6; 100 x 1000 x 1500 x 80 97.0 -> 93.7; causal 200 x 300 x 300 x 128
-    // 27.0 -> 26.0. With the middle one, which most steps of a single-step problem and the last of N % 128 > 96 take: 26 x 66 x
-    // 121 x 64 4.83 -> 4.62, 53 x 226 x 363 x 64 -> 128 11.3 -> 10.7; not for K and O past 64, whose other forms it slows down: 206 x 1803
-    // x 1803 x 128 560 -> 582.
-    // RAISE: MFMA sections at raised wave priority, so that the other wave of the SIMD does its softmax meanwhile: with K of 33
-    // to 64 355.8 -> 348.3 us at 64 x 4096 x 4096 x 64 (without the forms 351.9 -> 344.6); slower with K of 72 ... 128
-    // (32 x 2048 x 2048 x 72 90.2 -> 91.8, x 96 90.4 -> 92.8, x 128 93.3 -> 94.6; causal 64 x 1024 x 1024 x 80 32.2 -> 32.4) and 32 (72.1
-    // -> 73.0) and without softmax (128 x 1024 x 1024 x 64 38.2 -> 39.2).
+    // causal 200 x 300 x 300 x 128 27.0 -> 26.0 us. With the middle one, which most steps of a single-step problem and the last of
+    // N % 128 > 96 take: 26 x 66 x 121 x 64 4.83 -> 4.62, 53 x 226 x 363 x 64 -> 128 11.3 -> 10.7; not for K and O past 64, whose
+    // other forms it slows down (206 x 1803 x 1803 x 128 560 -> 582).
+    // RAISE: MFMA sections at raised wave priority, so that the other wave of the SIMD does its softmax meanwhile: faster with K of
+    // 33 to 64, slower with K of 72 ... 128 (32 x 2048 x 2048 x 128 93.3 -> 94.6) and 32 and without softmax (128 x 1024 x 1024 x 64
+    // 38.2 -> 39.2).
     constexpr bool RAISE = SOFTMAX && KS == 2;
     // One form, with the compares behind a branch, where more forms' registers cost a co-resident workgroup: 8 waves with
-    // K up to 32 and O up to 64 (122 registers, 150 with two forms: 200 x 500 x 500 x 32 24.4 -> 32.7 us, 256 x 2000 x 300 x 32 69 ->
-    // 93) and the 64-row instances.
-    constexpr bool FORMS = SOFTMAX && (NW == 8 ? !(KS == 1 && OG == 1) : MT == 2);
+    // K up to 32 and O up to 64 (122 registers, 150 with two forms: 200 x 500 x 500 x 32 24.4 -> 32.7 us) and the 64-row instances.
+    constexpr bool FORMS = SOFTMAX && NW == 8 && !(KS == 1 && OG == 1);
     constexpr bool MIDDLE_FORM = FORMS && !(KS == 4 && OG == 2);
     const int wave_m0    = m0 + wave * 16 * MT;
     const int wave_n_end = (p.mask_upper && wave_m0 + 16 * MT < p.N) ? wave_m0 + 16 * MT : p.N;
@@ -502,8 +498,32 @@ inline SlabOrder slab_order(int slabs, int batch)
     return SlabOrder{make_magic((uint32_t)size * (uint32_t)slabs), make_magic((uint32_t)size), make_magic((uint32_t)(batch - (groups - 1) * size)), groups};
 }
 
+template <int BM, int NT, int LDS>
+inline hipError_t gemm_gemm_launch_kernel(void (*kern)(GemmGemmArgs), GemmGemmArgs a, hipStream_t s)
+{
+    a.slabs = (a.M + BM - 1) / BM;
+    // (the threads of a grid dimension are counted in 32 bits, and a launch past them wraps around without an error: more batches
+    // than fit go out in launches of their own, whole groups of eight of them for the XCD mapping)
+    const long fit = ((1l << 32) - 1) / NT / a.slabs;
+    if(fit < 1)
+        return hipErrorInvalidValue;
+    const int most = (int)(fit >= a.batch ? a.batch : fit >= 8 ? fit & ~7l : fit);
+    for(int left = a.batch; left > 0; left -= most)
+    {
+        a.batch = left < most ? left : most;
+        if(a.mask_upper)
+            a.order = slab_order(a.slabs, a.batch);
+        hipLaunchKernelGGL(kern, dim3(a.slabs * a.batch), dim3(NT), LDS, s, a);
+        const hipError_t e = hipGetLastError();
+        if(e != hipSuccess)
+            return e;
+        a.a += most * a.bsa, a.b0 += most * a.bsb0, a.b1 += most * a.bsb1, a.c += most * a.bsc;
+    }
+    return hipSuccess;
+}
+
 template <int KS, int OG, int MT, int NW, bool SOFTMAX>
-inline hipError_t gemm_gemm_launch_t(GemmGemmArgs a, hipStream_t s)
+inline hipError_t gemm_gemm_launch_t(const GemmGemmArgs& a, hipStream_t s)
 {
     using Cfg  = GemmGemmCfg<KS, OG, MT, NW>;
     auto* kern = &gemm_gemm_kernel<KS, OG, MT, NW, SOFTMAX>;
@@ -515,25 +535,7 @@ inline hipError_t gemm_gemm_launch_t(GemmGemmArgs a, hipStream_t s)
     });
     if(attr_err != hipSuccess)
         return attr_err;
-    a.slabs = (a.M + Cfg::BM - 1) / Cfg::BM;
-    // (the threads of a grid dimension are counted in 32 bits, and a launch past them wraps around without an error: more batches
-    // than fit go out in launches of their own, whole groups of eight of them for the XCD mapping)
-    const long fit = ((1l << 32) - 1) / Cfg::NT / a.slabs;
-    if(fit < 1)
-        return hipErrorInvalidValue;
-    const int most = (int)(fit >= a.batch ? a.batch : fit >= 8 ? fit & ~7l : fit);
-    for(int left = a.batch; left > 0; left -= most)
-    {
-        a.batch = left < most ? left : most;
-        if(a.mask_upper)
-            a.order = slab_order(a.slabs, a.batch);
-        hipLaunchKernelGGL(kern, dim3(a.slabs * a.batch), dim3(Cfg::NT), Cfg::LDS, s, a);
-        const hipError_t e = hipGetLastError();
-        if(e != hipSuccess)
-            return e;
-        a.a += most * a.bsa, a.b0 += most * a.bsb0, a.b1 += most * a.bsb1, a.c += most * a.bsc;
-    }
-    return hipSuccess;
+    return gemm_gemm_launch_kernel<Cfg::BM, Cfg::NT, Cfg::LDS>(kern, a, s);
 }
 
 template <int MT, int NW, bool SOFTMAX>
@@ -546,6 +548,28 @@ inline hipError_t gemm_gemm_launch_mt(const GemmGemmArgs& g, hipStream_t s)
     if(ks == 2)
         return og == 1 ? gemm_gemm_launch_t<2, 1, MT, NW, SOFTMAX>(g, s) : gemm_gemm_launch_t<2, 2, MT, NW, SOFTMAX>(g, s);
     return og == 1 ? gemm_gemm_launch_t<4, 1, MT, NW, SOFTMAX>(g, s) : gemm_gemm_launch_t<4, 2, MT, NW, SOFTMAX>(g, s);
+}
+
+hipError_t gemm_softmax_gemm_launch(const GemmGemmArgs& a, hipStream_t s); // gemm_softmax_gemm.hip
+
+// Attention on waves of 16 rows (instance 2) instead of 32 (instance 0). Up to 256 slabs of 128 rows there is one workgroup to a CU: one
+// wave of 32 rows per SIMD, or two of 16, and the launch lasts as long as one wave's chain of steps. The shorter chain wins then, up to an
+// N from which the 32-row kernel's faster steps do; with heads past 96 at any N, and with the mask, whose launch ends with its longest
+// slabs alone on their CUs, up to 512 slabs. From there on, and with heads of 65 to 96, which the 16-row kernel pads to 128, 32 rows.
+// 16 / 32 rows, us: heads of 64: 64 x 512 x 512 10.6 / 11.2, 128 x 256 x 256 7.2 / 8.0, 42 x 768 x 768 causal 13.4 / 14.4, 8 x 1024 x 1024
+// causal 15.5 / 15.8, but 32 x 1024 x 1024 19.6 / 17.3, 5 x 1536 x 1536 21.8 / 21.2, 175 x 512 x 512 33.2 / 26.7, 350 x 256 x 256 21.4 / 18.2;
+// heads of 128: 64 x 512 x 512 17.1 / 18.1, 21 x 1536 x 1536 causal 37.9 / 38.6, 35 x 1362 x 1362 causal 37.5 / 40.2, but 36 x 1384 x 1384
+// 72.0 / 54.6, 63 x 1357 x 1357 causal 67.9 / 51.2; heads of 32: 128 x 256 x 256 5.6 / 5.8, but 64 x 512 x 512 8.3 / 8.1, 32 x 1024 x 1024
+// 15.6 / 12.5; of 80: 32 x 256 x 256 8.6 / 7.9.
+inline bool rows_in_16s(int M, int N, int K, int O, int batch, bool mask_upper)
+{
+    const int head   = K > O ? K : O;
+    const long slabs = (long)batch * ((M + 127) / 128);
+    if(head > 96)
+        return slabs <= (mask_upper ? 512 : 256);
+    if(mask_upper && head > 32 && head <= 64 && N <= 512) // (130 x 375 x 375 13.2 / 13.8 us)
+        return slabs <= 512;
+    return slabs <= 256 && (head > 64 ? false : head > 32 ? N <= (slabs <= 128 ? 1024 : 960) : N < 448);
 }
 
 // softmax: the attention variant with scores scale * (A * B0) and the optional upper-triangle mask
@@ -561,24 +585,25 @@ inline hipError_t gemm_gemm_launch(const void* a, const void* b0, const void* b1
     g.bsa = bsa, g.bsb0 = bsb0, g.bsb1 = bsb1, g.bsc = bsc;
     g.slabs = 0, g.order = SlabOrder{};
     g.scale = scale, g.mask_upper = mask_upper;
-    if(instance < 0)
-    {
-        // Many short waves (8 x 16 rows, the instance with two steps of prefetch where registers allow) are ahead on
-        // short problems: G 64, 512 x 64 x 512 x 64 plain 8.5 against 10.1 us, with softmax 10.9 against 13.0. Over a
-        // long N with small heads the 32-row waves read the B0 / B1 fragments half as often per row and win: G 64,
-        // 4096 x 64 x 4096 x 64 plain 267 against 302 us, softmax 367 against 433 (2048: 76 / 85 and 102 / 115; at
-        // N = 1024 plain 23.5 / 26.2, softmax 31.3 / 34.0).
-        // That needs workgroups to spare (two of them share a CU): below 256 slabs of 128 rows the 8-wave instance
-        // stays ahead with softmax (G 8, 2048 x 64 x 2048 x 64: 30.1 against 37.2 us), and without it, up to 128
-        // slabs of small heads, the 64-row instance, which doubles the workgroups (20.6 against 25.4 us).
-        const long slabs128 = (long)batch * ((M + 127) / 128);
-        const bool small_heads = K <= 64 && O <= 64;
-        instance = (!softmax && small_heads && slabs128 <= 128) ? 1 : (small_heads && N >= 1024 && slabs128 >= 256) ? 0 : 2;
-    }
     if(softmax)
-        return instance == 0 ? gemm_gemm_launch_mt<2, 4, true>(g, s)
+    {
+        if(instance < 0)
+            instance = rows_in_16s(M, N, K, O, batch, mask_upper) ? 2 : 0;
+        return instance == 0   ? gemm_softmax_gemm_launch(g, s)
                : instance == 1 ? gemm_gemm_launch_mt<1, 4, true>(g, s)
                                : gemm_gemm_launch_mt<1, 8, true>(g, s);
+    }
+    if(instance < 0)
+    {
+        // Many short waves (8 x 16 rows, the instance with two steps of prefetch where registers allow) are ahead on short
+        // problems: G 64, 512 x 64 x 512 x 64 8.5 against 10.1 us. Over a long N with small heads the 32-row waves read the B0 / B1
+        // fragments half as often per row and win: G 64, 4096 x 64 x 4096 x 64 267 against 302 us (2048: 76 / 85; at N = 1024
+        // 23.5 / 26.2). That needs workgroups to spare (two of them share a CU): up to 128 slabs of small heads the 64-row instance,
+        // which doubles the workgroups, is ahead (20.6 against 25.4 us).
+        const long slabs128 = (long)batch * ((M + 127) / 128);
+        const bool small_heads = K <= 64 && O <= 64;
+        instance = small_heads && slabs128 <= 128 ? 1 : small_heads && N >= 1024 && slabs128 >= 256 ? 0 : 2;
+    }
     return instance == 0 ? gemm_gemm_launch_mt<2, 4, false>(g, s)
            : instance == 1 ? gemm_gemm_launch_mt<1, 4, false>(g, s)
                            : gemm_gemm_launch_mt<1, 8, false>(g, s);

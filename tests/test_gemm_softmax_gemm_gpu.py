@@ -98,6 +98,76 @@ def test_gemm_softmax_gemm_edge_pairs(N, K):
             _close(_run(a, b0_gnk, b1, 0.3, mask, instance), ref)
 
 
+@pytest.mark.parametrize("K, O", [(32, 32), (16, 64), (64, 64), (72, 40), (80, 80), (96, 96), (24, 104), (128, 32), (128, 128), (32, 128)])
+def test_gemm_softmax_gemm_units(K, O):
+    """The 32-row kernel walks N in units of 64 columns (32 with K past 96 or O past 96), the first, an even number in the middle and
+    the last ones in code of their own: N around whole units, one to more than six of them, rows past the last wave's."""
+    for N in (1, 63, 64, 65, 127, 129, 191, 193, 257, 320, 385):
+        a, b0_gnk, b1 = (uniform_f16((2, x, y), -1, 1, 1970 + i) for i, (x, y) in enumerate(((133, K), (N, K), (N, O))))
+        for mask in (False, True):
+            _close(_run(a, b0_gnk, b1, 2.0 * K ** -0.5, mask, 0),
+                   lit.batched_gemm_softmax_gemm_f16(a, b0_gnk.transpose(0, 2, 1), b1, 2.0 * K ** -0.5, mask))
+
+
+@pytest.mark.parametrize("step", [0.01, 0.05, 0.2, 1.0])
+def test_gemm_softmax_gemm_growing_scores(step):
+    """The 32-row kernel rescales a unit after the maximum has risen, once the unit before has been added: scores that rise by step per
+    column, so that every unit raises it, in one row of a wave or in all of them. Against float64, within four times the difference
+    measured for scores that do not rise (2.5e-4 of the 2-norm; a probability is rounded to 2^-11 of itself)."""
+    G, M, N, K, O = 1, 96, 640, 16, 64
+    a = uniform_f16((G, M, K), -1, 1, 31)
+    a[..., 0] = 0
+    b0 = uniform_f16((G, N, K), -1, 1, 32)
+    b0[0, :, 0] = (step * np.arange(N)).astype(np.float16)
+    b1 = uniform_f16((G, N, O), -1, 1, 33)
+    for rows in (slice(0, M), slice(37, 38)):
+        x = a.copy()
+        x[0, rows, 0] = 1
+        for mask in (False, True):
+            s = x[0].astype(np.float64) @ b0[0].astype(np.float64).T
+            if mask:
+                s = np.where(np.arange(N)[None, :] > np.arange(M)[:, None], -np.inf, s)
+            p = np.exp(s - s.max(axis=1, keepdims=True))
+            ref = (p / p.sum(axis=1, keepdims=True)) @ b1[0].astype(np.float64)
+            out = _run(x, b0, b1, 1.0, mask, 0)[0].astype(np.float64)
+            assert np.linalg.norm(out - ref) <= 1e-3 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("instance", [0, 2])
+def test_gemm_softmax_gemm_nan_stays_in_its_row(instance):
+    """A NaN in a row of A reaches that row of C only, and an infinity in a row of B1 that is masked for a whole wave reaches none of
+    that wave's rows."""
+    G, M, N, K, O = 1, 256, 256, 64, 64
+    a, b0, b1 = (uniform_f16((G, x, 64), -1, 1, 41 + i) for i, x in enumerate((M, N, N)))
+    clean = _run(a, b0, b1, 0.125, True, instance)
+    for row in (0, 5, 21, 100, 255):
+        x = a.copy()
+        x[0, row, 3] = np.nan
+        out = _run(x, b0, b1, 0.125, True, instance)
+        assert np.all(np.isnan(out[0, row]))
+        keep = np.arange(M) != row
+        np.testing.assert_array_equal(out[0, keep].view(np.uint16), clean[0, keep].view(np.uint16))
+    for n in (32, 96, 224):
+        x = b1.copy()
+        x[0, n] = np.inf
+        out = _run(a, b0, x, 0.125, True, instance)
+        np.testing.assert_array_equal(out[0, :n].view(np.uint16), clean[0, :n].view(np.uint16))
+
+
+@pytest.mark.parametrize("G, M, N, K, mask, rows", [(2, 64, 1024, 64, False, 16), (2, 64, 1025, 64, False, 32), (129, 64, 960, 64, False, 16),
+                                                    (129, 64, 961, 64, False, 32), (512, 40, 64, 64, True, 16), (513, 40, 64, 64, True, 32),
+                                                    (257, 40, 513, 64, True, 32),
+                                                    (256, 100, 64, 128, False, 16), (257, 100, 64, 128, False, 32), (512, 40, 64, 128, True, 16),
+                                                    (513, 40, 64, 128, True, 32), (2, 64, 447, 32, False, 16), (2, 64, 448, 32, False, 32),
+                                                    (2, 64, 64, 80, False, 32), (2, 64, 64, 96, True, 32)])
+def test_gemm_softmax_gemm_auto_on_both_sides_of_its_rule(G, M, N, K, mask, rows):
+    """AUTO takes 16-row waves for few slabs of a short N, 32-row waves otherwise: bit for bit one of the two."""
+    a, b0, b1 = (uniform_f16((G, x, K), -1, 1, 51 + i) for i, x in enumerate((M, N, N)))
+    out = _run(a, b0, b1, K ** -0.5, mask)
+    np.testing.assert_array_equal(out.view(np.uint16), _run(a, b0, b1, K ** -0.5, mask, 2 if rows == 16 else 0).view(np.uint16))
+    _close(out[:2], lit.batched_gemm_softmax_gemm_f16(a[:2], b0[:2].transpose(0, 2, 1), b1[:2], K ** -0.5, mask))
+
+
 def test_gemm_softmax_gemm_closed_forms():
     """Zero scores: the uniform distribution, C = mean of B1's rows (exact: small integers over a power of
     two). Upper-triangle mask: row m averages rows 0..m, row 0 is B1[0] exactly. A dominant score selects
