@@ -664,7 +664,7 @@ __device__ __forceinline__ void store_row16_f16_fused(_Float16* crow, int n0, in
 // launches which never run it need not pay for. Its K loop is the plain one as long as the epilogue awaits
 // its D loads explicitly (see d_values_landed there).
 template <int DT, int BM, int BN, int WM, int WN, int BKB, int NST, int IM2COL, bool TA = false, bool TB = false,
-          bool FUSED = false>
+          bool FUSED = false, bool AHEAD = false>
 struct GemmTile
 {
     static constexpr int NW      = WM * WN;
@@ -692,7 +692,18 @@ struct GemmTile
     static constexpr int LDS_CU  = 160 * 1024;
     static constexpr bool USE_LUT = DT == DT_I8 && LDS_CU / (NST * STAGE) == LDS_CU / (NST * STAGE + 256);
     static constexpr int LUT     = USE_LUT ? 256 : 0;
-    static constexpr int LDS     = NST * STAGE + LUT;
+    // A third stage for the A tiles, which fills the LDS of a CU with the 256 x 256 tile's 64 KB stages: the loads of A are a K tile
+    // further ahead than those of B and have one more to arrive in. For strided convolutions, whose filter taps share few pixels: most
+    // of a K tile's A comes from beyond the L2 then and takes longer than the half to one K tile that two stages leave it (128 x 71 x 71, C
+    // 192 -> K 256, 3 x 3 stride 2, bias + ReLU 159 -> 152.6 us; 122 x 58 x 58, C 208 -> K 256 stride 2 116.5 -> 108.8). With unit stride the
+    // L2 has the pixels and the second load cursor costs up to 2 % (223 x 15 x 15, C 448 -> K 256 97.8 -> 99.7), as it does with dense K-major
+    // operands (f16 4096^3 km_nk 105.8 -> 107.1).
+    static_assert(!AHEAD || (ES == 2 && NST == 2), "the int8 epilogue's table finds no room");
+    static constexpr int NSTA     = NST + (AHEAD ? 1 : 0);
+    static constexpr int LDS      = NSTA * A_TILE + NST * B_TILE + LUT;
+    // LDS offsets of the stages: with as many of both kinds a K tile's A and B lie side by side, else all A tiles come first
+    __device__ static __forceinline__ int a_stage(int st) { return AHEAD ? st * A_TILE : st * STAGE; }
+    __device__ static __forceinline__ int b_stage(int st) { return AHEAD ? NSTA * A_TILE + st * B_TILE : st * STAGE + A_TILE; }
     // Workgroups of this instance that a CU's LDS and thread slots hold -- what launch_tile() sizes the persistent grid for --
     // and the waves per SIMD they come to. The register allocator is held to that many: a few registers more and the second
     // workgroup of every CU runs after the first instead of beside it. Left alone it gave fp16 128 x 128 with D operands 265
@@ -765,7 +776,7 @@ struct GemmTile
         {
             // (visible to every wave after the prologue's barrier, long before the first epilogue)
             if(p.epi == EPI_REQUANT_RND && p.ksplit == 1)
-                requant_lut_fill(smem + NST * STAGE, p.scale_relu, tid, NT);
+                requant_lut_fill(smem + LDS - LUT, p.scale_relu, tid, NT);
         }
 
         // ---- per-thread load slots -------------------------------------------------
@@ -783,7 +794,7 @@ struct GemmTile
         const uint32_t trow_b = TB ? (uint32_t)(wave * (1024 / (BN * ES)) + lane / (BN * ES / 16)) : 0u;
 
         // row / column offsets of the tile the LOAD cursor is on (tile >= ntiles: nothing valid)
-        auto setup_tile = [&](int tile_id) {
+        auto setup_tile = [&](int tile_id, auto with_a, auto with_b) {
             int tm = 0, tn = 0;
             const bool live = tile_id < ntiles_all;
             int g           = 0;
@@ -791,7 +802,7 @@ struct GemmTile
                 tile_of_block(tile_id, p.tiles_m, p.tiles_n, nbatch, g, tm, tn);
             const uint32_t a_batch = (uint32_t)((long)g * p.bsa * ES), b_batch = (uint32_t)((long)g * p.bsb * ES);
 #pragma unroll
-            for(int j = 0; j < NLA; ++j)
+            for(int j = 0; j < (decltype(with_a)::value ? NLA : 0); ++j)
             {
                 if constexpr(TA)
                 {
@@ -855,7 +866,7 @@ struct GemmTile
                 }
             }
 #pragma unroll
-            for(int j = 0; j < NLB; ++j)
+            for(int j = 0; j < (decltype(with_b)::value ? NLB : 0); ++j)
             {
                 if constexpr(TB)
                 {
@@ -879,7 +890,8 @@ struct GemmTile
         {
             uint8_t* sa;
             uint8_t* sb;
-            uint32_t k0;      // byte offset of the K tile
+            uint32_t k0;      // byte offset of the K tile (k0_b, k_oob_b: of B's, where A's loads are a K tile ahead)
+            uint32_t k0_b, k_oob_b;
             uint32_t k0a, k0b; // K-major operands: byte offset of the K tile's first k row
             int klim;          // K-major operands: k rows of this K tile that exist
             uint32_t k_oob;   // top bit set for chunks past K: OR-ed into the offset (arithmetic on
@@ -889,12 +901,14 @@ struct GemmTile
             uint32_t tap_off;
             bool tap_ok;
         };
-        auto load_ctx = [&](int kt, int stage) {
+        auto load_ctx = [&](int kt, int stage, int kt_b, int stage_b) {
             LoadCtx c;
-            c.sa    = smem + stage * STAGE;
-            c.sb    = c.sa + A_TILE;
+            c.sa    = smem + a_stage(stage);
+            c.sb    = AHEAD ? smem + b_stage(stage_b) : c.sa + A_TILE;
             c.k0    = (uint32_t)kt * BKB;
+            c.k0_b  = AHEAD ? (uint32_t)kt_b * BKB : c.k0;
             c.k_oob = (c.k0 + kb < kbytes) ? 0u : kOutOfRange;
+            c.k_oob_b = AHEAD ? (c.k0_b + kb < kbytes ? 0u : kOutOfRange) : c.k_oob;
             c.k0a   = TA ? (uint32_t)kt * KE * (uint32_t)p.lda * ES : 0u;
             c.k0b   = TB ? (uint32_t)kt * KE * (uint32_t)p.ldb * ES : 0u;
             c.klim  = p.K - kt * KE;
@@ -948,18 +962,11 @@ struct GemmTile
                 const int j         = slot - NLA;
                 const uint32_t voff =
                     TB ? (b_off[j] + c.k0b) | (~(uint32_t)((int)(trow_b + j * NW * (1024 / (BN * ES))) - c.klim) & kOutOfRange)
-                       : b_off[j] | c.k_oob;
+                       : b_off[j] | c.k_oob_b;
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (lds_ptr_t)(c.sb + (j * NW + wave) * 1024), 16,
-                                                         voff, TB ? 0 : (int)c.k0, 0, 0);
+                                                         voff, TB ? 0 : (int)c.k0_b, 0, 0);
             }
         };
-        auto issue_loads = [&](int kt, int stage) {
-            const LoadCtx c = load_ctx(kt, stage);
-#pragma unroll
-            for(int sl = 0; sl < LPT; ++sl)
-                issue_slot(c, sl);
-        };
-
         // A work unit is (K run s, C tile id): unit = s * ntiles_all + id, K tiles [s*nk_per, ...).
         const int nunits = ntiles_all * p.ksplit;
         auto unit_k_range = [&](int unit, int& k_begin, int& k_end) {
@@ -967,19 +974,37 @@ struct GemmTile
             k_begin      = sp * p.nk_per;
             k_end        = k_begin + p.nk_per < nk ? k_begin + p.nk_per : nk;
         };
-        // load cursor: (unit, kt) of the next K tile to request
-        int ld_unit = (int)blockIdx.x, ld_kt = 0, ld_end = nk;
-        unit_k_range(ld_unit, ld_kt, ld_end);
-        setup_tile(ld_unit < nunits ? ld_unit % ntiles_all : ntiles_all);
+        // load cursor: (unit, kt) of the next K tile to request. With AHEAD there are two, and A's is one K tile further: the loads
+        // of B have the time from this K tile's second half to the next one's middle, those of A a whole K tile more.
+        using std::false_type;
+        using std::true_type;
+        struct Cursor
+        {
+            int unit, kt, end;
+        };
+        auto tile_of_unit = [&](int unit) { return unit < nunits ? unit % ntiles_all : ntiles_all; };
+        Cursor ld{(int)blockIdx.x, 0, nk}, ld_b;
+        unit_k_range(ld.unit, ld.kt, ld.end);
+        ld_b = ld;
+        setup_tile(tile_of_unit(ld.unit), true_type{}, true_type{});
         // (kept apart from the issue itself: the branch would split the basic block in which the
         // loads are interleaved with MFMAs)
-        auto advance_load_cursor = [&]() {
-            if(++ld_kt >= ld_end)
+        auto advance = [&](Cursor& c, auto with_a, auto with_b) {
+            if(++c.kt >= c.end)
             {
-                ld_unit += gstride;
-                unit_k_range(ld_unit, ld_kt, ld_end);
-                setup_tile(ld_unit < nunits ? ld_unit % ntiles_all : ntiles_all);
+                c.unit += gstride;
+                unit_k_range(c.unit, c.kt, c.end);
+                setup_tile(tile_of_unit(c.unit), with_a, with_b);
             }
+        };
+        auto advance_load_cursor = [&]() {
+            if constexpr(AHEAD)
+            {
+                advance(ld, true_type{}, false_type{});
+                advance(ld_b, false_type{}, true_type{});
+            }
+            else
+                advance(ld, true_type{}, true_type{});
         };
 
         // ---- accumulators ------------------------------------------------------------
@@ -1025,20 +1050,21 @@ struct GemmTile
         // fragments and the first A fragment feed the first MFMA group, the last A fragment only
         // the last one, so the LDS latency of the late reads hides under the early groups.
         // stage_lds: LDS address of the stage.
-        auto read_one = [&](uint32_t stage_lds, auto ks_c, auto r_c, i32x4(&af)[MT], i32x4(&bf)[NG * 4]) {
+        constexpr int BIMM = AHEAD ? 0 : A_TILE; // (B's tile of the stage)
+        auto read_one = [&](uint32_t stage_lds, uint32_t stage_lds_b, auto ks_c, auto r_c, i32x4(&af)[MT], i32x4(&bf)[NG * 4]) {
             constexpr int KS = decltype(ks_c)::value, R = decltype(r_c)::value;
             if constexpr(R < NG * 4)
             {
-                const uint32_t base = stage_lds + (KS ? fb1 : fb0);
+                const uint32_t base = (AHEAD ? stage_lds_b : stage_lds) + (KS ? fb1 : fb0);
                 if constexpr(TB)
                 {
                     const uint32_t a = base ^ ((uint32_t)R << SEGSH);
-                    const i32x2 lo   = lds_read_tr_b64<ES, A_TILE + KS * TKS * BN * ES>(a);
-                    const i32x2 hi   = lds_read_tr_b64<ES, A_TILE + (KS * TKS + THALF) * BN * ES>(a);
+                    const i32x2 lo   = lds_read_tr_b64<ES, BIMM + KS * TKS * BN * ES>(a);
+                    const i32x2 hi   = lds_read_tr_b64<ES, BIMM + (KS * TKS + THALF) * BN * ES>(a);
                     bf[R]            = i32x4{lo[0], lo[1], hi[0], hi[1]};
                 }
                 else
-                    bf[R] = lds_read_b128<A_TILE + R * 16 * BKB>(base);
+                    bf[R] = lds_read_b128<BIMM + R * 16 * BKB>(base);
             }
             else
             {
@@ -1102,7 +1128,7 @@ struct GemmTile
         // fills the texture-address FIFOs (SQ_VMEM_TA_ADDR/CMD_FIFO_FULL), the in-order wave blocks
         // on VMEM issue, and its MFMAs wait behind it.
         auto half_step = [&](auto with_loads, const LoadCtx& lc, const i32x4(&caf)[MT], const i32x4(&cbf)[NG * 4],
-                             uint32_t nstage_lds, auto nks, i32x4(&naf)[MT], i32x4(&nbf)[NG * 4]) {
+                             uint32_t nstage_lds, uint32_t nstage_lds_b, auto nks, i32x4(&naf)[MT], i32x4(&nbf)[NG * 4]) {
             // The reads are over two groups before the end of the half; the first half of an iteration
             // starts its reads one group late.
             constexpr int NGRP = LPT, NR = MT + NG * 4, NM = MT * NG * 4;
@@ -1111,12 +1137,12 @@ struct GemmTile
             static_for<NGRP>([&](auto g_c) {
                 constexpr int g = decltype(g_c)::value;
                 if constexpr(decltype(with_loads)::value)
-                    issue_slot(lc, g);
+                    issue_slot(lc, AHEAD ? (g < NLB ? NLA + g : g - NLB) : g); // (AHEAD: B first, whose wait is the shorter)
                 constexpr int gr = g - RG0 < 0 ? 0 : (g - RG0 > RG ? RG : g - RG0); // read groups done before g
                 constexpr int gn = g + 1 - RG0 < 0 ? 0 : (g + 1 - RG0 > RG ? RG : g + 1 - RG0);
                 constexpr int r0 = gr * NR / RG, r1 = gn * NR / RG;
                 static_for<r1 - r0>([&](auto r_c) {
-                    read_one(nstage_lds, nks, std::integral_constant<int, r0 + decltype(r_c)::value>{}, naf, nbf);
+                    read_one(nstage_lds, nstage_lds_b, nks, std::integral_constant<int, r0 + decltype(r_c)::value>{}, naf, nbf);
                 });
 #pragma unroll
                 for(int m = g * NM / NGRP; m < (g + 1) * NM / NGRP; ++m)
@@ -1201,7 +1227,7 @@ struct GemmTile
                                                 acc[i][g * 4 + 3]};
                             if(p.epi == EPI_REQUANT_RND && USE_LUT)
                                 store_row16_i8_lut(crow, n0, p.N, v, p.scale_gemm,
-                                                   (uint32_t)(uintptr_t)(lds_ptr_t)smem + (uint32_t)(NST * STAGE), nt, whole);
+                                                   (uint32_t)(uintptr_t)(lds_ptr_t)smem + (uint32_t)(LDS - LUT), nt, whole);
                             else if(p.epi == EPI_REQUANT_RND)
                                 store_row16_i8<EPI_REQUANT_RND>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu, nt, whole);
                             else if(p.epi == EPI_REQUANT_CK)
@@ -1392,23 +1418,37 @@ struct GemmTile
 #pragma unroll
         for(int st = 0; st < NST; ++st)
         {
-            issue_loads(ld_kt, st);
+            const LoadCtx c = load_ctx(ld.kt, st, ld_b.kt, st);
+#pragma unroll
+            for(int sl = 0; sl < LPT; ++sl)
+                issue_slot(c, sl);
             advance_load_cursor();
         }
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 1) * LPT) : "memory");
+        if constexpr(AHEAD)
+        {
+            const LoadCtx c = load_ctx(ld.kt, NST, 0, 0);
+#pragma unroll
+            for(int sl = 0; sl < NLA; ++sl)
+                issue_slot(c, sl);
+            advance(ld, true_type{}, false_type{});
+        }
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 1) * LPT + (NSTA - NST) * NLA) : "memory");
         barrier();
-        static_for<MT + NG * 4>([&](auto r_c) { read_one(smem_lds, std::integral_constant<int, 0>{}, r_c, af0, bf0); });
+        static_for<MT + NG * 4>([&](auto r_c) {
+            read_one(smem_lds, smem_lds + (uint32_t)b_stage(0), std::integral_constant<int, 0>{}, r_c, af0, bf0);
+        });
 
         int kt = 0, kt_end = nk;
-        int st_cur = 0;       // stage of the K tile being multiplied
+        int st_cur = 0, sb_cur = 0; // stages of the K tile being multiplied: A's (and, without AHEAD, B's), B's
         bool drain = false;   // C stores are in flight: the next wait cannot count loads
         unit_k_range((int)blockIdx.x, kt, kt_end);
         for(int unit = (int)blockIdx.x; unit < nunits;)
         {
-            const int st_next  = st_cur + 1 == NST ? 0 : st_cur + 1;
+            const int st_next  = st_cur + 1 == NSTA ? 0 : st_cur + 1;
+            const int sb_next  = !AHEAD ? st_next : sb_cur + 1 == NST ? 0 : sb_cur + 1;
             // first fragments of this K tile (read in the previous half-iteration / the prologue)
             wait_frags();
-            half_step(std::false_type{}, LoadCtx{}, af0, bf0, smem_lds + (uint32_t)(st_cur * STAGE),
+            half_step(std::false_type{}, LoadCtx{}, af0, bf0, smem_lds + (uint32_t)a_stage(st_cur), smem_lds + (uint32_t)b_stage(sb_cur),
                       std::integral_constant<int, 1>{}, af1, bf1);
 
             // The direct loads of a wave retire in order: once at most NST-2 K tiles' worth are in
@@ -1418,17 +1458,17 @@ struct GemmTile
             if(drain)
                 asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
             else
-                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NST - 2) * LPT) : "memory");
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NST - 2) * LPT + (NSTA - NST) * NLA) : "memory");
             __builtin_amdgcn_sched_barrier(0);
             drain = false;
             barrier();
 
-            const LoadCtx lc = load_ctx(ld_kt, st_cur);
-            half_step(std::true_type{}, lc, af1, bf1, smem_lds + (uint32_t)(st_next * STAGE),
+            const LoadCtx lc = load_ctx(ld.kt, st_cur, ld_b.kt, sb_cur);
+            half_step(std::true_type{}, lc, af1, bf1, smem_lds + (uint32_t)a_stage(st_next), smem_lds + (uint32_t)b_stage(sb_next),
                       std::integral_constant<int, 0>{}, af0, bf0);
             advance_load_cursor();
 
-            st_cur = st_next;
+            st_cur = st_next, sb_cur = sb_next;
             if(++kt >= kt_end)
             {
                 acc_handover(std::true_type{});
@@ -1441,8 +1481,6 @@ struct GemmTile
                     else
                     {
                         using std::integral_constant;
-                        using std::false_type;
-                        using std::true_type;
                         // chunks of fragment rows whose D values are fetched together: all of them for a bias row alone,
                         // two with one per-row tensor, one with two
                         auto with_functor = [&](auto mode_c) {
@@ -1582,12 +1620,12 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs p)
 }
 
 template <int DT, int BM, int BN, int WM, int WN, int BKB, int NST, int IM2COL, bool TA = false, bool TB = false,
-          bool FUSED = false>
-__global__ __launch_bounds__((WM * WN * 64), (GemmTile<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED>::WAVES_EU))
+          bool FUSED = false, bool AHEAD = false>
+__global__ __launch_bounds__((WM * WN * 64), (GemmTile<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED, AHEAD>::WAVES_EU))
 void gemm_tile_kernel(const GemmArgs p)
 {
     extern __shared__ __attribute__((aligned(1024))) uint8_t ckx_smem[];
-    GemmTile<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED>::run(p, ckx_smem);
+    GemmTile<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED, AHEAD>::run(p, ckx_smem);
 }
 
 } // namespace ckx

@@ -41,11 +41,11 @@ inline int num_cus()
 // Persistent launch: at most (workgroups that fit a CU) x (CUs) workgroups, a multiple of 8 so
 // that workgroup b always lands on XCD b % 8 together with the tiles b, b + grid, ...
 template <int DT, int BM, int BN, int WM, int WN, int BKB, int NST, int IM2COL, bool TA = false, bool TB = false,
-          bool FUSED = false>
+          bool FUSED = false, bool AHEAD = false>
 hipError_t launch_tile(const GemmArgs& a, int tiles, hipStream_t s)
 {
-    using T              = GemmTile<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED>;
-    auto* kern           = &gemm_tile_kernel<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED>;
+    using T              = GemmTile<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED, AHEAD>;
+    auto* kern           = &gemm_tile_kernel<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED, AHEAD>;
     static std::once_flag once;
     static hipError_t attr_err = hipSuccess;
     std::call_once(once, [&] {

@@ -289,3 +289,29 @@ def test_conv2d_bias_relu_on_the_pointwise_kernel(shape):
     out = _conv(inp, wei, bias, None, s, (1, 1), (0, 0), inst)
     _close(out, ref)
     assert (out == 0).any() and (out > 0).any()
+
+
+# (N, C, Hi, filter, stride, K): whole K tiles and K tails, one K tile and fewer tiles than stages, ragged pixels, more tiles than CUs, and
+# two layers that the rule leaves to the plain 256 x 256 kernel (two column tiles; 5 x 5 stride 2)
+@pytest.mark.parametrize("case", [(1, 8, 9, 3, 2, 16), (2, 64, 15, 3, 2, 256), (3, 64, 33, 3, 2, 200), (1, 24, 20, 2, 2, 256), (2, 16, 30, 5, 3, 128),
+                                  (4, 192, 23, 3, 2, 256), (2, 128, 21, 3, 3, 256), (2, 64, 31, 3, 2, 512), (2, 16, 31, 5, 2, 256),
+                                  (600, 16, 31, 3, 2, 256)])
+def test_conv2d_strided_layers_on_the_256x256_tile(case):
+    """Strided layers on 256 x 256 tiles keep A in three LDS stages and B in two: small-integer operands, exact in any order, plain, with
+    bias and with bias and residual, against another tile instance bit for bit and (below 100 images) against the oracle."""
+    import gpu_util
+    n, c, hw, f, s, k = case
+    rng = np.random.default_rng(77)
+    inp, wei = rng.integers(-2, 3, (n, hw, hw, c)).astype(np.float16), rng.integers(-1, 2, (k, f, f, c)).astype(np.float16)
+    ho = (hw + 2 * (f // 2) - f) // s + 1
+    bias, resi = rng.integers(-3, 4, (k,)).astype(np.float16), rng.integers(-3, 4, (n, ho, ho, k)).astype(np.float16)
+    geom = ((s, s), (1, 1), (f // 2, f // 2))
+    out = gpu_util.conv2d_fwd(inp, wei, *geom, instance=0)
+    np.testing.assert_array_equal(out, gpu_util.conv2d_fwd(inp, wei, *geom, instance=8))
+    if n < 100:
+        np.testing.assert_array_equal(out, fast.conv2d_fwd_f16(inp, wei, *geom))
+    for r in (None, resi):
+        out = _conv(inp, wei, bias, r, *geom, instance=0)
+        np.testing.assert_array_equal(out, _conv(inp, wei, bias, r, *geom, instance=8))
+        if n < 100:
+            np.testing.assert_array_equal(out, fast.conv2d_fwd_bias_relu_f16(inp, wei, bias, r, *geom))
