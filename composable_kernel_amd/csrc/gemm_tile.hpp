@@ -899,7 +899,6 @@ struct GemmTile
             int tap_dh, tap_dw; // im2col: decoded ONCE per thread and K tile, every slot of a thread
             int tap_dd;         // sits at the same chunk position
             uint32_t tap_off;
-            bool tap_ok;
         };
         auto load_ctx = [&](int kt, int stage, int kt_b, int stage_b) {
             LoadCtx c;
@@ -914,7 +913,6 @@ struct GemmTile
             c.klim  = p.K - kt * KE;
             c.tap_dh = c.tap_dw = c.tap_dd = 0;
             c.tap_off                      = 0;
-            c.tap_ok            = true;
             if constexpr(IM2COL != 0)
             {
                 const uint32_t ke  = (c.k0 + kb) / ES; // element index along GEMM-K
@@ -932,7 +930,6 @@ struct GemmTile
                 c.tap_dh           = (int)y * p.cv.dH;
                 c.tap_dw           = (int)x * p.cv.dW;
                 c.tap_off          = ((uint32_t)((c.tap_dd * p.cv.Hi + c.tap_dh) * p.cv.Wi + c.tap_dw) * (uint32_t)p.cv.C + cc) * ES;
-                c.tap_ok           = ke < (uint32_t)p.K;
             }
             return c;
         };
@@ -948,11 +945,14 @@ struct GemmTile
                 else
                 {
                     const int hi0 = (int)a_hw0[j] >> 16, wi0 = (int)(a_hw0[j] << 16) >> 16;
-                    bool ok = c.tap_ok && (uint32_t)(hi0 + c.tap_dh) < (uint32_t)p.cv.Hi &&
-                              (uint32_t)(wi0 + c.tap_dw) < (uint32_t)p.cv.Wi;
+                    // (every condition is evaluated: with && the compiler put branches on the lane mask around each load of the 3-D
+                    // kernels, and a K tile's half was five basic blocks instead of one. 36 3-D problems 0.938 of the time, none slower: 16 x
+                    // 32^3, C 64 -> K 64 144.6 -> 137 us, 3 x 24^3, C 144 -> K 112 stride 2 31.2 -> 26.5. The tap itself is divided out anew for
+                    // every K tile: moved on digit by digit with carries, without a multiplication, it was slower, 1.002.)
+                    bool ok = ((uint32_t)(hi0 + c.tap_dh) < (uint32_t)p.cv.Hi) & ((uint32_t)(wi0 + c.tap_dw) < (uint32_t)p.cv.Wi);
                     if constexpr(IM2COL == 2)
-                        ok = ok && (uint32_t)(a_d0[j] + c.tap_dd) < (uint32_t)p.cv.Di;
-                    voff = (a_off[j] + c.tap_off) | (ok ? 0u : kOutOfRange);
+                        ok = ok & ((uint32_t)(a_d0[j] + c.tap_dd) < (uint32_t)p.cv.Di);
+                    voff = (a_off[j] + c.tap_off) | (ok ? 0u : kOutOfRange) | c.k_oob;
                 }
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_ptr_t)(c.sa + (j * NW + wave) * 1024), 16,
                                                          voff, (!TA && IM2COL == 0) ? (int)c.k0 : 0, 0, 0);
