@@ -7,11 +7,11 @@ namespace ckx {
 // The threads of a grid dimension are counted in 32 bits, and a launch past them wraps around without an error.
 constexpr long kMostBlocks = ((1l << 32) - 1) / 256;
 
-template <int DT, int B, bool TA, bool TB>
+template <int DT, int BM, int BN, bool TA, bool TB>
 static hipError_t launch_one(GemmArgs a, hipStream_t s)
 {
     constexpr long es = DT == DT_I8 ? 1 : 2;
-    a.tiles_m = (a.M + B - 1) / B, a.tiles_n = (a.N + B - 1) / B;
+    a.tiles_m = (a.M + BM - 1) / BM, a.tiles_n = (a.N + BN - 1) / BN;
     const long per_batch = (long)a.tiles_m * a.tiles_n, fit = kMostBlocks / per_batch;
     if(fit < 1)
         return hipErrorInvalidValue;
@@ -22,7 +22,7 @@ static hipError_t launch_one(GemmArgs a, hipStream_t s)
     {
         const int n = left < fit ? left : (int)fit;
         a.batch     = n;
-        hipLaunchKernelGGL((gemm_ragged_kernel<DT, B, B, TA, TB>), dim3((unsigned)(per_batch * n)), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((gemm_ragged_kernel<DT, BM, BN, TA, TB>), dim3((unsigned)(per_batch * n)), dim3(256), 0, s, a);
         const hipError_t e = hipGetLastError();
         if(e != hipSuccess)
             return e;
@@ -50,10 +50,36 @@ int ragged_tile(int M, int N, int batch)
     return (tiles128 >= 256 && 10 * tiles128 <= 3 * tiles64) || tiles64 / n > kMostBlocks ? 128 : 64;
 }
 
+RaggedTile ragged_small_tile(int M, int N, int batch)
+{
+    // The tile with the fewest operand rows through the busiest CU, its tiles times (m + n); a smaller one for a sixteenth less. A
+    // K tile takes 0.31 us of a CU for 64 + 64 rows, 0.24 for 64 + 32, 0.16 for 32 + 32, whether one workgroup or several ask for
+    // them. Of 43 random problems below the 128 x 128 line 26 run on one of the smaller two, none slower than on 64 x 64: 0.86
+    // of the time on average, 34 x 479 x 3569 20.9 -> 12.5 us, 1184 x 551 x 143 5.2 -> 4.6, 305 x 1011 x 2521 15.3 -> 12.0;
+    // 2001 x 1003 x 1025 stays (15.6 against 19.9 on 64 x 32, 23.7 on 32 x 32; 15.4 on a 128 x 64 one, which gains 10 % at most
+    // elsewhere and is not built).
+    const long n     = batch > 1 ? batch : 1;
+    const auto tiles = [&](RaggedTile t) { return (((long)M + t.m - 1) / t.m) * (((long)N + t.n - 1) / t.n) * n; };
+    RaggedTile best  = {64, 64};
+    long least       = (tiles(best) + 255) / 256 * 128;
+    for(const RaggedTile t : {RaggedTile{64, 32}, RaggedTile{32, 32}})
+    {
+        const long rows = (tiles(t) + 255) / 256 * (t.m + t.n);
+        if(16 * rows <= 15 * least && tiles(t) / n <= kMostBlocks)
+            best = t, least = rows;
+    }
+    return best;
+}
+
 template <int DT, bool TA, bool TB>
 static hipError_t launch_tile_size(const GemmArgs& a, hipStream_t s)
 {
-    return ragged_tile(a.M, a.N, a.batch) == 128 ? launch_one<DT, 128, TA, TB>(a, s) : launch_one<DT, 64, TA, TB>(a, s);
+    if(ragged_tile(a.M, a.N, a.batch) == 128)
+        return launch_one<DT, 128, 128, TA, TB>(a, s);
+    const RaggedTile t = ragged_small_tile(a.M, a.N, a.batch);
+    if(t.m == 32)
+        return launch_one<DT, 32, 32, TA, TB>(a, s);
+    return t.n == 32 ? launch_one<DT, 64, 32, TA, TB>(a, s) : launch_one<DT, 64, 64, TA, TB>(a, s);
 }
 
 template <int DT>

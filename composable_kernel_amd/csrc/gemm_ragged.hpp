@@ -17,14 +17,17 @@
 //     the last k row, which has no next one, is the checked one there, whether or not K ends in it.
 // Operands with less than one vector in the contiguous direction take the checked path element by element.
 //
-// What bounds it: with the 128 x 128 tile the operand bytes through a CU's L1 (32 KB per K tile; 0.27 of the MFMA rate at
-// 4001 x 4003 x 4095 fp16), with few tiles the latency of one K tile after the other. Against the element-by-element gather
+// What bounds it: the operand bytes through a CU's L1. A row that starts anywhere costs the L1 both lines that every 128
+// bytes of it touch: 35 to 49 bytes per ns and CU, 77 where rows start on a line (0.27 of the MFMA rate at 4001 x 4003 x
+// 4095 fp16). Reading whole lines and moving the chunks into place in registers took more than it saved (25 vector instructions
+// per 16 bytes; 2001 x 1003 x 1025 15.7 -> 19.3 us), unaligned LDS writes 50 to 120 cycles each instead of 13, and four K tiles in
+// flight instead of two nothing. Against the element-by-element gather
 // that served these shapes (one load instruction per element), fp16: 2001 x 1003 x 1025 98.7 -> 15.4 us, 4001 x 4003 x 4095
 // 2623 -> 197, 122 x 1283 x 3001 148 -> 17.4, 2049 x 2047 x 2047 with a K-major A 290 -> 55; int8 4001 x 4003 x 4095 3019 -> 118,
 // 40 x 333 x 3999 156 -> 16; bf16 3000 x 2999 x 1001 275 -> 47; one tile (32 x 33 x 65) 5.7, as before.
 //
-// Two tiles: 128 x 128 reads half the operand bytes per product, 64 x 64 gives four times the workgroups; ragged_tile() says
-// where the line lies.
+// Four tiles, 128 x 128 to 32 x 32: the larger read fewer operand bytes per product, the smaller fewer bytes per workgroup, which
+// is what a launch takes that does not fill the CUs; ragged_tile() and ragged_small_tile() say where the lines lie.
 #pragma once
 
 #include "gemm_tile.hpp"
@@ -69,7 +72,7 @@ struct RaggedOperand
     __device__ static __forceinline__ uint32_t tswz(uint32_t r)
     {
         constexpr int P     = BX * ES;
-        constexpr int LB    = P >= 256 ? 0 : (P == 128 ? 1 : 2);
+        constexpr int LB    = P >= 256 ? 0 : (P == 128 ? 1 : (P == 64 ? 2 : 3));
         const uint32_t full = ES == 2 ? ((r & 3u) | (((r >> 3) & 1u) << 2)) : ((r & 7u) | (((r >> 4) & 1u) << 3));
         return full >> LB;
     }
@@ -385,8 +388,13 @@ __global__ __launch_bounds__(256, 2) void gemm_ragged_kernel(const GemmArgs p)
     }
 }
 
-// rows and columns of the C tile a problem runs on: 128 or 64
+// rows and columns of the C tile a problem runs on: 128, or 64 and below (ragged_small_tile)
 int ragged_tile(int M, int N, int batch);
+struct RaggedTile
+{
+    int m, n;
+};
+RaggedTile ragged_small_tile(int M, int N, int batch);
 // ta / tb: the operand is K-major. tiles_m / tiles_n are set here.
 hipError_t launch_ragged(int dt, bool ta, bool tb, GemmArgs a, hipStream_t s);
 

@@ -1,5 +1,5 @@
-"""GPU parity of the GEMM for operands that are no whole 16-byte vectors (csrc/gemm_ragged.hpp) where it can go wrong: both of
-its tiles (128 x 128 from 256 C tiles on, 64 x 64 below), K below, at and just past one, two, three and four K tiles of 128
+"""GPU parity of the GEMM for operands that are no whole 16-byte vectors (csrc/gemm_ragged.hpp) where it can go wrong: all of
+its tiles (128 x 128 from 256 C tiles on, 64 x 64, 64 x 32 or 32 x 32 below, by their rows per CU), K below, at and just past one, two, three and four K tiles of 128
 bytes, extents one short of and one past a C tile, fewer elements than one vector in the contiguous direction, operands that
 end at their last element, all layouts. Integer operands small enough that every fp32 partial sum is exact: the result is the
 rounded exact product, whatever the order of the sum, and int8 is compared bit for bit after wrapping."""
@@ -62,6 +62,16 @@ def test_k_around_the_k_tiles(kind, layout):
 def test_tile_edges(kind, layout, shape):
     _run(kind, layout, *shape, off=0)
     _run(kind, layout, *shape, off=3)
+
+
+@pytest.mark.parametrize("layout", sorted(LAYOUTS))
+@pytest.mark.parametrize("kind", ["i8", "f16", "bf16"])
+@pytest.mark.parametrize("M, N", [(31, 33), (33, 31), (65, 1), (705, 497), (703, 511), (1021, 1003), (963, 1023)])
+def test_small_tiles(kind, layout, M, N):
+    """32 x 32 (the first three), 64 x 32 and 64 x 64 tiles at their edges, K around two K tiles"""
+    for K in (127, 129, 259):
+        _run(kind, layout, M, N, K, off=0)
+        _run(kind, layout, M, N, K, off=5)
 
 
 def test_batches_past_one_launch_dimension():
