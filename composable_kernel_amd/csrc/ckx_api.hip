@@ -125,6 +125,7 @@ struct TileInstance
 
 const TileInstance kTiles[] = {CKX_FOR_EACH_TILE(CKX_TILE)};
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
+static_assert(ckx::kFourStageTile == kNumTiles - 1, "the last tile of the list");
 
 // Launch plan: which tile instance, and into how many K runs each C tile is cut (split-K).
 struct Plan
@@ -671,8 +672,12 @@ int run_gemm(int dt, const void* a, const void* b, void* c, int M, int N, int K,
     // (its buffer resources start 3 KB before the operands and are that much longer: see kImmBias in gemm_w4.hpp)
     const bool w4 = ti == 0 && !kmajor && g.ksplit == 1 && g.a_bytes < (1u << 31) - 4096 && g.b_bytes < (1u << 31) - 4096 &&
                     (epi <= CKX_EPI_REQUANT_RND || (f16_fused(epi) && !uses_d1(epi))) && four_wave_body_pays(dt, K, (long)g.tiles_m * g.tiles_n * (batch > 1 ? batch : 1));
+    const bool pairs = ti == ckx::kFourStageTile && !kmajor && ckx::row_pairs_pay(M, N, (long)g.ksplit * (batch > 1 ? batch : 1));
+    if(pairs)
+        g.tiles_m = (M + 127) / 128;
     const tile_launch_fn launch = w4                   ? ckx::w4_tile(dt, fused)
                                   : kmajor             ? ckx::layout_tile(dt, ti, ta, tb)
+                                  : pairs              ? ckx::row_pairs_tile(dt, false, fused || (per_column_scale(epi) && g.ksplit == 1))
                                   : dt == ckx::DT_I8   ? (per_column_scale(epi) && g.ksplit == 1 ? t.dense_i8_fused : t.dense_i8)
                                   : dt == ckx::DT_BF16 ? t.dense_bf16
                                   : fused              ? t.dense_f16_fused
@@ -1077,7 +1082,12 @@ int run_conv(int op, const void* in, const void* wei, void* out, const ckx_conv2
     // but 49.5 -> 50.6, 5 x 5 stride 3, K 512 (1.8) 226 -> 233, 5 x 5 stride 2, K 256 (1.6) 141.3 -> 142.5.
     const int taps   = d->Y * d->X;
     const bool ahead = es == 2 && t.bm * t.bn == 256 * 256 && taps > 1 && 10l * d->stride_h * d->stride_w >= 3l * taps * g.tiles_n;
-    hipError_t e     = (ahead    ? (fused ? &launch_tile<ckx::DT_F16, 256, 256, 2, 4, 128, 2, 1, false, false, true, true>
+    const bool pairs = pl.tile == ckx::kFourStageTile && ckx::row_pairs_pay(M, N, g.ksplit);
+    if(pairs)
+        g.tiles_m = (M + 127) / 128;
+    hipError_t e     = (pairs    ? ckx::row_pairs_tile(es == 1 ? ckx::DT_I8 : ckx::DT_F16, true,
+                                                       es == 1 ? per_column_scale(epi) && g.ksplit == 1 : fused)
+                        : ahead  ? (fused ? &launch_tile<ckx::DT_F16, 256, 256, 2, 4, 128, 2, 1, false, false, true, true>
                                           : &launch_tile<ckx::DT_F16, 256, 256, 2, 4, 128, 2, 1, false, false, false, true>)
                         : es == 1  ? (per_column_scale(epi) && g.ksplit == 1 ? t.conv_i8_fused : t.conv_i8)
                         : fused ? t.conv_f16_fused
@@ -1249,7 +1259,11 @@ int run_convnd(int op, const void* in, const void* wei, void* out, const ckx_con
         hipError_t e = ckx::launch_generic(es == 1 ? ckx::DT_I8 : ckx::DT_F16, 2, g, lay, (hipStream_t)stream);
         return e == hipSuccess ? CKX_OK : hip_fail(e, kGenericName);
     }
-    const tile_launch_fn launch = ckx::conv3d_tile(es == 1 ? ckx::DT_I8 : ckx::DT_F16, pl.tile);
+    const bool pairs = pl.tile == ckx::kFourStageTile && ckx::row_pairs_pay(M, N, g.ksplit);
+    if(pairs)
+        g.tiles_m = (M + 127) / 128;
+    const tile_launch_fn launch = pairs ? ckx::row_pairs_conv3d_tile(es == 1 ? ckx::DT_I8 : ckx::DT_F16)
+                                        : ckx::conv3d_tile(es == 1 ? ckx::DT_I8 : ckx::DT_F16, pl.tile);
     if(!launch)
         return fail(CKX_UNSUPPORTED, "no kernel variant for this instance");
     hipError_t e = launch(g, g.tiles_m * g.tiles_n * g.ksplit, (hipStream_t)stream);

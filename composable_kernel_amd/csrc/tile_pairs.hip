@@ -1,0 +1,37 @@
+// Two row tiles of the four-stage 64 x 64 instance as one 128 x 64 workgroup of eight waves: a translation unit of its own so that its
+// kernels compile beside the others.
+#include "tile_launch.hpp"
+
+namespace ckx {
+namespace {
+
+template <int DT, int IM2COL, bool FUSED>
+constexpr tile_launch_fn pairs = &launch_tile<DT, 128, 64, 8, 1, 128, 3, IM2COL, false, false, FUSED>;
+
+} // namespace
+
+bool row_pairs_pay(long M, long N, long runs)
+{
+    // What bounds two co-resident 64 x 64 workgroups is the operand bytes that their CU loads (65 to 82 bytes per ns), and both load the same
+    // rows of B where they are above one another: a pair loads 192 rows per K tile where they load 256. So the line is
+    // where the busiest CU loads fewer: no gain with one workgroup per CU, with a single row tile, or with an odd number of row tiles that makes
+    // a second round. 43 of 52 random GEMMs and convolutions on the four-stage instance with more than one workgroup per CU are on this
+    // side, 0.69 to 1.00 of the time, 0.92 on average (int8 67 x 10990 x 9024 35.4 -> 24.5 us, 32 x 14 x 14, C = K = 256 13.0 -> 11.8, 128 x
+    // 4096 x 11008 21.3 -> 20.0); the others take 1.00 to 1.25 as pairs. Eight waves of 16 rows as in the 64 x 64 kernel (four of 32 take
+    // 1.2 to 1.5 times as long), three LDS stages (two workgroups per CU; four stages, and one: 2 % behind).
+    const long cus = num_cus(), cols = (N + 63) / 64 * runs, one = (M + 63) / 64 * cols, pair = (M + 127) / 128 * cols;
+    return (pair + cus - 1) / cus * (128 + 64) < (one + cus - 1) / cus * (64 + 64);
+}
+
+tile_launch_fn row_pairs_tile(int dt, bool im2col, bool fused)
+{
+    if(dt == DT_BF16)
+        return im2col || fused ? nullptr : pairs<DT_BF16, 0, false>;
+    if(dt == DT_I8)
+        return im2col ? (fused ? pairs<DT_I8, 1, true> : pairs<DT_I8, 1, false>) : fused ? pairs<DT_I8, 0, true> : pairs<DT_I8, 0, false>;
+    return im2col ? (fused ? pairs<DT_F16, 1, true> : pairs<DT_F16, 1, false>) : fused ? pairs<DT_F16, 0, true> : pairs<DT_F16, 0, false>;
+}
+
+tile_launch_fn row_pairs_conv3d_tile(int dt) { return dt == DT_I8 ? pairs<DT_I8, 2, false> : pairs<DT_F16, 2, false>; }
+
+} // namespace ckx

@@ -1,0 +1,143 @@
+"""GPU parity of the 128 x 64 row pairs that run behind the four-stage 64 x 64 instance (csrc/tile_pairs.hip): bit for bit what the
+two-stage 64 x 64 instance gives for the same problem (each element is the same sum in the same order), at the edges of the line between one
+tile and a pair, with rows that end in a pair's first half, one K tile and more than the three stages hold, K splits, every
+epilogue, convolutions and batches."""
+import ctypes
+
+import pytest
+
+import composable_kernel_amd as ck
+from composable_kernel_amd import capi
+
+pytestmark = pytest.mark.gpu
+FOUR_STAGE, TWO_STAGE = 8, 4
+
+
+def _pays(M, N, runs=1):
+    f = capi.lib()._ZN3ckx13row_pairs_payElll
+    f.argtypes, f.restype = [ctypes.c_long] * 3, ctypes.c_bool
+    return f(M, N, runs)
+
+
+def _both(make, c):
+    """make(instance) -> (operator, argument writing c); the results of both instances"""
+    import torch
+    import gpu_util
+    out = []
+    for instance in (FOUR_STAGE, TWO_STAGE):
+        c.fill_(77)
+        op, arg = make(instance)
+        assert op.IsSupportedArgument(arg), capi.last_error()
+        op.MakeInvokerPointer().Run(arg, ck.StreamConfig(gpu_util.stream()))
+        torch.cuda.synchronize()
+        out.append(c.clone())
+    assert torch.equal(out[0], out[1]), f"{int((out[0] != out[1]).sum())} elements differ"
+    return out[0]
+
+
+def _operand(kind, shape, seed):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    dt = {"i8": torch.int8, "f16": torch.float16, "bf16": torch.bfloat16}[kind]
+    return torch.randint(-9, 10, shape, generator=g, device="cuda").to(dt)
+
+
+def test_the_line():
+    assert not _pays(128, 64 * 128)                                    # one 64 x 64 workgroup per CU
+    assert _pays(128, 64 * 129) and not _pays(64, 64 * 300)            # two, one row tile
+    assert _pays(192, 64 * 100) and not _pays(192, 64 * 129)           # 200 pairs for 300; 258 for 387
+    assert _pays(128, 4096, 4) and not _pays(128, 4096, 2)
+
+
+@pytest.mark.parametrize("M, N, K", [(65, 8260, 128), (67, 9000, 64), (127, 8257, 1040), (128, 8256, 512), (150, 6000, 272), (700, 2500, 656), (1020, 1900, 400)])
+@pytest.mark.parametrize("form", ["i8", "i8_rounded", "i8_per_column", "f16", "f16_add_relu_add", "bf16"])
+def test_gemm(form, M, N, K):
+    import torch
+    assert _pays(M, N)
+    kind = form.split("_")[0]
+    a, b = _operand(kind, (M, K), 1), _operand(kind, (N, K), 2)
+    c = torch.empty((M + 1, N), dtype=a.dtype, device="cuda")
+    d = [_operand("f16", (N,), 3), _operand("f16", (M, N), 4)]
+    scales = torch.rand((N,), device="cuda") * 0.4
+
+    def make(instance):
+        if form == "i8_per_column":
+            op = ck.DeviceGemmMultipleDInt8(instance)
+            return op, op.MakeArgumentPointer(a, b, [scales], c, M, N, K, K, K, [0], N, None, None, ck.ActivationMul2Clamp(ck.Relu()))
+        if form == "f16_add_relu_add":
+            op = ck.DeviceGemmMultipleDF16(instance)
+            return op, op.MakeArgumentPointer(a, b, d, c, M, N, K, K, K, [0, N], N, None, None, ck.AddReluAdd())
+        op = {"i8": ck.DeviceGemmInt8, "f16": ck.DeviceGemmF16, "bf16": ck.DeviceGemmBF16}[kind](instance)
+        cop = ck.RequantReluRequant(0.02, 0.7, rounded=True) if form == "i8_rounded" else ck.PassThrough()
+        return op, op.MakeArgumentPointer(a, b, c, M, N, K, K, K, N, None, None, cop)
+
+    got = _both(make, c)
+    assert bool((got[M] == 77).all()), "wrote past the last row"
+    if form in ("f16", "bf16"):  # |sums| < 2^24: the rounded exact product
+        assert torch.equal(got[:M], (a.float() @ b.float().T.contiguous()).to(a.dtype))
+
+
+@pytest.mark.parametrize("kind", ["i8", "f16"])
+@pytest.mark.parametrize("M, N, K, runs", [(128, 4096, 1024, 4), (100, 2200, 2064, 5), (500, 1100, 1600, 3)])
+def test_k_split(kind, M, N, K, runs):
+    import torch
+    a, b = _operand(kind, (M, K), 5), _operand(kind, (N, K), 6)
+    c = torch.empty((M, N), dtype=a.dtype, device="cuda")
+    ws = torch.full((runs * M * N * 4 + 16,), 0x7F, dtype=torch.uint8, device="cuda")
+    assert _pays(M, N, runs)
+
+    def make(instance):
+        op = (ck.DeviceGemmInt8 if kind == "i8" else ck.DeviceGemmF16)(instance)
+        arg = op.MakeArgumentPointer(a, b, c, M, N, K, K, K, N, None, None, ck.PassThrough())
+        op.SetWorkSpacePointer(arg, ws, runs * M * N * 4)
+        return op, arg
+
+    before = capi.lib().ckx_set_forced_k_runs(runs)
+    try:
+        _both(make, c)
+    finally:
+        capi.lib().ckx_set_forced_k_runs(before)
+
+
+def test_batches():
+    import torch
+    G, M, N, K = 5, 120, 1900, 272
+    assert _pays(M, N, G)
+    a, b = _operand("f16", (G, M, K), 7), _operand("f16", (G, N, K), 8)
+    c = torch.empty((G, M, N), dtype=torch.float16, device="cuda")
+
+    def make(instance):
+        op = ck.DeviceBatchedGemmF16(instance)
+        return op, op.MakeArgumentPointer(a, b, c, M, N, K, K, K, N, M * K, N * K, M * N, G)
+    _both(make, c)
+
+
+@pytest.mark.parametrize("form", ["i8", "f16", "f16_bias_relu", "f16_bias_relu_add", "i8_3d", "f16_3d"])
+@pytest.mark.parametrize("N, C, K, hw, f, stride", [(32, 64, 256, 14, 3, 1), (9, 48, 72, 41, 5, 1), (5, 32, 264, 63, 3, 2)])
+def test_conv(form, N, C, K, hw, f, stride):
+    import torch
+    nd = 3 if form.endswith("3d") else 2
+    if nd == 3:
+        N, hw, K = 2, 13 * stride - (stride - 1), 264
+    ho = (hw + 2 * (f // 2) - f) // stride + 1
+    kind = form.split("_")[0]
+    x, w = _operand(kind, (N, *[hw] * nd, C), 9), _operand(kind, (K, *[f] * nd, C), 10)
+    bias, r = _operand("f16", (K,), 11), _operand("f16", (N, *[ho] * nd, K), 12)
+    y = torch.empty((N, *[ho] * nd, K), dtype=x.dtype, device="cuda")
+    geom = (N, K, C, [hw] * nd, [f] * nd, [ho] * nd, [stride] * nd, [1] * nd, [f // 2] * nd, [f // 2] * nd)
+
+    def make(instance):
+        if "bias" in form:
+            op = ck.DeviceConv2dFwdBiasActivationF16(instance)
+            if form.endswith("add"):
+                return op, op.MakeArgumentPointer(x, w, y, bias, r, *geom, None, None, ck.AddReluAdd())
+            return op, op.MakeArgumentPointer(x, w, y, bias, *geom, None, None, ck.AddRelu())
+        if nd == 3:
+            op = (ck.DeviceConvNdFwdInt8 if kind == "i8" else ck.DeviceConvNdFwdF16)(3, instance)
+        else:
+            op = (ck.DeviceConv2dFwdInt8 if kind == "i8" else ck.DeviceConv2dFwdF16)(instance)
+        cop = ck.RequantReluRequant(0.02, 0.7, rounded=True) if kind == "i8" else ck.PassThrough()
+        return op, op.MakeArgumentPointer(x, w, y, *geom, None, None, cop)
+
+    _both(make, y)
+    assert _pays(N * ho ** nd, K)
