@@ -672,10 +672,12 @@ int run_gemm(int dt, const void* a, const void* b, void* c, int M, int N, int K,
     // (its buffer resources start 3 KB before the operands and are that much longer: see kImmBias in gemm_w4.hpp)
     const bool w4 = ti == 0 && !kmajor && g.ksplit == 1 && g.a_bytes < (1u << 31) - 4096 && g.b_bytes < (1u << 31) - 4096 &&
                     (epi <= CKX_EPI_REQUANT_RND || (f16_fused(epi) && !uses_d1(epi))) && four_wave_body_pays(dt, K, (long)g.tiles_m * g.tiles_n * (batch > 1 ? batch : 1));
-    const bool pairs = ti == ckx::kFourStageTile && !kmajor && ckx::row_pairs_pay(M, N, (long)g.ksplit * (batch > 1 ? batch : 1));
+    // (not the K runs of a K-major A, whose pairs are level or behind: 640 x 256 x 4672 14.5 us and 14.8, 704 x 512 x 5696 19.3 and 19.8)
+    const bool pairs = ti == ckx::kFourStageTile && !(ta && g.ksplit > 1) && ckx::row_pairs_pay(M, N, (long)g.ksplit * (batch > 1 ? batch : 1));
     if(pairs)
         g.tiles_m = (M + 127) / 128;
     const tile_launch_fn launch = w4                   ? ckx::w4_tile(dt, fused)
+                                  : kmajor && pairs    ? ckx::row_pairs_layout_tile(dt, ta, tb)
                                   : kmajor             ? ckx::layout_tile(dt, ti, ta, tb)
                                   : pairs              ? ckx::row_pairs_tile(dt, false, fused || (per_column_scale(epi) && g.ksplit == 1))
                                   : dt == ckx::DT_I8   ? (per_column_scale(epi) && g.ksplit == 1 ? t.dense_i8_fused : t.dense_i8)

@@ -41,6 +41,7 @@ constexpr LayoutTile make_layout_tile()
 #define CKX_LAYOUT_TILE(BM, BN, WM, WN, NST, EFF) make_layout_tile<BM, BN, WM, WN, NST>(),
 const LayoutTile kLayoutTiles[] = {CKX_FOR_EACH_TILE(CKX_LAYOUT_TILE)};
 constexpr int kNumLayoutTiles = sizeof(kLayoutTiles) / sizeof(kLayoutTiles[0]);
+const LayoutTile kRowPairs = make_layout_tile<128, 64, 8, 1, 3>();
 
 } // namespace
 
@@ -49,6 +50,13 @@ tile_launch_fn layout_tile(int dt, int tile, bool a_kmajor, bool b_kmajor)
     if(dt < 0 || dt > 2 || tile < 0 || tile >= kNumLayoutTiles || (!a_kmajor && !b_kmajor))
         return nullptr;
     return kLayoutTiles[tile].fn[dt][a_kmajor && b_kmajor ? 2 : b_kmajor ? 1 : 0];
+}
+
+tile_launch_fn row_pairs_layout_tile(int dt, bool a_kmajor, bool b_kmajor)
+{
+    if(dt < 0 || dt > 2 || (!a_kmajor && !b_kmajor))
+        return nullptr;
+    return kRowPairs.fn[dt][a_kmajor && b_kmajor ? 2 : b_kmajor ? 1 : 0];
 }
 
 } // namespace ckx

@@ -71,12 +71,13 @@ tile_launch_fn layout_tile(int dt, int tile, bool a_kmajor, bool b_kmajor);
 // else null), with the D-operand epilogues
 tile_launch_fn w4_tile(int dt, bool fused);
 
-// 128 x 64 body of the four-stage 64 x 64 instance (tile_pairs.hip), K-contiguous operands, same results bit for bit: whether a launch of
+// 128 x 64 body of the four-stage 64 x 64 instance (tile_pairs.hip), same results bit for bit: whether a launch of
 // `runs` K runs (times batches) takes it, and the launchers; fused: the epilogues with D operands
 constexpr int kFourStageTile = 8; // (position in CKX_FOR_EACH_TILE)
 bool row_pairs_pay(long M, long N, long runs);
 tile_launch_fn row_pairs_tile(int dt, bool im2col, bool fused);
 tile_launch_fn row_pairs_conv3d_tile(int dt);
+tile_launch_fn row_pairs_layout_tile(int dt, bool a_kmajor, bool b_kmajor); // (gemm_layouts.hip)
 
 // weight-streaming GEMM for up to 128 rows (gemm_astream.hip): launcher for element type dt (DT_*) with 16 * nt output
 // columns per workgroup (nt = 3), grid = number of such column blocks

@@ -19,6 +19,8 @@ bool row_pairs_pay(long M, long N, long runs)
     // side, 0.69 to 1.00 of the time, 0.92 on average (int8 67 x 10990 x 9024 35.4 -> 24.5 us, 32 x 14 x 14, C = K = 256 13.0 -> 11.8, 128 x
     // 4096 x 11008 21.3 -> 20.0); the others take 1.00 to 1.25 as pairs. Eight waves of 16 rows as in the 64 x 64 kernel (four of 32 take
     // 1.2 to 1.5 times as long), three LDS stages (two workgroups per CU; four stages, and one: 2 % behind).
+    // With K-major operands 38 problems on this side 0.70 to 0.99, 0.88 on average: 512 x 2736 x 8160 fp16 B 72.0 -> 50.5, int8 640 x 2480 x
+    // 2944 B 17.3 -> 13.1, bf16 960 x 1904 x 2640 both 24.8 -> 22.0.
     const long cus = num_cus(), cols = (N + 63) / 64 * runs, one = (M + 63) / 64 * cols, pair = (M + 127) / 128 * cols;
     return (pair + cus - 1) / cus * (128 + 64) < (one + cus - 1) / cus * (64 + 64);
 }

@@ -77,6 +77,29 @@ def test_gemm(form, M, N, K):
         assert torch.equal(got[:M], (a.float() @ b.float().T.contiguous()).to(a.dtype))
 
 
+@pytest.mark.parametrize("kind", ["i8", "f16", "bf16"])
+@pytest.mark.parametrize("layout", ["km_nk", "mk_kn", "km_kn"])
+@pytest.mark.parametrize("M, N, K", [(80, 8272, 128), (176, 6000, 272), (1008, 1904, 528), (704, 2512, 64)])
+def test_k_major(kind, layout, M, N, K):
+    import torch
+    assert _pays(M, N)
+    la, lb = layout.split("_")
+    a, b = _operand(kind, (M, K) if la == "mk" else (K, M), 13), _operand(kind, (N, K) if lb == "nk" else (K, N), 14)
+    c = torch.empty((M + 1, N), dtype=a.dtype, device="cuda")
+    lay = dict(ALayout=ck.RowMajor if la == "mk" else ck.ColumnMajor, BLayout=ck.ColumnMajor if lb == "nk" else ck.RowMajor)
+
+    def make(instance):
+        op = {"i8": ck.DeviceGemmInt8, "f16": ck.DeviceGemmF16, "bf16": ck.DeviceGemmBF16}[kind](instance, **lay)
+        cop = ck.RequantReluRequant(0.02, 0.7, rounded=True) if kind == "i8" else ck.PassThrough()
+        return op, op.MakeArgumentPointer(a, b, c, M, N, K, a.shape[1], b.shape[1], N, None, None, cop)
+
+    got = _both(make, c)
+    assert bool((got[M] == 77).all()), "wrote past the last row"
+    if kind != "i8":  # |sums| < 2^24: the rounded exact product
+        a_mk, b_kn = (a if la == "mk" else a.T).float().contiguous(), (b.T if lb == "nk" else b).float().contiguous()
+        assert torch.equal(got[:M], (a_mk @ b_kn).to(a.dtype))
+
+
 @pytest.mark.parametrize("kind", ["i8", "f16"])
 @pytest.mark.parametrize("M, N, K, runs", [(128, 4096, 1024, 4), (100, 2200, 2064, 5), (500, 1100, 1600, 3)])
 def test_k_split(kind, M, N, K, runs):
