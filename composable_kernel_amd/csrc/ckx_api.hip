@@ -261,7 +261,7 @@ Plan make_plan(long M, int N, int kbytes, int only_tile, long workspace_bytes, i
             // Two four-stage 64 x 64 workgroups per CU without a split: 3 us and their K tiles' bytes at 82 GB/s, which is above the
             // estimate so far from 20 K tiles on. Measured over 257 ... 512 such tiles: 13 us at 24 K tiles, 16 ... 17 at 32, 25 ... 27
             // at 64, 32 ... 37 at 80, 49 ... 57 at 127, 80 at 200; half as much again with K-major operands, which keep this rate as
-            // their other instances are slower too. fp16 1222 x 960 x 8288 63 -> 45 us (three K runs of 128 x 64 tiles), bf16 2266 x
+            // their other instances are slower too (as single tiles; many of these launches now run as pairs, tile_pairs.hip, in 0.7 to 1.0 of it). fp16 1222 x 960 x 8288 63 -> 45 us (three K runs of 128 x 64 tiles), bf16 2266 x
             // 488 x 6656 K-major B 48.2 -> 39.0, int8 2800 x 376 x 16256 52.0 -> 45.3; 1024 x 1280 x 4096 stays (25.4, next 33.1).
             if(per_cu == 2 && nst > 2 && sp == 1 && !conv)
             {
@@ -676,7 +676,12 @@ int run_gemm(int dt, const void* a, const void* b, void* c, int M, int N, int K,
     const bool pairs = ti == ckx::kFourStageTile && !(ta && g.ksplit > 1) && ckx::row_pairs_pay(M, N, (long)g.ksplit * (batch > 1 ? batch : 1));
     if(pairs)
         g.tiles_m = (M + 127) / 128;
-    const tile_launch_fn launch = w4                   ? ckx::w4_tile(dt, fused)
+    const bool columns = ti == ckx::kFourStageTile && !pairs && !kmajor && !fused && !per_column_scale(epi) &&
+                         ckx::column_pairs_pay(M, N, g.ksplit, batch > 1 ? batch : 1);
+    if(columns)
+        g.tiles_n = (N + 127) / 128;
+    const tile_launch_fn launch = columns              ? ckx::column_pairs_tile(dt)
+                                  : w4                 ? ckx::w4_tile(dt, fused)
                                   : kmajor && pairs    ? ckx::row_pairs_layout_tile(dt, ta, tb)
                                   : kmajor             ? ckx::layout_tile(dt, ti, ta, tb)
                                   : pairs              ? ckx::row_pairs_tile(dt, false, fused || (per_column_scale(epi) && g.ksplit == 1))

@@ -78,6 +78,9 @@ bool row_pairs_pay(long M, long N, long runs);
 tile_launch_fn row_pairs_tile(int dt, bool im2col, bool fused);
 tile_launch_fn row_pairs_conv3d_tile(int dt);
 tile_launch_fn row_pairs_layout_tile(int dt, bool a_kmajor, bool b_kmajor); // (gemm_layouts.hip)
+// 64 x 128 body of the same instance: dense GEMMs with K-contiguous operands and a plain epilogue
+bool column_pairs_pay(long M, long N, long ksplit, long batch);
+tile_launch_fn column_pairs_tile(int dt);
 
 // weight-streaming GEMM for up to 128 rows (gemm_astream.hip): launcher for element type dt (DT_*) with 16 * nt output
 // columns per workgroup (nt = 3), grid = number of such column blocks

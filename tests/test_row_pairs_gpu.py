@@ -1,4 +1,4 @@
-"""GPU parity of the 128 x 64 row pairs that run behind the four-stage 64 x 64 instance (csrc/tile_pairs.hip): bit for bit what the
+"""GPU parity of the 128 x 64 row pairs and 64 x 128 column pairs that run behind the four-stage 64 x 64 instance (csrc/tile_pairs.hip): bit for bit what the
 two-stage 64 x 64 instance gives for the same problem (each element is the same sum in the same order), at the edges of the line between one
 tile and a pair, with rows that end in a pair's first half, one K tile and more than the three stages hold, K splits, every
 epilogue, convolutions and batches."""
@@ -17,6 +17,12 @@ def _pays(M, N, runs=1):
     f = capi.lib()._ZN3ckx13row_pairs_payElll
     f.argtypes, f.restype = [ctypes.c_long] * 3, ctypes.c_bool
     return f(M, N, runs)
+
+
+def _columns_pay(M, N, ksplit=1, batch=1):
+    f = capi.lib()._ZN3ckx16column_pairs_payEllll
+    f.argtypes, f.restype = [ctypes.c_long] * 4, ctypes.c_bool
+    return not _pays(M, N, ksplit * batch) and f(M, N, ksplit, batch)
 
 
 def _both(make, c):
@@ -47,13 +53,16 @@ def test_the_line():
     assert _pays(128, 64 * 129) and not _pays(64, 64 * 300)            # two, one row tile
     assert _pays(192, 64 * 100) and not _pays(192, 64 * 129)           # 200 pairs for 300; 258 for 387
     assert _pays(128, 4096, 4) and not _pays(128, 4096, 2)
+    assert _columns_pay(64, 64 * 300) and not _columns_pay(64, 64 * 256) and not _columns_pay(128, 64 * 129)
+    assert _columns_pay(64, 4096, 8) and not _columns_pay(192, 2048, 5) and _columns_pay(192, 2048, 1, 5)
 
 
-@pytest.mark.parametrize("M, N, K", [(65, 8260, 128), (67, 9000, 64), (127, 8257, 1040), (128, 8256, 512), (150, 6000, 272), (700, 2500, 656), (1020, 1900, 400)])
+@pytest.mark.parametrize("M, N, K", [(65, 8260, 128), (67, 9000, 64), (127, 8257, 1040), (128, 8256, 512), (150, 6000, 272), (700, 2500, 656), (1020, 1900, 400),
+                                     (1, 64 * 257, 128), (63, 20000, 272), (64, 32705, 64), (130, 8255, 528), (190, 8256, 1040), (300, 5000, 400)])
 @pytest.mark.parametrize("form", ["i8", "i8_rounded", "i8_per_column", "f16", "f16_add_relu_add", "bf16"])
 def test_gemm(form, M, N, K):
     import torch
-    assert _pays(M, N)
+    assert _pays(M, N) or _columns_pay(M, N)
     kind = form.split("_")[0]
     a, b = _operand(kind, (M, K), 1), _operand(kind, (N, K), 2)
     c = torch.empty((M + 1, N), dtype=a.dtype, device="cuda")
@@ -101,13 +110,13 @@ def test_k_major(kind, layout, M, N, K):
 
 
 @pytest.mark.parametrize("kind", ["i8", "f16"])
-@pytest.mark.parametrize("M, N, K, runs", [(128, 4096, 1024, 4), (100, 2200, 2064, 5), (500, 1100, 1600, 3)])
+@pytest.mark.parametrize("M, N, K, runs", [(128, 4096, 1024, 4), (100, 2200, 2064, 5), (500, 1100, 1600, 3), (40, 4100, 1552, 5), (64, 2816, 1024, 8)])
 def test_k_split(kind, M, N, K, runs):
     import torch
     a, b = _operand(kind, (M, K), 5), _operand(kind, (N, K), 6)
     c = torch.empty((M, N), dtype=a.dtype, device="cuda")
     ws = torch.full((runs * M * N * 4 + 16,), 0x7F, dtype=torch.uint8, device="cuda")
-    assert _pays(M, N, runs)
+    assert _pays(M, N, runs) or _columns_pay(M, N, runs)
 
     def make(instance):
         op = (ck.DeviceGemmInt8 if kind == "i8" else ck.DeviceGemmF16)(instance)
@@ -122,10 +131,10 @@ def test_k_split(kind, M, N, K, runs):
         capi.lib().ckx_set_forced_k_runs(before)
 
 
-def test_batches():
+@pytest.mark.parametrize("G, M, N, K, columns", [(5, 120, 1900, 272, False), (7, 60, 2700, 272, True)])
+def test_batches(G, M, N, K, columns):
     import torch
-    G, M, N, K = 5, 120, 1900, 272
-    assert _pays(M, N, G)
+    assert _columns_pay(M, N, 1, G) if columns else _pays(M, N, G)
     a, b = _operand("f16", (G, M, K), 7), _operand("f16", (G, N, K), 8)
     c = torch.empty((G, M, N), dtype=torch.float16, device="cuda")
 
