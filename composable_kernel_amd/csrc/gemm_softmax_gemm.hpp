@@ -60,9 +60,6 @@ struct SoftmaxGemmCfg
     __device__ static __forceinline__ uint32_t v_key(uint32_t r) { return VRS == 128 ? ((r >> 1) & 1u) << 2 : VRS == 256 ? (r & 3u) << 2 : 0u; }
 };
 
-// offset past every operand (below 2 GiB, whole 16-byte chunks) that stays out of range with up to 2 GiB added
-constexpr uint32_t kPastEnd = 0x7ffffff0u;
-
 template <int KS, int OT, int NW>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_softmax_gemm_kernel(const GemmGemmArgs p)
 {
@@ -106,8 +103,12 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     const uint32_t gk = live_k && (int)ck * 8 < p.K ? rk0 * (uint32_t)p.sb0 * 2u + ck * 16u : kOutOfRange;
     const uint32_t gv = live_v && (int)cv * 8 < p.O ? rv0 * (uint32_t)p.sb1 * 2u + cv * 16u : kOutOfRange;
     const uint32_t lk = rk0 * KRS + (ck ^ Cfg::k_key(rk0)) * 16, lv = rv0 * VRS + (cv ^ Cfg::v_key(rv0)) * 16;
-    // byte offset of a unit's first row in the operand; for units that do not exist one that no chunk's offset brings back into range
-    auto first = [&](int u, int stride) { return u * UC < p.N ? (uint32_t)(u * UC) * (uint32_t)stride * 2u : kPastEnd; };
+    // Byte offset of a unit's first row in the operand; a unit that does not exist starts at row N, the first past the end. Chunks past K or O
+    // begin at kOutOfRange and stay out of range with all rows up to 64 past N added, but for operands that end less than 64 rows
+    // below 2 GiB: there a sum may wrap around into the operand, for rows past N only. What is read then goes nowhere: columns past N get
+    // -inf for a score by a select (mask), whatever it was, output columns past O are not stored, and units that do not exist meet no
+    // product. (The out-of-range bit OR-ed into the sum instead, two to four instructions a unit: 1.03 of the time with one wave per SIMD.)
+    auto first = [&](int u, int stride) { return (uint32_t)(u * UC < p.N ? u * UC : p.N) * (uint32_t)stride * 2u; };
     // (rows past the last one read as zeros through the range check; CHECKED: they are found by their number, for strides whose
     // offsets of rows past the last one may wrap around)
     auto load_k = [&](int u, i32x4(&r)[NLK], auto checked) {

@@ -28,15 +28,15 @@ def _close(out, ref):
     assert bad == 0, f"{bad} outside tolerance, max err {max_err}"
 
 
-def _run(a_gmk, b0_gnk, b1_gno, scale=1.0, mask=False, instance=capi.INSTANCE_AUTO, pad=(0, 0, 0, 0)):
-    """pad: extra elements per row of A, B0, B1, C (row strides larger than the extents)."""
+def _run(a_gmk, b0_gnk, b1_gno, scale=1.0, mask=False, instance=capi.INSTANCE_AUTO, pad=(0, 0, 0, 0), gap=0.0):
+    """pad: extra elements per row of A, B0, B1, C (row strides larger than the extents), those of the operands filled with gap."""
     import torch
     import gpu_util
     G, M, K = a_gmk.shape
     N, O = b0_gnk.shape[1], b1_gno.shape[2]
 
     def padded(x, p):
-        out = np.zeros(x.shape[:2] + (x.shape[2] + p,), np.float16)
+        out = np.full(x.shape[:2] + (x.shape[2] + p,), gap, np.float16)
         out[..., :x.shape[2]] = x
         return out
 
@@ -107,6 +107,18 @@ def test_gemm_softmax_gemm_units(K, O):
         for mask in (False, True):
             _close(_run(a, b0_gnk, b1, 2.0 * K ** -0.5, mask, 0),
                    lit.batched_gemm_softmax_gemm_f16(a, b0_gnk.transpose(0, 2, 1), b1, 2.0 * K ** -0.5, mask))
+
+
+@pytest.mark.parametrize("K, O", [(8, 8), (24, 104), (40, 24), (72, 40), (104, 72)])
+def test_gemm_softmax_gemm_row_gaps_are_not_read(K, O):
+    """K and O that leave chunks of a padded fragment row empty, NaNs between the rows of A, B0 and B1: units before, at and past the
+    last one, whose rows and chunks that do not exist read as zeros."""
+    for N in (64, 200, 257, 385):
+        a, b0_gnk, b1 = (uniform_f16((2, x, y), -1, 1, 1980 + i) for i, (x, y) in enumerate(((133, K), (N, K), (N, O))))
+        for mask in (False, True):
+            ref = lit.batched_gemm_softmax_gemm_f16(a, b0_gnk.transpose(0, 2, 1), b1, K ** -0.5, mask)
+            for instance in (0, 2):
+                _close(_run(a, b0_gnk, b1, K ** -0.5, mask, instance, (8, 24, 16, 8), np.nan), ref)
 
 
 @pytest.mark.parametrize("step", [0.01, 0.05, 0.2, 1.0])
