@@ -567,8 +567,10 @@ inline bool rows_in_16s(int M, int N, int K, int O, int batch, bool mask_upper)
     const long slabs = (long)batch * ((M + 127) / 128);
     if(head > 96)
         return slabs <= (mask_upper ? 512 : 256);
-    if(mask_upper && head > 32 && head <= 64 && N <= 512) // (130 x 375 x 375 13.2 / 13.8 us)
-        return slabs <= 512;
+    // (130 x 375 x 375 13.2 / 13.8 us; longer N, where the second workgroup of some CUs comes late enough: 43 x 768 x 768 13.9 / 14.9, 64 x 768 x
+    // 768 13.5 / 14.7, 47 x 896 x 896 0.97 of the time, but 75 x 640 x 640 1.04, 67 x 768 x 768 1.00)
+    if(mask_upper && head > 32 && head <= 64 && N < 1024)
+        return slabs <= (N <= 512 ? 512 : N < 768 ? 304 + 3 * (N - 512) / 8 : 384);
     return slabs <= 256 && (head > 64 ? false : head > 32 ? N <= (slabs <= 128 ? 1024 : 960) : N < 448);
 }
 

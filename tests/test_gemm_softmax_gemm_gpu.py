@@ -167,16 +167,20 @@ def test_gemm_softmax_gemm_nan_stays_in_its_row(instance):
 
 
 @pytest.mark.parametrize("G, M, N, K, mask, rows", [(2, 64, 1024, 64, False, 16), (2, 64, 1025, 64, False, 32), (129, 64, 960, 64, False, 16),
-                                                    (129, 64, 961, 64, False, 32), (512, 40, 64, 64, True, 16), (513, 40, 64, 64, True, 32),
-                                                    (257, 40, 513, 64, True, 32),
-                                                    (256, 100, 64, 128, False, 16), (257, 100, 64, 128, False, 32), (512, 40, 64, 128, True, 16),
-                                                    (513, 40, 64, 128, True, 32), (2, 64, 447, 32, False, 16), (2, 64, 448, 32, False, 32),
-                                                    (2, 64, 64, 80, False, 32), (2, 64, 64, 96, True, 32)])
+                                                    (129, 64, 961, 64, False, 32), (512, 128, 192, 64, True, 16), (513, 128, 192, 64, True, 32),
+                                                    (304, 128, 513, 64, True, 16), (305, 128, 513, 64, True, 32), (352, 128, 640, 64, True, 16),
+                                                    (353, 128, 640, 64, True, 32), (384, 128, 1023, 40, True, 16), (385, 128, 768, 64, True, 32),
+                                                    (257, 128, 1024, 64, True, 32),
+                                                    (256, 100, 192, 128, False, 16), (257, 100, 192, 128, False, 32), (512, 128, 192, 128, True, 16),
+                                                    (513, 128, 192, 128, True, 32), (2, 64, 447, 32, False, 16), (2, 64, 448, 32, False, 32),
+                                                    (2, 64, 192, 80, False, 32), (2, 128, 192, 96, True, 32)])
 def test_gemm_softmax_gemm_auto_on_both_sides_of_its_rule(G, M, N, K, mask, rows):
-    """AUTO takes 16-row waves for few slabs of a short N, 32-row waves otherwise: bit for bit one of the two."""
+    """AUTO takes 16-row waves for few slabs of a short N, 32-row waves otherwise: bit for bit the one, and not the other."""
     a, b0, b1 = (uniform_f16((G, x, K), -1, 1, 51 + i) for i, x in enumerate((M, N, N)))
     out = _run(a, b0, b1, K ** -0.5, mask)
-    np.testing.assert_array_equal(out.view(np.uint16), _run(a, b0, b1, K ** -0.5, mask, 2 if rows == 16 else 0).view(np.uint16))
+    by_rows = {16: _run(a, b0, b1, K ** -0.5, mask, 2), 32: _run(a, b0, b1, K ** -0.5, mask, 0)}
+    np.testing.assert_array_equal(out.view(np.uint16), by_rows[rows].view(np.uint16))
+    assert np.any(out.view(np.uint16) != by_rows[48 - rows].view(np.uint16)), "both kernels give the same: this shape shows nothing"
     _close(out[:2], lit.batched_gemm_softmax_gemm_f16(a[:2], b0[:2].transpose(0, 2, 1), b1[:2], K ** -0.5, mask))
 
 
