@@ -184,7 +184,8 @@ def test_gemm_softmax_gemm_auto_on_both_sides_of_its_rule(G, M, N, K, mask, rows
     _close(out[:2], lit.batched_gemm_softmax_gemm_f16(a[:2], b0[:2].transpose(0, 2, 1), b1[:2], K ** -0.5, mask))
 
 
-def test_gemm_softmax_gemm_closed_forms():
+@pytest.mark.parametrize("instance", [0, 2])
+def test_gemm_softmax_gemm_closed_forms(instance):
     """Zero scores: the uniform distribution, C = mean of B1's rows (exact: small integers over a power of
     two). Upper-triangle mask: row m averages rows 0..m, row 0 is B1[0] exactly. A dominant score selects
     one row of B1 exactly."""
@@ -192,10 +193,10 @@ def test_gemm_softmax_gemm_closed_forms():
     b1 = (np.arange(G * N * O).reshape(G, N, O) % 7).astype(np.float16)
     a0 = np.zeros((G, M, K), np.float16)
     b0 = uniform_f16((G, N, K), -1, 1, 71)
-    out = _run(a0, b0, b1)
+    out = _run(a0, b0, b1, instance=instance)
     np.testing.assert_array_equal(out, np.broadcast_to(b1.astype(np.float32).mean(axis=1, keepdims=True),
                                                        (G, M, O)).astype(np.float16))
-    out = _run(a0, b0, b1, mask=True)
+    out = _run(a0, b0, b1, mask=True, instance=instance)
     np.testing.assert_array_equal(out[:, 0], b1[:, 0])
     for m in (1, 3, 7, 127, 159):        # m + 1 a power of two, or within fp16 rounding otherwise
         want = b1[:, :m + 1].astype(np.float64).mean(axis=1)
@@ -204,11 +205,12 @@ def test_gemm_softmax_gemm_closed_forms():
     a[:, np.arange(M), np.arange(M) % K] = 1
     b0h = np.zeros((G, N, K), np.float16)
     b0h[:, (np.arange(K) * 5) % N, np.arange(K)] = 40
-    out = _run(a, b0h, b1)
+    out = _run(a, b0h, b1, instance=instance)
     np.testing.assert_array_equal(out, b1[:, ((np.arange(M) % K) * 5) % N])
 
 
-def test_gemm_softmax_gemm_running_maximum_is_rescaled():
+@pytest.mark.parametrize("instance", [0, 2])
+def test_gemm_softmax_gemm_running_maximum_is_rescaled(instance):
     """The row maximum sits in the LAST 128-column step and the early steps hold large negative scores, and
     the other way round: the one-pass softmax must rescale what it accumulated."""
     G, M, N, K, O = 1, 64, 512, 16, 32
@@ -218,36 +220,38 @@ def test_gemm_softmax_gemm_running_maximum_is_rescaled():
     for ramp in (np.linspace(-30, 8, N), np.linspace(8, -30, N)):
         b0 = np.zeros((G, N, K), np.float16)
         b0[0, :, 0] = ramp.astype(np.float16)
-        out = _run(a, b0, b1)
+        out = _run(a, b0, b1, instance=instance)
         _close(out, lit.batched_gemm_softmax_gemm_f16(a, b0.transpose(0, 2, 1), b1))
         # scores far apart (neighbours differ by 0.074 * 300): the result is the row of B1 at the maximum
-        out = _run(a, b0, b1, scale=300.0)
+        out = _run(a, b0, b1, scale=300.0, instance=instance)
         np.testing.assert_array_equal(out[0], np.broadcast_to(b1[0, int(np.argmax(b0[0, :, 0]))], (M, O)))
 
 
-def test_gemm_softmax_gemm_negative_scale():
+@pytest.mark.parametrize("instance", [0, 2])
+def test_gemm_softmax_gemm_negative_scale(instance):
     """A negative scale turns the softmax towards the SMALLEST raw score (the kernel moves the sign into A)."""
     G, M, N, K, O = 2, 96, 300, 32, 32
     a = uniform_f16((G, M, K), -1, 1, 21)
     b0_gnk = uniform_f16((G, N, K), -1, 1, 22)
     b1 = uniform_f16((G, N, O), -1, 1, 23)
     for mask in (False, True):
-        out = _run(a, b0_gnk, b1, -0.7, mask)
+        out = _run(a, b0_gnk, b1, -0.7, mask, instance)
         _close(out, lit.batched_gemm_softmax_gemm_f16(a, b0_gnk.transpose(0, 2, 1), b1, -0.7, mask))
         # same as a positive scale on the negated A
-        np.testing.assert_array_equal(out.view(np.uint16), _run(-a, b0_gnk, b1, 0.7, mask).view(np.uint16))
+        np.testing.assert_array_equal(out.view(np.uint16), _run(-a, b0_gnk, b1, 0.7, mask, instance).view(np.uint16))
 
 
-def test_gemm_softmax_gemm_padded_strides_and_scale_zero():
+@pytest.mark.parametrize("instance", [0, 2])
+def test_gemm_softmax_gemm_padded_strides_and_scale_zero(instance):
     G, M, N, K, O = 3, 72, 200, 64, 48
     a = uniform_f16((G, M, K), -1, 1, 11)
     b0_gnk = uniform_f16((G, N, K), -1, 1, 12)
     b1 = uniform_f16((G, N, O), -1, 1, 13)
-    out = _run(a, b0_gnk, b1, 0.125, False, pad=(8, 16, 24, 8))
+    out = _run(a, b0_gnk, b1, 0.125, False, instance, pad=(8, 16, 24, 8))
     _close(out, lit.batched_gemm_softmax_gemm_f16(a, b0_gnk.transpose(0, 2, 1), b1, 0.125))
     # scale 0 makes the scores irrelevant: same result as A = 0
-    np.testing.assert_array_equal(_run(a, b0_gnk, b1, 0.0).view(np.uint16),
-                                  _run(np.zeros_like(a), b0_gnk, b1).view(np.uint16))
+    np.testing.assert_array_equal(_run(a, b0_gnk, b1, 0.0, False, instance).view(np.uint16),
+                                  _run(np.zeros_like(a), b0_gnk, b1, 1.0, False, instance).view(np.uint16))
 
 
 @pytest.mark.parametrize("mask", [False, True])
@@ -283,5 +287,6 @@ def test_gemm_softmax_gemm_refused_arguments_and_empty_sum():
     assert capi.lib().ckx_num_instances(capi.OP_BATCHED_GEMM_SOFTMAX_GEMM) == 3
     assert b"SoftmaxGemm" in capi.lib().ckx_instance_name(capi.OP_BATCHED_GEMM_SOFTMAX_GEMM, 0)
     # N = 0: an empty sum, C = 0
-    out = _run(np.ones((1, 16, 8), np.float16), np.zeros((1, 0, 8), np.float16), np.zeros((1, 0, 8), np.float16))
-    np.testing.assert_array_equal(out, np.zeros((1, 16, 8), np.float16))
+    for instance in (0, 2):
+        out = _run(np.ones((1, 16, 8), np.float16), np.zeros((1, 0, 8), np.float16), np.zeros((1, 0, 8), np.float16), instance=instance)
+        np.testing.assert_array_equal(out, np.zeros((1, 16, 8), np.float16))
