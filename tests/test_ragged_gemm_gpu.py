@@ -3,7 +3,8 @@ its tiles (128 x 128 from 256 C tiles on, 64 x 64, 64 x 32 or 32 x 32 below, by 
 bytes, extents one short of and one past a C tile, fewer elements than one vector in the contiguous direction, operands that
 end at their last element, all layouts. Integer operands small enough that every fp32 partial sum is exact: the result is the
 rounded exact product, whatever the order of the sum, and int8 is compared bit for bit after wrapping."""
-import numpy as np
+import ctypes
+
 import pytest
 
 import composable_kernel_amd as ck
@@ -13,6 +14,24 @@ pytestmark = pytest.mark.gpu
 
 LAYOUTS = {"mk_nk": (ck.RowMajor, ck.ColumnMajor), "km_kn": (ck.ColumnMajor, ck.RowMajor),
            "km_nk": (ck.ColumnMajor, ck.ColumnMajor), "mk_kn": (ck.RowMajor, ck.RowMajor)}
+
+
+# one problem for each tile below the 128 x 128 one, one element over or under whole tiles
+SMALL = {(32, 32): (67, 93), (64, 32): (705, 497), (64, 64): (1021, 1003)}
+
+
+class _Tile(ctypes.Structure):
+    _fields_ = [("m", ctypes.c_int), ("n", ctypes.c_int)]
+
+
+def _tile(M, N, batch=1):
+    """rows and columns of the C tile that the problem runs on"""
+    if capi.lib()._ZN3ckx11ragged_tileEiii(M, N, batch) == 128:
+        return 128, 128
+    f = capi.lib()._ZN3ckx17ragged_small_tileEiii
+    f.argtypes, f.restype = [ctypes.c_int] * 3, _Tile
+    t = f(M, N, batch)
+    return t.m, t.n
 
 
 def _run(kind, layout, M, N, K, off):
@@ -46,13 +65,16 @@ def _run(kind, layout, M, N, K, off):
 
 @pytest.mark.parametrize("layout", sorted(LAYOUTS))
 @pytest.mark.parametrize("kind", ["i8", "f16", "bf16"])
-def test_k_around_the_k_tiles(kind, layout):
+@pytest.mark.parametrize("tile", sorted(SMALL))
+def test_k_around_the_k_tiles(kind, layout, tile):
     kt = 128 if kind == "i8" else 64
+    M, N = SMALL[tile]
+    assert _tile(M, N) == tile
     for tiles in range(0, 7):
         for d in (-1, 0, 1):
             K = tiles * kt + d
             if K > 0:
-                _run(kind, layout, 67, 93, K, 1)
+                _run(kind, layout, M, N, K, 1)
 
 
 @pytest.mark.parametrize("layout", sorted(LAYOUTS))
@@ -66,9 +88,11 @@ def test_tile_edges(kind, layout, shape):
 
 @pytest.mark.parametrize("layout", sorted(LAYOUTS))
 @pytest.mark.parametrize("kind", ["i8", "f16", "bf16"])
-@pytest.mark.parametrize("M, N", [(31, 33), (33, 31), (65, 1), (705, 497), (703, 511), (1021, 1003), (963, 1023)])
-def test_small_tiles(kind, layout, M, N):
-    """32 x 32 (the first three), 64 x 32 and 64 x 64 tiles at their edges, K around two K tiles"""
+@pytest.mark.parametrize("M, N, tile", [(31, 33, (32, 32)), (33, 31, (32, 32)), (65, 1, (32, 32)), (705, 497, (64, 32)), (703, 511, (64, 32)),
+                                        (1021, 1003, (64, 64)), (963, 1023, (64, 64))])
+def test_small_tiles(kind, layout, M, N, tile):
+    """32 x 32, 64 x 32 and 64 x 64 tiles at their edges, K around two K tiles"""
+    assert _tile(M, N) == tile
     for K in (127, 129, 259):
         _run(kind, layout, M, N, K, off=0)
         _run(kind, layout, M, N, K, off=5)
@@ -96,13 +120,13 @@ def test_batches_past_one_launch_dimension():
 def test_k_below_one_vector_and_half_a_k_tile(kind, K):
     """Rows of less than one vector are read element by element (int8 with another order of the slots), and a second k-step past
     K is left out, in C tiles of full, partial and single rows."""
-    for M, N in ((147, 869), (64, 65), (1, 63), (130, 3)):
+    for M, N in ((147, 869), (64, 65), (1, 63), (130, 3), *SMALL.values()):
         _run(kind, "mk_nk", M, N, K, off=1)
         _run(kind, "km_nk", M, N, K, off=0)
         _run(kind, "mk_kn", M, N, K, off=1)
 
 
-# ---- the 128 x 128 tile (256 of them and more): its epilogue has 16 columns per lane where B is K-contiguous
+# ---- epilogues: 16 columns per lane on the 128 x 128 tile (256 of them and more) where B is K-contiguous, 8 on 64 x 64, 4 on 64 x 32 and 32 x 32
 def _big(kind, M, N, K, lda, ldb, seed):
     """Small integers with leading dimensions of their own: fp16 results and int8 accumulators are exact."""
     import torch
@@ -125,12 +149,13 @@ def _requant(acc, sg, sr, rounded):
 
 
 @pytest.mark.parametrize("epilogue", ["rounded", "literal", "per_column", "per_column_relu"])
-@pytest.mark.parametrize("shape", [(2047, 2049, 195, 201, 197, 2051), (2100, 2000, 65, 65, 67, 2003)])
-def test_large_tile_int8_epilogues(epilogue, shape):
+@pytest.mark.parametrize("shape, tile", [((2047, 2049, 195, 201, 197, 2051), (128, 128)), ((2100, 2000, 65, 65, 67, 2003), (128, 128))] +
+                         [((M, N, 451, 453, 455, N + 2), tile) for tile, (M, N) in sorted(SMALL.items())])
+def test_int8_epilogues(epilogue, shape, tile):
     import torch
     import gpu_util
     M, N, K, lda, ldb, ldc = shape
-    assert capi.lib()._ZN3ckx11ragged_tileEiii(M, N, 1) == 128
+    assert _tile(M, N) == tile
     a, b, acc = _big("i8", M, N, K, lda, ldb, 21)
     c = torch.full((M, ldc), 77, dtype=torch.int8, device="cuda")
     if epilogue.startswith("per_column"):
@@ -152,11 +177,12 @@ def test_large_tile_int8_epilogues(epilogue, shape):
 
 
 @pytest.mark.parametrize("functor", ["relu_add", "bilinear"])
-def test_large_tile_d_operands_on_any_element(functor):
+@pytest.mark.parametrize("M, N, K, tile", [(2049, 2047, 131, (128, 128))] + [(M, N, 227, tile) for tile, (M, N) in sorted(SMALL.items())])
+def test_d_operands_on_any_element(functor, M, N, K, tile):
     import torch
     import gpu_util
-    M, N, K, ldd, ldc = 2049, 2047, 131, 2053, 2049
-    assert capi.lib()._ZN3ckx11ragged_tileEiii(M, N, 1) == 128
+    ldd, ldc = N + 6, N + 2
+    assert _tile(M, N) == tile
     a, b, acc = _big("f16", M, N, K, K + 2, K + 4, 22)
     d = [torch.randint(-50, 51, (M * ldd + 1,), device="cuda").half() for _ in range(2)]
     rows = [x[1:].reshape(M, ldd)[:, :N].float() for x in d]
@@ -177,7 +203,7 @@ def test_batches_on_both_tiles(kind, G, M, N, K, large):
     """Batches whose tiles add up past 256 although one has a few; odd batch strides, the gaps between the C batches untouched."""
     import torch
     import gpu_util
-    assert capi.lib()._ZN3ckx11ragged_tileEiii(M, N, G) == (128 if large else 64)
+    assert _tile(M, N, G) == ((128, 128) if large else (64, 64))
     g = torch.Generator(device="cuda").manual_seed(23)
     dt = torch.int8 if kind == "i8" else torch.float16
     bsa, bsb, bsc = M * K + 3, N * K + 5, M * N + 7
