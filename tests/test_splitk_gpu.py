@@ -119,6 +119,52 @@ def test_conv2d_split_k(force_split, dtype):
         assert bad == 0, max_err
 
 
+# (N, C, Hi, filter, stride, K, runs): runs of one K tile, of two with a shorter last one, of three and five; a K tail; two units to a
+# workgroup and more, so that the load cursors pass from run to run
+@pytest.mark.parametrize("case", [(2, 56, 15, 3, 2, 256, 8), (1, 32, 20, 3, 2, 136, 5), (2, 64, 15, 3, 2, 256, 5), (3, 64, 33, 3, 2, 200, 3),
+                                  (2, 64, 15, 3, 2, 256, 2), (2, 16, 30, 5, 3, 128, 7), (8, 56, 71, 3, 2, 256, 8), (13, 64, 71, 3, 2, 256, 5)])
+def test_strided_conv2d_on_the_256x256_tile_split_k(force_split, case):
+    """Strided fp16 layers on 256 x 256 tiles load A a K tile further ahead than B, so that the two are in different K runs, and in
+    different tiles, at times. Small-integer operands, exact in any order: bit for bit the unsplit result, the two-stage 64 x 64 instance
+    at the same split and (small cases) the oracle, plain and with bias and residual."""
+    import torch
+    import gpu_util
+    n, c, hw, f, s, k, runs = case
+    rng = np.random.default_rng(78)
+    inp, wei = rng.integers(-2, 3, (n, hw, hw, c)).astype(np.float16), rng.integers(-1, 2, (k, f, f, c)).astype(np.float16)
+    ho = (hw + 2 * (f // 2) - f) // s + 1
+    bias, resi = rng.integers(-3, 4, (k,)).astype(np.float16), rng.integers(-3, 4, (n, ho, ho, k)).astype(np.float16)
+    dx, dw, db, dr = (gpu_util.dev(x) for x in (inp, wei, bias, resi))
+    geom = (n, k, c, [hw] * 2, [f] * 2, [ho] * 2, [s] * 2, [1] * 2, [f // 2] * 2, [f // 2] * 2)
+
+    def run(instance, fused, split):
+        force_split(runs if split else 0)
+        y = torch.full((n, ho, ho, k), float("nan"), dtype=torch.float16, device="cuda")
+        if fused:
+            op = ck.DeviceConv2dFwdBiasActivationF16(instance)
+            arg = op.MakeArgumentPointer(dx, dw, y, db, dr, *geom, None, None, ck.AddReluAdd())
+        else:
+            op = ck.DeviceConv2dFwdF16(instance)
+            arg = op.MakeArgumentPointer(dx, dw, y, *geom)
+        assert op.IsSupportedArgument(arg), capi.last_error()
+        if split:
+            need = op.GetWorkSpaceSize(arg)
+            assert need == runs * n * ho * ho * k * 4
+            op.SetWorkSpacePointer(arg, torch.full((need,), 0x7F, dtype=torch.uint8, device="cuda"))
+        op.MakeInvokerPointer().Run(arg, ck.StreamConfig(gpu_util.stream()))
+        torch.cuda.synchronize()
+        return y
+
+    for fused in (False, True):
+        got = run(0, fused, True)
+        assert torch.equal(got, run(0, fused, False)), "the split changes the result"
+        assert torch.equal(got, run(4, fused, True)), "differs from the 64 x 64 instance"
+        if n < 4:
+            geo = ((s, s), (1, 1), (f // 2, f // 2))
+            want = fast.conv2d_fwd_bias_relu_f16(inp, wei, bias, resi, *geo) if fused else fast.conv2d_fwd_f16(inp, wei, *geo)
+            np.testing.assert_array_equal(got.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("shape", [(8, 10300, 256), (9, 10300, 256), (16, 5200, 192), (16, 1000, 320), (17, 10300, 128),
                                    (32, 5200, 256), (33, 10300, 128), (48, 700, 4096), (64, 10304, 192), (65, 700, 2048),
                                    # few columns under a long K (tile kernel with a K split when the workspace is there),
