@@ -1,13 +1,15 @@
 """GPU parity of the 128 x 64 row pairs and 64 x 128 column pairs that run behind the four-stage 64 x 64 instance (csrc/tile_pairs.hip): bit for bit what the
 two-stage 64 x 64 instance gives for the same problem (each element is the same sum in the same order), at the edges of the line between one
 tile and a pair, with rows that end in a pair's first half, one K tile and more than the three stages hold, K splits, every
-epilogue, convolutions and batches."""
+epilogue, convolutions and batches, and the exact result (small integers) by another way."""
 import ctypes
 
+import numpy as np
 import pytest
 
 import composable_kernel_amd as ck
 from composable_kernel_amd import capi
+from oracle import fast
 
 pytestmark = pytest.mark.gpu
 FOUR_STAGE, TWO_STAGE = 8, 4
@@ -82,8 +84,14 @@ def test_gemm(form, M, N, K):
 
     got = _both(make, c)
     assert bool((got[M] == 77).all()), "wrote past the last row"
-    if form in ("f16", "bf16"):  # |sums| < 2^24: the rounded exact product
-        assert torch.equal(got[:M], (a.float() @ b.float().T.contiguous()).to(a.dtype))
+    acc = a.float() @ b.float().T.contiguous()  # |sums| < 2^24: the exact product
+    if kind == "i8":
+        acc = acc.to(torch.int32).cpu().numpy()
+        want = fast.epilogue_i8_mul2_clamp(acc, scales.cpu().numpy(), True) if form == "i8_per_column" else \
+            fast.epilogue_i8(acc, fast.EPI_REQUANT_RND if form == "i8_rounded" else fast.EPI_PASSTHROUGH, 0.02, 0.7)
+        np.testing.assert_array_equal(got[:M].cpu().numpy(), want)
+    else:
+        assert torch.equal(got[:M], ((acc + d[0].float()).clamp_min(0) + d[1].float() if form == "f16_add_relu_add" else acc).to(a.dtype))
 
 
 @pytest.mark.parametrize("kind", ["i8", "f16", "bf16"])
@@ -104,9 +112,42 @@ def test_k_major(kind, layout, M, N, K):
 
     got = _both(make, c)
     assert bool((got[M] == 77).all()), "wrote past the last row"
-    if kind != "i8":  # |sums| < 2^24: the rounded exact product
-        a_mk, b_kn = (a if la == "mk" else a.T).float().contiguous(), (b.T if lb == "nk" else b).float().contiguous()
-        assert torch.equal(got[:M], (a_mk @ b_kn).to(a.dtype))
+    a_mk, b_kn = (a if la == "mk" else a.T).float().contiguous(), (b.T if lb == "nk" else b).float().contiguous()
+    acc = a_mk @ b_kn  # |sums| < 2^24: the exact product
+    if kind == "i8":
+        np.testing.assert_array_equal(got[:M].cpu().numpy(), fast.epilogue_i8(acc.to(torch.int32).cpu().numpy(), fast.EPI_REQUANT_RND, 0.02, 0.7))
+    else:
+        assert torch.equal(got[:M], acc.to(a.dtype))
+
+
+@pytest.fixture
+def force_runs():
+    L = capi.lib()
+    before = L.ckx_set_forced_k_runs(0)
+    yield L.ckx_set_forced_k_runs
+    L.ckx_set_forced_k_runs(before)
+
+
+@pytest.mark.parametrize("kind", ["i8", "f16", "bf16"])
+@pytest.mark.parametrize("M, N, K, runs", [(128, 4096, 1024, 4), (500, 1104, 1600, 3), (112, 2208, 2064, 5)])
+def test_k_split_with_a_k_major_b(force_runs, kind, M, N, K, runs):
+    """B K-major keeps its pairs under a K split (A K-major does not)."""
+    import torch
+    assert _pays(M, N, runs)
+    a, b = _operand(kind, (M, K), 15), _operand(kind, (K, N), 16)
+    c = torch.empty((M, N), dtype=a.dtype, device="cuda")
+    force_runs(runs)
+
+    def make(instance):
+        op = {"i8": ck.DeviceGemmInt8, "f16": ck.DeviceGemmF16, "bf16": ck.DeviceGemmBF16}[kind](instance, BLayout=ck.RowMajor)
+        arg = op.MakeArgumentPointer(a, b, c, M, N, K, K, N, N, None, None, ck.PassThrough())
+        need = op.GetWorkSpaceSize(arg)
+        assert need == runs * M * N * 4
+        op.SetWorkSpacePointer(arg, torch.full((need,), 0x7F, dtype=torch.uint8, device="cuda"))
+        return op, arg
+
+    got, acc = _both(make, c), a.float() @ b.float()
+    assert torch.equal(got, acc.to(torch.int32).to(torch.int8) if kind == "i8" else acc.to(a.dtype))
 
 
 @pytest.mark.parametrize("kind", ["i8", "f16"])
@@ -145,31 +186,47 @@ def test_batches(G, M, N, K, columns):
 
 
 @pytest.mark.parametrize("form", ["i8", "f16", "f16_bias_relu", "f16_bias_relu_add", "i8_3d", "f16_3d"])
-@pytest.mark.parametrize("N, C, K, hw, f, stride", [(32, 64, 256, 14, 3, 1), (9, 48, 72, 41, 5, 1), (5, 32, 264, 63, 3, 2)])
-def test_conv(form, N, C, K, hw, f, stride):
+@pytest.mark.parametrize("N, C, K, hw, f, stride, runs", [(32, 64, 256, 14, 3, 1, 1), (9, 48, 72, 41, 5, 1, 1), (5, 32, 264, 63, 3, 2, 1),
+                                                          (8, 64, 256, 14, 3, 1, 3), (3, 48, 136, 29, 3, 1, 4)])
+def test_conv(force_runs, form, N, C, K, hw, f, stride, runs):
     import torch
     nd = 3 if form.endswith("3d") else 2
     if nd == 3:
-        N, hw, K = 2, 13 * stride - (stride - 1), 264
+        N, hw, K, runs = (2, 13 * stride - (stride - 1), 264, 1) if runs == 1 else (1, 12, 264, 3)
     ho = (hw + 2 * (f // 2) - f) // stride + 1
+    M = N * ho ** nd
+    assert _pays(M, K, runs)
     kind = form.split("_")[0]
     x, w = _operand(kind, (N, *[hw] * nd, C), 9), _operand(kind, (K, *[f] * nd, C), 10)
     bias, r = _operand("f16", (K,), 11), _operand("f16", (N, *[ho] * nd, K), 12)
     y = torch.empty((N, *[ho] * nd, K), dtype=x.dtype, device="cuda")
     geom = (N, K, C, [hw] * nd, [f] * nd, [ho] * nd, [stride] * nd, [1] * nd, [f // 2] * nd, [f // 2] * nd)
+    force_runs(runs if runs > 1 else 0)
 
     def make(instance):
         if "bias" in form:
             op = ck.DeviceConv2dFwdBiasActivationF16(instance)
             if form.endswith("add"):
-                return op, op.MakeArgumentPointer(x, w, y, bias, r, *geom, None, None, ck.AddReluAdd())
-            return op, op.MakeArgumentPointer(x, w, y, bias, *geom, None, None, ck.AddRelu())
-        if nd == 3:
-            op = (ck.DeviceConvNdFwdInt8 if kind == "i8" else ck.DeviceConvNdFwdF16)(3, instance)
+                arg = op.MakeArgumentPointer(x, w, y, bias, r, *geom, None, None, ck.AddReluAdd())
+            else:
+                arg = op.MakeArgumentPointer(x, w, y, bias, *geom, None, None, ck.AddRelu())
         else:
-            op = (ck.DeviceConv2dFwdInt8 if kind == "i8" else ck.DeviceConv2dFwdF16)(instance)
-        cop = ck.RequantReluRequant(0.02, 0.7, rounded=True) if kind == "i8" else ck.PassThrough()
-        return op, op.MakeArgumentPointer(x, w, y, *geom, None, None, cop)
+            if nd == 3:
+                op = (ck.DeviceConvNdFwdInt8 if kind == "i8" else ck.DeviceConvNdFwdF16)(3, instance)
+            else:
+                op = (ck.DeviceConv2dFwdInt8 if kind == "i8" else ck.DeviceConv2dFwdF16)(instance)
+            cop = ck.RequantReluRequant(0.02, 0.7, rounded=True) if kind == "i8" else ck.PassThrough()
+            arg = op.MakeArgumentPointer(x, w, y, *geom, None, None, cop)
+        if runs > 1:
+            need = op.GetWorkSpaceSize(arg)
+            assert need == runs * M * K * 4
+            op.SetWorkSpacePointer(arg, torch.full((need,), 0x7F, dtype=torch.uint8, device="cuda"))
+        return op, arg
 
-    _both(make, y)
-    assert _pays(N * ho ** nd, K)
+    got, (hx, hw_) = _both(make, y).cpu().numpy(), (t.cpu().numpy() for t in (x, w))  # |sums| < 2^24: exact
+    where = ([stride] * nd, [1] * nd, [f // 2] * nd)
+    if "bias" in form:
+        want = fast.conv2d_fwd_bias_relu_f16(hx, hw_, bias.cpu().numpy(), r.cpu().numpy() if form.endswith("add") else None, *where)
+    else:
+        want = fast.convnd_fwd(hx, hw_, *where, epi=fast.EPI_REQUANT_RND if kind == "i8" else fast.EPI_PASSTHROUGH, scale_gemm=0.02, scale_relu=0.7)
+    np.testing.assert_array_equal(got, want)
