@@ -1309,7 +1309,7 @@ const char* ckx_instance_name(int op, int instance)
         return nullptr;
     s = std::string(fam) + "<" +
         (op == CKX_OP_BATCHED_GEMM_GEMM || op == CKX_OP_BATCHED_GEMM_SOFTMAX_GEMM
-             ? ckx::gemm_gemm_instance_name(instance)
+             ? ckx::gemm_gemm_instance_name(instance, op == CKX_OP_BATCHED_GEMM_SOFTMAX_GEMM)
          : (op == CKX_OP_CONV2D_FWD_F16 || op == CKX_OP_CONV2D_FWD_I8) && instance >= kNumTiles
              ? (instance == kConvPatchInstance ? kPatchName : instance == kConvPointwiseInstance ? kPointwiseName
                 : instance == kConvStemInstance ? kStemName : instance == kConvRowsInstance ? kRowsName : kGenericName)

@@ -13,8 +13,8 @@
 //   round-to-nearest-even conversion to fp16. B1 is transposed while it is staged into LDS
 //   so that its fragment is one 16-byte read as well.
 //
-// SOFTMAX variant (upstream's DeviceBatchedGemmSoftmaxGemm, "attention") on 16 rows per wave, for problems too small to give every
-// SIMD two waves of 32 (gemm_softmax_gemm.hpp has the kernel for all others):
+// SOFTMAX variant (upstream's DeviceBatchedGemmSoftmaxGemm, "attention") on 16 rows per wave, for launches whose shorter
+// chain of steps wins: about one workgroup per CU and short N or wide heads, see rows_in_16s() (gemm_softmax_gemm.hpp has the kernel for all others):
 //   C[g] = half( half(softmax_n(scale * A[g] * B0[g], masked)) * B1[g] )
 // with the softmax along N in one pass over N (running row maximum and running sum): a step's
 // scores become p = exp(s - running max), the output accumulators and the running sum are rescaled
@@ -453,9 +453,10 @@ __global__ __launch_bounds__(NW * 64)
 // ---------------------------------------------------------------- host side
 constexpr int kNumGemmGemmInstances = 3;
 
-inline const char* gemm_gemm_instance_name(int i)
+inline const char* gemm_gemm_instance_name(int i, bool softmax)
 {
-    return i == 0   ? "MI355X_Mfma16_GemmGemm<128 rows, 4 waves x 32, 128-col steps, K<=128, O<=128>"
+    return i == 0 && softmax ? "MI355X_Mfma32_GemmSoftmaxGemm<128 rows, 4 waves x 32, steps of 64 or 32 cols, K<=128, O<=128>"
+           : i == 0 ? "MI355X_Mfma16_GemmGemm<128 rows, 4 waves x 32, 128-col steps, K<=128, O<=128>"
            : i == 1 ? "MI355X_Mfma16_GemmGemm<64 rows, 4 waves x 16, 128-col steps, K<=128, O<=128>"
                     : "MI355X_Mfma16_GemmGemm<128 rows, 8 waves x 16, 128-col steps, K<=128, O<=128>";
 }

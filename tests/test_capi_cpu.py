@@ -34,6 +34,11 @@ def test_instance_factory_lists_named_instances():
         names = [L.ckx_instance_name(op, i).decode() for i in range(n)]
         assert len(set(names)) == n
         assert L.ckx_instance_name(op, n) is None
+    # instance 0 of the softmax operator is a kernel of its own (32x32x16 MFMAs), the others are shared with GEMM-GEMM
+    plain, soft = ([L.ckx_instance_name(op, i).decode().split("<", 1)[1] for i in range(3)]
+                   for op in (capi.OP_BATCHED_GEMM_GEMM, capi.OP_BATCHED_GEMM_SOFTMAX_GEMM))
+    assert "Mfma32_GemmSoftmaxGemm<128 rows, 4 waves x 32" in soft[0] and "Mfma16_GemmGemm<128 rows, 4 waves x 32" in plain[0]
+    assert soft[1:] == plain[1:]
     assert L.ckx_num_instances(99) == 0
     assert len(ck.DeviceGemmInt8.GetInstances()) == L.ckx_num_instances(capi.OP_GEMM_I8)
 
