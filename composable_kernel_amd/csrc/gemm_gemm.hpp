@@ -31,6 +31,7 @@
 #include <string>
 
 #include "gemm_tile.hpp"
+#include "tile_launch.hpp"
 
 namespace ckx {
 
@@ -565,7 +566,7 @@ hipError_t gemm_softmax_gemm_launch(const GemmGemmArgs& a, hipStream_t s); // ge
 inline bool rows_in_16s(int M, int N, int K, int O, int batch, bool mask_upper)
 {
     const int head   = K > O ? K : O;
-    const long slabs = (long)batch * ((M + 127) / 128);
+    const long slabs = (long)batch * ((M + 127) / 128) * 256 / num_cus(); // (as on 256 CUs, which the lines here were measured on)
     if(head > 96)
         return slabs <= (mask_upper ? 512 : 256);
     // (130 x 375 x 375 13.2 / 13.8 us; longer N, where the second workgroup of some CUs comes late enough: 43 x 768 x 768 13.9 / 14.9, 64 x 768 x

@@ -1,6 +1,7 @@
 // Launcher of the GEMM for operands that are no whole 16-byte vectors (a translation unit of its own so that its kernels
 // compile beside the others).
 #include "gemm_ragged.hpp"
+#include "tile_launch.hpp"
 
 namespace ckx {
 
@@ -47,7 +48,7 @@ int ragged_tile(int M, int N, int batch)
     const long n        = batch > 1 ? batch : 1;
     const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128) * n, tiles64 = (long)((M + 63) / 64) * ((N + 63) / 64) * n;
     // (... or where one batch of the small ones is more than a launch holds)
-    return (tiles128 >= 256 && 10 * tiles128 <= 3 * tiles64) || tiles64 / n > kMostBlocks ? 128 : 64;
+    return (tiles128 >= num_cus() && 10 * tiles128 <= 3 * tiles64) || tiles64 / n > kMostBlocks ? 128 : 64;
 }
 
 RaggedTile ragged_small_tile(int M, int N, int batch)
@@ -58,13 +59,13 @@ RaggedTile ragged_small_tile(int M, int N, int batch)
     // of the time on average, 34 x 479 x 3569 20.9 -> 12.5 us, 1184 x 551 x 143 5.2 -> 4.6, 305 x 1011 x 2521 15.3 -> 12.0;
     // 2001 x 1003 x 1025 stays (15.6 against 19.9 on 64 x 32, 23.7 on 32 x 32; 15.4 on a 128 x 64 one, which gains 10 % at most
     // elsewhere and is not built).
-    const long n     = batch > 1 ? batch : 1;
+    const long n     = batch > 1 ? batch : 1, cus = num_cus();
     const auto tiles = [&](RaggedTile t) { return (((long)M + t.m - 1) / t.m) * (((long)N + t.n - 1) / t.n) * n; };
     RaggedTile best  = {64, 64};
-    long least       = (tiles(best) + 255) / 256 * 128;
+    long least       = (tiles(best) + cus - 1) / cus * 128;
     for(const RaggedTile t : {RaggedTile{64, 32}, RaggedTile{32, 32}})
     {
-        const long rows = (tiles(t) + 255) / 256 * (t.m + t.n);
+        const long rows = (tiles(t) + cus - 1) / cus * (t.m + t.n);
         if(16 * rows <= 15 * least && tiles(t) / n <= kMostBlocks)
             best = t, least = rows;
     }
