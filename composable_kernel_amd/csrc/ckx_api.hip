@@ -1085,7 +1085,7 @@ int run_conv(int op, const void* in, const void* wei, void* out, const ckx_conv2
     const bool fused = f16_fused(epi) && g.ksplit == 1;
     // A a K tile further ahead (AHEAD in gemm_tile.hpp): strides that leave a pixel to less than about three of the filter's taps, so that
     // 3/10 and more of every K tile's A are new to the L2, which the column tiles of a row of tiles share. us, tenths: 3 x 3 stride 2, K
-    // 256 (4.4) 158 -> 152, 193 -> 182, 117 -> 109; 5 x 5 stride 3, K 256 (3.6) 135 -> 124.5; below: 3 x 3 stride 2, K 512 (2.2) 341 -> 319
+    // 256 (4.4) 166.0 -> 159.9 (128 x 71 x 71, C 192), 112.7 -> 104.8 (122 x 58 x 58, C 208); 5 x 5 stride 3, K 256 (3.6) 128.6 -> 116.0; below: 3 x 3 stride 2, K 512 (2.2) 341 -> 319
     // but 49.5 -> 50.6, 5 x 5 stride 3, K 512 (1.8) 226 -> 233, 5 x 5 stride 2, K 256 (1.6) 141.3 -> 142.5.
     const int taps   = d->Y * d->X;
     const bool ahead = es == 2 && t.bm * t.bn == 256 * 256 && taps > 1 && 10l * d->stride_h * d->stride_w >= 3l * taps * g.tiles_n;

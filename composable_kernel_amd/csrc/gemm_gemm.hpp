@@ -562,7 +562,9 @@ hipError_t gemm_softmax_gemm_launch(const GemmGemmArgs& a, hipStream_t s); // ge
 // causal 15.5 / 15.8, but 32 x 1024 x 1024 19.6 / 17.3, 5 x 1536 x 1536 21.8 / 21.2, 175 x 512 x 512 33.2 / 26.7, 350 x 256 x 256 21.4 / 18.2;
 // heads of 128: 64 x 512 x 512 17.1 / 18.1, 21 x 1536 x 1536 causal 37.9 / 38.6, 35 x 1362 x 1362 causal 37.5 / 40.2, but 36 x 1384 x 1384
 // 72.0 / 54.6, 63 x 1357 x 1357 causal 67.9 / 51.2; heads of 32: 128 x 256 x 256 5.6 / 5.8, but 64 x 512 x 512 8.3 / 8.1, 32 x 1024 x 1024
-// 15.6 / 12.5; of 80: 32 x 256 x 256 8.6 / 7.9.
+// 15.6 / 12.5; of 80: 32 x 256 x 256 8.6 / 7.9. The lines in N lie on the careful side: with one slab to a batch (M = 128) 32 rows are level with 16 at N 768 and
+// 1.02 to 1.08 ahead from 832 on (heads of 64, 200 batches: 960 17.4 / 16.1, 968 17.7 / 16.8, 1024 17.6 / 16.7, 1032 18.7 / 17.6), and for heads of
+// 32 1.02 to 1.14 ahead from 320 on (128 batches: 384 6.8 / 6.5, 440 8.2 / 7.5, 448 8.3 / 7.2, 480 8.1 / 7.7).
 inline bool rows_in_16s(int M, int N, int K, int O, int batch, bool mask_upper)
 {
     const int head   = K > O ? K : O;

@@ -55,8 +55,8 @@ RaggedTile ragged_small_tile(int M, int N, int batch)
 {
     // The tile with the fewest operand rows through the busiest CU, its tiles times (m + n); a smaller one for a sixteenth less. A
     // K tile takes 0.31 us of a CU for 64 + 64 rows, 0.24 for 64 + 32, 0.16 for 32 + 32, whether one workgroup or several ask for
-    // them. Of 43 random problems below the 128 x 128 line 26 run on one of the smaller two, none slower than on 64 x 64: 0.86
-    // of the time on average, 34 x 479 x 3569 20.9 -> 12.5 us, 1184 x 551 x 143 5.2 -> 4.6, 305 x 1011 x 2521 15.3 -> 12.0;
+    // them. Of 137 random problems below the 128 x 128 line 115 run on 32 x 32 tiles, in 0.50 to 1.02 of the time on 64 x 64 ones, 0.84 on
+    // average, and four on 64 x 32, 0.92: 34 x 479 x 3569 20.8 -> 12.1 us, 1184 x 551 x 143 5.2 -> 4.6, 305 x 1011 x 2521 15.3 -> 12.0;
     // 2001 x 1003 x 1025 stays (15.6 against 19.9 on 64 x 32, 23.7 on 32 x 32; 15.4 on a 128 x 64 one, which gains 10 % at most
     // elsewhere and is not built).
     const long n     = batch > 1 ? batch : 1, cus = num_cus();

@@ -18,11 +18,13 @@
 // instructions of ANOTHER unit, and so on: unit u's softmax among the products of unit u + 1's scores and unit u - 1's output.
 // What is left over 4096 columns of heads of 64: the running maximum of some row of the wave rises in two units of three, and raising it and
 // rescaling what has been accumulated takes about 50 vector instructions (a maximum that lags behind, moved on a 2^8-fold excess only, would
-// take 332 and 176 us for the first two figures below, but its probabilities are rounded at less favourable places: 2-norm of the error
-// against float64 2.62e-4 where this one and the 16-row kernel have 2.53e-4); and the clock, which the power limit holds at 1.9 GHz (with
+// take 0.98 and 0.96 of the time of the first two figures below, but its probabilities are rounded at less favourable places: 2-norm of the
+// error against float64 2.62e-4 where this one and the 16-row kernel have 2.53e-4); and the clock, which the power limit holds at 1.9 GHz (with
 // operands of zeros the same launch takes 0.75 of the time).
-// 64 x 4096 x 4096 x 64 386 -> 340 us, causal 195 -> 184; 32 x 2048 x 2048 x 128 100 -> 83, x 80 95 -> 59, causal 52 -> 42; 64 x 2048 x 2048 x 32
-// 81 -> 60 (before: 16x16x32 MFMAs, sums by v_dot2, softmax and products one after the other).
+// Counters of 64 x 4096 x 4096 x 64 (of the time that two waves share a SIMD): matrix core busy 50 %, vector instructions active 71 %, 1.21 together; with
+// 16x16x32 MFMAs, sums by v_dot2 and softmax and products one after the other 34 and 64 %, 0.98. us, that kernel and this one in turn on one card:
+// 394.7 -> 359.1, causal 184.6 -> 179.4 (192.4 -> 189.5 with new operands in each pass); 32 x 2048 x 2048 x 128 92.4 -> 80.9, x 80 89.8 -> 58.8; 64 x 2048
+// x 2048 x 32 79.1 -> 59.2. 48 + 120 random problems 0.76 and 0.88 of the time.
 #pragma once
 
 #include "gemm_gemm.hpp"

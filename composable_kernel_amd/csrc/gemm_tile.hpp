@@ -695,7 +695,7 @@ struct GemmTile
     // A third stage for the A tiles, which fills the LDS of a CU with the 256 x 256 tile's 64 KB stages: the loads of A are a K tile
     // further ahead than those of B and have one more to arrive in. For strided convolutions, whose filter taps share few pixels: most
     // of a K tile's A comes from beyond the L2 then and takes longer than the half to one K tile that two stages leave it (128 x 71 x 71, C
-    // 192 -> K 256, 3 x 3 stride 2, bias + ReLU 159 -> 152.6 us; 122 x 58 x 58, C 208 -> K 256 stride 2 116.5 -> 108.8). With unit stride the
+    // 192 -> K 256, 3 x 3 stride 2, bias + ReLU 166.0 -> 159.9 us with new operands in each pass; 122 x 58 x 58, C 208 -> K 256 stride 2 112.7 -> 104.8). With unit stride the
     // L2 has the pixels and the second load cursor costs up to 2 % (223 x 15 x 15, C 448 -> K 256 97.8 -> 99.7), as it does with dense K-major
     // operands (f16 4096^3 km_nk 105.8 -> 107.1).
     static_assert(!AHEAD || (ES == 2 && NST == 2), "the int8 epilogue's table finds no room");
@@ -946,8 +946,8 @@ struct GemmTile
                 {
                     const int hi0 = (int)a_hw0[j] >> 16, wi0 = (int)(a_hw0[j] << 16) >> 16;
                     // (every condition is evaluated: with && the compiler put branches on the lane mask around each load of the 3-D
-                    // kernels, and a K tile's half was five basic blocks instead of one. 36 3-D problems 0.938 of the time, none slower: 16 x
-                    // 32^3, C 64 -> K 64 144.6 -> 137 us, 3 x 24^3, C 144 -> K 112 stride 2 31.2 -> 26.5. The tap itself is divided out anew for
+                    // kernels, and a K tile's half was five basic blocks instead of one. 60 3-D problems 0.93 of the time, none slower: 16 x
+                    // 32^3, C 64 -> K 64 152.3 -> 148.1 us (new operands in each pass), 3 x 24^3, C 144 -> K 112 stride 2 30.5 -> 25.4. The tap itself is divided out anew for
                     // every K tile: moved on digit by digit with carries, without a multiplication, it was slower, 1.002.)
                     bool ok = ((uint32_t)(hi0 + c.tap_dh) < (uint32_t)p.cv.Hi) & ((uint32_t)(wi0 + c.tap_dw) < (uint32_t)p.cv.Wi);
                     if constexpr(IM2COL == 2)

@@ -15,12 +15,11 @@ bool row_pairs_pay(long M, long N, long runs)
     // What bounds two co-resident 64 x 64 workgroups is the operand bytes that their CU loads (65 to 82 bytes per ns), and both load the same
     // rows of B where they are above one another: a pair loads 192 rows per K tile where they load 256. So the line is
     // where the busiest CU loads fewer: no gain with one workgroup per CU, with a single row tile, or with an odd number of row tiles that makes
-    // a second round. 43 of 52 random GEMMs and convolutions on the four-stage instance with more than one workgroup per CU are on this
-    // side, 0.69 to 1.00 of the time, 0.92 on average (int8 67 x 10990 x 9024 35.4 -> 24.5 us, 32 x 14 x 14, C = K = 256 13.0 -> 11.8, 128 x
-    // 4096 x 11008 21.3 -> 20.0); the others take 1.00 to 1.25 as pairs. Eight waves of 16 rows as in the 64 x 64 kernel (four of 32 take
-    // 1.2 to 1.5 times as long), three LDS stages (two workgroups per CU; four stages, and one: 2 % behind).
-    // With K-major operands 38 problems on this side 0.70 to 0.99, 0.88 on average: 512 x 2736 x 8160 fp16 B 72.0 -> 50.5, int8 640 x 2480 x
-    // 2944 B 17.3 -> 13.1, bf16 960 x 1904 x 2640 both 24.8 -> 22.0.
+    // a second round. Random problems on this side: 9 GEMMs 0.80 to 0.97 of the time, 0.88 on average, 11 convolutions 0.83 to 0.93 (0.96 of it their
+    // branch-free range checks), 12 GEMMs with K-major operands 0.79 to 1.02, 0.90 on average; on the other side single tiles as before, and pairs
+    // 1.00 to 1.25 of their time. us: int8 67 x 10992 x 9024 36.4 -> 24.2, 128 x 4096 x 11008 20.9 -> 19.5, 32 x 14 x 14, C = K = 256 12.2 -> 11.0, fp16
+    // 83 x 9560 x 4928 30.1 -> 25.7, 512 x 2736 x 8160 with a K-major B 71.3 -> 49.7. Eight waves of 16 rows as in the 64 x 64 kernel (four of 32
+    // take 1.2 to 1.5 times as long), three LDS stages (two workgroups per CU; four stages, and one: 2 % behind).
     const long cus = num_cus(), cols = (N + 63) / 64 * runs, one = (M + 63) / 64 * cols, pair = (M + 127) / 128 * cols;
     return (pair + cus - 1) / cus * (128 + 64) < (one + cus - 1) / cus * (64 + 64);
 }
@@ -28,7 +27,7 @@ bool row_pairs_pay(long M, long N, long runs)
 bool column_pairs_pay(long M, long N, long ksplit, long batch)
 {
     // Where row pairs do not pay -- a single row tile, an odd number of them -- two column tiles share their rows of A in the same way. 23
-    // random GEMMs on this side 0.81 to 0.99 of the time, 0.89 on average: int8 277 x 6261 x 4928 24.5 -> 19.7 us, 146 x 10644 x 8384 35.8 -> 29.1, fp16
+    // random GEMMs on this side 0.81 to 0.99 of the time, 0.89 on average: int8 277 x 6261 x 4928 22.6 -> 18.1 us, 146 x 10644 x 8384 35.8 -> 29.1, fp16
     // 26 x 2321 x 8736 in K runs 21.3 -> 19.2. K runs of several row tiles are level, 0.96 to 1.02 (157 x 1521 x 5696 19.1 -> 19.5), and stay.
     if(ksplit > 1 && M > 64)
         return false;
