@@ -5,7 +5,7 @@
 Flags: -ffp-contract=off keeps the requant epilogue's fp32 multiplies unfused;
 packed fp32 VALU forms are disabled for the device pass.
 
-Three guards protect the kernels' hand-managed waits (the MFMA fragment reads of gemm_tile.hpp, conv_patch.hpp and
+Three guards protect the kernels' hand-managed waits (the MFMA fragment reads of gemm_tile.hpp, conv_patch.hpp, conv_window.hpp and
 conv_pointwise.hpp are inline-assembly LDS reads that the compiler does not count in lgkmcnt; the kernels wait for
 them themselves, so no compiler-made copy or spill of such a register may run before that wait):
   * every kernel's register report (-Rpass-analysis=kernel-resource-usage) is read, and the build FAILS if one of
@@ -60,7 +60,7 @@ def check_compiler():
 
 # kernels whose LDS fragment reads are inline assembly waited for by hand (mangled-name fragments)
 HAND_WAITED_KERNELS = ("gemm_tile_kernel", "gemm_w4_kernel", "gemm_astream_kernel", "conv_patch_kernel", "conv_patch_wide_kernel",
-                       "conv_pointwise_kernel")
+                       "conv_pointwise_kernel", "conv_window_kernel")
 
 
 def vgpr_spills(compiler_output):

@@ -20,6 +20,7 @@
 #include "conv_patch_wide.hpp"
 #include "conv_pointwise.hpp"
 #include "conv_stem.hpp"
+#include "conv_window.hpp"
 #include "gemm_skinny.hpp"
 #include "gemm_generic.hpp"
 #include "gemm_ragged.hpp"
@@ -889,6 +890,31 @@ int check_conv(int op, const ckx_conv2d_desc* d, int epi, int instance)
     return CKX_OK;
 }
 
+// us that the tile kernel takes for a conv whose filter has several taps, by its plan: the MFMA and latency terms of make_plan, and a
+// K tile's operands through a CU's load path at 75 bytes per ns (within 0.8 ... 1.25 of the time of 60 of 70 layers above 14 us; more than
+// 500 int8 channels take up to twice as long, when a pixel's line has left the L2 before the next tap asks for it)
+double conv_tile_us(const Plan& pl, long M, int N, int kbytes)
+{
+    const TileInstance& t = kTiles[pl.tile];
+    const long cus = num_cus(), units = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * pl.ksplit;
+    const int nst  = t.lds / ((t.bm + t.bn) * 128);
+    long per_cu    = 160 * 1024 / t.lds < 2048 / t.threads ? 160 * 1024 / t.lds : 2048 / t.threads;
+    per_cu         = per_cu > 4 ? 4 : per_cu;
+    per_cu         = per_cu * cus > units ? (units + cus - 1) / cus : per_cu;
+    const long rounds = (units + cus * per_cu - 1) / (cus * per_cu);
+    const double eff = t.bm == 256 && t.bn == 64 ? t.eff * 1.1 : t.eff, floor_us = nst > 2 ? 0.30 : 0.42;
+    const double mfma_us = per_cu * (t.bm * t.bn / 65536.0) / eff * 1.1, load_us = per_cu * (double)(t.bm + t.bn) * 128.0 / 75.0e3;
+    const double iter_us = mfma_us > load_us ? (mfma_us > floor_us ? mfma_us : floor_us) : (load_us > floor_us ? load_us : floor_us);
+    return rounds * (iter_us * pl.nk_per + 6.0 / per_cu + 2.0);
+}
+// the windowed kernel's shape for a conv with unit strides that the tile kernel would run by `pl`, and its box in `w`; -1: the tile kernel
+int conv_window_shape(int dt, ckx::ConvWindowArgs& w, const Plan& pl, long M)
+{
+    if(pl.ksplit != 1 || w.taps < 9)
+        return -1;
+    return ckx::choose_conv_window(dt, w, conv_tile_us(pl, M, w.K, w.taps * w.pix_bytes));
+}
+
 long conv_workspace_bytes(int op, const ckx_conv2d_desc* d, int instance)
 {
     const int es = op == CKX_OP_CONV2D_FWD_I8 ? 1 : 2;
@@ -1082,6 +1108,23 @@ int run_conv(int op, const void* in, const void* wei, void* out, const ckx_conv2
     g.ksplit = pl.ksplit;
     g.nk_per = pl.nk_per;
     g.ws     = ws;
+    if(instance == CKX_INSTANCE_AUTO && d->stride_h == 1 && d->stride_w == 1 && dops.ldd0 == 0)
+    {
+        ckx::ConvWindowArgs w;
+        std::memset(&w, 0, sizeof(w));
+        w.in = in, w.wei = wei, w.out = out, w.d0 = g.d0, w.d1 = g.d1, w.ldd1 = g.ldd1;
+        w.in_bytes = g.a_bytes, w.wei_bytes = g.b_bytes;
+        w.N = d->N, w.Di = 1, w.Hi = d->Hi, w.Wi = d->Wi, w.Do = 1, w.Ho = d->Ho, w.Wo = d->Wo, w.K = N;
+        w.pix_bytes = d->C * es, w.units = w.pix_bytes / 16, w.Y = d->Y, w.X = d->X, w.taps = d->Y * d->X;
+        w.dD = 1, w.dH = d->dilation_h, w.dW = d->dilation_w, w.pT = d->pad_top, w.pL = d->pad_left;
+        w.epi = epi, w.scale_gemm = sg, w.scale_relu = sr, w.nt_store = g.nt_store;
+        const int dt = es == 1 ? ckx::DT_I8 : ckx::DT_F16, shape = conv_window_shape(dt, w, pl, M);
+        if(shape >= 0)
+        {
+            hipError_t e = ckx::launch_conv_window(dt, shape, w, (hipStream_t)stream);
+            return e == hipSuccess ? CKX_OK : hip_fail(e, t.name);
+        }
+    }
     const bool fused = f16_fused(epi) && g.ksplit == 1;
     // A a K tile further ahead (AHEAD in gemm_tile.hpp): strides that leave a pixel to less than about three of the filter's taps, so that
     // 3/10 and more of every K tile's A are new to the L2, which the column tiles of a row of tiles share. us, tenths: 3 x 3 stride 2, K
@@ -1265,6 +1308,23 @@ int run_convnd(int op, const void* in, const void* wei, void* out, const ckx_con
         lay.X = d->filter[2], lay.Y = d->filter[1];
         hipError_t e = ckx::launch_generic(es == 1 ? ckx::DT_I8 : ckx::DT_F16, 2, g, lay, (hipStream_t)stream);
         return e == hipSuccess ? CKX_OK : hip_fail(e, kGenericName);
+    }
+    if(instance == CKX_INSTANCE_AUTO && d->stride[0] == 1 && d->stride[1] == 1 && d->stride[2] == 1)
+    {
+        ckx::ConvWindowArgs w;
+        std::memset(&w, 0, sizeof(w));
+        w.in = in, w.wei = wei, w.out = out, w.in_bytes = g.a_bytes, w.wei_bytes = g.b_bytes;
+        w.three_d = 1, w.N = d->N, w.Di = d->in[0], w.Hi = d->in[1], w.Wi = d->in[2], w.Do = d->out[0], w.Ho = d->out[1], w.Wo = d->out[2], w.K = N;
+        w.pix_bytes = d->C * es, w.units = w.pix_bytes / 16, w.Y = d->filter[1], w.X = d->filter[2];
+        w.taps = d->filter[0] * d->filter[1] * d->filter[2], w.dD = d->dilation[0], w.dH = d->dilation[1], w.dW = d->dilation[2];
+        w.pF = d->pad_left[0], w.pT = d->pad_left[1], w.pL = d->pad_left[2];
+        w.epi = epi, w.scale_gemm = sg, w.scale_relu = sr, w.nt_store = g.nt_store;
+        const int dt = es == 1 ? ckx::DT_I8 : ckx::DT_F16, shape = conv_window_shape(dt, w, pl, M);
+        if(shape >= 0)
+        {
+            hipError_t e = ckx::launch_conv_window(dt, shape, w, (hipStream_t)stream);
+            return e == hipSuccess ? CKX_OK : hip_fail(e, t.name);
+        }
     }
     const bool pairs = pl.tile == ckx::kFourStageTile && ckx::row_pairs_pay(M, N, g.ksplit);
     if(pairs)
