@@ -92,14 +92,6 @@ using ckx::make_magic;
 using ckx::num_cus;
 using ckx::tile_launch_fn;
 
-template <int DT>
-hipError_t launch_reduce(const ckx::GemmArgs& a, hipStream_t s)
-{
-    const long groups = (long)a.M * ((a.N + 15) / 16);
-    hipLaunchKernelGGL((ckx::splitk_reduce_kernel<DT>), dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, s, a);
-    return hipGetLastError();
-}
-
 struct TileInstance
 {
     const char* name;
@@ -694,9 +686,7 @@ int run_gemm(int dt, const void* a, const void* b, void* c, int M, int N, int K,
         return fail(CKX_UNSUPPORTED, "no kernel variant for this layout");
     hipError_t e = launch(g, g.tiles_m * g.tiles_n * g.ksplit * batch, (hipStream_t)stream);
     if(e == hipSuccess && g.ksplit > 1)
-        e = dt == ckx::DT_I8     ? launch_reduce<ckx::DT_I8>(g, (hipStream_t)stream)
-            : dt == ckx::DT_BF16 ? launch_reduce<ckx::DT_BF16>(g, (hipStream_t)stream)
-                                 : launch_reduce<ckx::DT_F16>(g, (hipStream_t)stream);
+        e = ckx::launch_splitk_reduce(dt, g, (hipStream_t)stream);
     if(e != hipSuccess)
         return hip_fail(e, t.name);
     return CKX_OK;
@@ -1144,8 +1134,7 @@ int run_conv(int op, const void* in, const void* wei, void* out, const ckx_conv2
                                 : t.conv_f16)(g, g.tiles_m * g.tiles_n * g.ksplit,
                                                                                  (hipStream_t)stream);
     if(e == hipSuccess && g.ksplit > 1)
-        e = es == 1 ? launch_reduce<ckx::DT_I8>(g, (hipStream_t)stream)
-                    : launch_reduce<ckx::DT_F16>(g, (hipStream_t)stream);
+        e = ckx::launch_splitk_reduce(es == 1 ? ckx::DT_I8 : ckx::DT_F16, g, (hipStream_t)stream);
     if(e != hipSuccess)
         return hip_fail(e, t.name);
     return CKX_OK;
@@ -1335,7 +1324,7 @@ int run_convnd(int op, const void* in, const void* wei, void* out, const ckx_con
         return fail(CKX_UNSUPPORTED, "no kernel variant for this instance");
     hipError_t e = launch(g, g.tiles_m * g.tiles_n * g.ksplit, (hipStream_t)stream);
     if(e == hipSuccess && g.ksplit > 1)
-        e = es == 1 ? launch_reduce<ckx::DT_I8>(g, (hipStream_t)stream) : launch_reduce<ckx::DT_F16>(g, (hipStream_t)stream);
+        e = ckx::launch_splitk_reduce(es == 1 ? ckx::DT_I8 : ckx::DT_F16, g, (hipStream_t)stream);
     if(e != hipSuccess)
         return hip_fail(e, t.name);
     return CKX_OK;

@@ -1548,77 +1548,6 @@ struct GemmTile
     }
 };
 
-// Second pass of a split-K launch: C = epilogue(sum over the K runs of the workspace slices).
-// One thread per 16 consecutive columns of a row, slices added in run order (deterministic).
-template <int DT>
-__global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs p)
-{
-    using acc_t   = typename std::conditional<DT == DT_I8, i32x4, f32x4>::type;
-    constexpr int ES = DT == DT_I8 ? 1 : 2;
-    const int groups_per_row = (p.N + 15) / 16;
-    const long gid = (long)blockIdx.x * 256 + threadIdx.x;
-    if(gid >= (long)p.M * groups_per_row)
-        return;
-    const int m  = (int)(gid / groups_per_row);
-    const int n0 = (int)(gid - (long)m * groups_per_row) * 16;
-    acc_t v[4];
-#pragma unroll
-    for(int t = 0; t < 4; ++t)
-        v[t] = acc_t{0, 0, 0, 0};
-    const bool full = n0 + 16 <= p.N;
-    for(int sp = 0; sp < p.ksplit; ++sp)
-    {
-        const uint8_t* wrow = reinterpret_cast<const uint8_t*>(p.ws) + (((size_t)sp * p.M + m) * p.N + n0) * 4;
-        if(full)
-        {
-#pragma unroll
-            for(int t = 0; t < 4; ++t)
-            {
-                const acc_t w = load_vec<acc_t>(wrow + 16 * t);
-                v[t][0] += w[0], v[t][1] += w[1], v[t][2] += w[2], v[t][3] += w[3];
-            }
-        }
-        else
-        {
-#pragma unroll
-            for(int e = 0; e < 16; ++e)
-                if(n0 + e < p.N)
-                    v[e / 4][e % 4] += reinterpret_cast<const decltype(v[0][0] + 0)*>(wrow)[e];
-        }
-    }
-    if constexpr(DT == DT_I8)
-    {
-        int8_t* crow = reinterpret_cast<int8_t*>(p.c) + (size_t)m * p.ldc;
-        if(epi_per_column_scale(p.epi))
-        {
-            float sc[16];
-            load_col_scales(make_rsrc(p.d0, (uint32_t)p.N * 4u), n0, sc);
-            store_row16_i8_cols(crow, n0, p.N, v, sc, p.epi == EPI_RELU_MUL2_CLAMP);
-        }
-        else if(p.epi == EPI_REQUANT_RND)
-            store_row16_i8<EPI_REQUANT_RND>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu);
-        else if(p.epi == EPI_REQUANT_CK)
-            store_row16_i8<EPI_REQUANT_CK>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu);
-        else
-            store_row16_i8<EPI_PASSTHROUGH>(crow, n0, p.N, v, p.scale_gemm, p.scale_relu);
-    }
-    else if constexpr(DT == DT_BF16)
-        store_row16_f16(reinterpret_cast<__bf16*>(p.c) + (size_t)m * p.ldc, n0, p.N, v);
-    else
-    {
-        _Float16* crow = reinterpret_cast<_Float16*>(p.c) + (size_t)m * p.ldc;
-        if(p.epi == EPI_PASSTHROUGH)
-            store_row16_f16(crow, n0, p.N, v);
-        else
-        {
-            store_row16_f16_fused(crow, n0, p.N, v, p.epi,
-                                  reinterpret_cast<const _Float16*>(p.d0) + (size_t)m * p.ldd0,
-                                  p.d1 ? reinterpret_cast<const _Float16*>(p.d1) + (size_t)m * p.ldd1 : nullptr,
-                                  false, p.scale_gemm, p.scale_relu);
-        }
-    }
-}
-
 template <int DT, int BM, int BN, int WM, int WN, int BKB, int NST, int IM2COL, bool TA = false, bool TB = false,
           bool FUSED = false, bool AHEAD = false>
 __global__ __launch_bounds__((WM * WN * 64), (GemmTile<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED, AHEAD>::WAVES_EU))

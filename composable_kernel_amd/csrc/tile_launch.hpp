@@ -82,6 +82,9 @@ tile_launch_fn row_pairs_layout_tile(int dt, bool a_kmajor, bool b_kmajor); // (
 bool column_pairs_pay(long M, long N, long ksplit, long batch);
 tile_launch_fn column_pairs_tile(int dt);
 
+// second pass of a split-K launch (splitk_reduce.hip)
+hipError_t launch_splitk_reduce(int dt, const GemmArgs& a, hipStream_t s);
+
 // weight-streaming GEMM for up to 128 rows (gemm_astream.hip): launcher for element type dt (DT_*) with 16 * nt output
 // columns per workgroup (nt = 3), grid = number of such column blocks
 tile_launch_fn astream_launcher(int dt, int nt);

@@ -243,3 +243,46 @@ def test_device_gemm_splitk_rejects_missing_workspace_and_bad_kbatch():
     out, _ = _run_splitk(ck.DeviceGemmSplitKInt8(capi.lib().ckx_num_instances(capi.OP_GEMM_SPLITK)), a, b_nk,
                          torch.int8, 2, ck.PassThrough())
     assert out is None      # a skinny instance
+
+
+@pytest.mark.parametrize("split", [2, 4, 8])
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 66, 131])
+def test_second_pass_at_the_ends_of_rows(force_split, split, N):
+    """Rows that end inside the four columns of a thread of the second pass: integers, so every data type is exact."""
+    import torch
+    rng = np.random.default_rng(N)
+    a, b_nk = rng.integers(-4, 5, (37, 1024)).astype(np.int8), rng.integers(-4, 5, (N, 1024)).astype(np.int8)
+    force_split(split)
+    out, need = _run_gemm(ck.DeviceGemmInt8(4), a, b_nk, torch.int8, ck.RequantReluRequant(0.02, 0.4, rounded=True))
+    assert need > 0
+    np.testing.assert_array_equal(out, fast.gemm_i8(a, b_nk.T, lit.EPI_REQUANT_RND, 0.02, 0.4))
+    want = a.astype(np.float64) @ b_nk.T.astype(np.float64)
+    out, need = _run_gemm(ck.DeviceGemmF16(4), a.astype(np.float16), b_nk.astype(np.float16), torch.float16)
+    assert need > 0
+    np.testing.assert_array_equal(out, want.astype(np.float16))
+
+
+@pytest.mark.parametrize("K", [3, 40, 66])
+@pytest.mark.parametrize("residual", [False, True])
+def test_second_pass_with_d_operands(force_split, K, residual):
+    import torch
+    import gpu_util
+    rng = np.random.default_rng(K)
+    inp, wei, bias, resi = (rng.integers(-2, 3, s).astype(np.float16) for s in ((2, 9, 11, 64), (K, 3, 3, 64), (K,), (2, 9, 11, K)))
+    di, dw, db, dr = (gpu_util.dev(x) for x in (inp, wei, bias, resi))
+    do = torch.full((2, 9, 11, K), float("nan"), dtype=torch.float16, device="cuda")
+    force_split(3)
+    op = ck.DeviceConv2dFwdBiasActivationF16(4)
+    geom = (2, K, 64, [9, 11], [3, 3], [9, 11], [1, 1], [1, 1], [1, 1], [1, 1], None, None)
+    arg = op.MakeArgumentPointer(di, dw, do, db, dr, *geom, ck.AddReluAdd()) if residual else \
+        op.MakeArgumentPointer(di, dw, do, db, *geom, ck.AddRelu())
+    assert op.IsSupportedArgument(arg)
+    need = op.GetWorkSpaceSize(arg)
+    assert need > 0
+    ws = torch.full((need,), 0x7F, dtype=torch.uint8, device="cuda")
+    op.SetWorkSpacePointer(arg, ws)
+    op.MakeInvokerPointer().Run(arg, ck.StreamConfig(gpu_util.stream()))
+    torch.cuda.synchronize()
+    acc  = fast.conv2d_fwd_f16(inp, wei, (1, 1), (1, 1), (1, 1)).astype(np.float32)  # (integers below 2048: exact)
+    want = np.maximum(acc + bias.astype(np.float32), 0) + (resi.astype(np.float32) if residual else 0)
+    np.testing.assert_array_equal(do.cpu().numpy(), want.astype(np.float16))
