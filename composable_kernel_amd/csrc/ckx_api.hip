@@ -684,7 +684,9 @@ int run_gemm(int dt, const void* a, const void* b, void* c, int M, int N, int K,
                                                        : t.dense_f16;
     if(!launch)
         return fail(CKX_UNSUPPORTED, "no kernel variant for this layout");
-    hipError_t e = launch(g, g.tiles_m * g.tiles_n * g.ksplit * batch, (hipStream_t)stream);
+    const bool tail  = ti == 0 && !w4 && !kmajor && dt == ckx::DT_I8 && !per_column_scale(epi) && ckx::short_tail(g);
+    const int tiles  = g.tiles_m * g.tiles_n + g.tail_m * g.tail_n;
+    hipError_t e     = (tail ? ckx::short_tail_tile() : launch)(g, tiles * g.ksplit * batch, (hipStream_t)stream);
     if(e == hipSuccess && g.ksplit > 1)
         e = ckx::launch_splitk_reduce(dt, g, (hipStream_t)stream);
     if(e != hipSuccess)

@@ -237,6 +237,10 @@ struct GemmArgs
     uint32_t a_bytes;       // extent of the A / B allocations seen by the buffer resource
     uint32_t b_bytes;
     int tiles_m, tiles_n;
+    // SHORT kernels (one K run, no batch): the tiles of the last round, of fewer rows so that they occupy every CU (short_tail in
+    // tile_launch.hpp): tail_m x tail_n tiles of 2 * tail_h rows from row tail_row0 and column tile tail_col0 on, after
+    // the tiles_m x tiles_n whole ones. tail_m == 0: none.
+    int tail_m, tail_n, tail_row0, tail_col0, tail_h;
     int epi;
     float scale_gemm, scale_relu;
     int nt_store; // stream the C tile past L2 (large outputs)
@@ -664,7 +668,7 @@ __device__ __forceinline__ void store_row16_f16_fused(_Float16* crow, int n0, in
 // launches which never run it need not pay for. Its K loop is the plain one as long as the epilogue awaits
 // its D loads explicitly (see d_values_landed there).
 template <int DT, int BM, int BN, int WM, int WN, int BKB, int NST, int IM2COL, bool TA = false, bool TB = false,
-          bool FUSED = false, bool AHEAD = false>
+          bool FUSED = false, bool AHEAD = false, bool SHORT = false>
 struct GemmTile
 {
     static constexpr int NW      = WM * WN;
@@ -714,6 +718,10 @@ struct GemmTile
     static constexpr int NLA     = BM * CPR / NT; // 16-byte loads per thread and K tile, A
     static constexpr int NLB     = BN * CPR / NT;
     static constexpr int LPT     = NLA + NLB;
+    // Short tiles in the last round (GemmArgs::tail_m): their fragment rows past `rows` are neither multiplied nor stored. A kernel of its own,
+    // because the branches around each fragment row's MFMAs cost the launches that need none 2 to 7 %; one reason why K-major operands have
+    // none: their fragments are put together from two reads each, and a copy on the way, before the data is there, went by unseen.
+    static_assert(!SHORT || (!TA && !TB && IM2COL == 0 && !FUSED && !AHEAD), "dense GEMMs with K-contiguous operands and a plain epilogue");
     static_assert(BKB == 128 && KSTEPS == 2, "pipeline written for 128-byte K tiles");
     static_assert(NST >= 2 && (NST - 2) * LPT < 64, "vmcnt is a 6-bit counter");
     static_assert(WTM % 16 == 0 && WTN % 64 == 0, "wave tile must be 16k x 64k");
@@ -764,7 +772,8 @@ struct GemmTile
 
         const int ntiles      = p.tiles_m * p.tiles_n;
         const int nbatch      = p.batch > 0 ? p.batch : 1;
-        const int ntiles_all  = ntiles * nbatch; // C tiles of all batches: id = batch * ntiles + tile
+        const int nwhole      = ntiles * nbatch;
+        const int ntiles_all  = nwhole + (SHORT ? p.tail_m * p.tail_n : 0); // C tiles of all batches: id = batch * ntiles + tile
         const int gstride     = (int)gridDim.x;
         const uint32_t kbytes = (uint32_t)p.K * ES;
         const int nk_real     = (int)((kbytes + BKB - 1) / BKB);
@@ -793,13 +802,30 @@ struct GemmTile
         const uint32_t trow_a = TA ? (uint32_t)(wave * (1024 / (BM * ES)) + lane / (BM * ES / 16)) : 0u;
         const uint32_t trow_b = TB ? (uint32_t)(wave * (1024 / (BN * ES)) + lane / (BN * ES / 16)) : 0u;
 
+        // batch, first row and column tile of a C tile, and the rows that each row of waves has of it
+        auto tile_at = [&](int tile_id, int& g, int& row0, int& tn, int& h) {
+            int tm;
+            if(SHORT && tile_id >= nwhole)
+            {
+                tile_of_block(tile_id - nwhole, p.tail_m, p.tail_n, 1, g, tm, tn);
+                h    = p.tail_h;
+                row0 = p.tail_row0 + tm * (WM * h);
+                tn += p.tail_col0;
+            }
+            else
+            {
+                tile_of_block(tile_id, p.tiles_m, p.tiles_n, nbatch, g, tm, tn);
+                h    = WTM;
+                row0 = tm * BM;
+            }
+        };
         // row / column offsets of the tile the LOAD cursor is on (tile >= ntiles: nothing valid)
         auto setup_tile = [&](int tile_id, auto with_a, auto with_b) {
-            int tm = 0, tn = 0;
+            int row0 = 0, tn = 0, h = WTM;
             const bool live = tile_id < ntiles_all;
             int g           = 0;
             if(live)
-                tile_of_block(tile_id, p.tiles_m, p.tiles_n, nbatch, g, tm, tn);
+                tile_at(tile_id, g, row0, tn, h);
             const uint32_t a_batch = (uint32_t)((long)g * p.bsa * ES), b_batch = (uint32_t)((long)g * p.bsb * ES);
 #pragma unroll
             for(int j = 0; j < (decltype(with_a)::value ? NLA : 0); ++j)
@@ -808,14 +834,15 @@ struct GemmTile
                 {
                     uint32_t r, x;
                     tslot<BM>(j, wave, lane, r, x);
-                    const uint32_t gx = (uint32_t)tm * BM + x;
+                    const uint32_t gx = (uint32_t)row0 + x;
                     a_off[j] = (live && gx < (uint32_t)p.M) ? a_batch + (r * (uint32_t)p.lda + gx) * ES : kOutOfRange;
                     a_hw0[j] = 0;
                     continue;
                 }
                 const uint32_t r  = (uint32_t)((j * NW + wave) * RPI + lane / CPR);
-                const uint32_t gm = (uint32_t)tm * BM + r;
-                const bool ok     = live && gm < (uint32_t)p.M;
+                // (tile row of a staged row: a short tile's rows are the first h of every row of waves)
+                const uint32_t gm = (uint32_t)row0 + (SHORT ? r / WTM * (uint32_t)h + r % WTM : r);
+                const bool ok     = live && gm < (uint32_t)p.M && (!SHORT || r % WTM < (uint32_t)h);
                 if constexpr(IM2COL == 0)
                 {
                     a_off[j] = ok ? a_batch + gm * (uint32_t)p.lda * ES + kb : kOutOfRange;
@@ -1127,7 +1154,8 @@ struct GemmTile
         // k-step]. The loads must not be issued back to back: a burst of eight 1 KB loads per wave
         // fills the texture-address FIFOs (SQ_VMEM_TA_ADDR/CMD_FIFO_FULL), the in-order wave blocks
         // on VMEM issue, and its MFMAs wait behind it.
-        auto half_step = [&](auto with_loads, const LoadCtx& lc, const i32x4(&caf)[MT], const i32x4(&cbf)[NG * 4],
+        // rows: fragment rows of the tile that exist
+        auto half_step = [&](auto with_loads, int rows, const LoadCtx& lc, const i32x4(&caf)[MT], const i32x4(&cbf)[NG * 4],
                              uint32_t nstage_lds, uint32_t nstage_lds_b, auto nks, i32x4(&naf)[MT], i32x4(&nbf)[NG * 4]) {
             // The reads are over two groups before the end of the half; the first half of an iteration
             // starts its reads one group late.
@@ -1144,9 +1172,12 @@ struct GemmTile
                 static_for<r1 - r0>([&](auto r_c) {
                     read_one(nstage_lds, nstage_lds_b, nks, std::integral_constant<int, r0 + decltype(r_c)::value>{}, naf, nbf);
                 });
+                if(!SHORT || g * NM / NGRP / (NG * 4) < rows)
+                {
 #pragma unroll
-                for(int m = g * NM / NGRP; m < (g + 1) * NM / NGRP; ++m)
-                    mfma_one(m, caf, cbf);
+                    for(int m = g * NM / NGRP; m < (g + 1) * NM / NGRP; ++m)
+                        mfma_one(m, caf, cbf);
+                }
                 __builtin_amdgcn_sched_barrier(0);
             });
         };
@@ -1154,8 +1185,8 @@ struct GemmTile
         // ---- epilogue: registers -> global, 16 consecutive columns per lane -------------
         const bool nt     = p.nt_store != 0;
         auto epilogue = [&](int unit) {
-            int tm, tn, bi;
-            tile_of_block(unit % ntiles_all, p.tiles_m, p.tiles_n, nbatch, bi, tm, tn);
+            int row0, tn, bi, h;
+            tile_at(unit % ntiles_all, bi, row0, tn, h);
             // (a K split is never combined with a batch: the slices are [run][M][N])
             acc_t* slice = reinterpret_cast<acc_t*>(reinterpret_cast<uint8_t*>(p.ws) +
                                                     (size_t)(unit / ntiles_all) * p.M * p.N * 4);
@@ -1187,7 +1218,7 @@ struct GemmTile
 #pragma unroll
                         for(int i = 0; i < MT; ++i)
                         {
-                            const int m = tm * BM + wm * WTM + 16 * i + (lane & 15);
+                            const int m = row0 + wm * WTM + 16 * i + (lane & 15);
                             if(m < p.M && n0 < p.N)
                             {
                                 const i32x4 v[4] = {acc[i][g * 4], acc[i][g * 4 + 1], acc[i][g * 4 + 2], acc[i][g * 4 + 3]};
@@ -1205,12 +1236,12 @@ struct GemmTile
 #pragma unroll
             for(int i = 0; i < MT; ++i)
             {
-                const int m = tm * BM + wm * WTM + 16 * i + (lane & 15);
+                const int m = row0 + wm * (SHORT ? h : WTM) + 16 * i + (lane & 15);
 #pragma unroll
                 for(int g = 0; g < NG; ++g)
                 {
                     const int n0 = tn * BN + wn * WTN + 64 * g + 16 * (lane >> 4);
-                    if(m < p.M && n0 < p.N)
+                    if(m < p.M && n0 < p.N && (!SHORT || 16 * i < h))
                     {
                         if(p.ksplit > 1)
                         {
@@ -1444,11 +1475,12 @@ struct GemmTile
         unit_k_range((int)blockIdx.x, kt, kt_end);
         for(int unit = (int)blockIdx.x; unit < nunits;)
         {
+            const int rows     = SHORT && unit >= nwhole * p.ksplit ? p.tail_h / 16 : MT;
             const int st_next  = st_cur + 1 == NSTA ? 0 : st_cur + 1;
             const int sb_next  = !AHEAD ? st_next : sb_cur + 1 == NST ? 0 : sb_cur + 1;
             // first fragments of this K tile (read in the previous half-iteration / the prologue)
             wait_frags();
-            half_step(std::false_type{}, LoadCtx{}, af0, bf0, smem_lds + (uint32_t)a_stage(st_cur), smem_lds + (uint32_t)b_stage(sb_cur),
+            half_step(std::false_type{}, rows, LoadCtx{}, af0, bf0, smem_lds + (uint32_t)a_stage(st_cur), smem_lds + (uint32_t)b_stage(sb_cur),
                       std::integral_constant<int, 1>{}, af1, bf1);
 
             // The direct loads of a wave retire in order: once at most NST-2 K tiles' worth are in
@@ -1464,7 +1496,7 @@ struct GemmTile
             barrier();
 
             const LoadCtx lc = load_ctx(ld.kt, st_cur, ld_b.kt, sb_cur);
-            half_step(std::true_type{}, lc, af1, bf1, smem_lds + (uint32_t)a_stage(st_next), smem_lds + (uint32_t)b_stage(sb_next),
+            half_step(std::true_type{}, rows, lc, af1, bf1, smem_lds + (uint32_t)a_stage(st_next), smem_lds + (uint32_t)b_stage(sb_next),
                       std::integral_constant<int, 0>{}, af0, bf0);
             advance_load_cursor();
 
@@ -1549,12 +1581,12 @@ struct GemmTile
 };
 
 template <int DT, int BM, int BN, int WM, int WN, int BKB, int NST, int IM2COL, bool TA = false, bool TB = false,
-          bool FUSED = false, bool AHEAD = false>
-__global__ __launch_bounds__((WM * WN * 64), (GemmTile<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED, AHEAD>::WAVES_EU))
+          bool FUSED = false, bool AHEAD = false, bool SHORT = false>
+__global__ __launch_bounds__((WM * WN * 64), (GemmTile<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED, AHEAD, SHORT>::WAVES_EU))
 void gemm_tile_kernel(const GemmArgs p)
 {
     extern __shared__ __attribute__((aligned(1024))) uint8_t ckx_smem[];
-    GemmTile<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED, AHEAD>::run(p, ckx_smem);
+    GemmTile<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED, AHEAD, SHORT>::run(p, ckx_smem);
 }
 
 } // namespace ckx

@@ -41,11 +41,11 @@ inline int num_cus()
 // Persistent launch: at most (workgroups that fit a CU) x (CUs) workgroups, a multiple of 8 so
 // that workgroup b always lands on XCD b % 8 together with the tiles b, b + grid, ...
 template <int DT, int BM, int BN, int WM, int WN, int BKB, int NST, int IM2COL, bool TA = false, bool TB = false,
-          bool FUSED = false, bool AHEAD = false>
+          bool FUSED = false, bool AHEAD = false, bool SHORT = false>
 hipError_t launch_tile(const GemmArgs& a, int tiles, hipStream_t s)
 {
-    using T              = GemmTile<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED, AHEAD>;
-    auto* kern           = &gemm_tile_kernel<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED, AHEAD>;
+    using T              = GemmTile<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED, AHEAD, SHORT>;
+    auto* kern           = &gemm_tile_kernel<DT, BM, BN, WM, WN, BKB, NST, IM2COL, TA, TB, FUSED, AHEAD, SHORT>;
     static std::once_flag once;
     static hipError_t attr_err = hipSuccess;
     std::call_once(once, [&] {
@@ -60,6 +60,10 @@ hipError_t launch_tile(const GemmArgs& a, int tiles, hipStream_t s)
     hipLaunchKernelGGL(kern, dim3(grid), dim3(T::NT), T::LDS, s, a);
     return hipGetLastError();
 }
+
+// Short tiles in the last round of an int8 launch of 256 x 256 tiles (tile_pairs.hip): true, and `g`'s tiles set, where they pay
+bool short_tail(GemmArgs& g);
+tile_launch_fn short_tail_tile();
 
 // K-major operand layouts (gemm_layouts.hip): launcher of tile instance `tile` for element type dt
 // (DT_*), A K-major (a_kmajor: column-major "km") and / or B K-major (b_kmajor: row-major "kn");

@@ -10,6 +10,41 @@ constexpr tile_launch_fn pairs = &launch_tile<DT, 128, 64, 8, 1, 128, 3, IM2COL,
 
 } // namespace
 
+bool short_tail(GemmArgs& g)
+{
+    // Where the tiles are no whole number of rounds of the CUs, as many of them as the whole rounds hold keep 256 rows, and the columns (or
+    // rows) behind them are cut into tiles of the fewest rows, 128 to 224 by 32, that still fit one round: 4096 x 11008, 688 tiles in three
+    // rounds, as 512 tiles of 256 rows and 242 of 192. Any saving pays: 13 random problems 1.02 to 1.17 of the speed, 1.09 on average. us: int8
+    // 4096 x 11008 x 4096 152.6 -> 147.7, 2687 x 3214 x 2384 35.5 -> 30.3, 4910 x 1681 x 3072 34.7 -> 30.0, 3447 x 10022 x 3600 147 -> 135. fp16
+    // and bf16 stay on the four-wave body, which is ahead by more than that (28 problems: 0.82 to 1.10, 0.95 on average), and strided fp16
+    // convolutions on whole tiles: what a short tile saves them is products, and they wait for loads (648 tiles, 2.5 rounds: 153.8 and 153.1).
+    const long grid = num_cus() - num_cus() % 8, tm = g.tiles_m, tn = g.tiles_n, rounds = tm * tn / grid;
+    if(tm * tn == rounds * grid || g.ksplit != 1 || g.batch > 1)
+        return false;
+    const long columns = rounds * grid / tm, rows = rounds * grid / tn; // column tiles and row tiles that the whole rounds hold
+    for(int h = 64; h < 128; h += 16)
+    {
+        const long in_columns = (g.M + 2 * h - 1) / (2 * h), in_rows = (g.M - rows * 256 + 2 * h - 1) / (2 * h);
+        if(rows * tn + in_rows * tn <= (rounds + 1) * grid)
+        {
+            g.tail_m = (int)in_rows, g.tail_n = (int)tn, g.tail_row0 = (int)rows * 256;
+            g.tiles_m = (int)rows;
+        }
+        else if(columns * tm + in_columns * (tn - columns) <= (rounds + 1) * grid)
+        {
+            g.tail_m = (int)in_columns, g.tail_n = (int)(tn - columns), g.tail_col0 = (int)columns;
+            g.tiles_n = (int)columns;
+        }
+        else
+            continue;
+        g.tail_h = h;
+        return true;
+    }
+    return false;
+}
+
+tile_launch_fn short_tail_tile() { return &launch_tile<DT_I8, 256, 256, 2, 4, 128, 2, 0, false, false, false, false, true>; }
+
 bool row_pairs_pay(long M, long N, long runs)
 {
     // What bounds two co-resident 64 x 64 workgroups is the operand bytes that their CU loads (65 to 82 bytes per ns), and both load the same
