@@ -552,7 +552,7 @@ inline hipError_t gemm_gemm_launch_mt(const GemmGemmArgs& g, hipStream_t s)
     return og == 1 ? gemm_gemm_launch_t<4, 1, MT, NW, SOFTMAX>(g, s) : gemm_gemm_launch_t<4, 2, MT, NW, SOFTMAX>(g, s);
 }
 
-hipError_t gemm_softmax_gemm_launch(const GemmGemmArgs& a, hipStream_t s); // gemm_softmax_gemm.hip
+hipError_t gemm_softmax_gemm_launch(const GemmGemmArgs& a, int parts, hipStream_t s); // gemm_softmax_gemm.hip; parts: shares of the columns, 1, 2 or 4
 
 // Attention on waves of 16 rows (instance 2) instead of 32 (instance 0). Up to 256 slabs of 128 rows there is one workgroup to a CU: one
 // wave of 32 rows per SIMD, or two of 16, and the launch lasts as long as one wave's chain of steps. The shorter chain wins then, up to an
@@ -578,6 +578,33 @@ inline bool rows_in_16s(int M, int N, int K, int O, int batch, bool mask_upper)
     return slabs <= 256 && (head > 64 ? false : head > 32 ? N <= (slabs <= 128 ? 1024 : 960) : N < 448);
 }
 
+// Attention, the shares of the columns that a workgroup's groups of waves take side by side: 1, 2 (128 rows) or 4 (64 rows), see
+// gemm_softmax_gemm.hpp. With one workgroup or fewer to a CU the launch lasts as long as a wave's chain of units, which the shares shorten;
+// with more the CUs are busy anyway, and what the shares cost shows: the merge, and with 64 rows every column read twice as often. A launch
+// under the triangular mask may have more of them once its chain is long: they start longest first, and the short ones fit in behind. Below
+// the lines in the chain's length the first loads and the merge cost more than the shares give; heads of 65 to 96 in quarters pad to 128. Up
+// to 64 rows of heads of 33 to 64 the choice between 16 and 32 rows stands up to 1025 columns, bit for bit.
+// 1 part (the better of 16 and 32 rows as chosen below) / 2 / 4, us, full: batch x M x N 3 x 3034 x 3034 of heads 32 28.5 / 24.0 / 15.5, 6 x
+// 3760 x 1709 / 64 23.7 / 20.7 / 16.5, 14 x 802 x 802 / 64 14.7 / 13.4 / 12.7, 12 x 1275 x 1275 / 80 23.0 / 21.2 / 21.7, 8 x 1676 x 1676 / 128
+// 39.8 / 32.5 / 27.2, 4 x 991 x 3837 / 128 81.2 / 62.1 / 45.6, but 6 x 2806 x 2806 / 64 (264 slabs of 64) 35.4 / 29.4 / 43.1, 8 x 1918 x 490 / 64 9.7 /
+// 10.2 / 9.6, 125 x 70 x 931 / 128 25.2 / 21.2 / 25.7 (two slabs of 64 for one of 128). Causal: 6 x 3772 / 64 44.9 / 37.0 / 28.3 (354 slabs of
+// 64), 25 x 936 / 64 16.3 / 15.0 / 19.7 (375), 15 x 591 / 64 11.0 / 11.4 / 11.8, 6 x 3707 / 128 78.7 / 60.8 / 47.9, 18 x 573 / 128 16.5 / 16.3 / 16.7.
+// Over 340 random problems none of the routes below is slower than one part beyond the noise; 2 parts gave up to 1.34, 4 up to 1.84 times.
+inline int column_parts(int M, int N, int K, int O, int batch, bool mask_upper)
+{
+    const int head     = K > O ? K : O;
+    const bool tri     = mask_upper && M <= N;
+    const int chain    = mask_upper && M < N ? M : N;
+    const long by64    = (long)batch * ((M + 63) / 64) * 256 / num_cus(), by128 = (long)batch * ((M + 127) / 128) * 256 / num_cus();
+    const long most    = tri && chain >= 1792 ? 384 : tri && chain >= 1024 ? 320 : 256;
+    const int line64   = M <= 64 ? 1026 : 640;
+    const int from4    = head <= 32 ? 576 : head <= 64 ? line64 : head <= 96 ? 1536 : 640;
+    const int from2    = head <= 32 ? 576 : head <= 64 ? (mask_upper && line64 < 768 ? 768 : line64) : head <= 96 ? 768 : 576;
+    if(chain >= from4 && by64 <= (M > 64 && M <= 128 ? 192 : most))
+        return 4;
+    return chain >= from2 && by128 <= (chain < 1024 ? 224 : most) ? 2 : 1;
+}
+
 // softmax: the attention variant with scores scale * (A * B0) and the optional upper-triangle mask
 inline hipError_t gemm_gemm_launch(const void* a, const void* b0, const void* b1, void* c, int M, int N, int K,
                                    int O, int batch, int sa, int sb0, int sb1, int sc, int64_t bsa,
@@ -594,8 +621,13 @@ inline hipError_t gemm_gemm_launch(const void* a, const void* b0, const void* b1
     if(softmax)
     {
         if(instance < 0)
+        {
+            const int parts = column_parts(M, N, K, O, batch, mask_upper);
+            if(parts > 1)
+                return gemm_softmax_gemm_launch(g, parts, s);
             instance = rows_in_16s(M, N, K, O, batch, mask_upper) ? 2 : 0;
-        return instance == 0   ? gemm_softmax_gemm_launch(g, s)
+        }
+        return instance == 0   ? gemm_softmax_gemm_launch(g, 1, s)
                : instance == 1 ? gemm_gemm_launch_mt<1, 4, true>(g, s)
                                : gemm_gemm_launch_mt<1, 8, true>(g, s);
     }

@@ -5,25 +5,49 @@ namespace ckx {
 
 namespace {
 
-template <int KS, int OT, int NW>
+// NS parts of the columns, on 4 or (NS = 4) 2 waves of rows each
+template <int KS, int OT, int NS>
 hipError_t launch(const GemmGemmArgs& a, hipStream_t s)
 {
-    using Cfg = SoftmaxGemmCfg<KS, OT, NW>;
-    return gemm_gemm_launch_kernel<Cfg::BM, Cfg::NT, Cfg::LDS>(&gemm_softmax_gemm_kernel<KS, OT, NW>, a, s);
+    constexpr int NW  = NS == 4 ? 2 : 4;
+    using Cfg         = SoftmaxGemmCfg<KS, OT, NW>;
+    constexpr int LDS = SoftmaxGemmSplit<KS, OT, NW, NS>::LDS;
+    auto* kern        = &gemm_softmax_gemm_kernel<KS, OT, NW, NS>;
+    if constexpr(LDS > 64 * 1024)
+    {
+        static std::once_flag once;
+        static hipError_t attr_err = hipSuccess;
+        std::call_once(once, [&] {
+            attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+        });
+        if(attr_err != hipSuccess)
+            return attr_err;
+    }
+    return gemm_gemm_launch_kernel<Cfg::BM, Cfg::NT * NS, LDS>(kern, a, s);
 }
 
-template <int KS, int NW>
+template <int KS, int NS>
 hipError_t launch_ks(const GemmGemmArgs& a, hipStream_t s)
 {
-    return a.O <= 32 ? launch<KS, 1, NW>(a, s) : a.O <= 64 ? launch<KS, 2, NW>(a, s) : a.O <= 96 ? launch<KS, 3, NW>(a, s) : launch<KS, 4, NW>(a, s);
+    return a.O <= 32 ? launch<KS, 1, NS>(a, s) : a.O <= 64 ? launch<KS, 2, NS>(a, s) : a.O <= 96 ? launch<KS, 3, NS>(a, s) : launch<KS, 4, NS>(a, s);
+}
+
+template <int NS>
+hipError_t launch_any(const GemmGemmArgs& a, hipStream_t s)
+{
+    return a.K <= 32 ? launch_ks<2, NS>(a, s) : a.K <= 64 ? launch_ks<4, NS>(a, s) : a.K <= 80 ? launch_ks<5, NS>(a, s)
+         : a.K <= 96 ? launch_ks<6, NS>(a, s) : launch_ks<8, NS>(a, s);
 }
 
 } // namespace
 
-hipError_t gemm_softmax_gemm_launch(const GemmGemmArgs& a, hipStream_t s)
+hipError_t gemm_softmax_gemm_launch(const GemmGemmArgs& a, int parts, hipStream_t s)
 {
-    return a.K <= 32 ? launch_ks<2, 4>(a, s) : a.K <= 64 ? launch_ks<4, 4>(a, s) : a.K <= 80 ? launch_ks<5, 4>(a, s)
-         : a.K <= 96 ? launch_ks<6, 4>(a, s) : launch_ks<8, 4>(a, s);
+    if(parts == 4) // (rows of 192 bytes are not laid out for two waves)
+        return a.K <= 32   ? (a.O <= 32 ? launch<2, 1, 4>(a, s) : a.O <= 64 ? launch<2, 2, 4>(a, s) : launch<2, 4, 4>(a, s))
+               : a.K <= 64 ? (a.O <= 32 ? launch<4, 1, 4>(a, s) : a.O <= 64 ? launch<4, 2, 4>(a, s) : launch<4, 4, 4>(a, s))
+                           : (a.O <= 32 ? launch<8, 1, 4>(a, s) : a.O <= 64 ? launch<8, 2, 4>(a, s) : launch<8, 4, 4>(a, s));
+    return parts == 2 ? launch_any<2>(a, s) : launch_any<1>(a, s);
 }
 
 } // namespace ckx

@@ -49,7 +49,9 @@ struct SoftmaxGemmCfg
     static constexpr int ROWS_K = KCH == 12 ? 16 * (NT / 192) : NT / KCH, ROWS_V = VCH == 12 ? 16 * (NT / 192) : NT / VCH; // rows per load
     static constexpr int NLK = (UC + ROWS_K - 1) / ROWS_K, NLV = (UC + ROWS_V - 1) / ROWS_V;
     static_assert((UC % ROWS_K == 0 || NLK == 1) && (UC % ROWS_V == 0 || NLV == 1), "");
-    static_assert((ROWS_K % 16 == 0 || NLK == 1) && (ROWS_V % 16 == 0 || NLV == 1), "the keys repeat after 16 rows");
+    static_assert((ROWS_K % 16 == 0 || NLK == 1 || (KRS == 256 && ROWS_K == 8)) && (ROWS_V % 4 == 0 || NLV == 1), "the keys repeat after 16 and 4 rows");
+    // (in steps of eight rows the key of a 256-byte row flips its highest bit every time)
+    static constexpr uint32_t k_flip(int i) { return ROWS_K == 8 && (i & 1) ? 128u : 0u; }
     static constexpr int KSLOT = UC * KRS, VSLOT = UC * VRS;
     static constexpr int LDS = 2 * KSLOT + 2 * VSLOT;
     // XOR on the chunk position of row r. A ds_read_b128 is served 16 lanes at a time, those with equal (lane bit 5, parity of lane
@@ -62,19 +64,34 @@ struct SoftmaxGemmCfg
     __device__ static __forceinline__ uint32_t v_key(uint32_t r) { return VRS == 128 ? ((r >> 1) & 1u) << 2 : VRS == 256 ? (r & 3u) << 2 : 0u; }
 };
 
-template <int KS, int OT, int NW>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_softmax_gemm_kernel(const GemmGemmArgs p)
+// NS > 1: NS groups of NW waves own the same rows and take a share of the columns each, with slices of B0 and B1 of their own; at the end
+// the other groups' maxima, sums and accumulators cross over to the first through LDS. For launches of few workgroups, which last as long as a
+// wave's chain of units: a part of the chain, and a second wave on every SIMD to fill the first one's waits.
+// (two groups of four waves, or four of two, which halves the rows of a workgroup too). One group / two / four, us: 1 x 2995 x 2995 of heads of 128
+// 65.4 / 50.4 / 38.5, 1 x 3082 x 3082 / 64 38.3 / 31.4 / 24.0; 170 random problems up to 540 slabs,
+// as column_parts() chooses, 1.17 times as fast on average, up to 1.84. The merge: 2-norm of the error against float32 as with one group (2.8e-4).
+template <int KS, int OT, int NW, int NS = 1>
+struct SoftmaxGemmSplit
+{
+    using Cfg = SoftmaxGemmCfg<KS, OT, NW>;
+    static constexpr int CROSS = (NS - 1) * NW * (16 * OT + 2) * 256; // bytes that cross over
+    static constexpr int LDS   = NS * Cfg::LDS > CROSS ? NS * Cfg::LDS : CROSS;
+};
+
+template <int KS, int OT, int NW, int NS = 1>
+__global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_softmax_gemm_kernel(const GemmGemmArgs p)
 {
     using Cfg = SoftmaxGemmCfg<KS, OT, NW>;
     constexpr int NT = Cfg::NT, UC = Cfg::UC, NB = Cfg::NB, NK2 = Cfg::NK2, KRS = Cfg::KRS, VRS = Cfg::VRS, KCH = Cfg::KCH, VCH = Cfg::VCH,
                   NLK = Cfg::NLK, NLV = Cfg::NLV, ROWS_K = Cfg::ROWS_K, ROWS_V = Cfg::ROWS_V;
     extern __shared__ __attribute__((aligned(16))) uint8_t gg_smem[];
-    uint8_t* const sK = gg_smem;
-    uint8_t* const sV = gg_smem + 2 * Cfg::KSLOT;
-
-    const int tid  = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int all_waves = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int part      = NS == 1 ? 0 : all_waves / NW; // which columns
+    const int wave      = all_waves - part * NW;
+    const int tid       = threadIdx.x - part * NT;
+    const int lane      = tid & 63;
+    uint8_t* const sK   = gg_smem + part * Cfg::LDS;
+    uint8_t* const sV   = sK + 2 * Cfg::KSLOT;
     const int row  = lane & 31; // this lane's row of the wave's 32
     const int h    = lane >> 5; // K-slot half
 
@@ -82,21 +99,25 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     slab_of_block<true>((int)blockIdx.x, p, g, slab);
     const int m0       = slab * Cfg::BM;
     const _Float16* A  = p.a + (int64_t)g * p.bsa;
-    const _Float16* B0 = p.b0 + (int64_t)g * p.bsb0;
-    const _Float16* B1 = p.b1 + (int64_t)g * p.bsb1;
     _Float16* C        = p.c + (int64_t)g * p.bsc;
 
     // with the upper-triangle mask, columns past the last row are masked for every row
     const int wave_m0 = m0 + wave * 32;
     const int n_end   = p.mask_upper && m0 + Cfg::BM < p.N ? m0 + Cfg::BM : p.N;
-    const int w_end   = p.mask_upper && wave_m0 + 32 < p.N ? wave_m0 + 32 : p.N;
-    const int full    = p.mask_upper && wave_m0 + 1 < p.N ? wave_m0 + 1 : p.N; // columns below are unmasked for every row of the wave
-    const int units   = (n_end + UC - 1) / UC;
-    const int w_units = wave_m0 < p.M ? (w_end + UC - 1) / UC : 0;
+    // units that every wave takes part in; this part's first column, and its columns (everything below counts columns from there)
+    const int all_units = (n_end + UC - 1) / UC, units = (all_units + NS - 1) / NS;
+    const int n_first   = part * units * UC;
+    const int N         = NS == 1 ? p.N : p.N <= n_first ? 0 : part < NS - 1 && p.N - n_first > units * UC ? units * UC : p.N - n_first;
+    const int wave_c0   = wave_m0 - n_first;
+    const _Float16* B0  = p.b0 + (int64_t)g * p.bsb0 + (int64_t)(NS == 1 ? 0 : n_first) * p.sb0;
+    const _Float16* B1  = p.b1 + (int64_t)g * p.bsb1 + (int64_t)(NS == 1 ? 0 : n_first) * p.sb1;
+    const int w_end     = p.mask_upper && wave_c0 + 32 < N ? wave_c0 + 32 : N;
+    const int full      = p.mask_upper && wave_c0 + 1 < N ? wave_c0 + 1 : N; // columns below are unmasked for every row of the wave
+    const int w_units   = wave_m0 < p.M && (NS == 1 || w_end > 0) ? (w_end + UC - 1) / UC : 0;
 
     // ---- B0 / B1 on their way: global -> registers -> LDS -----------------------------------------------------------------
-    const __amdgpu_buffer_rsrc_t rsrc_k = make_rsrc(B0, p.N > 0 ? (uint32_t)(((int64_t)(p.N - 1) * p.sb0 + p.K) * 2) : 0u);
-    const __amdgpu_buffer_rsrc_t rsrc_v = make_rsrc(B1, p.N > 0 ? (uint32_t)(((int64_t)(p.N - 1) * p.sb1 + p.O) * 2) : 0u);
+    const __amdgpu_buffer_rsrc_t rsrc_k = make_rsrc(B0, N > 0 ? (uint32_t)(((int64_t)(N - 1) * p.sb0 + p.K) * 2) : 0u);
+    const __amdgpu_buffer_rsrc_t rsrc_v = make_rsrc(B1, N > 0 ? (uint32_t)(((int64_t)(N - 1) * p.sb1 + p.O) * 2) : 0u);
     // (thread t takes chunk t % KCH of row t / KCH and of the same row ROWS_K further on: one offset into the operand and one into a
     // slot, whose keys repeat after 16 rows)
     const uint32_t rk0 = tid / KCH, ck = tid - rk0 * KCH, rv0 = tid / VCH, cv = tid - rv0 * VCH;
@@ -110,7 +131,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     // below 2 GiB: there a sum may wrap around into the operand, for rows past N only. What is read then goes nowhere: columns past N get
     // -inf for a score by a select (mask), whatever it was, output columns past O are not stored, and units that do not exist meet no
     // product. (The out-of-range bit OR-ed into the sum instead, two to four instructions a unit: 1.03 of the time with one wave per SIMD.)
-    auto first = [&](int u, int stride) { return (uint32_t)(u * UC < p.N ? u * UC : p.N) * (uint32_t)stride * 2u; };
+    auto first = [&](int u, int stride) { return (uint32_t)(u * UC < N ? u * UC : N) * (uint32_t)stride * 2u; };
     // (rows past the last one read as zeros through the range check; CHECKED: they are found by their number, for strides whose
     // offsets of rows past the last one may wrap around)
     auto load_k = [&](int u, i32x4(&r)[NLK], auto checked) {
@@ -120,7 +141,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
         {
             uint32_t off = gk + (step + (uint32_t)(i * ROWS_K) * (uint32_t)p.sb0 * 2u);
             if(decltype(checked)::value)
-                off = tid < (p.N - u * UC - i * ROWS_K) * KCH ? off : kOutOfRange;
+                off = tid < (N - u * UC - i * ROWS_K) * KCH ? off : kOutOfRange;
             r[i] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_k, off, 0, 0));
         }
     };
@@ -131,7 +152,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
         {
             uint32_t off = gv + (step + (uint32_t)(i * ROWS_V) * (uint32_t)p.sb1 * 2u);
             if(decltype(checked)::value)
-                off = tid < (p.N - u * UC - i * ROWS_V) * VCH ? off : kOutOfRange;
+                off = tid < (N - u * UC - i * ROWS_V) * VCH ? off : kOutOfRange;
             r[i] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_v, off, 0, 0));
         }
     };
@@ -139,7 +160,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
         for(int i = 0; i < NLK; ++i)
             if(live_k)
-                *reinterpret_cast<i32x4*>(sK + slot * Cfg::KSLOT + lk + i * ROWS_K * KRS) = r[i];
+                *reinterpret_cast<i32x4*>(sK + slot * Cfg::KSLOT + (lk ^ Cfg::k_flip(i)) + i * ROWS_K * KRS) = r[i];
     };
     auto store_v = [&](int slot, const i32x4(&r)[NLV]) {
 #pragma unroll
@@ -277,8 +298,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
         const int n0 = u * UC;
         if(n0 + UC <= full)
             return;
-        const int m     = wave_m0 + row;
-        const int n_lim = (p.mask_upper && m + 1 < p.N ? m + 1 : p.N) - n0 - 4 * h; // columns from here on are masked
+        const int c     = wave_c0 + row;
+        const int n_lim = (p.mask_upper && c + 1 < N ? c + 1 : N) - n0 - 4 * h; // columns from here on are masked
 #pragma unroll
         for(int b = 0; b < NB; ++b)
 #pragma unroll
@@ -463,7 +484,41 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     const int m       = wave_m0 + row;
     auto halves       = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, sum[0]), __builtin_bit_cast(uint32_t, sum[0]), false, false);
     const uint32_t s0 = halves[0], s1 = halves[1];
-    const float total = __builtin_bit_cast(float, s0) + __builtin_bit_cast(float, s1);
+    float total       = __builtin_bit_cast(float, s0) + __builtin_bit_cast(float, s1);
+    if constexpr(NS > 1)
+    {
+        constexpr int OVER = (16 * OT + 2) * 64; // floats of a wave
+        float* const over  = reinterpret_cast<float*>(gg_smem) + wave * OVER + lane;
+        __syncthreads();
+        if(part)
+        {
+            float* const to = over + (part - 1) * (NW * OVER);
+#pragma unroll
+            for(int t = 0; t < OT; ++t)
+#pragma unroll
+                for(int i = 0; i < 16; ++i)
+                    to[(16 * t + i) * 64] = acc[t][i];
+            to[16 * OT * 64]       = m_run;
+            to[(16 * OT + 1) * 64] = total;
+        }
+        __syncthreads();
+        if(part)
+            return;
+#pragma unroll
+        for(int q = 0; q < NS - 1; ++q)
+        {
+            const float* const from = over + q * (NW * OVER);
+            const float m_other = from[16 * OT * 64], m_both = __builtin_fmaxf(m_run, m_other), m_to = m_both == ninf ? 0.0f : m_both;
+            const float mine = __builtin_amdgcn_exp2f(m_run - m_to), other = __builtin_amdgcn_exp2f(m_other - m_to);
+            m_run = m_both;
+            total = total * mine + from[(16 * OT + 1) * 64] * other;
+#pragma unroll
+            for(int t = 0; t < OT; ++t)
+#pragma unroll
+                for(int i = 0; i < 16; ++i)
+                    acc[t][i] = acc[t][i] * mine + from[(16 * t + i) * 64] * other;
+        }
+    }
     const float inv   = total > 0.0f ? 1.0f / total : 0.0f; // N == 0: an empty sum, C = 0
     if(m >= p.M)
         return;

@@ -290,3 +290,25 @@ def test_gemm_softmax_gemm_refused_arguments_and_empty_sum():
     for instance in (0, 2):
         out = _run(np.ones((1, 16, 8), np.float16), np.zeros((1, 0, 8), np.float16), np.zeros((1, 0, 8), np.float16), instance=instance)
         np.testing.assert_array_equal(out, np.zeros((1, 16, 8), np.float16))
+
+
+@pytest.mark.parametrize("G, M, N, K, O", [
+    (2, 1, 576, 32, 32), (2, 133, 600, 16, 24), (1, 200, 641, 64, 64), (3, 64, 1026, 40, 24), (3, 65, 700, 40, 72), (1, 320, 673, 128, 128), (2, 64, 645, 24, 104),
+    (1, 129, 999, 128, 32), (1, 66, 1536, 80, 80), (2, 70, 1570, 96, 72), (1, 1100, 1100, 64, 32),             # four shares of the columns
+    (2, 133, 769, 80, 80), (1, 260, 801, 72, 96), (97, 65, 641, 64, 64), (97, 66, 577, 32, 32), (98, 70, 608, 128, 120), (99, 65, 800, 48, 104),
+    (97, 128, 900, 104, 16), (1, 300, 1030, 96, 40),                                                           # two
+    (193, 129, 640, 32, 32), (2, 100, 575, 32, 32), (2, 133, 639, 64, 64)])                                    # one (past the lines, and below)
+def test_gemm_softmax_gemm_column_shares(G, M, N, K, O):
+    """Launches of few workgroups deal the columns out to groups of waves and merge their sums: shares without columns (a causal slab's
+    later ones, units that do not divide), rows past M, scores that rise so that the last share holds every maximum or fall so that the
+    first does, NaNs between the rows. Against the oracle, and against the kernel with one share (instance 0): both round p to 2^-11 of
+    itself, at different running maxima, and the result to 2^-11, so they differ by at most 2^-9 of the sum of p |B1| <= 1."""
+    a, b0, b1 = (uniform_f16((G, x, y), -1, 1, 1990 + i) for i, (x, y) in enumerate(((M, K), (N, K), (N, O))))
+    a[..., 0] = 1
+    for mask in (False, True):
+        for slope in (0, 8, -8):
+            b0[..., 0] = (slope * np.arange(N) / N).astype(np.float16)
+            out = _run(a, b0, b1, K ** -0.5, mask, pad=(8, 24, 16, 8), gap=np.nan)
+            one = _run(a, b0, b1, K ** -0.5, mask, 0)
+            assert np.max(np.abs(out.astype(np.float64) - one)) <= 2.0 ** -9
+            _close(out[-1:], lit.batched_gemm_softmax_gemm_f16(a[-1:], b0[-1:].transpose(0, 2, 1), b1[-1:], K ** -0.5, mask))
