@@ -565,12 +565,18 @@ hipError_t gemm_softmax_gemm_launch(const GemmGemmArgs& a, int parts, hipStream_
 // 15.6 / 12.5; of 80: 32 x 256 x 256 8.6 / 7.9. The lines in N lie on the careful side: with one slab to a batch (M = 128) 32 rows are level with 16 at N 768 and
 // 1.02 to 1.08 ahead from 832 on (heads of 64, 200 batches: 960 17.4 / 16.1, 968 17.7 / 16.8, 1024 17.6 / 16.7, 1032 18.7 / 17.6), and for heads of
 // 32 1.02 to 1.14 ahead from 320 on (128 batches: 384 6.8 / 6.5, 440 8.2 / 7.5, 448 8.3 / 7.2, 480 8.1 / 7.7).
+// Past 256 slabs the mask's line holds only while there are enough slabs to a batch for the longest ones to come early (measured at M = N; with
+// columns past the last row, masked for all, the line stays): heads of 128, 297 x 104
+// x 104 15.3 / 11.9, 114 x 280 x 280 19.3 / 13.4, 83 x 606 x 606 28.5 / 23.0, 66 x 812 x 812 34.7 / 27.8, but 40 x 946 x 946 24.5 / 26.4 and 48 x 952 x 952 level;
+// heads of 64, 134 x 158 x 158 9.8 / 8.2, 442 x 128 x 128 11.1 / 9.4, 112 x 353 x 353 11.2 / 10.4, but with K 32 and O 64 104 x 352 x 352 8.3 / 8.9.
 inline bool rows_in_16s(int M, int N, int K, int O, int batch, bool mask_upper)
 {
     const int head   = K > O ? K : O;
     const long slabs = (long)batch * ((M + 127) / 128) * 256 / num_cus(); // (as on 256 CUs, which the lines here were measured on)
     if(head > 96)
-        return slabs <= (mask_upper ? 512 : 256);
+        return slabs <= (!mask_upper ? 256 : M < N ? 512 : N >= 896 ? 384 : 256);
+    if(slabs > 256 && M >= N && N <= 352 && K > 32)
+        return false;
     // (130 x 375 x 375 13.2 / 13.8 us; longer N, where the second workgroup of some CUs comes late enough: 43 x 768 x 768 13.9 / 14.9, 64 x 768 x
     // 768 13.5 / 14.7, 47 x 896 x 896 0.97 of the time, but 75 x 640 x 640 1.04, 67 x 768 x 768 1.00)
     if(mask_upper && head > 32 && head <= 64 && N < 1024)
