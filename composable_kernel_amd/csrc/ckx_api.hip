@@ -23,6 +23,7 @@
 #include "conv_window.hpp"
 #include "gemm_skinny.hpp"
 #include "gemm_generic.hpp"
+#include "gemm_pack.hpp"
 #include "gemm_ragged.hpp"
 
 // Workspace of ckx_gemm_i8_splitk_noalloc: device memory that belongs to the library, one copy per GPU,
@@ -458,10 +459,50 @@ int check_gemm_shape(int dt, int M, int N, int K, int sa, int sb, int sc, int al
     return CKX_OK;
 }
 
+// Copies of operands whose K is no whole number of 16-byte vectors (gemm_pack.hpp): elements of K and of a row, bytes of both copies
+struct PackPlan
+{
+    int K, pitch;
+    long a_bytes, bytes;
+};
+PackPlan pack_plan(int es, int M, int N, int K)
+{
+    const int vec = 16 / es, line = 128 / es;
+    PackPlan p;
+    p.K = (K + vec - 1) / vec * vec, p.pitch = (K + line - 1) / line * line;
+    p.a_bytes = (long)M * p.pitch * es, p.bytes = p.a_bytes + (long)N * p.pitch * es;
+    return p;
+}
+// The padding instance is bound by the operand rows through the busiest CU, whose K tiles take 0.32 to 0.45 us per 128 rows where whole lines
+// take about half; the copies cost a launch (3.4 us), their bytes, and what a product as small as its launch has to fill the CUs with. Padding
+// instance / copies and the instance for whole vectors, us: fp16 4001 x 4003 x 4095 196 / 130, 2049 x 2047 x 2047 55.0 / 39.8, 3001 x 333 x 3001
+// 33.9 / 25.9, 1500 x 901 x 2001 24.5 / 20.0, 1707 x 1491 x 1011 20.0 / 19.2, 2001 x 1003 x 1025 15.4 / 15.0, int8 4001 x 4003 x 4095 112 / 61.0, 1500
+// x 901 x 2001 16.2 / 15.4, but by rows: 1000 x 4001 x 513 (18 K tiles of 128) 16.0 / 16.7, int8 2474 x 765 x 1509 (24) 13.5 / 14.1, and by products: 700 x
+// 701 x 3001 (2.9e9 operations) 18.4 / 19.7, 2205 x 131 x 3491 (2.0) 20.9 / 23.5, and by products per
+// operand byte: fp16 3934 x 139 x 3815 (134) 25.7 / 28.3. 49 random problems on the near side of the lines take 0.77 of the time on average, 0.95 at most. K-major operands, transposed on the way: int8 1543 x 3503 x 1023 22.9 / 17.7
+// (11.1e9), 1066 x 3695 x 4069 82.4 / 64.8, but 3031 x 901 x 1055 (5.8) 20.6 / 21.2, 2924 x 981 x 1755 (10.1) 28.6 / 29.2.
+bool packing_pays(int es, int M, int N, int K, bool kmajor)
+{
+    const int vec     = 16 / es;
+    const double work = 2.0 * M * N * K;
+    if(K % vec == 0 || K < vec || work < (kmajor ? 11e9 : 4e9) || work < 200.0 * ((double)M + N) * K * es)
+        return false;
+    const long m = ckx::ragged_tile(M, N, 1) == 128 ? 128 : ckx::ragged_small_tile(M, N, 1).m;
+    const long n = m == 128 ? 128 : ckx::ragged_small_tile(M, N, 1).n;
+    const long rows = ((M + m - 1) / m * ((N + n - 1) / n) + num_cus() - 1) / num_cus() * (m + n); // of the busiest CU
+    const PackPlan p = pack_plan(es, M, N, K);
+    return rows * (((long)K * es + 127) / 128) >= 32 * 128 && p.a_bytes < (1l << 31) && p.bytes - p.a_bytes < (1l << 31);
+}
+
 // workspace need of the launch plan for this GEMM (0: none)
 long gemm_workspace_bytes(int dt, int M, int N, int K, int instance)
 {
     const int es = dt == ckx::DT_I8 ? 1 : 2;
+    if(M > 0 && N > 0 && instance == CKX_INSTANCE_AUTO && packing_pays(es, M, N, K, false)) // (K-major operands: fewer problems, the same copies)
+    {
+        const PackPlan p = pack_plan(es, M, N, K);
+        return p.bytes + gemm_workspace_bytes(dt, M, N, p.K, instance);
+    }
     // (up to 16 rows go to the skinny kernels, which take none -- except few columns under a long K: see run_gemm)
     const bool few_cols = M >= 8 && (N + 15) / 16 < (M > 16 ? 257 : 128) && (long)K * es >= 16384;
     if(M <= 0 || N <= 0 || (instance == CKX_INSTANCE_AUTO && M <= 16 && !few_cols) || instance >= kNumTiles ||
@@ -614,6 +655,19 @@ int run_gemm(int dt, const void* a, const void* b, void* c, int M, int N, int K,
         if(batch > 65535) // (the documented limit; the kernel itself counts batches in its linear grid)
             return fail(CKX_UNSUPPORTED, "the padding instance (operands that are not 16-byte aligned vectors) "
                                          "takes at most 65535 batches per launch");
+        // With a workspace, copies whose rows are whole vectors (a plan query names the padding instance all the same, which takes the operands as they are)
+        const PackPlan p = pack_plan(es, M, N, K);
+        if(instance == CKX_INSTANCE_AUTO && batch == 1 && k_batch == 0 && ws && !(reinterpret_cast<uintptr_t>(ws) & 15) && ws_bytes >= p.bytes &&
+           packing_pays(es, M, N, K, kmajor) && (!ta || M * es >= 16) && (!tb || N * es >= 16))
+        {
+            uint8_t* const to = reinterpret_cast<uint8_t*>(ws);
+            const hipError_t e =
+                ckx::launch_gemm_pack(ckx::GemmPack{a, b, to, to + p.a_bytes, es, M, N, K, sa, sb, ta, tb, p.pitch}, (hipStream_t)stream);
+            if(e != hipSuccess)
+                return hip_fail(e, kGenericName);
+            return run_gemm(dt, to, to + p.a_bytes, c, M, N, p.K, p.pitch, p.pitch, sc, CKX_ROW_MAJOR, CKX_COL_MAJOR, cl, epi, sg, sr, instance,
+                            ws_bytes > p.bytes ? to + p.bytes : nullptr, ws_bytes - p.bytes, stream, dops);
+        }
         hipError_t e = ckx::launch_ragged(dt, ta, tb, g, (hipStream_t)stream);
         return e == hipSuccess ? CKX_OK : hip_fail(e, kGenericName);
     }

@@ -21,7 +21,7 @@
 // bytes of it touch: 35 to 49 bytes per ns and CU, 77 where rows start on a line (0.27 of the MFMA rate at 4001 x 4003 x
 // 4095 fp16). Reading whole lines and moving the chunks into place in registers took more than it saved (25 vector instructions
 // per 16 bytes; 2001 x 1003 x 1025 15.7 -> 19.3 us), unaligned LDS writes 50 to 120 cycles each instead of 13, and four K tiles in
-// flight instead of two nothing. Against the element-by-element gather
+// flight instead of two nothing. (Large products with a workspace: gemm_pack.hpp copies the operands to whole lines first.) Against the element-by-element gather
 // that served these shapes (one load instruction per element), fp16: 2001 x 1003 x 1025 98.7 -> 15.4 us, 4001 x 4003 x 4095
 // 2623 -> 197, 122 x 1283 x 3001 148 -> 17.4, 2049 x 2047 x 2047 with a K-major A 290 -> 55; int8 4001 x 4003 x 4095 3019 -> 118,
 // 40 x 333 x 3999 156 -> 16; bf16 3000 x 2999 x 1001 275 -> 47; one tile (32 x 33 x 65) 5.7, as before.

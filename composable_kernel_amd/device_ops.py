@@ -163,7 +163,7 @@ class BaseOperator:
         return capi.lib().ckx_instance_name(self.op_family, self.instance).decode()
 
     def GetWorkSpaceSize(self, arg):
-        """Bytes of optional device scratch (split-K); 0 for most problems."""
+        """Bytes of optional device scratch (split-K, copies of operands that are no whole vectors); 0 for most problems."""
         return 0
 
     def SetWorkSpacePointer(self, arg, p, nbytes=None):
