@@ -552,6 +552,7 @@ inline hipError_t gemm_gemm_launch_mt(const GemmGemmArgs& g, hipStream_t s)
     return og == 1 ? gemm_gemm_launch_t<4, 1, MT, NW, SOFTMAX>(g, s) : gemm_gemm_launch_t<4, 2, MT, NW, SOFTMAX>(g, s);
 }
 
+hipError_t gemm_gemm_wide_launch(const GemmGemmArgs& a, int parts, hipStream_t s); // gemm_gemm_wide.hip: the same kernel without its softmax
 hipError_t gemm_softmax_gemm_launch(const GemmGemmArgs& a, int parts, hipStream_t s); // gemm_softmax_gemm.hip; parts: shares of the columns, 1, 2 or 4
 
 // Attention on waves of 16 rows (instance 2) instead of 32 (instance 0). Up to 256 slabs of 128 rows there is one workgroup to a CU: one
@@ -611,6 +612,33 @@ inline int column_parts(int M, int N, int K, int O, int batch, bool mask_upper)
     return chain >= from2 && by128 <= (chain < 1024 ? 224 : most) ? 2 : 1;
 }
 
+// Without softmax: shares of the columns (1, 2 or 4, as above) on the 32-row kernel, or 0 for the kernels of 128-column steps.
+// The 32-row waves read B0 and B1 fragments half as often per product and keep other units' reads and conversions between their MFMAs; their
+// units of 32 or 64 columns pad N less than steps of 128. The kernels of 128-column steps have more waves per row, and stay ahead on short chains
+// and, with heads of 33 to 64, while few workgroups leave the CUs to one wave of 32 rows per SIMD. us, steps of 128 / 1 / 2 / 4 shares, by slabs of
+// 128 rows and N: heads of 32: 351 slabs, 299 8.0 / 6.3 / 9.5 / 13.3; 408, 1087 16.3 / 11.7 / 15.2 / 27.4; 109, 975 9.6 / 8.3 / 6.9 / 8.2; 96, 1388 11.7 / 9.8 / 8.1 / 7.7;
+// but 72, 402 level. Of 64: 328, 747 16.6 / 15.1 / 20.1 / 22.1; 180, 946 12.0 / 11.2 / 12.3 / 21.5; 147, 1997 19.3 / 17.5 / 16.9 / 22.9; 50, 1753 15.3 / 15.6 / 14.8 /
+// 13.6, but 99, 811 9.3 / 9.8 / 10.2 / 9.9; 256, 512 7.7 / 8.4 / 9.1 / 14.9; 576, 275 13.5 / 14.5; 84, 1881 (168 slabs of 64) 16.9 and 17.4 in four shares. Of 128: 592,
+// 294 36.4 / 25.4 / 34.1 / 52.8; 51, 692 16.6 / 14.0 / 14.7 / 14.6; 45, 1946 36.5 / 29.2 / 27.1 / 23.4; 45, 142 7.8 / 7.3, but 27, 235, which fills its steps,
+// 7.2 / 7.6; 63, 111 6.0 / 6.9; of K 128 and O 32, 75, 738 12.4 / 12.8. 190 random problems up to 1400 slabs: 1.12 times as fast on average, up to 1.95.
+inline int wide_parts(int M, int N, int K, int O, int batch)
+{
+    const int head   = K > O ? K : O;
+    const long by64  = (long)batch * ((M + 63) / 64) * 256 / num_cus(), by128 = (long)batch * ((M + 127) / 128) * 256 / num_cus();
+    const bool few   = by128 <= 256;
+    if(N >= (head <= 32 ? 1024 : head <= 64 ? 1152 : 1280) && by64 <= (head > 32 && head <= 64 ? 160 : 192))
+        return 4;
+    if(head <= 32)
+        return few && N >= 768 ? 2 : N >= (few ? 448 : 288) ? 1 : 0;
+    if(head <= 64)
+        return few ? (by128 <= 128 || N < 768 ? 0 : N < 1400 ? 1 : 2) : N >= 576 ? 1 : 0;
+    if(few && N >= 1280)
+        return 2;
+    if(few && N < 1024 && (K <= 32 || O <= 32))
+        return 0;
+    return N >= 264 || (K > 64 && O > 64 && (!few || (N > 128 && N <= 192))) ? 1 : 0;
+}
+
 // softmax: the attention variant with scores scale * (A * B0) and the optional upper-triangle mask
 inline hipError_t gemm_gemm_launch(const void* a, const void* b0, const void* b1, void* c, int M, int N, int K,
                                    int O, int batch, int sa, int sb0, int sb1, int sc, int64_t bsa,
@@ -640,13 +668,14 @@ inline hipError_t gemm_gemm_launch(const void* a, const void* b0, const void* b1
     if(instance < 0)
     {
         // Many short waves (8 x 16 rows, the instance with two steps of prefetch where registers allow) are ahead on short
-        // problems: G 64, 512 x 64 x 512 x 64 8.5 against 10.1 us. Over a long N with small heads the 32-row waves read the B0 / B1
-        // fragments half as often per row and win: G 64, 4096 x 64 x 4096 x 64 267 against 302 us (2048: 76 / 85; at N = 1024
-        // 23.5 / 26.2). That needs workgroups to spare (two of them share a CU): up to 128 slabs of small heads the 64-row instance,
-        // which doubles the workgroups, is ahead (20.6 against 25.4 us).
+        // problems: G 64, 512 x 64 x 512 x 64 8.5 against 10.1 us. Up to 128 slabs of small heads the 64-row instance, which doubles
+        // the workgroups, is (20.6 against 25.4 us).
         const long slabs128 = (long)batch * ((M + 127) / 128);
         const bool small_heads = K <= 64 && O <= 64;
-        instance = small_heads && slabs128 <= 128 ? 1 : small_heads && N >= 1024 && slabs128 >= 256 ? 0 : 2;
+        const int parts        = wide_parts(M, N, K, O, batch);
+        if(parts > 0)
+            return gemm_gemm_wide_launch(g, parts, s);
+        instance = small_heads && slabs128 <= 128 ? 1 : 2;
     }
     return instance == 0 ? gemm_gemm_launch_mt<2, 4, false>(g, s)
            : instance == 1 ? gemm_gemm_launch_mt<1, 4, false>(g, s)

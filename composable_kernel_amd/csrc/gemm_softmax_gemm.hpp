@@ -25,6 +25,7 @@
 // 16x16x32 MFMAs, sums by v_dot2 and softmax and products one after the other 34 and 64 %, 0.98. us, that kernel and this one in turn on one card:
 // 394.7 -> 359.1, causal 184.6 -> 179.4 (192.4 -> 189.5 with new operands in each pass); 32 x 2048 x 2048 x 128 92.4 -> 80.9, x 80 89.8 -> 58.8; 64 x 2048
 // x 2048 x 32 79.1 -> 59.2. 48 + 120 random problems 0.76 and 0.88 of the time.
+// SM = false: the same kernel without the softmax, for the fused pair of GEMMs (gemm_gemm_wide.hip; wide_parts() has its figures).
 #pragma once
 
 #include "gemm_gemm.hpp"
@@ -78,7 +79,8 @@ struct SoftmaxGemmSplit
     static constexpr int LDS   = NS * Cfg::LDS > CROSS ? NS * Cfg::LDS : CROSS;
 };
 
-template <int KS, int OT, int NW, int NS = 1>
+// SM: with the softmax; without, the scores rounded to fp16 take the probabilities' place (C = half( half(A * B0) * B1 ))
+template <int KS, int OT, int NW, int NS = 1, bool SM = true>
 __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_softmax_gemm_kernel(const GemmGemmArgs p)
 {
     using Cfg = SoftmaxGemmCfg<KS, OT, NW>;
@@ -260,7 +262,8 @@ __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
             for(int t = 0; t < OT; ++t)
                 acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v_frag(slot, k2, t), pr[k2], acc[t], 0, 0, 0);
-            sum = add_up(sum, pr[k2]);
+            if constexpr(SM)
+                sum = add_up(sum, pr[k2]);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -291,7 +294,11 @@ __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2,
     auto softmax = [&](f32x16(&s)[NB], f16x8(&pr)[NK2]) {
 #pragma unroll
         for(int q = 0; q < NP; ++q)
-            stage_fma(s, q), stage_exp(s, q), stage_half(s, pr, q);
+        {
+            if constexpr(SM)
+                stage_fma(s, q), stage_exp(s, q);
+            stage_half(s, pr, q);
+        }
         pin(pr);
     };
     auto mask = [&](int u, f32x16(&s)[NB]) {
@@ -304,7 +311,7 @@ __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2,
         for(int b = 0; b < NB; ++b)
 #pragma unroll
             for(int i = 0; i < 16; ++i)
-                s[b][i] = 32 * b + 8 * (i / 4) + i % 4 < n_lim ? s[b][i] : ninf;
+                s[b][i] = 32 * b + 8 * (i / 4) + i % 4 < n_lim ? s[b][i] : SM ? ninf : 0.0f;
     };
 
     // ---- the units ----------------------------------------------------------------------------------------------------------
@@ -343,7 +350,7 @@ __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2,
         {
             i32x4 v = __builtin_bit_cast(i32x4, af[ks]);
             v       = 16 * ks + 8 * h < p.K ? v : i32x4{0, 0, 0, 0};
-            af[ks]  = __builtin_bit_cast(f16x8, p.scale < 0.0f ? v ^ (int)0x80008000 : v); // scale * (A * B0) = |scale| * ((-A) * B0)
+            af[ks]  = __builtin_bit_cast(f16x8, SM && p.scale < 0.0f ? v ^ (int)0x80008000 : v); // scale * (A * B0) = |scale| * ((-A) * B0)
         }
     }
     __syncthreads();
@@ -357,7 +364,8 @@ __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2,
         __syncthreads();
         stage(0, 0, kChecked);
         mask(0, sa);
-        raise(max_of(sa)); // (nothing accumulated yet)
+        if constexpr(SM)
+            raise(max_of(sa)); // (nothing accumulated yet)
         softmax(sa, pa);
         if(w_units > 1)
             scores(1, sa);
@@ -376,14 +384,14 @@ __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2,
     bool pending = false; // wave-uniform: acc still waits for corr
     auto middle = [&](int u, auto parity, f32x16(&s)[NB], f32x16(&s_next)[NB], f16x8(&pr)[NK2], f16x8(&p_prev)[NK2]) {
         constexpr int W = decltype(parity)::value, R = 1 - W; // slots written and read
-        constexpr int G0 = NB * KS, L = G0 + NK2 * (OT + 1), AHEAD = 4;
+        constexpr int OTS = OT + SM, G0 = NB * KS, L = G0 + NK2 * OTS, AHEAD = 4; // (OTS: the row sums have a step of their own)
         f16x8 frag[L];
         auto fetch = [&](auto ic) {
             constexpr int i = decltype(ic)::value;
             if constexpr(i < G0)
                 frag[i] = k_frag(R, i % NB, i / NB);
-            else if constexpr(i < L && (i - G0) % (OT + 1) < OT)
-                frag[i] = v_frag(R, (i - G0) / (OT + 1), (i - G0) % (OT + 1));
+            else if constexpr(i < L && (i - G0) % OTS < OT)
+                frag[i] = v_frag(R, (i - G0) / OTS, (i - G0) % OTS);
         };
         __builtin_amdgcn_s_setprio(0);
         __syncthreads();
@@ -391,17 +399,25 @@ __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2,
         __builtin_amdgcn_sched_barrier(0);
         // (four units and more here: at least 3 * UC rows, and the offsets of 64 more stay below 2^32)
         stage(u, W, std::false_type{});
-        if(pending)
-            rescale(corr);
-        pending = exceeded(mx);
-        if(pending)
-            corr = raise(mx);
+        if constexpr(SM)
+        {
+            if(pending)
+                rescale(corr);
+            pending = exceeded(mx);
+            if(pending)
+                corr = raise(mx);
+        }
         __builtin_amdgcn_s_setprio(1); // (32 x 2048 x 2048 x 80 61.4 -> 58.8 us, x 128 86.4 -> 82.9, 64 x 4096 x 4096 x 64 346 -> 340)
         auto vector_work = [&](auto ic) {
-            constexpr int i = decltype(ic)::value, q0 = i * (NP + 2) / L, q1 = (i + 1) * (NP + 2) / L;
+            constexpr int i = decltype(ic)::value, steps = SM ? NP + 2 : NP, q0 = i * steps / L, q1 = (i + 1) * steps / L;
 #pragma unroll
             for(int q = q0; q < q1; ++q)
             {
+                if constexpr(!SM)
+                {
+                    stage_half(s, pr, q);
+                    continue;
+                }
                 if(q >= 2)
                     stage_half(s, pr, q - 2);
                 if(q >= 1 && q - 1 < NP)
@@ -419,7 +435,7 @@ __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2,
         });
         float mxa, mxb;
         static_for<L - G0>([&](auto jc) {
-            constexpr int j = decltype(jc)::value, k2 = j / (OT + 1), t = j % (OT + 1);
+            constexpr int j = decltype(jc)::value, k2 = j / OTS, t = j % OTS;
             fetch(std::integral_constant<int, G0 + j + AHEAD>{});
             if constexpr(t < OT)
                 acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag[G0 + j], p_prev[k2], acc[t], 0, 0, 0);
@@ -427,7 +443,7 @@ __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2,
                 sum = add_up(sum, p_prev[k2]);
             vector_work(std::integral_constant<int, G0 + j>{});
             // (the next scores are complete: their maximum)
-            constexpr int NM = NB * 16 / 4, r0 = j * NM / (L - G0), r1 = (j + 1) * NM / (L - G0);
+            constexpr int NM = SM ? NB * 16 / 4 : 0, r0 = j * NM / (L - G0), r1 = (j + 1) * NM / (L - G0);
 #pragma unroll
             for(int r = r0; r < r1; ++r)
             {
@@ -440,11 +456,12 @@ __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2,
                 asm volatile("" : "+v"(mxa), "+v"(mxb));
             __builtin_amdgcn_sched_barrier(0);
         });
-        mx = score_max(mxa, mxb);
+        if constexpr(SM)
+            mx = score_max(mxa, mxb);
         pin(pr);
     };
     // (two units at a time, so that scores and probabilities change places without copies; what is left goes step after step)
-    if(w_units > 3)
+    if(SM && w_units > 3)
         mx = max_of(sa);
     for(; u + 2 < w_units; u += 2)
     {
@@ -452,7 +469,7 @@ __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2,
         middle(u + 1, std::integral_constant<int, 0>{}, sb, sa, pa, pb);
     }
     __builtin_amdgcn_s_setprio(0);
-    if(pending)
+    if(SM && pending)
         rescale(corr);
     for(; u < w_units; ++u)
     {
@@ -460,9 +477,12 @@ __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2,
         stage(u, u & 1, kChecked);
         accumulate((u + 1) & 1, pa, NB);
         mask(u, sa);
-        const float top = max_of(sa);
-        if(exceeded(top))
-            rescale(raise(top));
+        if constexpr(SM)
+        {
+            const float top = max_of(sa);
+            if(exceeded(top))
+                rescale(raise(top));
+        }
         softmax(sa, pa);
         if(u + 1 < w_units)
             scores((u + 1) & 1, sa);
@@ -498,8 +518,8 @@ __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
                 for(int i = 0; i < 16; ++i)
                     to[(16 * t + i) * 64] = acc[t][i];
-            to[16 * OT * 64]       = m_run;
-            to[(16 * OT + 1) * 64] = total;
+            if constexpr(SM)
+                to[16 * OT * 64] = m_run, to[(16 * OT + 1) * 64] = total;
         }
         __syncthreads();
         if(part)
@@ -508,6 +528,15 @@ __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2,
         for(int q = 0; q < NS - 1; ++q)
         {
             const float* const from = over + q * (NW * OVER);
+            if constexpr(!SM)
+            {
+#pragma unroll
+                for(int t = 0; t < OT; ++t)
+#pragma unroll
+                    for(int i = 0; i < 16; ++i)
+                        acc[t][i] += from[(16 * t + i) * 64];
+                continue;
+            }
             const float m_other = from[16 * OT * 64], m_both = __builtin_fmaxf(m_run, m_other), m_to = m_both == ninf ? 0.0f : m_both;
             const float mine = __builtin_amdgcn_exp2f(m_run - m_to), other = __builtin_amdgcn_exp2f(m_other - m_to);
             m_run = m_both;
@@ -531,7 +560,7 @@ __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2,
         f32x4 v[4];
 #pragma unroll
         for(int i = 0; i < 16; ++i)
-            v[i / 4][i % 4] = acc[t][i] * inv;
+            v[i / 4][i % 4] = SM ? acc[t][i] * inv : acc[t][i];
         store_row16_f16(C + (int64_t)m * p.sc, o0, p.O, v);
     }
 }

@@ -131,3 +131,53 @@ def test_batches_past_one_launch(softmax):
     op.MakeInvokerPointer().Run(arg, ck.StreamConfig(gpu_util.stream()))
     torch.cuda.synchronize()
     assert torch.equal(c, want)
+
+
+@pytest.mark.parametrize("G, M, N, K, O", [
+    (4, 130, 1025, 32, 32), (3, 65, 1152, 64, 64), (1, 64, 1290, 64, 24), (2, 33, 1300, 128, 128), (1, 200, 1311, 96, 40), (2, 1, 1281, 24, 104),   # 4 shares
+    (110, 129, 770, 32, 32), (129, 128, 1400, 40, 64), (100, 130, 1281, 128, 120), (98, 65, 1295, 80, 72),                                      # 2
+    (2, 129, 448, 32, 32), (2, 133, 479, 8, 24), (257, 33, 289, 32, 32), (129, 1, 768, 64, 40), (257, 65, 577, 64, 64), (2, 133, 264, 128, 128),
+    (2, 31, 161, 72, 128), (257, 40, 66, 128, 128), (3, 97, 327, 40, 128), (1, 260, 385, 128, 72),                                              # 1
+    (2, 129, 447, 32, 32), (2, 64, 1100, 64, 64), (2, 65, 200, 128, 128), (2, 130, 1000, 128, 32)])                                             # steps of 128
+def test_gemm_gemm_on_both_sides_of_the_32_row_kernels_rule(G, M, N, K, O):
+    """Units, shares and rows that end anywhere, NaNs between the rows of A, B0 and B1, nothing written between those of C."""
+    import torch
+    import gpu_util
+    pads = (8, 24, 16, 8)
+    ops = [uniform_f16((G, x, y), -0.5, 0.5, 930 + i) for i, (x, y) in enumerate(((M, K), (N, K), (N, O)))]
+    dev = []
+    for x, pad in zip(ops, pads):
+        buf = np.full(x.shape[:2] + (x.shape[2] + pad,), np.nan, np.float16)
+        buf[..., :x.shape[2]] = x
+        dev.append(torch.from_numpy(buf.view(np.int16)).cuda())
+    c = torch.full((G, M, O + pads[3]), 0x7E00, dtype=torch.int16, device="cuda")
+    sa, sb0, sb1, sc = K + pads[0], K + pads[1], O + pads[2], O + pads[3]
+    op = ck.DeviceBatchedGemmGemmF16()
+    arg = op.MakeArgumentPointer(*dev, c, M, N, K, O, G, sa, sb0, sb1, sc, M * sa, N * sb0, N * sb1, M * sc)
+    assert op.IsSupportedArgument(arg), capi.last_error()
+    op.MakeInvokerPointer().Run(arg, ck.StreamConfig(gpu_util.stream()))
+    torch.cuda.synchronize()
+    out = c.cpu().numpy().view(np.float16)
+    assert np.all(out[..., O:].view(np.uint16) == 0x7E00), "wrote between the C rows"
+    a, b0, b1 = ops
+    for g in {0, G - 1}:
+        _close(out[g:g + 1, :, :O], lit.batched_gemm_gemm_f16(a[g:g + 1], b0[g:g + 1].transpose(0, 2, 1), b1[g:g + 1]))
+    # against float64, with the intermediate rounded to fp16 as the operator rounds it: a fp32 sum that lies next to a rounding boundary may
+    # round to the neighbour, 2^-11 of itself (|.| <= K / 4), once in about 2^11 / K of them, and the result to 2^-11 of itself
+    s = (a[0].astype(np.float64) @ b0[0].astype(np.float64).T).astype(np.float32).astype(np.float16)
+    want = s.astype(np.float64) @ b1[0].astype(np.float64)
+    assert np.linalg.norm(out[0, :, :O] - want) <= 6e-4 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("G, M, N, K", [(2, 133, 479, 32), (4, 130, 1025, 32), (1, 260, 385, 128)])
+def test_gemm_gemm_nan_row_stays_in_its_row(G, M, N, K):
+    import gpu_util
+    a, b0, b1 = (uniform_f16((G, x, K), -0.5, 0.5, 940 + i) for i, x in enumerate((M, N, N)))
+    clean = gpu_util.gemm_gemm_f16(a, b0, b1)
+    for row in (0, 31, M - 1):
+        x = a.copy()
+        x[0, row, 3] = np.nan
+        out = gpu_util.gemm_gemm_f16(x, b0, b1)
+        assert np.all(np.isnan(out[0, row]))
+        keep = np.arange(M) != row
+        np.testing.assert_array_equal(out[:, keep].view(np.uint16), clean[:, keep].view(np.uint16))
