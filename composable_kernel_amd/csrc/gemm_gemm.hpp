@@ -591,12 +591,12 @@ inline bool rows_in_16s(int M, int N, int K, int O, int batch, bool mask_upper)
 // under the triangular mask may have more of them once its chain is long: they start longest first, and the short ones fit in behind. Below
 // the lines in the chain's length the first loads and the merge cost more than the shares give; heads of 65 to 96 in quarters pad to 128. Up
 // to 64 rows of heads of 33 to 64 the choice between 16 and 32 rows stands up to 1025 columns, bit for bit.
-// 1 part (the better of 16 and 32 rows as chosen below) / 2 / 4, us, full: batch x M x N 3 x 3034 x 3034 of heads 32 28.5 / 24.0 / 15.5, 6 x
+// 1 part (16 or 32 rows as rows_in_16s() chooses) / 2 / 4, us, full: batch x M x N 3 x 3034 x 3034 of heads 32 28.5 / 24.0 / 15.5, 6 x
 // 3760 x 1709 / 64 23.7 / 20.7 / 16.5, 14 x 802 x 802 / 64 14.7 / 13.4 / 12.7, 12 x 1275 x 1275 / 80 23.0 / 21.2 / 21.7, 8 x 1676 x 1676 / 128
 // 39.8 / 32.5 / 27.2, 4 x 991 x 3837 / 128 81.2 / 62.1 / 45.6, but 6 x 2806 x 2806 / 64 (264 slabs of 64) 35.4 / 29.4 / 43.1, 8 x 1918 x 490 / 64 9.7 /
 // 10.2 / 9.6, 125 x 70 x 931 / 128 25.2 / 21.2 / 25.7 (two slabs of 64 for one of 128). Causal: 6 x 3772 / 64 44.9 / 37.0 / 28.3 (354 slabs of
 // 64), 25 x 936 / 64 16.3 / 15.0 / 19.7 (375), 15 x 591 / 64 11.0 / 11.4 / 11.8, 6 x 3707 / 128 78.7 / 60.8 / 47.9, 18 x 573 / 128 16.5 / 16.3 / 16.7.
-// Over 340 random problems none of the routes below is slower than one part beyond the noise; 2 parts gave up to 1.34, 4 up to 1.84 times.
+// Of 340 random problems none that takes parts is slower than with one; 2 parts give up to 1.34, 4 up to 1.84 times.
 inline int column_parts(int M, int N, int K, int O, int batch, bool mask_upper)
 {
     const int head     = K > O ? K : O;
