@@ -237,10 +237,6 @@ struct GemmArgs
     uint32_t a_bytes;       // extent of the A / B allocations seen by the buffer resource
     uint32_t b_bytes;
     int tiles_m, tiles_n;
-    // SHORT kernels (one K run, no batch): the tiles of the last round, of fewer rows so that they occupy every CU (short_tail in
-    // tile_launch.hpp): tail_m x tail_n tiles of 2 * tail_h rows from row tail_row0 and column tile tail_col0 on, after
-    // the tiles_m x tiles_n whole ones. tail_m == 0: none.
-    int tail_m, tail_n, tail_row0, tail_col0, tail_h;
     int epi;
     float scale_gemm, scale_relu;
     int nt_store; // stream the C tile past L2 (large outputs)
@@ -259,6 +255,11 @@ struct GemmArgs
     int batch;
     long bsa, bsb, bsc;
     ConvGeom cv;
+    // SHORT kernels (one K run, no batch): the tiles of the last round, of fewer rows so that they occupy every CU (short_tail in
+    // tile_launch.hpp): tail_m x tail_n tiles of 2 * tail_h rows from row tail_row0 and column tile tail_col0 on, after
+    // the tiles_m x tiles_n whole ones. tail_m == 0: none. (At the end: in front of cv, which then
+    // began in another line of the kernel's arguments, they cost every im2col launch 0.2 us.)
+    int tail_m, tail_n, tail_row0, tail_col0, tail_h;
 };
 
 constexpr uint32_t kOutOfRange = 0x80000000u;
