@@ -167,7 +167,8 @@ def time_launches(fn, n_warmup, n_repeat, stream):
 
 def gemm_plan(op, M, N, K, sa=None, sb=None, sc=None, a_layout=ROW_MAJOR, b_layout=COL_MAJOR, epilogue=EPI_PASSTHROUGH,
               batch=1, workspace_bytes=0, instance=INSTANCE_AUTO):
-    """(instance, K runs) a launch of this GEMM would use (ckx_gemm_plan); strides default to the dense ones."""
+    """(instance, K runs) a launch of this GEMM would use (ckx_gemm_plan); strides default to the dense ones. INSTANCE_AUTO: the operands
+    are copied to the workspace first, which only the automatic choice does."""
     sa = sa if sa is not None else (K if a_layout == ROW_MAJOR else M)
     sb = sb if sb is not None else (K if b_layout == COL_MAJOR else N)
     sc = sc if sc is not None else N

@@ -494,6 +494,13 @@ bool packing_pays(int es, int M, int N, int K, bool kmajor)
     return rows * (((long)K * es + 127) / 128) >= 32 * 128 && p.a_bytes < (1l << 31) && p.bytes - p.a_bytes < (1l << 31);
 }
 
+// AUTO copies the operands of this product, which needs the padding instance, to a workspace of ws_bytes bytes (copies end with a line of 16
+// bytes and more)
+bool copies_operands(int es, int M, int N, int K, bool ta, bool tb, long ws_bytes)
+{
+    return packing_pays(es, M, N, K, ta || tb) && ws_bytes >= pack_plan(es, M, N, K).bytes && (!ta || M * es >= 16) && (!tb || N * es >= 16);
+}
+
 // workspace need of the launch plan for this GEMM (0: none)
 long gemm_workspace_bytes(int dt, int M, int N, int K, int instance)
 {
@@ -655,11 +662,11 @@ int run_gemm(int dt, const void* a, const void* b, void* c, int M, int N, int K,
         if(batch > 65535) // (the documented limit; the kernel itself counts batches in its linear grid)
             return fail(CKX_UNSUPPORTED, "the padding instance (operands that are not 16-byte aligned vectors) "
                                          "takes at most 65535 batches per launch");
-        // With a workspace, copies whose rows are whole vectors (a plan query names the padding instance all the same, which takes the operands as they are)
-        const PackPlan p = pack_plan(es, M, N, K);
-        if(instance == CKX_INSTANCE_AUTO && batch == 1 && k_batch == 0 && ws && !(reinterpret_cast<uintptr_t>(ws) & 15) && ws_bytes >= p.bytes &&
-           packing_pays(es, M, N, K, kmajor) && (!ta || M * es >= 16) && (!tb || N * es >= 16))
+        // With a workspace, copies whose rows are whole vectors
+        if(instance == CKX_INSTANCE_AUTO && batch == 1 && k_batch == 0 && ws && !(reinterpret_cast<uintptr_t>(ws) & 15) &&
+           copies_operands(es, M, N, K, ta, tb, ws_bytes))
         {
+            const PackPlan p  = pack_plan(es, M, N, K);
             uint8_t* const to = reinterpret_cast<uint8_t*>(ws);
             const hipError_t e =
                 ckx::launch_gemm_pack(ckx::GemmPack{a, b, to, to + p.a_bytes, es, M, N, K, sa, sb, ta, tb, p.pitch}, (hipStream_t)stream);
@@ -1410,6 +1417,11 @@ const char* ckx_instance_name(int op, int instance)
 {
     static thread_local std::string s;
     const char* fam = family_prefix(op);
+    if(fam && instance == CKX_INSTANCE_AUTO)
+    {
+        s = std::string(fam) + "<auto>";
+        return s.c_str();
+    }
     if(!fam || instance < 0 || instance >= ckx_num_instances(op))
         return nullptr;
     s = std::string(fam) + "<" +
@@ -1475,6 +1487,14 @@ int ckx_gemm_plan(int op, int32_t M, int32_t N, int32_t K, int32_t sa, int32_t s
     if(*instance == kGenericGemmInstance ||
        (*instance == CKX_INSTANCE_AUTO && gemm_needs_generic(dt, M, N, K, sa, sb, ta, tb, epilogue)))
     {
+        const int es = dt == ckx::DT_I8 ? 1 : 2;
+        if(*instance == CKX_INSTANCE_AUTO && batch == 1 && copies_operands(es, M, N, K, ta, tb, workspace_bytes))
+        {
+            // (the instance that runs on the copies refuses the operands themselves: only AUTO makes this launch)
+            const PackPlan p = pack_plan(es, M, N, K);
+            *k_runs          = choose_gemm(dt, M, N, p.K, false, CKX_INSTANCE_AUTO, workspace_bytes - p.bytes, 0, 1).ksplit;
+            return CKX_OK;
+        }
         *instance = kGenericGemmInstance, *k_runs = 1;
         return CKX_OK;
     }

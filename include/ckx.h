@@ -108,7 +108,7 @@ const char* ckx_last_error(void);
  * DeviceOperationInstanceFactory<DeviceOp>::GetInstances() enumerates
  * (library/include/ck/library/tensor_operation_instance/gpu/gemm.hpp:233-379).
  * ckx_instance_name() is the GetTypeString() of that instance
- * (device_gemm_xdl_cshuffle.hpp:655-672). */
+ * (device_gemm_xdl_cshuffle.hpp:655-672), "<family><auto>" for CKX_INSTANCE_AUTO. */
 int ckx_num_instances(int op);
 const char* ckx_instance_name(int op, int instance);
 
@@ -128,8 +128,9 @@ const char* ckx_instance_name(int op, int instance);
  * K-major operand (km / kn) on the tile instances of 64 rows and more, with the PassThrough / requant
  * epilogues. The LAST instance of every GEMM family is the padding instance (any K, M, N, strides and base
  * addresses, all four layouts, every epilogue of the data type: the reference's KPadding / MNKPadding
- * instances, device_gemm_xdl_cshuffle.hpp:99-184) and CKX_INSTANCE_AUTO sends there exactly the problems
- * the vectorised instances refuse, so AUTO supports every shape. This holds for every ckx_gemm_* and
+ * instances, device_gemm_xdl_cshuffle.hpp:99-184) and CKX_INSTANCE_AUTO sends there the problems the vectorised
+ * instances refuse, so AUTO supports every shape -- but for large products whose K is no whole vector and that come
+ * with a workspace: their operands are copied there to rows that are, for the vectorised instances. This holds for every ckx_gemm_* and
  * ckx_batched_gemm_* entry point below. */
 int ckx_gemm_i8_is_supported(int32_t M, int32_t N, int32_t K, int32_t stride_a, int32_t stride_b,
                              int32_t stride_c, int a_layout, int b_layout, int c_layout, int epilogue,
@@ -140,7 +141,7 @@ int ckx_gemm_i8(const void* p_a, const void* p_b, void* p_c, int32_t M, int32_t 
                 void* p_workspace, int64_t workspace_bytes, void* stream);
 /* BaseOperator::GetWorkSpaceSize (device_base.hpp:47): bytes of device scratch with which the
  * launch may cut K into several runs (split-K: problems with too few C tiles to occupy the
- * machine). The workspace is OPTIONAL: with p_workspace == NULL, or fewer bytes than asked for,
+ * machine), or copy operands whose K is no whole vector (large products on CKX_INSTANCE_AUTO). The workspace is OPTIONAL: with p_workspace == NULL, or fewer bytes than asked for,
  * the launch uses a plan that needs none. It needs no initialisation and holds nothing between
  * calls; two launches that share one workspace must not overlap. */
 int64_t ckx_gemm_i8_workspace_bytes(int32_t M, int32_t N, int32_t K, int instance);
@@ -392,7 +393,8 @@ int ckx_batched_gemm_softmax_gemm_f16(const void* p_a, const void* p_b0, const v
  * the instance and the number of K runs that ckx_gemm_* / ckx_batched_gemm_* (op = CKX_OP_GEMM_I8 / _F16 / _BF16) or
  * ckx_conv2d_fwd_* would use for this problem with `workspace_bytes` of 16-byte aligned workspace (0: none).
  * *instance is in / out: CKX_INSTANCE_AUTO asks for the automatic choice, an instance index for that instance's K
- * split. Operand addresses are taken to be 16-byte aligned (a launch sends misaligned ones to the padding
+ * split. CKX_INSTANCE_AUTO comes back where that launch has no index: a GEMM whose operands are copied to the workspace
+ * first (*k_runs: the runs on the copies). Operand addresses are taken to be 16-byte aligned (a launch sends misaligned ones to the padding
  * instance). The automatic choice is a cost model; tests/golden/planner_audit.json holds what it was measured against. */
 int ckx_gemm_plan(int op, int32_t M, int32_t N, int32_t K, int32_t stride_a, int32_t stride_b, int32_t stride_c,
                   int a_layout, int b_layout, int c_layout, int epilogue, int32_t batch, int64_t workspace_bytes,

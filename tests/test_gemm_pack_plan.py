@@ -16,3 +16,26 @@ def test_workspace_for_copies(es, query):
     assert need(2049, 2047, 2047, generic) == 0                                # AUTO only
     split = need(600, 600, 16000, -1)
     assert split > 0 and need(600, 600, 15999, -1) == split + 1200 * 16000 * es # the copies come on top of the K runs' slices
+
+
+@pytest.mark.parametrize("op, es", [(capi.OP_GEMM_I8, 1), (capi.OP_GEMM_F16, 2), (capi.OP_GEMM_BF16, 2)])
+def test_plan_of_a_copied_product(op, es):
+    """The query answers for the launch with copies: no instance index has it, and its K runs are those on the copies."""
+    def plan(M, N, K, ws, **kw):
+        return capi.gemm_plan(op, M, N, K, workspace_bytes=ws, **kw)
+    generic = capi.lib().ckx_num_instances(op) - 1
+    M, N, K = 2049, 2047, 2047
+    copies = (M + N) * 2048 * es
+    assert plan(M, N, K, copies) == (capi.INSTANCE_AUTO, 1)
+    assert plan(M, N, K, copies - 1) == plan(M, N, K, 0) == (generic, 1)        # no room for both copies
+    assert plan(M, N, K, 1 << 30, instance=generic) == (generic, 1)            # as asked for
+    assert plan(M, N, K, 1 << 30, batch=2, sa=K, sb=K) == (generic, 1)          # batches are not copied
+    assert plan(64, 3001, 2049, 1 << 30) == (generic, 1)                       # little work
+    kn = dict(b_layout=capi.ROW_MAJOR)
+    assert plan(2049, 2047, 1023, 1 << 30, **kn) == (generic, 1) and plan(2049, 2047, 2047, 1 << 30, **kn)[0] == capi.INSTANCE_AUTO
+    # what is left of the workspace holds the K runs' slices, or not
+    copies, room = 1200 * 16000 * es, 1 << 28
+    runs = plan(600, 600, 16000, room)[1]
+    assert runs > 1
+    assert plan(600, 600, 15999, copies + room) == (capi.INSTANCE_AUTO, runs) and plan(600, 600, 15999, copies) == (capi.INSTANCE_AUTO, 1)
+    assert capi.lib().ckx_instance_name(op, capi.INSTANCE_AUTO).endswith(b"<auto>")
