@@ -29,7 +29,7 @@ SYMBOLS = [
     "ckx_gemm_f16_is_supported", "ckx_gemm_f16", "ckx_gemm_f16_workspace_bytes",
     "ckx_gemm_bf16_is_supported", "ckx_gemm_bf16", "ckx_gemm_bf16_workspace_bytes",
     "ckx_batched_gemm_is_supported", "ckx_batched_gemm_i8", "ckx_batched_gemm_f16",
-    "ckx_gemm_splitk_workspace_bytes", "ckx_gemm_i8_splitk", "ckx_gemm_f16_splitk", "ckx_gemm_i8_splitk_noalloc",
+    "ckx_gemm_workspace_bytes", "ckx_gemm_splitk_workspace_bytes", "ckx_gemm_i8_splitk", "ckx_gemm_f16_splitk", "ckx_gemm_i8_splitk_noalloc",
     "ckx_gemm_f16_multiple_d_is_supported", "ckx_gemm_f16_multiple_d", "ckx_gemm_f16_bilinear", "ckx_conv2d_fwd_bias_activation_f16",
     "ckx_gemm_i8_multiple_d_is_supported", "ckx_gemm_i8_multiple_d", "ckx_conv2d_fwd_i8_multiple_d",
     "ckx_conv2d_fwd_is_supported", "ckx_conv2d_fwd_i8", "ckx_conv2d_fwd_f16", "ckx_conv2d_fwd_workspace_bytes",
@@ -99,6 +99,8 @@ def lib():
     for fn in (L.ckx_gemm_i8_workspace_bytes, L.ckx_gemm_f16_workspace_bytes, L.ckx_gemm_bf16_workspace_bytes):
         fn.restype = i64
         fn.argtypes = [i32, i32, i32, C.c_int]
+    L.ckx_gemm_workspace_bytes.restype = i64
+    L.ckx_gemm_workspace_bytes.argtypes = [C.c_int, i32, i32, i32] + [C.c_int] * 3
     L.ckx_gemm_f16_is_supported.argtypes = shape + [C.c_int]
     L.ckx_gemm_f16.argtypes = [vp, vp, vp] + shape + [C.c_int, vp, i64, vp]
     L.ckx_gemm_bf16_is_supported.argtypes = shape + [C.c_int]

@@ -502,10 +502,10 @@ bool copies_operands(int es, int M, int N, int K, bool ta, bool tb, long ws_byte
 }
 
 // workspace need of the launch plan for this GEMM (0: none)
-long gemm_workspace_bytes(int dt, int M, int N, int K, int instance)
+long gemm_workspace_bytes(int dt, int M, int N, int K, int instance, bool kmajor = false)
 {
     const int es = dt == ckx::DT_I8 ? 1 : 2;
-    if(M > 0 && N > 0 && instance == CKX_INSTANCE_AUTO && packing_pays(es, M, N, K, false)) // (K-major operands: fewer problems, the same copies)
+    if(M > 0 && N > 0 && instance == CKX_INSTANCE_AUTO && packing_pays(es, M, N, K, kmajor))
     {
         const PackPlan p = pack_plan(es, M, N, K);
         return p.bytes + gemm_workspace_bytes(dt, M, N, p.K, instance);
@@ -1456,6 +1456,14 @@ int ckx_gemm_i8(const void* a, const void* b, void* c, int32_t M, int32_t N, int
 {
     return run_gemm(ckx::DT_I8, a, b, c, M, N, K, sa, sb, sc, al, bl, cl, epilogue, scale_gemm, scale_relu,
                     instance, workspace, workspace_bytes, stream);
+}
+
+int64_t ckx_gemm_workspace_bytes(int op, int32_t M, int32_t N, int32_t K, int a_layout, int b_layout, int instance)
+{
+    if(op != CKX_OP_GEMM_I8 && op != CKX_OP_GEMM_F16 && op != CKX_OP_GEMM_BF16)
+        return 0;
+    return gemm_workspace_bytes(op == CKX_OP_GEMM_I8 ? ckx::DT_I8 : op == CKX_OP_GEMM_BF16 ? ckx::DT_BF16 : ckx::DT_F16, M, N, K, instance,
+                                a_layout == CKX_COL_MAJOR || b_layout == CKX_ROW_MAJOR);
 }
 
 int ckx_set_big_tile_waves(int waves)

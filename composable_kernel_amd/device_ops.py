@@ -217,7 +217,7 @@ class DeviceGemmInt8(_DeviceGemm):
                                                    *self.layouts, a.c_op.epilogue, self.instance)
 
     def GetWorkSpaceSize(self, a):
-        return int(capi.lib().ckx_gemm_i8_workspace_bytes(a.M, a.N, a.K, self.instance))
+        return int(capi.lib().ckx_gemm_workspace_bytes(capi.OP_GEMM_I8, a.M, a.N, a.K, *self.layouts[:2], self.instance))
 
     def _launch(self, a, stream):
         return capi.lib().ckx_gemm_i8(a.p_a, a.p_b, a.p_c, a.M, a.N, a.K, a.StrideA, a.StrideB, a.StrideC,
@@ -238,7 +238,7 @@ class DeviceGemmF16(_DeviceGemm):
                                                     *self.layouts, self.instance)
 
     def GetWorkSpaceSize(self, a):
-        return int(capi.lib().ckx_gemm_f16_workspace_bytes(a.M, a.N, a.K, self.instance))
+        return int(capi.lib().ckx_gemm_workspace_bytes(capi.OP_GEMM_F16, a.M, a.N, a.K, *self.layouts[:2], self.instance))
 
     def _launch(self, a, stream):
         return capi.lib().ckx_gemm_f16(a.p_a, a.p_b, a.p_c, a.M, a.N, a.K, a.StrideA, a.StrideB, a.StrideC,
@@ -307,7 +307,7 @@ class DeviceGemmBF16(_DeviceGemm):
                                                      *self.layouts, self.instance)
 
     def GetWorkSpaceSize(self, a):
-        return int(capi.lib().ckx_gemm_bf16_workspace_bytes(a.M, a.N, a.K, self.instance))
+        return int(capi.lib().ckx_gemm_workspace_bytes(capi.OP_GEMM_BF16, a.M, a.N, a.K, *self.layouts[:2], self.instance))
 
     def _launch(self, a, stream):
         return capi.lib().ckx_gemm_bf16(a.p_a, a.p_b, a.p_c, a.M, a.N, a.K, a.StrideA, a.StrideB, a.StrideC,
@@ -386,7 +386,7 @@ class DeviceGemmMultipleDF16(BaseOperator):
             a.c_op.cde_epilogue, self.instance)
 
     def GetWorkSpaceSize(self, a):
-        return int(capi.lib().ckx_gemm_f16_workspace_bytes(a.M, a.N, a.K, self.instance))
+        return int(capi.lib().ckx_gemm_workspace_bytes(capi.OP_GEMM_F16, a.M, a.N, a.K, *self.layouts[:2], self.instance))
 
     def _launch(self, a, stream):
         if isinstance(a.c_op, Bilinear):
@@ -428,7 +428,7 @@ class DeviceGemmMultipleDInt8(BaseOperator):
             self.instance)
 
     def GetWorkSpaceSize(self, a):
-        return int(capi.lib().ckx_gemm_i8_workspace_bytes(a.M, a.N, a.K, self.instance))
+        return int(capi.lib().ckx_gemm_workspace_bytes(capi.OP_GEMM_I8, a.M, a.N, a.K, *self.layouts[:2], self.instance))
 
     def _launch(self, a, stream):
         return capi.lib().ckx_gemm_i8_multiple_d(

@@ -545,9 +545,8 @@ struct DeviceGemmMfma : public DeviceGemm<ALayout, BLayout, CLayout, ADataType, 
     }
     static int64_t WorkSpaceBytes(const Argument& a, int inst)
     {
-        return is_i8     ? ckx_gemm_i8_workspace_bytes(a.M, a.N, a.K, inst)
-               : is_bf16 ? ckx_gemm_bf16_workspace_bytes(a.M, a.N, a.K, inst)
-                         : ckx_gemm_f16_workspace_bytes(a.M, a.N, a.K, inst);
+        return ckx_gemm_workspace_bytes(is_i8 ? CKX_OP_GEMM_I8 : is_bf16 ? CKX_OP_GEMM_BF16 : CKX_OP_GEMM_F16, a.M, a.N, a.K, ALayout::code,
+                                        BLayout::code, inst);
     }
     size_t GetWorkSpaceSize(const BaseArgument* p) const override
     {
@@ -978,6 +977,10 @@ struct DeviceGemmMultipleDMfma
         index_t M, N, K, StrideA, StrideB, StrideD0, StrideD1, StrideE;
         CDEElementwiseOperation cde_element_op_;
     };
+    static int64_t WorkSpaceBytes(const Argument& a, int inst)
+    {
+        return ckx_gemm_workspace_bytes(CKX_OP_GEMM_F16, a.M, a.N, a.K, ALayout::code, BLayout::code, inst);
+    }
     static int Supported(const Argument& a, int inst)
     {
         return ckx_gemm_f16_multiple_d_is_supported(a.M, a.N, a.K, a.StrideA, a.StrideB, a.StrideD0, a.StrideD1,
@@ -986,7 +989,7 @@ struct DeviceGemmMultipleDMfma
     }
     static int Launch(const Argument& a, int inst, void* stream)
     {
-        const int64_t ws_bytes = a.p_workspace_ ? ckx_gemm_f16_workspace_bytes(a.M, a.N, a.K, inst) : 0;
+        const int64_t ws_bytes = a.p_workspace_ ? WorkSpaceBytes(a, inst) : 0;
         if constexpr(is_bilinear)
             return ckx_gemm_f16_bilinear(a.p_a, a.p_b, a.p_d0, a.p_e, a.M, a.N, a.K, a.StrideA, a.StrideB, a.StrideD0,
                                          a.StrideE, ALayout::code, BLayout::code, DELayout::code,
@@ -1023,7 +1026,7 @@ struct DeviceGemmMultipleDMfma
     size_t GetWorkSpaceSize(const BaseArgument* p) const override
     {
         const auto* a = dynamic_cast<const Argument*>(p);
-        return a ? (size_t)ckx_gemm_f16_workspace_bytes(a->M, a->N, a->K, instance_) : 0;
+        return a ? (size_t)WorkSpaceBytes(*a, instance_) : 0;
     }
     std::unique_ptr<BaseArgument>
     MakeArgumentPointer(const void* p_a, const void* p_b, std::array<const void*, NumDTensor> p_ds, void* p_e,
@@ -1065,6 +1068,10 @@ struct DeviceGemmMultipleDInt8Mfma
         void* p_e;
         index_t M, N, K, StrideA, StrideB, StrideD0, StrideE;
     };
+    static int64_t WorkSpaceBytes(const Argument& a, int inst)
+    {
+        return ckx_gemm_workspace_bytes(CKX_OP_GEMM_I8, a.M, a.N, a.K, ALayout::code, BLayout::code, inst);
+    }
     static int Supported(const Argument& a, int inst)
     {
         return ckx_gemm_i8_multiple_d_is_supported(a.M, a.N, a.K, a.StrideA, a.StrideB, a.StrideD0, a.StrideE,
@@ -1072,7 +1079,7 @@ struct DeviceGemmMultipleDInt8Mfma
     }
     static int Launch(const Argument& a, int inst, void* stream)
     {
-        const int64_t ws_bytes = a.p_workspace_ ? ckx_gemm_i8_workspace_bytes(a.M, a.N, a.K, inst) : 0;
+        const int64_t ws_bytes = a.p_workspace_ ? WorkSpaceBytes(a, inst) : 0;
         return ckx_gemm_i8_multiple_d(a.p_a, a.p_b, a.p_d0, a.p_e, a.M, a.N, a.K, a.StrideA, a.StrideB, a.StrideD0,
                                       a.StrideE, ALayout::code, BLayout::code, DELayout::code, cde_code, inst,
                                       a.p_workspace_, ws_bytes, stream);
@@ -1099,7 +1106,7 @@ struct DeviceGemmMultipleDInt8Mfma
     size_t GetWorkSpaceSize(const BaseArgument* p) const override
     {
         const auto* a = dynamic_cast<const Argument*>(p);
-        return a ? (size_t)ckx_gemm_i8_workspace_bytes(a->M, a->N, a->K, instance_) : 0;
+        return a ? (size_t)WorkSpaceBytes(*a, instance_) : 0;
     }
     std::unique_ptr<BaseArgument>
     MakeArgumentPointer(const void* p_a, const void* p_b, std::array<const void*, 1> p_ds, void* p_e, index_t M,

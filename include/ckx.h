@@ -143,8 +143,11 @@ int ckx_gemm_i8(const void* p_a, const void* p_b, void* p_c, int32_t M, int32_t 
  * launch may cut K into several runs (split-K: problems with too few C tiles to occupy the
  * machine), or copy operands whose K is no whole vector (large products on CKX_INSTANCE_AUTO). The workspace is OPTIONAL: with p_workspace == NULL, or fewer bytes than asked for,
  * the launch uses a plan that needs none. It needs no initialisation and holds nothing between
- * calls; two launches that share one workspace must not overlap. */
+ * calls; two launches that share one workspace must not overlap. The queries of one data type answer for A row-major,
+ * B column-major, which is enough for every layout; ckx_gemm_workspace_bytes (op = CKX_OP_GEMM_I8 / _F16 /
+ * _BF16) answers for the layouts: fewer products with a K-major operand are copied. */
 int64_t ckx_gemm_i8_workspace_bytes(int32_t M, int32_t N, int32_t K, int instance);
+int64_t ckx_gemm_workspace_bytes(int op, int32_t M, int32_t N, int32_t K, int a_layout, int b_layout, int instance);
 
 /* ---- fp16 GEMM:  C = half(A * B), fp32 accumulation -----------------------
  * Replaces DeviceGemm<..., half_t, half_t, half_t, PassThrough x3>

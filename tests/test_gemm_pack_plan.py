@@ -1,6 +1,7 @@
 """Which GEMMs ask for a workspace for copies of their operands: K no whole number of 16-byte vectors, and work enough. Runs on the CPU."""
 import pytest
 
+import composable_kernel_amd as ck
 from composable_kernel_amd import capi
 
 
@@ -39,3 +40,23 @@ def test_plan_of_a_copied_product(op, es):
     assert runs > 1
     assert plan(600, 600, 15999, copies + room) == (capi.INSTANCE_AUTO, runs) and plan(600, 600, 15999, copies) == (capi.INSTANCE_AUTO, 1)
     assert capi.lib().ckx_instance_name(op, capi.INSTANCE_AUTO).endswith(b"<auto>")
+
+
+@pytest.mark.parametrize("device_op, functor", [
+    (ck.DeviceGemmInt8, None), (ck.DeviceGemmF16, None), (ck.DeviceGemmBF16, None), (ck.DeviceGemmMultipleDF16, ck.Bilinear(0.5, 2.0)),
+    (ck.DeviceGemmMultipleDInt8, ck.ActivationMul2Clamp(ck.Relu()))])
+def test_workspace_of_k_major_operands(device_op, functor):
+    """The operators ask for room for copies where their layouts are copied, and for none where they are not."""
+    def need(al, bl, M, N, K):
+        op = device_op(ALayout=al, BLayout=bl)
+        a, b = (M if al is ck.ColumnMajor else K), (N if bl is ck.RowMajor else K)
+        if functor is None:
+            return op.GetWorkSpaceSize(op.MakeArgumentPointer(0, 0, 0, M, N, K, a, b, N))
+        return op.GetWorkSpaceSize(op.MakeArgumentPointer(0, 0, [0], 0, M, N, K, a, b, [0], N, None, None, functor))
+    row, col = ck.RowMajor, ck.ColumnMajor
+    es = 1 if "Int8" in device_op.__name__ else 2
+    copies = lambda M, N, K: (M + N) * -(-K * es // 128) * 128
+    assert need(row, col, 2049, 2047, 1023) == copies(2049, 2047, 1023)
+    for al, bl in ((row, row), (col, col), (col, row)):
+        assert need(al, bl, 2049, 2047, 1023) == 0                             # 8.6e9 operations
+        assert need(al, bl, 2049, 2047, 2047) == copies(2049, 2047, 2047)      # 17e9
