@@ -969,7 +969,7 @@ double conv_tile_us(const Plan& pl, long M, int N, int kbytes)
 // the windowed kernel's shape for a conv with unit strides that the tile kernel would run by `pl`, and its box in `w`; -1: the tile kernel
 int conv_window_shape(int dt, ckx::ConvWindowArgs& w, const Plan& pl, long M)
 {
-    if(pl.ksplit != 1 || w.taps < 9)
+    if(pl.ksplit != 1)
         return -1;
     return ckx::choose_conv_window(dt, w, conv_tile_us(pl, M, w.K, w.taps * w.pix_bytes));
 }

@@ -54,8 +54,8 @@ double plan_conv_window(int dt, int shape, ConvWindowArgs& a)
     const Shape& sh = shape_of(dt, shape);
     a.total         = a.taps * a.units;
     a.nk            = (a.total + 7) / 8;
-    // (entries of the K table have 16 bits for the unit of a weight row; a chunk's K tiles have to outlast the one they share with the next)
-    if(a.taps < 8 || a.total >= 65536 || a.nk < 4)
+    // (nine taps: a 3 x 3 filter is the smallest that this was measured on; entries of the K table have 16 bits for the unit of a weight row; a chunk's K tiles have to outlast the one they share with the next)
+    if(a.taps < 9 || a.total >= 65536 || a.nk < 4)
         return -1.0;
     const int fz = a.taps / (a.Y * a.X), outer = a.three_d ? a.Do : a.N, planes = (a.units + 1) / 2;
     const int space = (kLdsCu - sh.fixed_lds - (a.nk * 32 + 255) / 256 * 256) / 2048; // KB of a window buffer

@@ -1,4 +1,4 @@
-// Conv forward with the input under a box of output pixels in LDS: 2-D and 3-D, NHWC / NDHWC, unit strides, filters of eight and more taps,
+// Conv forward with the input under a box of output pixels in LDS: 2-D and 3-D, NHWC / NDHWC, unit strides, filters of nine and more taps,
 // fp16 and int8, gfx950.
 //
 // Takes the place of the same reference kernels as the tile kernel's im2col view

@@ -53,4 +53,6 @@ def test_the_line():
     assert at(138.0, *few_channels) == 0 and at(90.0, *few_channels) == -1
     assert at(290.0, (43, 43, 43), 4, 176, 32, (3, 3, 3), (1, 1, 1), (1, 1, 1)) == 2
     assert at(1e9, (32, 32), 16, 64, 64, (1, 7), (1, 1), (0, 3)) == -1       # too few taps
+    assert at(1e9, (32, 32), 16, 128, 64, (2, 4), (1, 1), (0, 1)) == -1 and at(1e9, (32, 32), 16, 128, 64, (1, 9), (1, 1), (0, 4)) >= 0
+    assert at(1e9, (16, 16, 16), 4, 128, 64, (2, 2, 2), (1, 1, 1), (1, 1, 1)) == -1
     assert at(13.9, (8, 8), 1, 32, 32, (3, 3), (1, 1), (1, 1)) == -1          # small calls are not searched
