@@ -212,6 +212,11 @@ Plan make_plan(long M, int N, int kbytes, int only_tile, long workspace_bytes, i
     const long cus  = num_cus(); // (the time constants below were measured on a 256-CU part)
     const int nk    = (kbytes + 127) / 128 > 0 ? (kbytes + 127) / 128 : 1;
     const int force = k_batch > 0 ? splitk_runs(kbytes, k_batch) : force_ksplit();
+    if(M <= 0 || N <= 0) // (a plan query for an empty problem: no tiles to rate)
+    {
+        best.tile = only_tile >= 0 ? only_tile : 0, best.nk_per = nk;
+        return best;
+    }
     for(int i = 0; i < kNumTiles; ++i)
     {
         if(only_tile >= 0 && i != only_tile)

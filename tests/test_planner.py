@@ -134,3 +134,25 @@ def test_short_conv_loops_with_d_operands_take_the_128x128_tile():
         ho = (hw - 1) // 2 + 1
         d = capi.Conv2dDesc(N, K, C, hw, hw, 1, 1, ho, ho, 2, 2, 1, 1, 0, 0, 0, 0)
         assert capi.conv2d_fwd_plan(capi.OP_CONV2D_FWD_F16, d, epi, WORKSPACE) == (2, 1)
+
+
+def test_plan_of_an_empty_problem():
+    """Supported, and launched as nothing: the queries answer with one K run (and some instance) too. In a process of its own, which a
+    division by the number of tiles would end."""
+    import subprocess
+    import sys
+    code = """
+from composable_kernel_amd import capi
+for op in (capi.OP_GEMM_I8, capi.OP_GEMM_F16, capi.OP_GEMM_BF16):
+    for M, N in ((0, 128), (128, 0), (0, 0), (1000, 0)):
+        for kw in (dict(), dict(workspace_bytes=1 << 20), dict(b_layout=capi.ROW_MAJOR), dict(instance=3)):
+            assert capi.gemm_plan(op, M, N, 128, **kw)[1] == 1
+for stride in (1, 2):
+    for N, K, Hi, Ho, pad in ((0, 64, 8, 8 // stride, 1), (4, 0, 8, 8 // stride, 1), (4, 64, 3 - stride, 0, 0)):
+        d = capi.Conv2dDesc(N, K, 64, Hi, 8, 3, 3, Ho, 8 // stride, stride, stride, 1, 1, pad, 1, pad, 1)
+        for op in (capi.OP_CONV2D_FWD_I8, capi.OP_CONV2D_FWD_F16):
+            for inst in (-1, 3):
+                assert capi.conv2d_fwd_plan(op, d, instance=inst, workspace_bytes=1 << 20)[1] == 1
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(HERE), capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
