@@ -595,7 +595,7 @@ def resnet50_sweep(args):
         epi = {None: capi.EPI_REQUANT_RND if w["dtype"] == "i8" else capi.EPI_PASSTHROUGH,
                "bias_relu": capi.EPI_ADD_RELU, "bias_relu_add": capi.EPI_ADD_RELU_ADD}[w["fused"]]
         inst, runs = capi.conv2d_fwd_plan(op, desc, epi, 1 << 30)
-        name = L.ckx_instance_name(op, inst).decode()
+        name = "MI355X_Mfma16_Window" if inst == capi.INSTANCE_AUTO else L.ckx_instance_name(op, inst).decode()
         frac = max(x["mfma_frac"], x["hbm_frac"])
         row = {"workload": w["name"], "dtype": w["dtype"], "op": "conv_fwd" + ("_" + w["fused"] if w["fused"] else ""),
                "instance": name, "k_runs": runs, "us": round(x["ms"] * 1e3, 2), "value": round(x["tput"], 1),

@@ -181,6 +181,7 @@ def gemm_plan(op, M, N, K, sa=None, sb=None, sc=None, a_layout=ROW_MAJOR, b_layo
 
 
 def conv2d_fwd_plan(op, desc, epilogue=EPI_PASSTHROUGH, workspace_bytes=0, instance=INSTANCE_AUTO):
+    """As gemm_plan, for a convolution (ckx_conv2d_fwd_plan); INSTANCE_AUTO: the windowed kernel."""
     inst, runs = C.c_int(instance), C.c_int(0)
     check(lib().ckx_conv2d_fwd_plan(op, C.byref(desc), epilogue, int(workspace_bytes), C.byref(inst), C.byref(runs)))
     return inst.value, runs.value

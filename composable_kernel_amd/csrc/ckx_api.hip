@@ -962,6 +962,8 @@ double conv_tile_us(const Plan& pl, long M, int N, int kbytes)
     const TileInstance& t = kTiles[pl.tile];
     const long cus = num_cus(), units = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * pl.ksplit;
     const int nst  = t.lds / ((t.bm + t.bn) * 128);
+    if(units < 1) // (a plan query for an empty layer)
+        return 0.0;
     long per_cu    = 160 * 1024 / t.lds < 2048 / t.threads ? 160 * 1024 / t.lds : 2048 / t.threads;
     per_cu         = per_cu > 4 ? 4 : per_cu;
     per_cu         = per_cu * cus > units ? (units + cus - 1) / cus : per_cu;
@@ -971,12 +973,30 @@ double conv_tile_us(const Plan& pl, long M, int N, int kbytes)
     const double iter_us = mfma_us > load_us ? (mfma_us > floor_us ? mfma_us : floor_us) : (load_us > floor_us ? load_us : floor_us);
     return rounds * (iter_us * pl.nk_per + 6.0 / per_cu + 2.0);
 }
-// the windowed kernel's shape for a conv with unit strides that the tile kernel would run by `pl`, and its box in `w`; -1: the tile kernel
-int conv_window_shape(int dt, ckx::ConvWindowArgs& w, const Plan& pl, long M)
+// The windowed kernel's shape for a layer that the tile kernel would run by `pl`, and the layer and its box in `w` (operands and epilogue are
+// the launcher's); -1: the tile kernel. Two dimensions, and three convolved ones.
+int conv_window_shape(int es, const ckx_conv2d_desc* d, const Plan& pl, ckx::ConvWindowArgs& w)
 {
-    if(pl.ksplit != 1)
+    if(d->stride_h != 1 || d->stride_w != 1 || pl.ksplit != 1)
         return -1;
-    return ckx::choose_conv_window(dt, w, conv_tile_us(pl, M, w.K, w.taps * w.pix_bytes));
+    std::memset(&w, 0, sizeof(w));
+    w.N = d->N, w.Di = 1, w.Hi = d->Hi, w.Wi = d->Wi, w.Do = 1, w.Ho = d->Ho, w.Wo = d->Wo, w.K = d->K;
+    w.pix_bytes = d->C * es, w.units = w.pix_bytes / 16, w.Y = d->Y, w.X = d->X, w.taps = d->Y * d->X;
+    w.dD = 1, w.dH = d->dilation_h, w.dW = d->dilation_w, w.pT = d->pad_top, w.pL = d->pad_left;
+    return ckx::choose_conv_window(es == 1 ? ckx::DT_I8 : ckx::DT_F16, w,
+                                   conv_tile_us(pl, (long)d->N * d->Ho * d->Wo, w.K, w.taps * w.pix_bytes));
+}
+int conv_window_shape(int es, const ckx_convnd_desc* d, const Plan& pl, ckx::ConvWindowArgs& w)
+{
+    if(d->stride[0] != 1 || d->stride[1] != 1 || d->stride[2] != 1 || pl.ksplit != 1)
+        return -1;
+    std::memset(&w, 0, sizeof(w));
+    w.three_d = 1, w.N = d->N, w.Di = d->in[0], w.Hi = d->in[1], w.Wi = d->in[2], w.Do = d->out[0], w.Ho = d->out[1], w.Wo = d->out[2], w.K = d->K;
+    w.pix_bytes = d->C * es, w.units = w.pix_bytes / 16, w.Y = d->filter[1], w.X = d->filter[2];
+    w.taps = d->filter[0] * d->filter[1] * d->filter[2], w.dD = d->dilation[0], w.dH = d->dilation[1], w.dW = d->dilation[2];
+    w.pF = d->pad_left[0], w.pT = d->pad_left[1], w.pL = d->pad_left[2];
+    return ckx::choose_conv_window(es == 1 ? ckx::DT_I8 : ckx::DT_F16, w,
+                                   conv_tile_us(pl, (long)d->N * w.Do * w.Ho * w.Wo, w.K, w.taps * w.pix_bytes));
 }
 
 long conv_workspace_bytes(int op, const ckx_conv2d_desc* d, int instance)
@@ -1172,22 +1192,15 @@ int run_conv(int op, const void* in, const void* wei, void* out, const ckx_conv2
     g.ksplit = pl.ksplit;
     g.nk_per = pl.nk_per;
     g.ws     = ws;
-    if(instance == CKX_INSTANCE_AUTO && d->stride_h == 1 && d->stride_w == 1 && dops.ldd0 == 0)
+    ckx::ConvWindowArgs w;
+    const int window = instance == CKX_INSTANCE_AUTO && dops.ldd0 == 0 ? conv_window_shape(es, d, pl, w) : -1;
+    if(window >= 0)
     {
-        ckx::ConvWindowArgs w;
-        std::memset(&w, 0, sizeof(w));
         w.in = in, w.wei = wei, w.out = out, w.d0 = g.d0, w.d1 = g.d1, w.ldd1 = g.ldd1;
         w.in_bytes = g.a_bytes, w.wei_bytes = g.b_bytes;
-        w.N = d->N, w.Di = 1, w.Hi = d->Hi, w.Wi = d->Wi, w.Do = 1, w.Ho = d->Ho, w.Wo = d->Wo, w.K = N;
-        w.pix_bytes = d->C * es, w.units = w.pix_bytes / 16, w.Y = d->Y, w.X = d->X, w.taps = d->Y * d->X;
-        w.dD = 1, w.dH = d->dilation_h, w.dW = d->dilation_w, w.pT = d->pad_top, w.pL = d->pad_left;
         w.epi = epi, w.scale_gemm = sg, w.scale_relu = sr, w.nt_store = g.nt_store;
-        const int dt = es == 1 ? ckx::DT_I8 : ckx::DT_F16, shape = conv_window_shape(dt, w, pl, M);
-        if(shape >= 0)
-        {
-            hipError_t e = ckx::launch_conv_window(dt, shape, w, (hipStream_t)stream);
-            return e == hipSuccess ? CKX_OK : hip_fail(e, t.name);
-        }
+        hipError_t e = ckx::launch_conv_window(es == 1 ? ckx::DT_I8 : ckx::DT_F16, window, w, (hipStream_t)stream);
+        return e == hipSuccess ? CKX_OK : hip_fail(e, t.name);
     }
     const bool fused = f16_fused(epi) && g.ksplit == 1;
     // A a K tile further ahead (AHEAD in gemm_tile.hpp): strides that leave a pixel to less than about three of the filter's taps, so that
@@ -1372,22 +1385,14 @@ int run_convnd(int op, const void* in, const void* wei, void* out, const ckx_con
         hipError_t e = ckx::launch_generic(es == 1 ? ckx::DT_I8 : ckx::DT_F16, 2, g, lay, (hipStream_t)stream);
         return e == hipSuccess ? CKX_OK : hip_fail(e, kGenericName);
     }
-    if(instance == CKX_INSTANCE_AUTO && d->stride[0] == 1 && d->stride[1] == 1 && d->stride[2] == 1)
+    ckx::ConvWindowArgs w;
+    const int window = instance == CKX_INSTANCE_AUTO ? conv_window_shape(es, d, pl, w) : -1;
+    if(window >= 0)
     {
-        ckx::ConvWindowArgs w;
-        std::memset(&w, 0, sizeof(w));
         w.in = in, w.wei = wei, w.out = out, w.in_bytes = g.a_bytes, w.wei_bytes = g.b_bytes;
-        w.three_d = 1, w.N = d->N, w.Di = d->in[0], w.Hi = d->in[1], w.Wi = d->in[2], w.Do = d->out[0], w.Ho = d->out[1], w.Wo = d->out[2], w.K = N;
-        w.pix_bytes = d->C * es, w.units = w.pix_bytes / 16, w.Y = d->filter[1], w.X = d->filter[2];
-        w.taps = d->filter[0] * d->filter[1] * d->filter[2], w.dD = d->dilation[0], w.dH = d->dilation[1], w.dW = d->dilation[2];
-        w.pF = d->pad_left[0], w.pT = d->pad_left[1], w.pL = d->pad_left[2];
         w.epi = epi, w.scale_gemm = sg, w.scale_relu = sr, w.nt_store = g.nt_store;
-        const int dt = es == 1 ? ckx::DT_I8 : ckx::DT_F16, shape = conv_window_shape(dt, w, pl, M);
-        if(shape >= 0)
-        {
-            hipError_t e = ckx::launch_conv_window(dt, shape, w, (hipStream_t)stream);
-            return e == hipSuccess ? CKX_OK : hip_fail(e, t.name);
-        }
+        hipError_t e = ckx::launch_conv_window(es == 1 ? ckx::DT_I8 : ckx::DT_F16, window, w, (hipStream_t)stream);
+        return e == hipSuccess ? CKX_OK : hip_fail(e, t.name);
     }
     const bool pairs = pl.tile == ckx::kFourStageTile && ckx::row_pairs_pay(M, N, g.ksplit);
     if(pairs)
@@ -1405,6 +1410,18 @@ int run_convnd(int op, const void* in, const void* wei, void* out, const ckx_con
 }
 
 } // namespace
+
+namespace ckx {
+// the windowed kernel's shape that AUTO takes for a layer with three convolved dimensions and no workspace; -1: the tile kernel
+int auto_conv3d_window(int op, const ckx_convnd_desc* d)
+{
+    const int es  = op == CKX_OP_CONV2D_FWD_I8 ? 1 : 2;
+    const Plan pl = make_plan((long)d->N * d->out[0] * d->out[1] * d->out[2], d->K, d->filter[0] * d->filter[1] * d->filter[2] * d->C * es,
+                              CKX_INSTANCE_AUTO, 0, 0, false, true);
+    ConvWindowArgs w;
+    return conv_window_shape(es, d, pl, w);
+}
+} // namespace ckx
 
 extern "C" {
 
@@ -1554,6 +1571,9 @@ int ckx_conv2d_fwd_plan(int op, const ckx_conv2d_desc* d, int epilogue, int64_t 
     {
         const Plan pl = make_plan((long)d->N * d->Ho * d->Wo, d->K, d->Y * d->X * d->C * es, *instance,
                                   workspace_bytes > 0 ? workspace_bytes : 0, 0, false, true, d->Y * d->X);
+        ckx::ConvWindowArgs w;
+        if(*instance == CKX_INSTANCE_AUTO && conv_window_shape(es, d, pl, w) >= 0)
+            return CKX_OK; // (the windowed kernel has no index: only AUTO makes this launch)
         *instance = pl.tile, *k_runs = pl.ksplit;
     }
     return CKX_OK;

@@ -56,3 +56,22 @@ def test_the_line():
     assert at(1e9, (32, 32), 16, 128, 64, (2, 4), (1, 1), (0, 1)) == -1 and at(1e9, (32, 32), 16, 128, 64, (1, 9), (1, 1), (0, 4)) >= 0
     assert at(1e9, (16, 16, 16), 4, 128, 64, (2, 2, 2), (1, 1, 1), (1, 1, 1)) == -1
     assert at(13.9, (8, 8), 1, 32, 32, (3, 3), (1, 1), (1, 1)) == -1          # small calls are not searched
+
+
+def test_plan_query_of_a_windowed_layer():
+    """No instance index makes that launch: the query answers with the automatic choice. By index, with a K split and for layers past the
+    lines it answers with the tile instance."""
+    from composable_kernel_amd import capi
+
+    def query(N, C, K, hw, stride=1, op=capi.OP_CONV2D_FWD_F16, **kw):
+        ho = (hw - 1) // stride + 1
+        return capi.conv2d_fwd_plan(op, capi.Conv2dDesc(N, K, C, hw, hw, 3, 3, ho, ho, stride, stride, 1, 1, 1, 1, 1, 1), **kw)
+    assert query(48, 88, 24, 57) == (capi.INSTANCE_AUTO, 1) and query(48, 88, 24, 57, instance=7) == (7, 1)
+    assert query(32, 176, 24, 57, op=capi.OP_CONV2D_FWD_I8, instance=7) == (7, 1) and query(32, 176, 24, 57, op=capi.OP_CONV2D_FWD_I8) == (capi.INSTANCE_AUTO, 1)
+    assert query(48, 88, 24, 57, stride=2)[0] >= 0 and query(1, 88, 24, 57)[0] >= 0
+    capi.lib().ckx_set_forced_k_runs(2)
+    try:
+        inst, runs = query(48, 88, 24, 57, workspace_bytes=1 << 30)
+        assert inst >= 0 and runs == 2
+    finally:
+        capi.lib().ckx_set_forced_k_runs(0)
