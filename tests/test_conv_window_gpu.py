@@ -88,14 +88,63 @@ def test_an_infinite_pixel_stays_in_its_windows(shape, C):
         np.testing.assert_array_equal(out[~hit], clean[~hit])
 
 
-@pytest.mark.parametrize("dtype", ["i8", "f16"])
-@pytest.mark.parametrize("nd", [2, 3])
-def test_the_automatic_choice_agrees_with_the_tile_kernel(dtype, nd):
-    """Layers that the library runs on the windowed kernel (its rule is the host's), against a tile instance by name."""
+# data type, form, spatial, N, C, K, filter, dilation, pads, right pads: layers that the library's rule runs on the windowed kernel
+AUTO = [
+    ("i8", "requant", (57, 57), 32, 176, 24, (3, 3), (1, 1), (1, 1), (1, 1)),
+    ("i8", "columns", (41, 41), 64, 304, 24, (3, 3), (1, 1), (1, 1), (1, 1)),
+    ("i8", "plain", (96, 96), 240, 176, 32, (3, 3), (1, 1), (1, 1), (1, 1)),     # 68 MB: stored past the L2
+    ("i8", "requant", (34, 33, 35), 4, 112, 32, (3, 3, 3), (1, 1, 1), (1, 1, 1), (1, 1, 1)),
+    ("f16", "plain", (93, 93), 26, 48, 32, (5, 5), (1, 1), (2, 2), (2, 2)),
+    ("f16", "plain", (61, 50), 24, 208, 32, (3, 5), (1, 2), (2, 1), (0, 5)),
+    ("f16", "bias", (33, 33), 64, 104, 24, (3, 3), (1, 1), (1, 1), (1, 1)),
+    ("f16", "residual", (57, 57), 48, 88, 24, (3, 3), (1, 1), (1, 1), (1, 1)),
+    ("f16", "plain", (34, 33, 35), 4, 112, 32, (3, 3, 3), (1, 1, 1), (1, 1, 1), (1, 1, 1)),
+]
+
+
+@pytest.mark.parametrize("at", range(len(AUTO)))
+def test_the_automatic_choice_agrees_with_the_tile_kernel(at):
+    """The operators with the automatic choice, on layers where it is the windowed kernel, against a tile instance by name."""
+    import ctypes as C
+
+    import torch
+
     import gpu_util
-    shape = (26, 93, 93, 48) if nd == 2 else (4, 34, 33, 35, 112)
-    filt  = (5, 5) if nd == 2 else (3, 3, 3)
-    inp, wei = _ints(shape, 13, dtype), _ints((32, *filt, shape[-1]), 14, dtype)
-    args = (inp, wei, (1,) * nd, (1,) * nd, tuple(f // 2 for f in filt))
-    op   = ck.RequantReluRequant(0.05, 0.7, rounded=True) if dtype == "i8" else None
-    np.testing.assert_array_equal(gpu_util.convnd_fwd(*args, out_op=op), gpu_util.convnd_fwd(*args, out_op=op, instance=7))
+    from composable_kernel_amd import capi
+    dtype, form, spatial, N, channels, K, filt, dil, pads, right = AUTO[at]
+    nd, family = len(spatial), capi.OP_CONV2D_FWD_I8 if dtype == "i8" else capi.OP_CONV2D_FWD_F16
+    out_len = [spatial[i] + pads[i] + right[i] - (filt[i] - 1) * dil[i] for i in range(nd)]
+    geom = (N, K, channels, list(spatial), list(filt), out_len, [1] * nd, list(dil), list(pads), list(right))
+    if nd == 3:
+        chosen = capi.lib()._ZN3ckx18auto_conv3d_windowEiPK15ckx_convnd_desc
+        chosen.restype, chosen.argtypes = C.c_int, [C.c_int, C.POINTER(capi.ConvNdDesc)]
+        assert chosen(family, C.byref(capi.ConvNdDesc.make(*geom))) >= 0
+    else:
+        epi  = {"plain": capi.EPI_PASSTHROUGH, "requant": capi.EPI_REQUANT_RND, "columns": capi.EPI_RELU_MUL2_CLAMP, "bias": capi.EPI_ADD_RELU,
+                "residual": capi.EPI_ADD_RELU_ADD}[form]
+        desc = capi.Conv2dDesc(N, K, channels, *spatial, *filt, *out_len, 1, 1, *dil, *pads, *right)
+        assert capi.conv2d_fwd_plan(family, desc, epi) == (capi.INSTANCE_AUTO, 1)
+    g    = torch.Generator(device="cuda").manual_seed(at)
+    td   = torch.int8 if dtype == "i8" else torch.float16
+    ints = lambda *s: torch.randint(-2, 3, s, generator=g, device="cuda", dtype=torch.int8).to(td)
+    x, w, bias, resi = ints(N, *spatial, channels), ints(K, *filt, channels), ints(K), ints(N, *out_len, K)
+    scales = torch.rand(K, generator=g, device="cuda") * 0.2 + 0.01
+
+    def result(instance):
+        y = torch.full((N, *out_len, K), 77, dtype=td, device="cuda")
+        if form == "columns":
+            op  = ck.DeviceConv2dFwdMultipleDInt8(instance)
+            arg = op.MakeArgumentPointer(x, w, y, scales, *geom, None, None, ck.ActivationMul2Clamp(ck.Relu()))
+        elif form in ("bias", "residual"):
+            op  = ck.DeviceConv2dFwdBiasActivationF16(instance)
+            arg = op.MakeArgumentPointer(x, w, y, bias, resi, *geom, None, None, ck.AddReluAdd()) if form == "residual" else \
+                op.MakeArgumentPointer(x, w, y, bias, *geom, None, None, ck.AddRelu())
+        else:
+            op  = (ck.DeviceConvNdFwdInt8 if dtype == "i8" else ck.DeviceConvNdFwdF16)(nd, instance)
+            arg = op.MakeArgumentPointer(x, w, y, *geom, None, None, ck.RequantReluRequant(0.05, 0.7, rounded=True) if form == "requant" else None)
+        assert op.IsSupportedArgument(arg), capi.last_error()
+        op.MakeInvokerPointer().Run(arg, ck.StreamConfig(gpu_util.stream()))
+        torch.cuda.synchronize()
+        return y
+    got = result(capi.INSTANCE_AUTO)
+    assert torch.equal(got, result(7)) and int((got != 0).sum()) > got.numel() // 8
