@@ -591,12 +591,6 @@ struct FunctorOf
     }
 };
 
-// 16 consecutive fp16 outputs of one row with D operands; d0row / d1row point at column 0 of the
-// row's D values (d1row may be null)
-__device__ __forceinline__ void store_row16_f16_fused(_Float16* crow, int n0, int N, f32x4 (&v)[4],
-                                                      int mode, const _Float16* d0row, const _Float16* d1row,
-                                                      bool nt, float alpha, float beta);
-
 // T = _Float16 or __bf16
 template <typename T>
 __device__ __forceinline__ void store_row16_f16(T* crow, int n0, int N, const f32x4 (&v)[4],
@@ -622,29 +616,6 @@ __device__ __forceinline__ void store_row16_f16(T* crow, int n0, int N, const f3
         store_room<2>(crow + n0, lo, (N - n0) * 2, nt);
         store_room<2>(crow + n0 + 8, hi, (N - n0 - 8) * 2, nt);
     }
-}
-
-__device__ __forceinline__ void store_row16_f16_fused(_Float16* crow, int n0, int N, f32x4 (&v)[4],
-                                                      int mode, const _Float16* d0row, const _Float16* d1row,
-                                                      bool nt, float alpha, float beta)
-{
-    const bool has_d1 = epi_has_d1(mode);
-    const f16x8 z     = {0, 0, 0, 0, 0, 0, 0, 0};
-    const int room    = (N - n0) * 2;
-    const f16x8 b_lo = load_head16<f16x8>(d0row + n0, room);
-    const f16x8 b_hi = load_head16<f16x8>(d0row + n0 + 8, room - 16);
-    const f16x8 r_lo = has_d1 ? load_head16<f16x8>(d1row + n0, room) : z;
-    const f16x8 r_hi = has_d1 ? load_head16<f16x8>(d1row + n0 + 8, room - 16) : z;
-#pragma unroll
-    for(int t = 0; t < 4; ++t)
-#pragma unroll
-        for(int j = 0; j < 4; ++j)
-        {
-            const int e = t * 4 + j;
-            v[t][j]     = epi_f16_value(mode, v[t][j], (float)(e < 8 ? b_lo[e] : b_hi[e - 8]),
-                                        (float)(e < 8 ? r_lo[e] : r_hi[e - 8]), alpha, beta);
-        }
-    store_row16_f16(crow, n0, N, v, nt);
 }
 
 // ------------------------------------------------------------------- kernel
