@@ -589,8 +589,12 @@ inline bool rows_in_16s(int M, int N, int K, int O, int batch, bool mask_upper)
 // gemm_softmax_gemm.hpp. With one workgroup or fewer to a CU the launch lasts as long as a wave's chain of units, which the shares shorten;
 // with more the CUs are busy anyway, and what the shares cost shows: the merge, and with 64 rows every column read twice as often. A launch
 // under the triangular mask may have more of them once its chain is long: they start longest first, and the short ones fit in behind. Below
-// the lines in the chain's length the first loads and the merge cost more than the shares give; heads of 65 to 96 in quarters pad to 128. Up
-// to 64 rows of heads of 33 to 64 the choice between 16 and 32 rows stands up to 1025 columns, bit for bit.
+// the lines in the chain's length the first loads and the merge cost more than the shares give; heads of 65 to 96 in quarters pad to 128. Behind
+// every line: S shares take (1 - 1 / S) of a chain's units away and add a merge that grows with the head, and in quarters the first
+// loads of twice the workgroups; a CU with a second workgroup has the units' waits filled already.
+// Up to 64 rows of heads of 33 to 64 have one share up to 1025 columns, because outputs there are held bit for bit to those of the 16-row
+// kernel, and at 1025 of the 32-row one. From 736 columns on that costs time: batch x 64 x N of heads 64, one share / four, us: 16 x 736 12.1 / 10.7, 16 x
+// 960 15.0 / 11.8, 96 x 1024 15.6 / 12.6, 224 x 960 16.8 / 14.9, 224 x 1024 15.5 / 15.2; below not: 16 x 640 10.3 / 10.5, 224 x 640 12.2 / 12.9.
 // 1 part (16 or 32 rows as rows_in_16s() chooses) / 2 / 4, us, full: batch x M x N 3 x 3034 x 3034 of heads 32 28.5 / 24.0 / 15.5, 6 x
 // 3760 x 1709 / 64 23.7 / 20.7 / 16.5, 14 x 802 x 802 / 64 14.7 / 13.4 / 12.7, 12 x 1275 x 1275 / 80 23.0 / 21.2 / 21.7, 8 x 1676 x 1676 / 128
 // 39.8 / 32.5 / 27.2, 4 x 991 x 3837 / 128 81.2 / 62.1 / 45.6, but 6 x 2806 x 2806 / 64 (264 slabs of 64) 35.4 / 29.4 / 43.1, 8 x 1918 x 490 / 64 9.7 /

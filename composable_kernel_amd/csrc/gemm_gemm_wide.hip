@@ -7,21 +7,7 @@ namespace {
 template <int KS, int OT, int NS>
 hipError_t launch(const GemmGemmArgs& a, hipStream_t s)
 {
-    constexpr int NW  = NS == 4 ? 2 : 4;
-    using Cfg         = SoftmaxGemmCfg<KS, OT, NW>;
-    constexpr int LDS = SoftmaxGemmSplit<KS, OT, NW, NS>::LDS;
-    auto* kern        = &gemm_softmax_gemm_kernel<KS, OT, NW, NS, false>;
-    if constexpr(LDS > 64 * 1024)
-    {
-        static std::once_flag once;
-        static hipError_t attr_err = hipSuccess;
-        std::call_once(once, [&] {
-            attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-        });
-        if(attr_err != hipSuccess)
-            return attr_err;
-    }
-    return gemm_gemm_launch_kernel<Cfg::BM, Cfg::NT * NS, LDS>(kern, a, s);
+    return gemm_softmax_gemm_launch_one<KS, OT, NS, false>(a, s);
 }
 
 template <int NS>

@@ -565,4 +565,25 @@ __global__ __launch_bounds__(NW * NS * 64) __attribute__((amdgpu_waves_per_eu(2,
     }
 }
 
+// NS parts of the columns, on 4 or (NS = 4) 2 waves of rows each
+template <int KS, int OT, int NS, bool SM>
+hipError_t gemm_softmax_gemm_launch_one(const GemmGemmArgs& a, hipStream_t s)
+{
+    constexpr int NW  = NS == 4 ? 2 : 4;
+    using Cfg         = SoftmaxGemmCfg<KS, OT, NW>;
+    constexpr int LDS = SoftmaxGemmSplit<KS, OT, NW, NS>::LDS;
+    auto* kern        = &gemm_softmax_gemm_kernel<KS, OT, NW, NS, SM>;
+    if constexpr(LDS > 64 * 1024)
+    {
+        static std::once_flag once;
+        static hipError_t attr_err = hipSuccess;
+        std::call_once(once, [&] {
+            attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+        });
+        if(attr_err != hipSuccess)
+            return attr_err;
+    }
+    return gemm_gemm_launch_kernel<Cfg::BM, Cfg::NT * NS, LDS>(kern, a, s);
+}
+
 } // namespace ckx
