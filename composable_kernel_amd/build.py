@@ -7,7 +7,9 @@ packed fp32 VALU forms are disabled for the device pass.
 
 Three guards protect the kernels' hand-managed waits (the MFMA fragment reads of gemm_tile.hpp, conv_patch.hpp, conv_window.hpp and
 conv_pointwise.hpp are inline-assembly LDS reads that the compiler does not count in lgkmcnt; the kernels wait for
-them themselves, so no compiler-made copy or spill of such a register may run before that wait):
+them themselves, so no compiler-made copy or spill of such a register may run before that wait). They see spills, scratch
+memory and AccVGPR counts; a copy between two vector registers, which a branch around the products can bring about, they do
+not see: the bit-exact integer-operand GPU tests are what finds it, so they are run for every change to such a kernel:
   * every kernel's register report (-Rpass-analysis=kernel-resource-usage) is read, and the build FAILS if one of
     those kernels spills vector registers;
   * the four-wave GEMM body (gemm_w4.hpp) also issues its MFMAs and direct loads as inline assembly: its kernels must

@@ -566,16 +566,33 @@ hipError_t gemm_softmax_gemm_launch(const GemmGemmArgs& a, int parts, hipStream_
 // 15.6 / 12.5; of 80: 32 x 256 x 256 8.6 / 7.9. The lines in N lie on the careful side: with one slab to a batch (M = 128) 32 rows are level with 16 at N 768 and
 // 1.02 to 1.08 ahead from 832 on (heads of 64, 200 batches: 960 17.4 / 16.1, 968 17.7 / 16.8, 1024 17.6 / 16.7, 1032 18.7 / 17.6), and for heads of
 // 32 1.02 to 1.14 ahead from 320 on (128 batches: 384 6.8 / 6.5, 440 8.2 / 7.5, 448 8.3 / 7.2, 480 8.1 / 7.7).
-// Past 256 slabs the mask's line holds only while there are enough slabs to a batch for the longest ones to come early (measured at M = N; with
-// columns past the last row, masked for all, the line stays): heads of 128, 297 x 104
-// x 104 15.3 / 11.9, 114 x 280 x 280 19.3 / 13.4, 83 x 606 x 606 28.5 / 23.0, 66 x 812 x 812 34.7 / 27.8, but 40 x 946 x 946 24.5 / 26.4 and 48 x 952 x 952 level;
+// Past 256 slabs of heads past 96 the masked 16-row kernel, of which a CU holds one workgroup, stays ahead from 896 columns up to 384 slabs (40 x 946 x 946
+// 24.5 / 26.4, level at 48 x 952 x 952), and up to 512 where the launch lasts no longer than its longest chain (second_slabs_fit()) and either the
+// chains are long or every XCD has whole batches, whose columns stay in its L2. us, 16 rows / 32 rows, heads of 128: 24 x 2304 x 2304 54.5 / 60.8, 16 x 3102 x
+// 3102 68.5 / 75.0, 28 x 1909 x 1909 46.8 / 51.2, 32 x 1588 x 1588 38.0 / 40.9, 48 x 869 x 869 24.0 / 26.5, 64 x 611 x 611 18.5 / 20.4; where they do not
+// fit: 48 x 1030 x 1030 32.2 / 29.7, 51 x 1244 x 1244 45.2 / 40.1, 54 x 815 x 815 28.8 / 25.4, 112 x 397 x 397 22.9 / 16.5, 297 x 104 x 104 15.3 / 11.9; with a
+// few batches more on some XCDs: 51 x 813 x 813 29.0 / 25.9, 46 x 858 x 858 26.3 / 26.0, 37 x 1365 x 1365 39.8 / 38.5. (With columns past the last row, masked for all,
+// its line is 512 slabs.) Of 195 random problems with M = N > 576 the choice is at most 4 % behind the other kernel but for four (up to 8 %), and up to 1.29 ahead;
 // heads of 64, 134 x 158 x 158 9.8 / 8.2, 442 x 128 x 128 11.1 / 9.4, 112 x 353 x 353 11.2 / 10.4, but with K 32 and O 64 104 x 352 x 352 8.3 / 8.9.
+//
+// Masked slabs, M >= N, one workgroup to a CU, up to two rounds, longest chains first: the k-th slab past the CUs starts where the k-th slab ends
+// from the back. Whether they all end before the longest one, with 80 columns' time for a slab's first loads.
+inline bool second_slabs_fit(int M, int N, int batch)
+{
+    const long per_batch = (M + 127) / 128, cus = num_cus(), slabs = batch * per_batch;
+    const auto chain = [&](long rank) { const long c = 128 * (per_batch - rank / batch); return c < N ? c : (long)N; };
+    for(long k = 0; cus + k < slabs; ++k)
+        if(k >= cus || chain(cus + k) + chain(cus - 1 - k) + 80 > N)
+            return false;
+    return true;
+}
 inline bool rows_in_16s(int M, int N, int K, int O, int batch, bool mask_upper)
 {
     const int head   = K > O ? K : O;
     const long slabs = (long)batch * ((M + 127) / 128) * 256 / num_cus(); // (as on 256 CUs, which the lines here were measured on)
     if(head > 96)
-        return slabs <= (!mask_upper ? 256 : M < N ? 512 : N >= 896 ? 384 : 256);
+        return slabs <= (!mask_upper ? 256 : M < N ? 512 : N >= 896 ? 384 : 256) ||
+               (mask_upper && M >= N && N > 576 && (N >= 1600 || batch % 8 == 0) && second_slabs_fit(M, N, batch));
     if(slabs > 256 && M >= N && N <= 352 && K > 32)
         return false;
     // (130 x 375 x 375 13.2 / 13.8 us; longer N, where the second workgroup of some CUs comes late enough: 43 x 768 x 768 13.9 / 14.9, 64 x 768 x

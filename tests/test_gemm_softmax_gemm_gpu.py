@@ -312,3 +312,15 @@ def test_gemm_softmax_gemm_column_shares(G, M, N, K, O):
             one = _run(a, b0, b1, K ** -0.5, mask, 0)
             assert np.max(np.abs(out.astype(np.float64) - one)) <= 2.0 ** -9
             _close(out[-1:], lit.batched_gemm_softmax_gemm_f16(a[-1:], b0[-1:].transpose(0, 2, 1), b1[-1:], K ** -0.5, mask))
+
+
+@pytest.mark.parametrize("G, M, N, rows", [(48, 865, 865, 16), (52, 772, 772, 32), (44, 794, 794, 32), (24, 2083, 2083, 16), (24, 2499, 2499, 32), (28, 1909, 1909, 16),
+                                           (31, 1970, 1970, 32), (45, 1066, 1066, 32), (32, 1588, 1588, 16), (40, 946, 946, 16), (64, 577, 577, 16), (64, 576, 576, 32),
+                                           (8, 6472, 809, 32), (33, 1160, 893, 32), (16, 3101, 3101, 16)])
+def test_causal_wide_heads_past_one_workgroup_a_cu(G, M, N, rows):
+    """256 to 512 slabs: 16-row waves where the slabs that start second end before the longest chain, and the chains are long or the XCDs have whole
+    batches, 32-row waves otherwise (csrc/gemm_gemm.hpp, rows_in_16s). Bit for bit the one kernel, and not the other."""
+    a, b0, b1 = (uniform_f16((G, x, 128), -1, 1, 61 + i) for i, x in enumerate((M, N, N)))
+    out = _run(a, b0, b1, 128 ** -0.5, True).view(np.uint16)
+    by_rows = {16: _run(a, b0, b1, 128 ** -0.5, True, 2).view(np.uint16), 32: _run(a, b0, b1, 128 ** -0.5, True, 0).view(np.uint16)}
+    assert np.array_equal(out, by_rows[rows]) and np.any(out != by_rows[48 - rows])
