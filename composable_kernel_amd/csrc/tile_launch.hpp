@@ -61,8 +61,10 @@ hipError_t launch_tile(const GemmArgs& a, int tiles, hipStream_t s)
     return hipGetLastError();
 }
 
-// Short tiles in the last round of an int8 launch of 256 x 256 tiles (tile_pairs.hip): true, and `g`'s tiles set, where they pay
+// Short tiles in the last round of an int8 launch of 256 x 256 tiles (tile_pairs.hip): true, and `g`'s tiles set, where they pay. Their rows, 0
+// where whole tiles stay; below: rows behind the whole tiles, else columns beside them
 bool short_tail(GemmArgs& g);
+int short_tail_rows(int M, int N, int K, bool& below);
 tile_launch_fn short_tail_tile();
 
 // K-major operand layouts (gemm_layouts.hip): launcher of tile instance `tile` for element type dt

@@ -1,5 +1,5 @@
 """GPU parity of the short tiles in the last round of int8 GEMMs on 256 x 256 tiles (csrc/tile_pairs.hip, short_tail): less than a round of tiles,
-tails below and beside whole tiles, every tail height, M and N that end inside a tile and a vector, all plain epilogues. Bit for bit."""
+tails below and beside whole tiles, every tail height, shapes around the rule, M and N that end inside a tile and a vector, all plain epilogues. Bit for bit."""
 import numpy as np
 import pytest
 
@@ -9,28 +9,27 @@ from oracle import fast, lit
 
 pytestmark = pytest.mark.gpu
 
-# M, N, K; what the rule makes of them on 256 CUs is worked out in _tail() below
 SHAPES = [(1300, 7600, 160), (1296, 7632, 992), (5000, 5103, 144), (4096, 11008, 128), (2687, 3214, 304), (3447, 10021, 400), (257, 65800, 272),
-          (8200, 2060, 1040), (6144, 4096, 256), (300, 33000, 144), (3500, 4000, 208)]
+          (8200, 2060, 1040), (6144, 4096, 256), (300, 33000, 144), (3500, 4000, 208), (2675, 9622, 272), (3810, 6671, 320)]
 
 
-def _tail(M, N, grid=256):
-    """The rule restated: (whole row tiles, whole column tiles, rows of a short tile, tails beside rather than below)."""
-    tm, tn = -(-M // 256), -(-N // 256)
-    rounds = tm * tn // grid
-    columns, rows = rounds * grid // tm, rounds * grid // tn
-    for h in (64, 80, 96, 112):
-        if rows * tn + -(-(M - rows * 256) // (2 * h)) * tn <= (rounds + 1) * grid:
-            return rows, tn, 2 * h, False
-        if columns * tm + -(-M // (2 * h)) * (tn - columns) <= (rounds + 1) * grid:
-            return tm, columns, 2 * h, True
-    return None
+def _tail(M, N, K):
+    """The library's rule: rows of a short tile (0: whole tiles), below the whole tiles rather than beside them."""
+    import ctypes as C
+
+    from composable_kernel_amd import capi
+    rule = capi.lib()._ZN3ckx15short_tail_rowsEiiiRb
+    rule.restype, rule.argtypes = C.c_int, [C.c_int] * 3 + [C.POINTER(C.c_bool)]
+    below = C.c_bool()
+    return rule(M, N, K, C.byref(below)), below.value
 
 
 def test_the_shapes_are_what_they_are_meant_to_be():
-    kinds = [_tail(M, N) for M, N, _ in SHAPES]
-    assert {k[2] for k in kinds if k} == {128, 160, 192, 224}
-    assert any(k and k[3] for k in kinds) and any(k and not k[3] and k[0] for k in kinds) and any(k and k[0] == 0 for k in kinds)
+    """Every height, below whole tiles and beside them, and less than a round of tiles; whole tiles where a tail does not pay."""
+    tails = {s: _tail(*s) for s in SHAPES}
+    assert {h for h, _ in tails.values()} == {0, 128, 160, 192}
+    assert any(h and not below for h, below in tails.values()) and any(h and below and -(-M // 256) * -(-N // 256) > 256 for (M, N, _), (h, below) in tails.items())
+    assert any(h and -(-M // 256) * -(-N // 256) < 256 for (M, N, _), (h, _) in tails.items())
 
 
 @pytest.mark.parametrize("shape", SHAPES)
