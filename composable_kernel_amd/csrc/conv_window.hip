@@ -128,10 +128,13 @@ double plan_conv_window(int dt, int shape, ConvWindowArgs& a)
 
 int choose_conv_window(int dt, ConvWindowArgs& a, double tile_us)
 {
-    // Above this the windowed kernel won on 25 of 27 random layers (1.02 to 2.46, 1.27 on average; 0.99 on the other two), from 1.0 to 1.15 on
-    // half of them (0.83 to 1.18), below on none but two (1.07, 1.10). The 14 us spare small calls the search for a box.
-    // (Below twelve K tiles a tile's ends outweigh them: 15 x 27^3, C 16 -> K 16, seven of them, 25.3 -> 27.0 us though rated faster.)
-    constexpr double margin = 1.15;
+    // Above this the windowed kernel won on 67 of 70 random layers (1.02 to 2.80, 1.34 on average), from 1.0 to 1.15 on half of 27 (0.83 to
+    // 1.18), below on none but two (1.07, 1.10). The 14 us spare small calls the search for a box.
+    // (Below twelve K tiles a tile's ends outweigh them: 15 x 27^3, C 16 -> K 16, seven of them, 25.3 -> 27.0 us though rated faster. From there to
+    // fifteen that is so where a pixel is a single chunk, and the next tile's whole window has to come in behind them: C 32, 14 of them, 25 x 18^3 -> K 16
+    // 24.6 -> 26.0 us rated 1.31, 4 x 33^3 -> K 32 26.2 -> 27.4 rated 1.28, 3 x 45^3 -> K 16 level rated 1.29; int8 23 x 35^3, C 64 -> K 16 130.5 -> 109.3 rated 1.39.
+    // The third layer that lost: int8 8 x 102^2, C 512 -> K 72, 62.8 -> 68.3, three column tiles that load the window each.)
+    constexpr double margin = 1.15, margin_short = 1.35;
     if(tile_us < 14.0 || a.taps * a.units < 12 * 8)
         return -1;
     ConvWindowArgs best = a;
@@ -140,8 +143,9 @@ int choose_conv_window(int dt, ConvWindowArgs& a, double tile_us)
     {
         ConvWindowArgs w = a;
         const double us  = plan_conv_window(dt, i, w);
-        if(us >= 0.0 && us * margin < tile_us)
-            best = w, shape = i, tile_us = us * margin;
+        const double m  = w.chunks == 1 && w.nk < 16 ? margin_short : margin;
+        if(us >= 0.0 && us * m < tile_us)
+            best = w, shape = i, tile_us = us * m;
     }
     a = best;
     return shape;

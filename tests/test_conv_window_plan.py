@@ -55,6 +55,9 @@ def test_the_line():
     assert at(1e9, (32, 32), 16, 64, 64, (1, 7), (1, 1), (0, 3)) == -1       # too few taps
     assert at(1e9, (32, 32), 16, 128, 64, (2, 4), (1, 1), (0, 1)) == -1 and at(1e9, (32, 32), 16, 128, 64, (1, 9), (1, 1), (0, 4)) >= 0
     assert at(1e9, (16, 16, 16), 4, 128, 64, (2, 2, 2), (1, 1, 1), (1, 1, 1)) == -1
+    # one chunk of fourteen K tiles: the next window has little time to come in
+    assert at(35.5, (18, 18, 18), 25, 32, 16, (3, 3, 3), (1, 1, 1), (1, 1, 1)) == -1 and at(39.0, (18, 18, 18), 25, 32, 16, (3, 3, 3), (1, 1, 1), (1, 1, 1)) == 2
+    assert choose("i8", layer("i8", (35, 35, 35), 23, 64, 16, (3, 3, 3), (1, 1, 1), (1, 1, 1))[0], 162.3) == 2
     assert at(13.9, (8, 8), 1, 32, 32, (3, 3), (1, 1), (1, 1)) == -1          # small calls are not searched
 
 
