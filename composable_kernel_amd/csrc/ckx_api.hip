@@ -480,15 +480,17 @@ PackPlan pack_plan(int es, int M, int N, int K)
 }
 // The padding instance is bound by the operand rows through the busiest CU, whose K tiles take 0.32 to 0.45 us per 128 rows where whole lines
 // take about half; the copies cost a launch (3.4 us), their bytes, and what a product as small as its launch has to fill the CUs with. 16-bit
-// operands: where CUs have one 64 x 64 tile each, both kernels wait for their K tiles' latency, and little pays for the copies; two or
-// three tiles with a short K are level. Padding instance / copies and the instance for whole vectors, us: fp16 4001 x 4003 x 4095 211 / 135, 2049 x 2047 x
-// 2047 55.2 / 40.3, 3001 x 333 x 3001 33.8 / 25.9, 1500 x 901 x 2001 24.5 / 20.1, int8 4001 x 4003 x 4095 115 / 64.6, 1856 x 729 x 2111 16.9 / 13.7.
-// On the other side of the lines, by work: fp16 700 x 701 x 3001 (2.9e9 operations) 18.4 / 19.7; by operations per operand byte: 251 x 3973 x 3783 (236)
-// 26.0 / 29.2, 4004 x 285 x 1969 (266) level; by tiles and CUs: 316 x 3263 x 2979 (255 tiles) 22.2 / 23.6, 794 x 1205 x 2409 (247) 18.5 / 18.3, but 797 x 903 x
-// 4069 (195) 27.9 / 25.0, 1000 x 1000 x 8001 (256, 126 K tiles) 49.3 / 44.0 and int8 900 x 1000 x 6001 (240) 23.9 / 20.9; by K tiles: 2001 x 1003 x 1025 (two a CU, 17) 15.6 / 15.2, 3878 x 661 x 1053 (three, 17) 20.9 / 21.0, but 485 x 3861 x 1339
-// (two, 21) 18.4 / 17.8, 838 x 3089 x 1289 (three, 21) 24.8 / 23.1, 2428 x 1503 x 577 (four, 10) 17.7 / 16.6 and int8 2107 x 991 x 1497 (three, 12) 17.3 / 15.5; by
-// rows: int8 2474 x 765 x 1509 (24) 13.5 / 14.1. K-major operands, transposed on the way: int8 1704 x 2145 x 2155 29.3 / 21.2 (15.8e9), fp16 655 x 2425 x 3557
-// 39.0 / 33.7 (11.3e9), but int8 3031 x 901 x 1055 (5.8) 20.6 / 21.2, 2924 x 981 x 1755 (10.1) 28.6 / 29.2.
+// operands: where CUs have one 64 x 64 tile each, both kernels wait for their K tiles' latency, and little pays for the copies; three tiles
+// with a short K are level. Padding instance / copies and the instance for whole vectors, us: fp16 4001 x 4003 x 4095 200 / 129, 2049 x 2047 x
+// 2047 55.0 / 39.6, 3001 x 333 x 3001 33.8 / 25.8, 1500 x 901 x 2001 24.5 / 19.8, int8 4001 x 4003 x 4095 112 / 61.8, 1856 x 729 x 2111 16.9 /
+// 13.5. On the other side of the lines, by work: fp16 700 x 701 x 3001 (2.9e9 operations) 18.4 / 19.7; by operations per operand byte: 251 x
+// 3973 x 3783 (236) 26.0 / 29.2, 4004 x 285 x 1969 (266) level; by tiles and CUs: 316 x 3263 x 2979 (255 tiles) 22.2 / 23.6, 794 x 1205 x 2409
+// (247) 18.5 / 18.3, but 797 x 903 x 4069 (195) 27.9 / 25.0, 1000 x 1000 x 8001 (256, 126 K tiles) 49.3 / 44.0 and int8 900 x 1000 x 6001
+// (240) 23.9 / 20.9; by K tiles: 3878 x 661 x 1053 (three a CU, 17) 20.9 / 21.0, 2030 x 1381 x 791 (three, 13) 17.2 / 17.3, but 2001 x 1003 x
+// 1025 (two, 17) 15.34 / 14.49 ... 15.04 on three cards, 838 x 3089 x 1289 (three, 21) 24.8 / 23.1, 2428 x 1503 x 577 (four, 10) 17.7 / 16.6
+// and int8 2107 x 991 x 1497 (three, 12) 17.3 / 15.5; by rows: int8 2474 x 765 x 1509 (24) 13.5 / 14.1. K-major operands, transposed on the
+// way: int8 1704 x 2145 x 2155 29.3 / 21.2 (15.8e9), fp16 655 x 2425 x 3557 39.0 / 33.7 (11.3e9), but int8 3031 x 901 x 1055 (5.8) 20.6 /
+// 21.2, 2924 x 981 x 1755 (10.1) 28.6 / 29.2.
 bool packing_pays(int es, int M, int N, int K, bool kmajor)
 {
     const int vec     = 16 / es;
@@ -499,7 +501,7 @@ bool packing_pays(int es, int M, int N, int K, bool kmajor)
     const long n = m == 128 ? 128 : ckx::ragged_small_tile(M, N, 1).n;
     const long tiles = (M + m - 1) / m * ((N + n - 1) / n), per_cu = (tiles + num_cus() - 1) / num_cus(), k_tiles = ((long)K * es + 127) / 128;
     if(!kmajor && es == 2 && m + n == 128 &&
-       (per_cu == 1 ? 5 * tiles > 4l * num_cus() && k_tiles < 64 : per_cu < 4 && k_tiles < 20 && 2 * tiles > 3l * num_cus()))
+       (per_cu == 1 ? 5 * tiles > 4l * num_cus() && k_tiles < 64 : per_cu == 3 && k_tiles < 20))
         return false;
     const PackPlan p = pack_plan(es, M, N, K);
     return per_cu * (m + n) * k_tiles >= 32 * 128 && p.a_bytes < (1l << 31) && p.bytes - p.a_bytes < (1l << 31);
