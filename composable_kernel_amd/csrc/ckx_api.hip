@@ -487,7 +487,7 @@ PackPlan pack_plan(int es, int M, int N, int K)
 // 3973 x 3783 (236) 26.0 / 29.2, 4004 x 285 x 1969 (266) level; by tiles and CUs: 316 x 3263 x 2979 (255 tiles) 22.2 / 23.6, 794 x 1205 x 2409
 // (247) 18.5 / 18.3, but 797 x 903 x 4069 (195) 27.9 / 25.0, 1000 x 1000 x 8001 (256, 126 K tiles) 49.3 / 44.0 and int8 900 x 1000 x 6001
 // (240) 23.9 / 20.9; by K tiles: 3878 x 661 x 1053 (three a CU, 17) 20.9 / 21.0, 2030 x 1381 x 791 (three, 13) 17.2 / 17.3, but 2001 x 1003 x
-// 1025 (two, 17) 15.34 / 14.49 ... 15.04 on three cards, 838 x 3089 x 1289 (three, 21) 24.8 / 23.1, 2428 x 1503 x 577 (four, 10) 17.7 / 16.6
+// 1025 (two, 17) 15.35 / 14.50, 838 x 3089 x 1289 (three, 21) 24.8 / 23.1, 2428 x 1503 x 577 (four, 10) 17.7 / 16.6
 // and int8 2107 x 991 x 1497 (three, 12) 17.3 / 15.5; by rows: int8 2474 x 765 x 1509 (24) 13.5 / 14.1. K-major operands, transposed on the
 // way: int8 1704 x 2145 x 2155 29.3 / 21.2 (15.8e9), fp16 655 x 2425 x 3557 39.0 / 33.7 (11.3e9), but int8 3031 x 901 x 1055 (5.8) 20.6 /
 // 21.2, 2924 x 981 x 1755 (10.1) 28.6 / 29.2.

@@ -15,7 +15,7 @@
 //   * GEMM-K runs over (chunk, tap, unit), 8 units per K tile, without padding: a table in LDS has for each unit its offset in the window and
 //     in a weight row. The weights come through a ring of three stages of 128 bytes per channel, as in the tile kernel.
 //
-// us, tile kernel and this one in turn on one card: 16 x 32^3, C 64 -> K 64 150 -> 121; 18 x 42^3, 160 -> 16 849 -> 529; 7 x 34^3, 112 -> 32 148 -> 105; int8
+// us, tile kernel and this one in turn on one card: 16 x 32^3, C 64 -> K 64 149 -> 117; 18 x 42^3, 160 -> 16 849 -> 529; 7 x 34^3, 112 -> 32 148 -> 105; int8
 // 12 x 96^2, 992 -> 24, 3 x 3 148 -> 62; 115 x 32^2, 592 -> 280 with bias, ReLU and residual 603 -> 453; 23 x 110^2, 272 -> 160 399 -> 329.
 // What bounds it: of the first one's time a tile's ends take a sixth (every CU stores at once) and loading the windows, which are read in pieces
 // of 64 of a line's 128 bytes, a fifth; the K loop keeps the matrix cores 60 % busy, the rest being the barrier and the wait for the

@@ -576,13 +576,16 @@ hipError_t gemm_softmax_gemm_launch(const GemmGemmArgs& a, int parts, hipStream_
 // heads of 64, 134 x 158 x 158 9.8 / 8.2, 442 x 128 x 128 11.1 / 9.4, 112 x 353 x 353 11.2 / 10.4, but with K 32 and O 64 104 x 352 x 352 8.3 / 8.9.
 //
 // Masked slabs, M >= N, one workgroup to a CU, up to two rounds, longest chains first: the k-th slab past the CUs starts where the k-th slab ends
-// from the back. Whether they all end before the longest one, with 80 columns' time for a slab's first loads.
+// from the back. Whether they all end before the longest one, with 80 columns' time for a slab's first loads: looked at where the first slab's
+// chain becomes a longer one, as the second's only become shorter.
 inline bool second_slabs_fit(int M, int N, int batch)
 {
     const long per_batch = (M + 127) / 128, cus = num_cus(), slabs = batch * per_batch;
+    if(slabs > 2 * cus)
+        return false;
     const auto chain = [&](long rank) { const long c = 128 * (per_batch - rank / batch); return c < N ? c : (long)N; };
-    for(long k = 0; cus + k < slabs; ++k)
-        if(k >= cus || chain(cus + k) + chain(cus - 1 - k) + 80 > N)
+    for(long k = 0; cus + k < slabs; k = cus - (cus - 1 - k) / batch * batch)
+        if(chain(cus + k) + chain(cus - 1 - k) + 80 > N)
             return false;
     return true;
 }

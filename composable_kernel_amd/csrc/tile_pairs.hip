@@ -19,7 +19,7 @@ int short_tail_rows(int M, int N, int K, bool& below)
     // (0.97 to 1.09), 3 1.04 from nine K tiles on (0.98 to 1.04 below); 160 rows 0 1.08 to 1.17, 1 1.03 (0.98 to 1.07), 2 1.02 (0.97 to 1.06), 3
     // 1.01 (0.97 below eight K tiles); 192 rows 0 1.05, from 24 K tiles on 1 and 2 1.005 (0.99 to 1.03), 3 1.06, below 0.96 to 1.03; 224 rows 0.92
     // to 1.02. us: int8 2687 x 3214 x 2384 35.7 -> 30.6, 4910 x 1681 x 3072 34.8 -> 30.9, 3447 x 10022 x 3600 146.4 -> 136.0, 4096 x 11008 x 4096
-    // (192 rows behind two rounds) 157.3 -> 153.5, but 4852 x 5968 x 544 28.0 / 30.4, 7430 x 3687 x 2176 58.9 / 61.5. fp16 and bf16 stay on the
+    // (192 rows behind two rounds) 152.9 -> 148.1, but 4852 x 5968 x 544 28.0 / 30.4, 7430 x 3687 x 2176 58.9 / 61.5. fp16 and bf16 stay on the
     // four-wave body, which is ahead by more than that (28 problems: 0.82 to 1.10, 0.95 on average), and strided fp16 convolutions on whole tiles:
     // what a short tile saves them is products, and they wait for loads (648 tiles, 2.5 rounds: 153.8 and 153.1).
     const long grid = num_cus() - num_cus() % 8, tm = (M + 255l) / 256, tn = (N + 255l) / 256, rounds = tm * tn / grid;

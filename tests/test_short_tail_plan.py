@@ -16,7 +16,7 @@ def test_short_tiles_only_where_they_win():
     assert _rows(1610, 7437, 1568) == 0     # 224 rows, less than a round: 27.2 / 27.8
     assert _rows(7430, 3687, 2176) == 0     # 192 rows behind one round: 58.9 / 61.5
     assert _rows(4100, 10272, 368) == 0     # 192 rows behind two, few K tiles: 31.5 / 32.5
-    assert _rows(4096, 11008, 4096) == 192  # 192 rows behind two, 32 K tiles: 157.3 / 153.5
+    assert _rows(4096, 11008, 4096) == 192  # 192 rows behind two, 32 K tiles: 152.9 / 148.1
     assert _rows(8156, 6764, 640) == 0      # 128 rows behind three, few K tiles: 50.2 / 51.4
     assert _rows(8076, 7252, 688) == 0      # 160 rows behind three, few K tiles: 58.9 / 60.7
     assert _rows(2687, 3214, 2384) == 160   # less than a round: 35.7 / 30.6
