@@ -130,8 +130,8 @@ const char* ckx_instance_name(int op, int instance);
  * addresses, all four layouts, every epilogue of the data type: the reference's KPadding / MNKPadding
  * instances, device_gemm_xdl_cshuffle.hpp:99-184) and CKX_INSTANCE_AUTO sends there the problems the vectorised
  * instances refuse, so AUTO supports every shape -- but for large products whose K is no whole vector and that come
- * with a workspace: their operands are copied there to rows that are, for the vectorised instances. This holds for every ckx_gemm_* and
- * ckx_batched_gemm_* entry point below. */
+ * with a workspace: their operands are copied there to rows that are, for the vectorised instances. This holds
+ * for every ckx_gemm_* and ckx_batched_gemm_* entry point below (batches are not copied). */
 int ckx_gemm_i8_is_supported(int32_t M, int32_t N, int32_t K, int32_t stride_a, int32_t stride_b,
                              int32_t stride_c, int a_layout, int b_layout, int c_layout, int epilogue,
                              int instance);
@@ -141,11 +141,12 @@ int ckx_gemm_i8(const void* p_a, const void* p_b, void* p_c, int32_t M, int32_t 
                 void* p_workspace, int64_t workspace_bytes, void* stream);
 /* BaseOperator::GetWorkSpaceSize (device_base.hpp:47): bytes of device scratch with which the
  * launch may cut K into several runs (split-K: problems with too few C tiles to occupy the
- * machine), or copy operands whose K is no whole vector (large products on CKX_INSTANCE_AUTO). The workspace is OPTIONAL: with p_workspace == NULL, or fewer bytes than asked for,
- * the launch uses a plan that needs none. It needs no initialisation and holds nothing between
- * calls; two launches that share one workspace must not overlap. The queries of one data type answer for A row-major,
- * B column-major, which is enough for every layout; ckx_gemm_workspace_bytes (op = CKX_OP_GEMM_I8 / _F16 /
- * _BF16) answers for the layouts: fewer products with a K-major operand are copied. */
+ * machine), or copy operands whose K is no whole vector (large products on CKX_INSTANCE_AUTO). The
+ * workspace is OPTIONAL: with p_workspace == NULL, or fewer bytes than asked for, the launch uses a plan
+ * that needs none. It needs no initialisation and holds nothing between calls; two launches that share one
+ * workspace must not overlap. The queries of one data type answer for A row-major, B column-major, which is
+ * enough for every layout; ckx_gemm_workspace_bytes (op = CKX_OP_GEMM_I8 / _F16 / _BF16) answers for the
+ * layouts: fewer products with a K-major operand are copied. */
 int64_t ckx_gemm_i8_workspace_bytes(int32_t M, int32_t N, int32_t K, int instance);
 int64_t ckx_gemm_workspace_bytes(int op, int32_t M, int32_t N, int32_t K, int a_layout, int b_layout, int instance);
 
@@ -397,8 +398,8 @@ int ckx_batched_gemm_softmax_gemm_f16(const void* p_a, const void* p_b0, const v
  * ckx_conv2d_fwd_* would use for this problem with `workspace_bytes` of 16-byte aligned workspace (0: none).
  * *instance is in / out: CKX_INSTANCE_AUTO asks for the automatic choice, an instance index for that instance's K
  * split. CKX_INSTANCE_AUTO comes back where that launch has no index: a GEMM whose operands are copied to the workspace
- * first (*k_runs: the runs on the copies), a convolution whose input goes through LDS window by window. Operand addresses are taken to be 16-byte aligned (a launch sends misaligned ones to the padding
- * instance). The automatic choice is a cost model; tests/golden/planner_audit.json holds what it was measured against. */
+ * first (*k_runs: the runs on the copies), a convolution whose input goes through LDS window by window. Operand
+ * addresses are taken to be 16-byte aligned (a launch sends misaligned ones to the padding instance). The automatic choice is a cost model; tests/golden/planner_audit.json holds what it was measured against. */
 int ckx_gemm_plan(int op, int32_t M, int32_t N, int32_t K, int32_t stride_a, int32_t stride_b, int32_t stride_c,
                   int a_layout, int b_layout, int c_layout, int epilogue, int32_t batch, int64_t workspace_bytes,
                   int* instance, int* k_runs);
