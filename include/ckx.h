@@ -399,7 +399,8 @@ int ckx_batched_gemm_softmax_gemm_f16(const void* p_a, const void* p_b0, const v
  * *instance is in / out: CKX_INSTANCE_AUTO asks for the automatic choice, an instance index for that instance's K
  * split. CKX_INSTANCE_AUTO comes back where that launch has no index: a GEMM whose operands are copied to the workspace
  * first (*k_runs: the runs on the copies), a convolution whose input goes through LDS window by window. Operand
- * addresses are taken to be 16-byte aligned (a launch sends misaligned ones to the padding instance). The automatic choice is a cost model; tests/golden/planner_audit.json holds what it was measured against. */
+ * addresses are taken to be 16-byte aligned (a launch sends misaligned ones to the padding instance). The automatic
+ * choice is a cost model; tests/golden/planner_audit.json holds what it was measured against. */
 int ckx_gemm_plan(int op, int32_t M, int32_t N, int32_t K, int32_t stride_a, int32_t stride_b, int32_t stride_c,
                   int a_layout, int b_layout, int c_layout, int epilogue, int32_t batch, int64_t workspace_bytes,
                   int* instance, int* k_runs);
